@@ -53,6 +53,31 @@ def build_rate_probe(verbose: bool = True) -> str:
     return RATE_PROBE
 
 
+NATIVE_SRC = os.path.join(CSRC, "intfa_torch.cpp")
+NATIVE = os.path.join(HERE, "_native.so")
+
+
+def build_native(verbose: bool = True) -> str:
+    """Compiles the extension module behind the Python entry points (host code only: g++ against libtorch) beside libintfa.so."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    lib = os.path.join(root, "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-isystem", "/opt/rocm/include", "-I", sysconfig.get_paths()["include"], NATIVE_SRC, "-o", NATIVE,
+           "-L", HERE, "-lintfa", "-L", lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + lib]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for {NATIVE_SRC}:\n{r.stderr[-4000:]}")
+    if verbose:
+        print(f"built {NATIVE}")
+    return NATIVE
+
+
 def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
     """Compiles every source and links the library.  `only` (development): a list of name fragments - sources whose file
     name contains none of them keep their existing object file."""
@@ -96,6 +121,7 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
     if verbose:
         print(f"built {OUT} from {len(srcs)} source file(s), {len(todo)} compiled")
+    build_native(verbose)
     if os.path.exists(C_CALLER_SRC):
         build_c_caller(verbose)
     if os.path.exists(RATE_PROBE_SRC) and not only:

@@ -1,8 +1,9 @@
 """Drop-in for the reference module of the same name: ``attention_full_int8`` (flash_atten_full_int8.py:186-223)."""
 import torch
 
-from . import _capi
-from ._host import launch_forward
+from . import _capi, _host
+
+_PROUND = {"rne": _capi.PROUND_RNE, "reference": _capi.PROUND_REFERENCE}
 
 
 def attention_full_int8(q, k, v, q_scale, k_scale, v_scale, causal, sm_scale, *, out_dtype=torch.float16,
@@ -29,7 +30,6 @@ def attention_full_int8(q, k, v, q_scale, k_scale, v_scale, causal, sm_scale, *,
     ``p_round``: "reference" (the default) reproduces the fp16 sequence of flash_atten_full_int8.py:49-51 when P is
     requantised; "rne" is an opt-in that folds 127 into the exponent and rounds to nearest-even in fp32.
     """
-    pr = {"rne": _capi.PROUND_RNE, "reference": _capi.PROUND_REFERENCE}[p_round]
-    return launch_forward("full", q, k, v, q_scale, k_scale, v_scale, causal, sm_scale, out_dtype,
-                          num_splits=num_splits, p_round=pr, return_lse=return_lse, v_scale_block=v_scale_block,
-                          seqlens_k=seqlens_k)
+    native = _host._native or _host.native()
+    return native.forward(_capi.VARIANT_FULL_INT8, q, k, v, q_scale, k_scale, v_scale, causal, sm_scale, out_dtype,
+                          num_splits, _PROUND[p_round], return_lse, v_scale_block, seqlens_k)

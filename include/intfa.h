@@ -179,6 +179,12 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
 /* Bytes of workspace the forward needs for p->num_splits (0 when num_splits <= 1). */
 size_t intfa_fwd_workspace_bytes(const intfa_fwd_params* p);
 
+/* Bytes of workspace with which the split-KV forward merges the partials itself instead of launching a merge kernel
+ * behind it: intfa_fwd_workspace_bytes() plus 8 bytes per 32 query rows of every head (0 when num_splits <= 1).  Nothing has to be
+ * cleared; with less, down to intfa_fwd_workspace_bytes(), the merge is a second launch.  Two launches that may run at the
+ * same time must not share a workspace, with or without the merge. */
+size_t intfa_fwd_merge_workspace_bytes(const intfa_fwd_params* p);
+
 /* attention_full_int8(q, k, v, q_scale, k_scale, v_scale, causal, sm_scale) -> o
  * replaces _attention_full_int8.forward + _attn_fwd_full_int8 (flash_atten_full_int8.py:73-221);
  * native counterpart run_mha_fwd_full_qi8_ (csrc/flash_fwd_launch_template.h:503-523). */

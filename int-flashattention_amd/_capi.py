@@ -55,7 +55,8 @@ class AppendParams(ctypes.Structure):
 
 VARIANT_FULL_INT8, VARIANT_HALF_INT8, VARIANT_FP16 = 0, 1, 2
 
-EXPORTS = ("intfa_version", "intfa_error_string", "intfa_fwd_block_n", "intfa_fwd_workspace_bytes", "intfa_fwd_suggest_splits",
+EXPORTS = ("intfa_version", "intfa_error_string", "intfa_fwd_block_n", "intfa_fwd_workspace_bytes",
+           "intfa_fwd_merge_workspace_bytes", "intfa_fwd_suggest_splits",
            "intfa_fwd_full_int8", "intfa_fwd_half_int8", "intfa_fwd_fp16", "intfa_fwd_full_int8_static", "intfa_debug_qk_int32",
            "intfa_quant_pertoken", "intfa_quant_pertensor_workspace_bytes", "intfa_quant_pertensor",
            "intfa_quant_perblock_channel", "intfa_kvcache_append_int8")
@@ -84,6 +85,8 @@ def load():
     lib.intfa_fwd_suggest_splits.argtypes = [pp, ctypes.c_int, ctypes.c_int]
     lib.intfa_fwd_workspace_bytes.restype = ctypes.c_size_t
     lib.intfa_fwd_workspace_bytes.argtypes = [pp]
+    lib.intfa_fwd_merge_workspace_bytes.restype = ctypes.c_size_t
+    lib.intfa_fwd_merge_workspace_bytes.argtypes = [pp]
     for name in ("intfa_fwd_full_int8", "intfa_fwd_half_int8", "intfa_fwd_fp16", "intfa_fwd_full_int8_static"):
         fn = getattr(lib, name)
         fn.restype = ctypes.c_int

@@ -5,6 +5,7 @@
 #include "intfa_splitkv.h"
 
 #include <atomic>
+#include <random>
 
 using namespace intfa;
 
@@ -34,8 +35,6 @@ int static_scratch_ptr(void** out) {
     *out = ptr;
     return INTFA_OK;
 }
-
-constexpr int kMaxSplits = 64;
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -124,6 +123,20 @@ size_t workspace_bytes_for(const intfa_fwd_params* p) {
     return rows * (size_t)p->head_dim * sizeof(float) + rows * sizeof(float);
 }
 
+// One 8-byte arrival word per query block of at least kDecodeRows rows, behind the partials.
+size_t ticket_offset(const intfa_fwd_params* p) { return (workspace_bytes_for(p) + 7) & ~(size_t)7; }
+size_t merge_workspace_bytes_for(const intfa_fwd_params* p) {
+    if (workspace_bytes_for(p) == 0) return 0;
+    return ticket_offset(p) + (size_t)p->batch * p->heads * ((p->seqlen + kDecodeRows - 1) / kDecodeRows) * sizeof(uint64_t);
+}
+
+// Epochs of the launches that merge their splits themselves: 56 bits in the upper bits of the word, counted from a random
+// start so that a ticket word holding old data of another process's making is not taken for one of ours.
+uint64_t next_epoch() {
+    static std::atomic<uint64_t> count{((uint64_t)std::random_device{}() << 32 | std::random_device{}()) | 1u};
+    return count.fetch_add(1, std::memory_order_relaxed) << 8;
+}
+
 int setup_split(const intfa_fwd_params* p, int block_n, KParams* kp) {
     if (p->num_splits <= 1) return INTFA_OK;
     if (p->num_splits > kMaxSplits) return INTFA_ERR_SPLITS;
@@ -135,6 +148,11 @@ int setup_split(const intfa_fwd_params* p, int block_n, KParams* kp) {
     const size_t rows = (size_t)p->num_splits * p->batch * p->heads * p->seqlen;
     kp->o_part = (float*)p->workspace;
     kp->lse_part = kp->o_part + rows * (size_t)p->head_dim;
+    // (the merge addresses the partials with 32-bit offsets)
+    if (p->workspace_bytes >= merge_workspace_bytes_for(p) && need < (1ull << 32)) {
+        kp->ticket = (uint64_t*)((char*)p->workspace + ticket_offset(p));
+        kp->epoch = next_epoch();
+    }
     return INTFA_OK;
 }
 
@@ -155,6 +173,10 @@ int launch_combine(const intfa_fwd_params* p, const KParams& kp, hipStream_t str
 // instead of each taking 32 query rows (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h).
 constexpr int kDecodeMaxRows = 2 * kDecodeRows;
 bool decode_shaped(int seqlen) { return seqlen <= kDecodeMaxRows; }
+// (scale rows of 64 keys under the 128-key block: the decode kernel has one scale row per block)
+bool decode_kernel_takes(int variant, const KParams& kp) {
+    return decode_shaped(kp.seqlen) && !(variant == INTFA_VARIANT_FULL_INT8 && kp.vs_sub == 2);
+}
 
 int dispatch(int variant, const intfa_fwd_params* p, const KParams& kp, bool dump_s, hipStream_t stream) {
     const bool vblk = variant == INTFA_VARIANT_FULL_INT8 && !dump_s && kp.vs_g > 0;
@@ -165,9 +187,9 @@ int dispatch(int variant, const intfa_fwd_params* p, const KParams& kp, bool dum
     sel.split = kp.num_splits > 1;
     sel.dump_s = dump_s;
     const int d = kp.head_dim;
-    if (vblk && kp.vs_sub == 2) {              // (also for few query rows: the decode kernel has one scale row per block)
+    if (vblk && kp.vs_sub == 2) {
         if (d == 128) return launch_full_int8_vblk64_d128(kp, sel, stream);
-    } else if (!dump_s && decode_shaped(kp.seqlen)) {
+    } else if (!dump_s && decode_kernel_takes(variant, kp)) {
         if (variant == INTFA_VARIANT_FULL_INT8) {
             if (d == 64) return launch_decode_full_int8_d64(kp, sel, stream);
             if (d == 128) return launch_decode_full_int8_d128(kp, sel, stream);
@@ -214,8 +236,11 @@ int run_forward(int variant, const intfa_fwd_params* p, int qk_bytes, int v_byte
     rc = setup_split(p, block_n_for(variant, kp.head_dim), &kp);
     if (rc != INTFA_OK) return rc;
     kp.pair_mblocks = (kp.causal && kp.num_splits <= 1 && ((kp.seqlen + kBlockM - 1) / kBlockM) % 2 == 0) ? 1 : 0;
+    // (the decode-shaped kernels merge; the general ones leave it to the merge kernel)
+    const bool merges = decode_kernel_takes(variant, kp);
+    if (!merges) kp.ticket = nullptr;
     rc = dispatch(variant, p, kp, false, stream);
-    if (rc != INTFA_OK || kp.num_splits <= 1) return rc;
+    if (rc != INTFA_OK || kp.num_splits <= 1 || kp.ticket != nullptr) return rc;
     return launch_combine(p, kp, stream);
 }
 
@@ -249,6 +274,8 @@ const char* intfa_error_string(int code) {
 }
 
 size_t intfa_fwd_workspace_bytes(const intfa_fwd_params* p) { return workspace_bytes_for(p); }
+
+size_t intfa_fwd_merge_workspace_bytes(const intfa_fwd_params* p) { return p == nullptr ? 0 : merge_workspace_bytes_for(p); }
 
 int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus) {
     if (p == nullptr) return INTFA_ERR_NULL;

@@ -54,6 +54,7 @@ struct KParams {
     const int32_t* seqlens_k;              // optional [batch]: number of keys per batch entry (<= seqlen_k)
     int32_t* s_dump;                       // debug: int32 S [B,H,N,N]
     float* o_part; float* lse_part;        // split-KV partials [S,B,H,N,D] fp32 / [S,B,H,N]
+    uint64_t* ticket; uint64_t epoch;      // arrival words of the query blocks, the launch's epoch (intfa_splitkv.h); nullptr: no merge here
     int64_t q_sb, q_sh, q_sn;              // bytes
     int64_t k_sb, k_sh, k_sn;
     int64_t v_sb, v_sh, v_sn;

@@ -22,6 +22,7 @@
 #pragma once
 #include "intfa_device.h"
 #include "intfa_launch.h"
+#include "intfa_splitkv.h"
 
 namespace intfa {
 
@@ -307,8 +308,9 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
         }
     };
 
+    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    if (SPLIT && p.ticket != nullptr && tid == 0) splitkv_open_tickets(p, (b * p.heads + h) * n_mblk + mb);
     if (nb_begin < nb_end) {
-        issue_loads(nb_begin, 0);
         if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(load_ks(nb_begin));
         if (vs_thread) {
 #pragma unroll
@@ -339,25 +341,30 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const float out_scale = !seen ? 0.f : (PROUND == 0) ? (vs / l_tot) : (vs / (127.f * l_tot));
     const float l_true = (PROUND == 0) ? l_tot * (1.f / 127.f) : l_tot;
     const float lse = seen ? m_run + __builtin_log2f(l_true) : -INFINITY;
-    if (!q_valid) return;
     if (SPLIT) {
-        const int64_t row = ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + q_row;
-        float* op = p.o_part + row * D;
+        const SplitPartials part(p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
+        if (q_valid) {
 #pragma unroll
-        for (int j = 0; j < DTW; ++j) {
-            const int dt = wave + 4 * j;
-            if (dt >= DT) continue;
+            for (int j = 0; j < DTW; ++j) {
+                const int dt = wave + 4 * j;
+                if (dt >= DT) continue;
 #pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-                v4f o;
+                for (int a4 = 0; a4 < 4; ++a4) {
+                    v4f o;
 #pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * out_scale : 0.f;
-                *(v4f*)(op + 32 * dt + 8 * a4 + 4 * lh) = o;
+                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * out_scale : 0.f;
+                    part.put(lq, D, 32 * dt + 8 * a4 + 4 * lh, o);
+                }
             }
+            if (wave == 0 && lh == 0) part.put_lse(lq, seen ? lse : -INFINITY);
         }
-        if (wave == 0 && lh == 0) p.lse_part[row] = seen ? lse : -INFINITY;
+        if (p.ticket == nullptr || !splitkv_last_arrival(p, smem, (b * p.heads + h) * n_mblk + mb)) return;
+        static_assert(kMergeLds <= LDS_BYTES, "the merge fits the tile memory");
+        const int row0 = mb * kDecodeRows;
+        splitkv_merge_rows<D, OUT_DT>(p, smem, b, h, row0, p.seqlen - row0 < kDecodeRows ? p.seqlen - row0 : kDecodeRows);
         return;
     }
+    if (!q_valid) return;
     char* orow = p.out + b * p.o_sb + h * p.o_sh + (int64_t)q_row * p.o_sn;
 #pragma unroll
     for (int j = 0; j < DTW; ++j) {

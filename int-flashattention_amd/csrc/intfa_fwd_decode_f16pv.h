@@ -23,6 +23,7 @@
 #pragma once
 #include "intfa_device.h"
 #include "intfa_launch.h"
+#include "intfa_splitkv.h"
 #include "intfa_fwd_f16pv.h"
 
 namespace intfa {
@@ -276,8 +277,9 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
         if (QK_INT8 && more && ks_wave) *(float*)(smem + ks_wr + (BUF ^ 1) * BN * 4) = cvt_ks(ks_next);
     };
 
+    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    if (SPLIT && p.ticket != nullptr && tid == 0) splitkv_open_tickets(p, (b * p.heads + h) * n_mblk + mb);
     if (nb_begin < nb_end) {
-        issue_loads(nb_begin, 0);
         if (QK_INT8) {
             const uint32_t s0 = load_ks(nb_begin);
             if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(s0);
@@ -305,24 +307,29 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const bool seen = nb_begin < nb_end && m_run > -INFINITY;
     const float inv = seen ? 1.f / l_tot : 0.f;
     const float lse = seen ? m_run + __builtin_log2f(l_tot) : -INFINITY;
-    if (!q_valid) return;
     if (SPLIT) {
-        const int64_t row = ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + q_row;
-        float* op = p.o_part + row * D;
-        if (own_tile) {
+        const SplitPartials part(p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
+        if (q_valid) {
+            if (own_tile) {
 #pragma unroll
-            for (int j = 0; j < DTW; ++j)
+                for (int j = 0; j < DTW; ++j)
 #pragma unroll
-                for (int a4 = 0; a4 < 4; ++a4) {
-                    v4f o;
+                    for (int a4 = 0; a4 < 4; ++a4) {
+                        v4f o;
 #pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * inv : 0.f;
-                    *(v4f*)(op + 32 * (wave + 4 * j) + 8 * a4 + 4 * lh) = o;
-                }
+                        for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * inv : 0.f;
+                        part.put(lq, D, 32 * (wave + 4 * j) + 8 * a4 + 4 * lh, o);
+                    }
+            }
+            if (wave == 0 && lh == 0) part.put_lse(lq, seen ? lse : -INFINITY);
         }
-        if (wave == 0 && lh == 0) p.lse_part[row] = lse;
+        if (p.ticket == nullptr || !splitkv_last_arrival(p, smem, (b * p.heads + h) * n_mblk + mb)) return;
+        static_assert(kMergeLds <= LDS_BYTES, "the merge fits the tile memory");
+        const int row0 = mb * kDecodeRows;
+        splitkv_merge_rows<D, IO_DT>(p, smem, b, h, row0, p.seqlen - row0 < kDecodeRows ? p.seqlen - row0 : kDecodeRows);
         return;
     }
+    if (!q_valid) return;
     char* orow = p.out + b * p.o_sb + h * p.o_sh + (int64_t)q_row * p.o_sn;
     if (own_tile) {
 #pragma unroll

@@ -1,11 +1,181 @@
 // Merge of split-KV partial results (algorithm of csrc/flash_fwd_kernel.h:1212-1235 and :1264-1283 in the
-// reference, evaluated in base 2 because the forward kernels keep log2-domain statistics).
+// reference, evaluated in base 2 because the forward kernels keep log2-domain statistics): inside the forward kernel by
+// the workgroup that finishes a query block last, or, for callers whose workspace has no room for the arrival tickets, by a
+// kernel of its own.
 #pragma once
 #include "intfa_device.h"
 
 namespace intfa {
 
-// D / 4 lanes per output row (one 16-byte load per lane and split, one 8-byte store), 256 / (D / 4) rows per workgroup;
+// ---- Merge inside the forward kernel.
+// A merge kernel costs a decoding step 3.4 - 8 us of GPU time and 3.7 us of host time for its launch, half as much as the
+// pass itself.  Instead every workgroup publishes its partial and takes a ticket of its query block; the one that draws the
+// last ticket merges the block while the other workgroups of the launch still run.
+//   * Partials are written and read at agent scope (sc1: past the L2 of the XCD, which is not coherent with the seven
+//     others); the ticket is an atomic at the same scope, drawn after the writes have been acknowledged.
+//   * A ticket word is the launch's epoch (upper 56 bits, never the same twice in a process) and the arrivals so far.  The
+//     workspace is not cleared: every workgroup of the block looks at the word when it starts and exchanges anything that
+//     is not of this epoch for (epoch, 0) - under the first tiles' way from HBM, so that the arrival itself is one atomic add
+//     (a compare-and-swap loop there, with all splits of a block arriving together, cost 5 us with eight of them).  The last
+//     arrival stores zero, so the replays of a captured graph, whose epoch is a constant, find no word of an earlier one.
+constexpr int kSplitAux = 16;                  // sc1 in the cache-policy operand of the buffer intrinsics
+typedef __amdgpu_buffer_rsrc_t BufferRsrc;
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+// The partials from row `first` (wave-uniform) of the [split][batch][head][row] axis onward.  A writer starts at its own
+// workgroup's first row; the merge addresses all of them from row 0 (the host gives tickets only when they span less than 4 GiB).
+struct SplitPartials {
+    BufferRsrc o, l;
+    uint32_t rows;                             // batch * heads * seqlen: rows of one split
+    __device__ __forceinline__ explicit SplitPartials(const KParams& p, int D, int64_t first) {
+        rows = (uint32_t)(p.batch * p.heads) * (uint32_t)p.seqlen;
+        const int64_t left = (int64_t)rows * p.num_splits - first, ob = left * D * 4, lb = left * 4;
+        o = __builtin_amdgcn_make_buffer_rsrc(p.o_part + first * D, 0, (int)(uint32_t)(ob < 0xffffffffll ? ob : 0xffffffffll), 0x00020000);
+        l = __builtin_amdgcn_make_buffer_rsrc(p.lse_part + first, 0, (int)(uint32_t)(lb < 0xffffffffll ? lb : 0xffffffffll), 0x00020000);
+    }
+    __device__ __forceinline__ void put(uint32_t row, int D, int col, v4f x) const {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, x), o, (row * (uint32_t)D + (uint32_t)col) * 4u, 0, kSplitAux);
+    }
+    __device__ __forceinline__ void put_lse(uint32_t row, float x) const {
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), l, row * 4u, 0, kSplitAux);
+    }
+    __device__ __forceinline__ v4f get(uint32_t row, int D, int col) const {
+        return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(o, (row * (uint32_t)D + (uint32_t)col) * 4u, 0, kSplitAux));
+    }
+    __device__ __forceinline__ float get_lse(uint32_t row) const {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(l, row * 4u, 0, kSplitAux));
+    }
+};
+
+template <int OUT_DT> __device__ __forceinline__ void store_out4(char* dst, v4f acc) {
+    if (OUT_DT == 0) {
+        v4h o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = (_Float16)acc[i];
+        *(v4h*)dst = o;
+    } else {
+        v4s o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = f32_to_bf16(acc[i]);
+        *(v4s*)dst = o;
+    }
+}
+
+// Thread 0, at the start: the ticket word of query block `group` becomes this epoch's.
+__device__ __forceinline__ void splitkv_open_tickets(const KParams& p, int group) {
+    uint64_t* t = p.ticket + group;
+    uint64_t seen = __hip_atomic_load(t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((seen ^ p.epoch) >= 256u)
+        __hip_atomic_compare_exchange_strong(t, &seen, p.epoch, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Takes this workgroup's ticket of query block `group`; true for the last of the block's num_splits workgroups.
+// Called by every thread of the workgroup after its stores; `smem` is free (16 bytes of it are used).
+__device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* smem, int group) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's partials have reached the point of coherence
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t* t = p.ticket + group;
+        const uint64_t before = __hip_atomic_fetch_add(t, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = before == (p.epoch | (uint64_t)(p.num_splits - 1));
+        if (last) __hip_atomic_store(t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *(int*)smem = last;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*(const int*)smem) != 0;
+}
+
+// Reductions over eight consecutive lanes (quad_perm 1,0,3,2 / 2,3,0,1, then the mirrored half row).
+template <typename F> __device__ __forceinline__ float reduce8(float x, F op) {
+    x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true)));
+    x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true)));
+    return op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true)));
+}
+
+// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; 256 threads.
+// LDS: kMergeLds bytes of `smem`.  Eight lanes per row read the row's log-sum-exps (all in flight at once) and leave the
+// weights in LDS; then D / 4 lanes take a row, four columns each, 256 / (D / 4) rows side by side.  With fewer rows than that the
+// idle threads share the splits of a row and their sums are added in LDS.  Everything that can be requested before the
+// weights are known is: this runs once, at the end of a block, and its time is a chain of latencies.
+constexpr int kMaxSplits = 64;
+constexpr int kMergeLds = 16 + 32 * kMaxSplits * 4 + 256 * 16;
+template <int D, int OUT_DT>
+__device__ __forceinline__ void splitkv_merge_rows(const KParams& p, char* smem, int b, int h, int row0, int nrows) {
+    constexpr int LPR = D / 4, RP = 256 / LPR, KL = kMaxSplits / 8, U = 4;
+    const SplitPartials part(p, D, 0);
+    const int ns = p.num_splits, tid = threadIdx.x;
+    float* w = (float*)(smem + 16);                        // [split][32]
+    v4f* red = (v4f*)(smem + 16 + 32 * kMaxSplits * 4);
+    const uint32_t base = (uint32_t)(b * p.heads + h) * (uint32_t)p.seqlen + (uint32_t)row0;
+    // rows side by side: a power of two; G threads share one (row, columns)
+    int rs_log = 0;
+    while ((1 << rs_log) < nrows && (1 << rs_log) < RP) ++rs_log;
+    const int rs = 1 << rs_log, G = RP >> rs_log;
+    const int slot = tid / LPR, col = (tid % LPR) * 4, g = slot >> rs_log, r_first = slot & (rs - 1);
+    const int wr = tid >> 3, wj = tid & 7;
+    const uint32_t wrow = base + (wr < nrows ? wr : nrows - 1);
+    float lse[KL];
+#pragma unroll
+    for (int k = 0; k < KL; ++k) {
+        const int s = 8 * k + wj;
+        lse[k] = part.get_lse((uint32_t)(s < ns ? s : ns - 1) * part.rows + wrow);
+    }
+    v4f x[U];
+    auto request = [&](int r, int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int s = s0 + u * G;                      // past the end: any partial, its weight is zero
+            x[u] = part.get((uint32_t)(s < ns ? s : ns - 1) * part.rows + base + (r < nrows ? r : nrows - 1), D, col);
+        }
+    };
+    request(r_first, g);
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        float mx = -INFINITY, sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < KL; ++k) {
+            lse[k] = 8 * k + wj < ns ? lse[k] : -INFINITY;
+            mx = fmaxf(mx, lse[k]);
+        }
+        mx = reduce8(mx, [](float a, float c) { return fmaxf(a, c); });
+        // A row no split saw a key for: zeros with lse = -inf, as in splitkv_combine_kernel.
+        const bool empty = mx == -INFINITY;
+        if (empty) mx = 0.f;
+#pragma unroll
+        for (int k = 0; k < KL; ++k) sum += fast_exp2(lse[k] - mx);
+        sum = reduce8(sum, [](float a, float c) { return a + c; });
+        const float total = empty ? -INFINITY : __builtin_log2f(sum) + mx;
+#pragma unroll
+        for (int k = 0; k < KL; ++k) w[(8 * k + wj) * 32 + wr] = empty ? 0.f : fast_exp2(lse[k] - total);      // (0 past the last split)
+        if (p.lse != nullptr && wj == 0 && wr < nrows) p.lse[wrow] = total;
+    }
+    __syncthreads();
+    char* out0 = p.out + b * p.o_sb + h * p.o_sh + (int64_t)row0 * p.o_sn;
+    for (int r = r_first; r < nrows || G > 1; r += rs) {   // (G > 1: one trip for every thread, there is a barrier in it)
+        const bool on = r < nrows;
+        v4f acc = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = g; s0 < ns; s0 += U * G) {
+            if (s0 != g || r != r_first) request(r, s0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int s = s0 + u * G;
+                const float wt = s < ns ? w[s * 32 + (on ? r : 0)] : 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt, x[u][i], acc[i]);
+            }
+        }
+        if (G > 1) {
+            red[tid] = acc;
+            __syncthreads();
+            if (g == 0)
+                for (int k = 1; k < G; ++k) acc += red[tid + k * rs * LPR];
+        }
+        if (on && g == 0) store_out4<OUT_DT>(out0 + (int64_t)r * p.o_sn + col * 2, acc);
+        if (G > 1) break;
+    }
+}
+
+// ---- Merge in a launch of its own: D / 4 lanes per output row (one 16-byte load per lane and split, one 8-byte store), 256 / (D / 4) rows per workgroup;
 // the loads of four splits are in flight together.
 template <int D, int OUT_DT>
 __global__ void __launch_bounds__(256) splitkv_combine_kernel(const KParams p) {
@@ -46,17 +216,7 @@ __global__ void __launch_bounds__(256) splitkv_combine_kernel(const KParams p) {
     const int64_t bh = row / p.seqlen, n = row % p.seqlen;
     const int64_t b = bh / p.heads, h = bh % p.heads;
     char* orow = p.out + b * p.o_sb + h * p.o_sh + n * p.o_sn + sub * 8;
-    if (OUT_DT == 0) {
-        v4h o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = (_Float16)acc[i];
-        *(v4h*)orow = o;
-    } else {
-        v4s o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = f32_to_bf16(acc[i]);
-        *(v4s*)orow = o;
-    }
+    store_out4<OUT_DT>(orow, acc);
     if (p.lse != nullptr && sub == 0) p.lse[row] = lse;
 }
 

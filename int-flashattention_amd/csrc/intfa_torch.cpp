@@ -261,7 +261,7 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     Tensor ws;
     if (p.num_splits > 1) {
-        p.workspace_bytes = intfa_fwd_workspace_bytes(&p);
+        p.workspace_bytes = intfa_fwd_merge_workspace_bytes(&p);
         ws = dev.empty({(int64_t)p.workspace_bytes}, ScalarType::Byte);
         p.workspace = ws.data_ptr();
     }

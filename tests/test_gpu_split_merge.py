@@ -1,0 +1,110 @@
+"""Split-KV: the forward that merges its partials itself (a workspace of intfa_fwd_merge_workspace_bytes) against the one
+that leaves the merge to a second launch (intfa_fwd_workspace_bytes), on workspaces that hold arbitrary old data, and through
+the replays of a captured graph."""
+import ctypes
+
+import pytest
+import torch
+
+import int_flashattention_amd as M
+from int_flashattention_amd import _capi
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def problem(variant, B, H, Nq, Nk, D, seed, lens=None):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = ((torch.randn((B, H, n, D), generator=g)).half().to(DEV) for n in (Nq, Nk, Nk))
+    out, lse = torch.empty_like(q), torch.empty((B, H, Nq), device=DEV)
+    p = _capi.FwdParams()
+    keep = [q, k, v, out, lse]
+    if variant != "fp":
+        (q, qs), (k, ks) = M.quant_pertoken(q), M.quant_pertoken(k)
+        p.q_scale, p.k_scale = qs.data_ptr(), ks.data_ptr()
+        p.qs_stride_b, p.qs_stride_h, p.qs_stride_n = qs.stride()
+        p.ks_stride_b, p.ks_stride_h, p.ks_stride_n = ks.stride()
+        keep += [q, k, qs, ks]
+    if variant == "full":
+        v, vs = M.quant_pertensor(v)
+        p.v_scale, (p.vs_stride_b, p.vs_stride_h) = vs.data_ptr(), vs.stride()
+        keep += [v, vs]
+    for name, t in (("q", q), ("k", k), ("v", v), ("o", out)):
+        for axis, s in zip("bhn", t.stride()):
+            setattr(p, f"{name}_stride_{axis}", s)
+    p.q, p.k, p.v, p.out, p.lse = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr()
+    p.batch, p.heads, p.seqlen, p.seqlen_k, p.head_dim = B, H, Nq, Nk, D
+    p.scale_dtype = p.io_dtype = _capi.INTFA_F16
+    p.sm_scale, p.p_round = D ** -0.5, _capi.PROUND_REFERENCE
+    if lens is not None:
+        t = torch.tensor(lens, dtype=torch.int32, device=DEV)
+        p.seqlens_k = t.data_ptr()
+        keep.append(t)
+    return p, out, lse, keep
+
+
+def call(variant, p, ws, nbytes):
+    lib = _capi.load()
+    p.workspace, p.workspace_bytes = ws.data_ptr(), nbytes
+    fn = {"full": lib.intfa_fwd_full_int8, "half": lib.intfa_fwd_half_int8, "fp": lib.intfa_fwd_fp16}[variant]
+    assert fn(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+
+
+def close(a, b):
+    assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+    f = torch.isfinite(b)
+    assert (a[f].float() - b[f].float()).abs().max().item() <= 2e-3
+    assert ((a[f].float() - b[f].float()).norm() / b[f].float().norm()).item() <= 1e-4
+
+
+# rows of a 32-row block: one, a few (idle threads share the splits), a full block, a second block with one row; splits:
+# the fewest, one more than a multiple of what a thread has in flight, the most, more than there are blocks
+@pytest.mark.parametrize("variant,D,Nq,Nk,splits", [
+    ("full", 128, 1, 1024, 2), ("full", 128, 33, 4096, 17), ("full", 64, 5, 8200, 64), ("full", 256, 32, 1500, 9),
+    ("half", 64, 1, 5000, 33), ("half", 128, 17, 700, 5), ("half", 256, 3, 2050, 16),
+    ("fp", 128, 64, 1300, 64), ("fp", 64, 9, 3001, 8), ("fp", 256, 1, 300, 3),
+])
+def test_merge_in_the_kernel_equals_the_merge_launch(variant, D, Nq, Nk, splits):
+    lib = _capi.load()
+    p, out, lse, keep = problem(variant, 2, 3, Nq, Nk, D, 7 * splits + Nq, lens=[Nk, max(1, Nk // 3)])
+    p.num_splits = splits
+    small, need = lib.intfa_fwd_workspace_bytes(ctypes.byref(p)), lib.intfa_fwd_merge_workspace_bytes(ctypes.byref(p))
+    assert need > small
+    ws = torch.empty((need,), dtype=torch.uint8, device=DEV)
+    call(variant, p, ws, small)
+    torch.cuda.synchronize()
+    want, want_lse = out.clone(), lse.clone()
+    for fill in (0, 255, None, 1):                 # None: what the call before left behind
+        if fill is not None:
+            ws.fill_(fill)
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        call(variant, p, ws, need)
+        torch.cuda.synchronize()
+        close(out, want)
+        close(lse, want_lse)
+
+
+def test_merge_replays_from_a_graph_beside_other_calls():
+    lib = _capi.load()
+    p, out, lse, keep = problem("half", 1, 4, 4, 4096, 128, 3)
+    p.num_splits = 8
+    need = lib.intfa_fwd_merge_workspace_bytes(ctypes.byref(p))
+    ws = torch.full((need,), 171, dtype=torch.uint8, device=DEV)
+    call("half", p, ws, need)
+    torch.cuda.synchronize()
+    want, want_lse = out.clone(), lse.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call("half", p, ws, need)
+    for i in range(4):
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(lse, want_lse), i
+        if i == 1:
+            ws.fill_(171)                          # the workspace is the caller's between replays
+        call("half", p, ws, need)                  # an eager call on the same workspace
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i

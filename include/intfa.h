@@ -231,6 +231,9 @@ int intfa_quant_pertoken(const void* x, int64_t stride_b, int64_t stride_h, int6
  * [batch, heads] in x's type.  Needs intfa_quant_pertensor_workspace_bytes() bytes of device scratch (4-byte
  * aligned) for the per-slice maxima. */
 size_t intfa_quant_pertensor_workspace_bytes(int32_t batch, int32_t heads);
+/* A workspace of this many bytes (at least intfa_quant_pertensor_workspace_bytes()) holds the maxima of the parts of a slice
+ * instead, which saves the launch that clears the per-slice words. */
+size_t intfa_quant_pertensor_parts_workspace_bytes(int32_t batch, int32_t heads, int32_t seqlen, int32_t head_dim);
 int intfa_quant_pertensor(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_n, void* q8, void* scale,
                           int32_t batch, int32_t heads, int32_t seqlen, int32_t head_dim, int32_t dtype,
                           void* workspace, size_t workspace_bytes, void* stream);

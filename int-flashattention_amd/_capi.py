@@ -58,7 +58,8 @@ VARIANT_FULL_INT8, VARIANT_HALF_INT8, VARIANT_FP16 = 0, 1, 2
 EXPORTS = ("intfa_version", "intfa_error_string", "intfa_fwd_block_n", "intfa_fwd_workspace_bytes",
            "intfa_fwd_merge_workspace_bytes", "intfa_fwd_suggest_splits",
            "intfa_fwd_full_int8", "intfa_fwd_half_int8", "intfa_fwd_fp16", "intfa_fwd_full_int8_static", "intfa_debug_qk_int32",
-           "intfa_quant_pertoken", "intfa_quant_pertensor_workspace_bytes", "intfa_quant_pertensor",
+           "intfa_quant_pertoken", "intfa_quant_pertensor_workspace_bytes",
+           "intfa_quant_pertensor_parts_workspace_bytes", "intfa_quant_pertensor",
            "intfa_quant_perblock_channel", "intfa_kvcache_append_int8")
 
 _lib = None
@@ -98,6 +99,8 @@ def load():
     lib.intfa_quant_pertoken.argtypes = [vp, i64, i64, i64, vp, vp, i32, i32, i32, i32, i32, vp]
     lib.intfa_quant_pertensor_workspace_bytes.restype = ctypes.c_size_t
     lib.intfa_quant_pertensor_workspace_bytes.argtypes = [i32, i32]
+    lib.intfa_quant_pertensor_parts_workspace_bytes.restype = ctypes.c_size_t
+    lib.intfa_quant_pertensor_parts_workspace_bytes.argtypes = [i32, i32, i32, i32]
     lib.intfa_quant_pertensor.restype = ctypes.c_int
     lib.intfa_quant_pertensor.argtypes = [vp, i64, i64, i64, vp, vp, i32, i32, i32, i32, i32, vp, ctypes.c_size_t, vp]
     lib.intfa_quant_perblock_channel.restype = ctypes.c_int

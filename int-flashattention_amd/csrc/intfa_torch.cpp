@@ -352,7 +352,7 @@ PyObject* quant_pertensor(PyObject*, PyObject* arg) {
     const Tensor x = quant_input(tensor_arg(arg, "x"));
     const CallDevice dev(x);
     Tensor q8 = dev.empty(x.sizes(), ScalarType::Char), scale = dev.empty(x.sizes().slice(0, 2), x.scalar_type());
-    const size_t need = intfa_quant_pertensor_workspace_bytes((int)x.size(0), (int)x.size(1));
+    const size_t need = intfa_quant_pertensor_parts_workspace_bytes((int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3));
     const Tensor ws = dev.empty({(int64_t)need}, ScalarType::Byte);
     void* const st = dev.raw_stream();
     const int rc = unlocked([&] {

@@ -1,0 +1,42 @@
+"""The per-(batch, head) quantiser around the sizes where its launches change: a slice in the registers of one workgroup, the
+two launches with a word per part, and the three with one word per slice (the smaller workspace of the C interface)."""
+import ctypes
+
+import pytest
+import torch
+
+import intfa_oracle as O
+import int_flashattention_amd as M
+from int_flashattention_amd import _capi
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# (N * d * 2 bytes around 128 KiB; one row; more slices than workgroups are wanted; a last chunk with one row)
+@pytest.mark.parametrize("B,H,N,d", [(1, 2, 1, 16), (2, 3, 511, 128), (1, 2, 512, 128), (1, 2, 513, 128), (1, 1, 1025, 64),
+                                     (3, 1, 257, 256), (1, 1, 4097, 16), (1, 5, 2049, 128), (40, 64, 520, 128)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_quant_pertensor_slice_sizes_bit_exact(B, H, N, d, dtype):
+    g = torch.Generator(device=DEV).manual_seed(N + d)
+    x = torch.randn((B, H, N, d), generator=g, device=DEV).to(dtype)
+    x[:, :, N // 2] *= 3                                    # the maximum lies inside
+    x[0, 0, -1, -1] = 30                                    # and in the very last element of one slice
+    q8, s = M.quant_pertensor(x)
+    cut = (slice(0, 2), slice(0, 5))
+    ref8, ref_s = O.quant_pertensor(x[cut].cpu())
+    assert torch.equal(s[cut].cpu(), ref_s) and torch.equal(q8[cut].cpu(), ref8)
+    if B * H > 10:
+        ref8, ref_s = O.quant_pertensor(x[-1:, -1:].cpu())
+        assert torch.equal(s[-1:, -1:].cpu(), ref_s) and torch.equal(q8[-1:, -1:].cpu(), ref8)
+    # the C interface with the smallest workspace, filled with old data
+    lib = _capi.load()
+    need = lib.intfa_quant_pertensor_workspace_bytes(B, H)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+    q8b, sb = torch.empty_like(q8), torch.empty_like(s)
+    dt = _capi.INTFA_F16 if dtype == torch.float16 else _capi.INTFA_BF16
+    rc = lib.intfa_quant_pertensor(x.data_ptr(), *x.stride()[:3], q8b.data_ptr(), sb.data_ptr(), B, H, N, d, dt, ws.data_ptr(), need,
+                                   ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert torch.equal(q8b, q8) and torch.equal(sb, s)

@@ -169,13 +169,26 @@ int launch_combine(const intfa_fwd_params* p, const KParams& kp, hipStream_t str
     return e == hipSuccess ? INTFA_OK : (int)e;
 }
 
-// Few query rows per head (decoding against a cache): the pass runs a kernel whose waves share the keys of a block
-// instead of each taking 32 query rows (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h).
-constexpr int kDecodeMaxRows = 2 * kDecodeRows;
+// The pass runs a kernel whose four waves share the keys of a block and own 32 query rows together, instead of 32 each
+// (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h), where the latter would leave waves without rows or compute units without a
+// workgroup:
+//   * few query rows per head (decoding against a cache), at any size;
+//   * small problems in a single pass: four times the workgroups, each walking its keys in a fraction of the time, as
+//     long as all of them are resident at once.  That is two per compute unit at head_dim 64 and for full-int8 at head_dim 128,
+//     one at head_dim 256 (a workgroup fills the LDS).  Measured around the line (general -> this, us): full-int8 d128
+//     causal B1 H16 N1024 22.7 -> 17.4, B3 H32 N256 (768 workgroups) 10.8 -> 12.8; full-int8 d256 B1 H8 N1024 31.5 -> 20.3,
+//     B1 H16 N1024 32.8 -> 37.6; B1 H8 N256 d64 7.6 -> 5.5.
+// Not half-int8 and fp16 at head_dim 128: there two of the four waves have no share of Q K^T, the gain ends at 10 %, and the
+// kernels differ in the rounding of P.  Everywhere else both kernels give the same bits, so that an output does not depend on how
+// many heads and batch entries it is computed with.
+constexpr int kComputeUnits = 256;
 bool decode_shaped(int seqlen) { return seqlen <= kDecodeMaxRows; }
 // (scale rows of 64 keys under the 128-key block: the decode kernel has one scale row per block)
 bool decode_kernel_takes(int variant, const KParams& kp) {
-    return decode_shaped(kp.seqlen) && !(variant == INTFA_VARIANT_FULL_INT8 && kp.vs_sub == 2);
+    const int per_cu = kp.head_dim == 64 ? 2 : kp.head_dim == 256 ? 1 : variant == INTFA_VARIANT_FULL_INT8 ? 2 : 0;
+    const int64_t wgs = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kDecodeRows - 1) / kDecodeRows);
+    const bool small = kp.num_splits <= 1 && wgs <= per_cu * kComputeUnits;
+    return (decode_shaped(kp.seqlen) || small) && !(variant == INTFA_VARIANT_FULL_INT8 && kp.vs_sub == 2);
 }
 
 int dispatch(int variant, const intfa_fwd_params* p, const KParams& kp, bool dump_s, hipStream_t stream) {
@@ -235,7 +248,11 @@ int run_forward(int variant, const intfa_fwd_params* p, int qk_bytes, int v_byte
     }
     rc = setup_split(p, block_n_for(variant, kp.head_dim), &kp);
     if (rc != INTFA_OK) return rc;
-    kp.pair_mblocks = (kp.causal && kp.num_splits <= 1 && ((kp.seqlen + kBlockM - 1) / kBlockM) % 2 == 0) ? 1 : 0;
+    // Causal passes of more workgroups than compute units give one workgroup the query blocks i and n-1-i (even counts).  At one
+    // workgroup per compute unit or less the pairs would only halve the number that work: B2 H32 N512 d128 full-int8
+    // 20.5 us in pairs, 15.0 without; B4 H32 N512 21.7 and 21.7; B8 H32 N512 30.6 and 37.6.
+    const int n_mblk = (kp.seqlen + kBlockM - 1) / kBlockM;
+    kp.pair_mblocks = kp.causal && kp.num_splits <= 1 && n_mblk % 2 == 0 && (int64_t)kp.batch * kp.heads * n_mblk > kComputeUnits ? 1 : 0;
     // (the decode-shaped kernels merge; the general ones leave it to the merge kernel)
     const bool merges = decode_kernel_takes(variant, kp);
     if (!merges) kp.ticket = nullptr;

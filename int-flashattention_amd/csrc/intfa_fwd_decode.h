@@ -7,11 +7,12 @@
 // query rows and its four waves share every key block:
 //   * wave w computes S^T for keys 32w .. 32w+31 of the block (KS MFMAs), dequantises and takes the partial row maxima;
 //   * the partial maxima meet in LDS (barrier), every wave then holds the block's row maximum;
-//   * wave w exponentiates and requantises its 32 keys and publishes its P8 fragment in LDS (barrier);
+//   * wave w exponentiates and requantises its 32 keys and publishes its P8 fragment and row sums in LDS (barrier);
 //   * wave w multiplies the whole block's P (all four fragments) with ITS 32-column slice of V and updates its slice of
-//     the fp32 output; the partial row sums of P meet once, in the epilogue.
-// The int32 sums run over the same 128 keys as in the general kernel, so results agree with it up to the order of the
-// fp32 additions of the row sums.  K/V tiles are double-buffered in LDS and the whole next tile is requested at the
+//     the fp32 output.
+// The int32 sums run over the same 128 keys as in the general kernel, and the waves exchange the row sums of their keys with
+// the P8 fragments and add them in that kernel's order: the results are the same bits, and which of the two runs may depend on
+// the number of heads and batch entries.  K/V tiles are double-buffered in LDS and the whole next tile is requested at the
 // start of a block (the data comes from HBM, not from a cache shared with other query blocks).
 // Head dims 64 and 256: the general kernels' key block is 64 there (the reference admits no key block longer than head_dim,
 // flash_atten_full_int8.py:88; at 256 registers set the limit), so a 128-key step of this
@@ -42,9 +43,10 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     constexpr int SWM = CH - 1;                  // swizzle mask of V rows
     // LDS map (bytes)
     constexpr int OFF_KS = 0;                            // two fp32 k_scale vectors
-    constexpr int OFF_XM = 2 * BN * 4;                   // 4 waves x 32 rows fp32: partial row maxima / row sums
+    constexpr int OFF_XM = 2 * BN * 4;                   // 4 waves x 32 rows fp32: partial row maxima
     constexpr int OFF_XP = OFF_XM + 4 * 32 * 4;          // 4 waves x 64 lanes x 16 bytes: the waves' P8 fragments
-    constexpr int OFF_VS = OFF_XP + 4 * 64 * 16;         // VBLK: two vectors of NBS * D fp32 channel scales (one row per block)
+    constexpr int OFF_XS = OFF_XP + 4 * 64 * 16;         // 64 lanes x 4 waves fp32: row sums of the waves' keys
+    constexpr int OFF_VS = OFF_XS + 4 * 64 * 4;          // VBLK: two vectors of NBS * D fp32 channel scales (one row per block)
     constexpr int NV = NBS * D;                          // channel scales per step
     constexpr int OFF_K = OFF_VS + (VBLK ? 2 * NV * 4 : 0);
     constexpr int OFF_V = OFF_K + 2 * KT;
@@ -87,7 +89,8 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);
     const float qsc = load_q_scale_log2(p, b, h, q_ld);
 
-    float m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only
+    float m_run = -INFINITY, l_run = 0.f;
+    float l_odd = 0.f;                           // head_dim 256: row sums of the odd sub-tiles (a wave of its own in that general kernel)
     float o_acc[DTW][16];
 #pragma unroll
     for (int j = 0; j < DTW; ++j)
@@ -153,6 +156,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const uint32_t xm_rd = OFF_XM + 4 * lq;                          // + 128 per wave
     const uint32_t xp_wr = OFF_XP + 1024 * wave + 16 * lane;
     const uint32_t xp_rd = OFF_XP + 16 * lane;                       // + 1024 per wave
+    const uint32_t xs_rd = OFF_XS + 16 * lane, xs_wr = xs_rd + 4 * wave;
     const uint32_t vs_wr = OFF_VS + 4 * vs_i;                        // + 4 * kThreads per further value
     const uint32_t vs_rd = OFF_VS + 16 * lh;                         // + 4 * (D*blk + 32*dt + 8*a4) per read
     // head_dim 64 has two output tiles for four waves: waves 2 and 3 compute tiles 0 and 1 a second time and store
@@ -256,6 +260,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
             }
         }
         *(v4i*)(smem + xp_wr) = p8;
+        *(float*)(smem + xs_wr) = lsum;
         v4f vsc[NBS][DTW][4];                              // channel scales of the step's blocks for this wave's output tiles
         if (VBLK) {
 #pragma unroll
@@ -270,6 +275,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
         v4i pall[NST];
 #pragma unroll
         for (int st = 0; st < NST; ++st) pall[st] = *(const v4i*)(smem + xp_rd + 1024 * st);
+        const v4f ls = *(const v4f*)(smem + xs_rd);
         // -------- this wave's output columns: O^T[d, q] += V^T[d, key] P^T[key, q] over the whole block
 #pragma unroll
         for (int j = 0; j < DTW; ++j) {
@@ -296,8 +302,12 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
                 }
             }
         }
-        if (NBS == 1) l_run = fmaf(l_run, alpha, lsum);
-        else l_run = blk_a ? fmaf(l_run, alpha, lsum) * alpha_b : fmaf(l_run * alpha, alpha_b, lsum);
+        if (D == 128) l_run = fmaf(l_run, alpha, (ls[0] + ls[1]) + (ls[2] + ls[3]));
+        else if (D == 64) l_run = fmaf(fmaf(l_run, alpha, ls[0] + ls[1]), alpha_b, ls[2] + ls[3]);
+        else {
+            l_run = fmaf(fmaf(l_run, alpha, ls[0]), alpha_b, ls[2]);
+            l_odd = fmaf(fmaf(l_odd, alpha, ls[1]), alpha_b, ls[3]);
+        }
         // (the raw scale is made opaque here, behind the step's last barrier: its conversion waits for the load, and with it
         // for the next step's tile copies that were issued ahead of it - that wait belongs at the end of the step)
         asm volatile("" : "+v"(ks_next));
@@ -327,13 +337,8 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
         }
     }
 
-    // ---- epilogue: the waves' partial row sums meet in LDS; every wave scales and stores its own output columns
-    __syncthreads();
-    const float l_pair = half_pair_sum(l_run);
-    if (lh == 0) *(float*)(smem + xm_wr) = l_pair;
-    __syncthreads();
-    const float l_tot = (*(const float*)(smem + xm_rd) + *(const float*)(smem + xm_rd + 128)) +
-                        (*(const float*)(smem + xm_rd + 256) + *(const float*)(smem + xm_rd + 384));   // units of 1/127 when PROUND == 0
+    // ---- epilogue: every wave scales and stores its own output columns
+    const float l_tot = half_pair_sum(l_run) + (D == 256 ? half_pair_sum(l_odd) : 0.f);      // units of 1/127 when PROUND == 0
     const float vs = VBLK ? 1.f : load_scale(p.v_scale, b * p.vs_sb + hk * p.vs_sh, p.scale_dtype);
     // false: an empty split range, an empty cache entry, or a causal row above the first key (zeros, lse = -inf; such a
     // row's accumulators hold NaN from exp2(-inf - -inf), hence the selects below)

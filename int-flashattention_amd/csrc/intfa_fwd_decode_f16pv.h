@@ -17,8 +17,10 @@
 // every wave owns one (two at head_dim 256) 32-column output tile.  The smaller step is what the stream wants there: 24
 // to 32 KiB of tiles per step let two or three workgroups share a compute unit at head_dim 128 (6.0 TB/s of K+V against
 // 5.4 - 5.9 with 128-key steps and one workgroup), and at head_dim 256 two steps of 128 keys would not fit the LDS.
-// Every block is evaluated with the same maximum, the same P and the same order of MFMA steps as in the general kernel;
-// only the row sums are added in another order (per wave, joined in the epilogue).  K/V tiles of a step are
+// In calls that the general kernels could have taken, at head_dim 64 and 256, every block is evaluated with the same frame, the same P, the same order of MFMA steps and of the row
+// sums as in the general kernels, so that the results are the same bits and which of the two runs may depend on the number of
+// heads and batch entries.  (At head_dim 128 and in decode-shaped calls the frame is the running maximum of every block,
+// which moves P's 16-bit rounding against the general kernel's lazy frame.)  K/V tiles of a step are
 // double-buffered in LDS and the whole next step is requested at the start of a step.
 #pragma once
 #include "intfa_device.h"
@@ -51,7 +53,8 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     constexpr int OFF_XM = 2 * BN * 4;                    // 4 waves x 32 rows fp32: partial row maxima / row sums
     constexpr int OFF_XP = OFF_XM + 4 * 32 * 4;           // NG operands of 64 lanes x 16 bytes: the waves' 16-bit P
     static_assert(QKW == 4 || QKW == 2, "a step is four or two 32-key sub-tiles");
-    constexpr int OFF_K = OFF_XP + NG * 1024;
+    constexpr int OFF_XS = OFF_XP + NG * 1024;            // head_dim 64: 64 lanes x 4 waves fp32, row sums of the waves' keys
+    constexpr int OFF_K = OFF_XS + (NBS == 2 ? 1024 : 0);
     constexpr int OFF_V = OFF_K + 2 * KT;
     constexpr int LDS_BYTES = OFF_V + 2 * VT;
     static_assert(OFF_K % 256 == 0, "tiles keep the bank alignment the swizzles assume");
@@ -95,7 +98,7 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     }
     const float qsc = QK_INT8 ? load_q_scale_log2(p, b, h, q_ld) : p.qk_scale_log2;
 
-    float m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only
+    float m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only (head_dim 64: all keys)
     v16f o_acc[DTW];
 #pragma unroll
     for (int j = 0; j < DTW; ++j)
@@ -148,10 +151,19 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const uint32_t xm_rd = OFF_XM + 4 * lq;                          // + 128 per wave
     const uint32_t xp_wr = OFF_XP + 2048 * wave + 16 * lane;         // + 1024 for the second operand
     const uint32_t xp_rd = OFF_XP + 16 * lane;                       // + 1024 per MFMA step
+    const uint32_t xs_rd = OFF_XS + 16 * lane, xs_wr = xs_rd + 4 * wave;
     // the smallest and this lane's own last visible key
     const int first_lim = p.causal ? (fold ? 0 : mb * kDecodeRows) + causal_off : 0x3fffffff;
     const int row_lim = p.causal ? (fold ? q_row % fold : q_row) + causal_off : 0x3fffffff;
     const bool blk_a = NBS == 1 || wave < 2;          // this wave's keys belong to the first block of a step
+    // head_dim 64, where fwd_f16pv_kernel could have taken the call (more than kDecodeMaxRows query rows), its lazy frame: it follows a row's maximum when that exceeds it by more than
+    // kFrameSlack in some row of the 32, and in the blocks that kernel masks (of its 128-row query blocks): the causal
+    // diagonal's, or the ragged last one
+    const int masked_first = p.seqlen <= kDecodeMaxRows ? 0 : p.causal ? ((mb * kDecodeRows / kBlockM) * kBlockM + causal_off + 1) / BNB : seqlen_k / BNB;
+    auto frame = [&](float m, float mxs, int blk) __attribute__((always_inline)) -> float {
+        const bool move = blk >= masked_first || __builtin_amdgcn_ballot_w64(mxs > m + kFrameSlack) != 0;
+        return move ? fmaxf(m, mxs) : m;
+    };
 
     auto mfma16 = [&](v4i a, v4i bb, v16f c) __attribute__((always_inline)) -> v16f {
         if (IO_DT == 0) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, bb), c, 0, 0, 0);
@@ -225,12 +237,12 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
         }
         __syncthreads();                                   // the partial maxima are in LDS
         const float mx_a = fmaxf(*(const float*)(smem + xm_rd), *(const float*)(smem + xm_rd + 128));
-        const float m_a = fmaxf(m_run, mx_a * qsc);
+        const float m_a = NBS == 2 ? frame(m_run, mx_a * qsc, nb) : fmaxf(m_run, mx_a * qsc);
         const float alpha_a = fast_exp2(m_run - m_a);
         float m_b = m_a, alpha_b = 1.f;                    // one block per step: no second factor
         if (NBS == 2) {
             const float mx_b = fmaxf(*(const float*)(smem + xm_rd + 256), *(const float*)(smem + xm_rd + 384));
-            m_b = fmaxf(m_a, mx_b * qsc);
+            m_b = frame(m_a, mx_b * qsc, nb + 1);
             alpha_b = fast_exp2(m_a - m_b);
         }
         m_run = m_b;
@@ -248,6 +260,7 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
             for (int u = 0; u < 2; ++u)
                 *(v4i*)(smem + xp_wr + 1024 * u) = IO_DT == 0 ? __builtin_bit_cast(v4i, pack_p_f16(e + 8 * u))
                                                               : __builtin_bit_cast(v4i, pack_p_bf16(e + 8 * u));
+            if (NBS == 2) *(float*)(smem + xs_wr) = lsum;
         }
         __syncthreads();                                   // the P operands are in LDS
         // -------- this wave's output columns: O^T[d, q] = (O^T alpha_A + V_A^T P_A^T) alpha_B + V_B^T P_B^T
@@ -260,7 +273,11 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o_acc[j][r] *= alpha_a;
 #pragma unroll
-                for (int g = 0; g < NG / NBS; ++g) o_acc[j] = mfma16(vf[j][g], pall[g], o_acc[j]);
+                for (int i = 0; i < NG / NBS; ++i) {
+                    // (the waves of fwd_f16pv_pair_kernel start with the keys of their own column half)
+                    const int g = D == 256 && j == 1 ? i ^ 2 : i;
+                    o_acc[j] = mfma16(vf[j][g], pall[g], o_acc[j]);
+                }
                 if (NBS == 2) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) o_acc[j][r] *= alpha_b;
@@ -270,7 +287,12 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
             }
         }
         if (NBS == 1) l_run = fmaf(l_run, alpha_a, lsum);
-        else l_run = blk_a ? fmaf(l_run, alpha_a, lsum) * alpha_b : fmaf(l_run * alpha_a, alpha_b, lsum);
+        else {
+#pragma clang fp contract(off)
+            const v4f ls = *(const v4f*)(smem + xs_rd);
+            l_run = l_run * alpha_a + (ls[0] + ls[1]);
+            l_run = l_run * alpha_b + (ls[2] + ls[3]);
+        }
         // (the raw scale is made opaque here, behind the step's last barrier: its conversion waits for the load, and with it
         // for the next step's tile copies that were issued ahead of it - that wait belongs at the end of the step)
         if (QK_INT8) asm volatile("" : "+v"(ks_next));
@@ -295,13 +317,15 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
         }
     }
 
-    // ---- epilogue: the waves' partial row sums meet in LDS; every wave scales and stores its own output columns
-    __syncthreads();
-    const float l_pair = half_pair_sum(l_run);
-    if (lh == 0) *(float*)(smem + xm_wr) = l_pair;
-    __syncthreads();
-    const float l_tot = (*(const float*)(smem + xm_rd) + *(const float*)(smem + xm_rd + 128)) +
-                        (*(const float*)(smem + xm_rd + 256) + *(const float*)(smem + xm_rd + 384));
+    // ---- epilogue: every wave scales and stores its own output columns (the waves' partial row sums meet in LDS first)
+    float l_tot = half_pair_sum(l_run);
+    if (NBS == 1) {
+        __syncthreads();
+        if (lh == 0) *(float*)(smem + xm_wr) = l_tot;
+        __syncthreads();
+        l_tot = (*(const float*)(smem + xm_rd) + *(const float*)(smem + xm_rd + 128)) +
+                (*(const float*)(smem + xm_rd + 256) + *(const float*)(smem + xm_rd + 384));
+    }
     // false: an empty split range, an empty cache entry, or a causal row above the first key (zeros, lse = -inf; such a
     // row's accumulators hold NaN from exp2(-inf - -inf), hence the selects below)
     const bool seen = nb_begin < nb_end && m_run > -INFINITY;

@@ -252,7 +252,10 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
             const float m_mv = fmaxf(m_run, mxs);
             const float a_mv = fast_exp2(m_run - m_mv);
             m_run = m_mv;
-            l_run *= a_mv;
+            {
+#pragma clang fp contract(off)
+                l_run *= a_mv;                   // (not fused with the addition below, here or in the decode-shaped kernel)
+            }
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -260,21 +263,30 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
         }
         const float m_new = m_run;
         // -------- pass 2: P = exp2(x*qsc - m), row sum, cast to the 16-bit type
-        float lsum = 0.f;
+        // (head_dim 64: a sum per sub-tile, then their sum - the order of the decode-shaped kernel, whose waves hold a sub-tile each;
+        // both give the same bits)
+        float lsum = 0.f, lfirst = 0.f;
         v4i pf[NST][2];                                   // B operands: 8 x 16-bit per 16-key step
 #pragma unroll
         for (int st = 0; st < NST; ++st) {
             if (DIAG && st > gw) continue;
             __builtin_amdgcn_sched_barrier(0);
             float e[16];
+            if (D == 64 && st == 1) lfirst = lsum;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) { e[r] = fast_exp2(fmaf(t[st][r], qsc, -m_new)); lsum += e[r]; }
+            for (int r = 0; r < 16; ++r) {
+                e[r] = fast_exp2(fmaf(t[st][r], qsc, -m_new));
+                lsum = r == 0 && (st == 0 || D == 64) ? e[r] : lsum + e[r];
+            }
 #pragma unroll
             for (int u = 0; u < 2; ++u)
                 pf[st][u] = IO_DT == 0 ? __builtin_bit_cast(v4i, pack_p_f16(e + 8 * u)) : __builtin_bit_cast(v4i, pack_p_bf16(e + 8 * u));
             asm volatile("" : "+v"(lsum));
         }
-        l_run += lsum;
+        {
+#pragma clang fp contract(off)
+            l_run += D == 64 ? lfirst + lsum : lsum;
+        }
         // -------- O^T[d, q] += V^T[d, key] P^T[key, q] (the fp32 accumulators of the MFMAs are the running output)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

@@ -313,7 +313,9 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         asm volatile("" : "+v"(alpha));
         m_run = m_new;
         // -------- pass 2: P = exp2(x*qsc - m), row sum, requantise
-        float lsum = 0.f;
+        // (sums per sub-tile, added in pairs: the order in which the waves of the decode-shaped kernel, which hold a sub-tile each,
+        // can add them too, so that both kernels give the same bits)
+        float lsum = 0.f, lpair = 0.f;
         v4i p8[NST];
         v16i oacc[2];
         const float bias = (PROUND == 0 ? kLog2_127 : 0.f) - m_new;
@@ -324,6 +326,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             // when the next block waits for it (its buffer was last read before this block's barrier)
             if (!DIAG) issue_v_slice(v_next, nb + 1, BUF ^ 1, st, NST);
             __builtin_amdgcn_sched_barrier(0);
+            float ls = 0.f;
             if (PROUND == 0) {
 #pragma unroll
                 for (int w4 = 0; w4 < 4; ++w4) {
@@ -331,7 +334,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 #pragma unroll
                     for (int b4 = 0; b4 < 4; ++b4) {
                         const float e = fast_exp2(fmaf(t[st][4 * w4 + b4], qsc, bias));   // 127 * p
-                        lsum += e;
+                        ls = w4 + b4 ? ls + e : e;
                         pk = __builtin_amdgcn_cvt_pk_u8_f32(e, b4, pk);
                     }
                     p8[st][w4] = (int)pk;
@@ -342,11 +345,13 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     e[r] = fast_exp2(fmaf(t[st][r], qsc, bias));                          // p
-                    lsum += e[r];
+                    ls = r ? ls + e[r] : e[r];
                 }
                 p8[st] = requant_p_reference16(e);
             }
-            asm volatile("" : "+v"(lsum));      // keep the row-sum chain inside its stage
+            lpair = (st & 1) ? lpair + ls : ls;
+            if (st & 1) lsum = st > 1 ? lsum + lpair : lpair;
+            asm volatile("" : "+v"(lpair), "+v"(lsum));      // keep the row-sum chain inside its stage
             // the P V chain of the first d-tile advances by one MFMA as soon as this sub-tile's P8 is packed: it runs
             // under the exponentials of the next sub-tile instead of in a burst behind the pass
             if (VBLK == 2) {                     // keys 0..63 of the block only: the second half is a chain (and a scale row) of its own

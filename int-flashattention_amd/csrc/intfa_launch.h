@@ -5,6 +5,7 @@
 
 namespace intfa {
 
+constexpr int kDecodeMaxRows = 64;    // most query rows per head of a decode-shaped call
 constexpr int kDecodeRows = 32;       // query rows per workgroup of the decode-shaped kernel (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h)
 
 // Launch switches resolved to template arguments inside the instance files.

@@ -111,6 +111,7 @@ int make_kparams(const intfa_fwd_params* p, int qk_bytes, int v_bytes, bool need
     k.batch = p->batch; k.heads = p->heads; k.seqlen = p->seqlen; k.seqlen_k = seqlen_k; k.head_dim = p->head_dim;
     k.scale_dtype = p->scale_dtype; k.causal = p->causal ? 1 : 0;
     k.kv_group = p->heads / heads_kv;
+    k.kv_key_bytes = p->head_dim * (qk_bytes + v_bytes);
     k.num_splits = 1; k.blocks_per_split = p->seqlen;   // single pass: never the limit
     k.qk_scale_log2 = p->sm_scale * 1.44269504f;      // flash_atten_full_int8.py:156-157
     *kp = k;
@@ -248,11 +249,6 @@ int run_forward(int variant, const intfa_fwd_params* p, int qk_bytes, int v_byte
     }
     rc = setup_split(p, block_n_for(variant, kp.head_dim), &kp);
     if (rc != INTFA_OK) return rc;
-    // Causal passes of more workgroups than compute units give one workgroup the query blocks i and n-1-i (even counts).  At one
-    // workgroup per compute unit or less the pairs would only halve the number that work: B2 H32 N512 d128 full-int8
-    // 20.5 us in pairs, 15.0 without; B4 H32 N512 21.7 and 21.7; B8 H32 N512 30.6 and 37.6.
-    const int n_mblk = (kp.seqlen + kBlockM - 1) / kBlockM;
-    kp.pair_mblocks = kp.causal && kp.num_splits <= 1 && n_mblk % 2 == 0 && (int64_t)kp.batch * kp.heads * n_mblk > kComputeUnits ? 1 : 0;
     // (the decode-shaped kernels merge; the general ones leave it to the merge kernel)
     const bool merges = decode_kernel_takes(variant, kp);
     if (!merges) kp.ticket = nullptr;

@@ -67,7 +67,6 @@ struct KParams {
     int32_t seqlen_k;                      // number of keys (= seqlen unless the caller passes separate lengths)
     int32_t scale_dtype, causal, num_splits, blocks_per_split;
     int32_t kv_group;                      // query heads per K/V head (1 = every query head has its own K/V)
-    int32_t pair_mblocks;                  // causal single-pass launches: one workgroup takes query blocks i and n-1-i
     int32_t vs_g;                          // blocked V scales: key blocks of the kernel per scale row (0 = scalar V scale)
     int32_t vs_sub;                        // blocked V scales: 2 when a scale row covers 64 keys, half of the 128-key block
     int32_t causal_rows;                   // decode kernel: query positions per folded query head (0 = the row is the position)
@@ -78,6 +77,11 @@ struct KParams {
     int32_t xcd_whole_wgs;                 // workgroups of the K/V heads that are dealt whole to the 8 XCDs (a multiple of 8)
     int32_t xcd_rem_chunk;                 // the remaining heads: consecutive workgroups per XCD (0: dealt one by one)
     FastDiv d_per_kv, d_heads_kv, d_per_head, d_n_split, d_heads, d_kv_group;
+    // causal launches: the K/V heads of an XCD in groups of run_units (the last one run_units_last), query-block-major in each
+    int32_t run_units, run_units_last, run_last_slot;      // run_last_slot: first slot of the last group
+    int32_t rem_wgs;                                       // workgroups of the K/V heads that are not dealt whole
+    int32_t kv_key_bytes;                                  // bytes of one key's K and V rows
+    FastDiv d_run, d_run_heads, d_run_heads_last, d_rem_heads;
 };
 
 // The kernel's own argument block as the epilogues re-read it: the pointer keeps the constant address space, so its
@@ -104,28 +108,62 @@ __device__ __forceinline__ float load_scale(const char* base, int64_t idx, int d
 // When the number of (batch, K/V head) pairs is no multiple of 8, the first 8 * floor(pairs / 8) are dealt whole as above and
 // the workgroups of the remaining pairs, taken in head order, are cut into 8 equal runs, one per XCD: a remaining head's
 // K/V then reaches two or three L2s instead of all eight.
+// Causal launches: query blocks differ in work by a factor of their number, so the order decides how long the last ones run
+// alone.  The K/V heads of an XCD are taken in groups of a few rounds of its workgroup slots; inside a group the heaviest
+// query blocks of all its heads come first (a head's own blocks one after the other leave the last heads' heavy blocks to the
+// end: N 3333, 64 heads on 16 K/V heads, fp16 d128 223 -> 200 us).  The remaining pairs are one such group over all XCDs,
+// ahead of the others: their heavy blocks must not come last either.
 // (All divisors are fixed per launch: fast_div.)
 struct WorkgroupJob { int b, h, hk, rem; };      // batch entry, query head, K/V head, index among the head's workgroups
 __device__ __forceinline__ WorkgroupJob deal_workgroup(const KParams& p, int bid) {
     const int kv_group = p.kv_group;
     const int per_head = p.per_head;
     const int per_kv = per_head * kv_group;              // workgroups per K/V head
-    int kv_lin, r;
-    if (bid < p.xcd_whole_wgs) {
-        const int xcd = bid & 7, slot = bid >> 3;
-        const int q = fast_div(slot, p.d_per_kv);
-        kv_lin = q * 8 + xcd;
-        r = slot - q * per_kv;
+    int kv_lin, hq, rem;
+    if (p.causal) {
+        int idx, first, unit_step, heads;
+        FastDiv d_heads;
+        if (bid >= p.rem_wgs) {
+            const int slot = (bid - p.rem_wgs) >> 3;
+            unit_step = 8;
+            if (slot < p.run_last_slot) {
+                const int g = fast_div(slot, p.d_run);
+                idx = slot - g * p.run_units * per_kv;
+                first = g * p.run_units; heads = p.run_units * kv_group; d_heads = p.d_run_heads;
+            } else {
+                idx = slot - p.run_last_slot;
+                first = fast_div(p.run_last_slot, p.d_per_kv); heads = p.run_units_last * kv_group; d_heads = p.d_run_heads_last;
+            }
+            first = first * 8 + ((bid - p.rem_wgs) & 7);
+        } else {
+            idx = bid;
+            unit_step = 1;
+            first = fast_div(p.xcd_whole_wgs, p.d_per_kv);
+            heads = (p.batch * p.heads_kv - first) * kv_group; d_heads = p.d_rem_heads;
+        }
+        rem = fast_div(idx, d_heads);
+        const int u = idx - rem * heads, unit = fast_div(u, p.d_kv_group);
+        kv_lin = first + unit * unit_step;
+        hq = u - unit * kv_group;
     } else {
-        const int j = bid - p.xcd_whole_wgs;                        // (xcd_whole_wgs is a multiple of 8: j & 7 is the XCD)
-        const int idx = p.xcd_rem_chunk ? (j & 7) * p.xcd_rem_chunk + (j >> 3) : j;
-        const int q = fast_div(idx, p.d_per_kv);
-        kv_lin = fast_div(p.xcd_whole_wgs, p.d_per_kv) + q;
-        r = idx - q * per_kv;
+        int r;
+        if (bid < p.xcd_whole_wgs) {
+            const int xcd = bid & 7, slot = bid >> 3;
+            const int q = fast_div(slot, p.d_per_kv);
+            kv_lin = q * 8 + xcd;
+            r = slot - q * per_kv;
+        } else {
+            const int j = bid - p.xcd_whole_wgs;                        // (xcd_whole_wgs is a multiple of 8: j & 7 is the XCD)
+            const int idx = p.xcd_rem_chunk ? (j & 7) * p.xcd_rem_chunk + (j >> 3) : j;
+            const int q = fast_div(idx, p.d_per_kv);
+            kv_lin = fast_div(p.xcd_whole_wgs, p.d_per_kv) + q;
+            r = idx - q * per_kv;
+        }
+        hq = fast_div(r, p.d_per_head);                  // query head inside the group
+        rem = r - hq * per_head;
     }
     const int bb = fast_div(kv_lin, p.d_heads_kv), hk = kv_lin - bb * p.heads_kv;
-    const int hq = fast_div(r, p.d_per_head);            // query head inside the group
-    return {bb, hk * kv_group + hq, hk, r - hq * per_head};
+    return {bb, hk * kv_group + hq, hk, rem};
 }
 
 // Number of keys of batch entry b: one length for all, or per batch (a cache filled to different lengths), clamped to

@@ -63,7 +63,8 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const int n_split = SPLIT ? p.num_splits : 1;
     const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
     const int rem = wg.rem, head = wg.b * p.heads + wg.h;
-    const int mb = fast_div(rem, p.d_n_split), split = rem - mb * n_split;
+    const int mb_idx = fast_div(rem, p.d_n_split), split = rem - mb_idx * n_split;
+    const int mb = p.causal ? n_mblk - 1 - mb_idx : mb_idx;     // heaviest query blocks first
     const int b = wg.b, h = wg.h;
     const int hk = wg.hk;
 

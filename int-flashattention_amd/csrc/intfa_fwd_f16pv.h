@@ -67,20 +67,12 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
 
     const int n_mblk = (p.seqlen + kBlockM - 1) / kBlockM;      // the last query block may be partial
     const int n_split = SPLIT ? p.num_splits : 1;
-    // Causal single-pass launches pair query block i with query block n-1-i in one workgroup (heavy one first): every
-    // workgroup then walks the same number of key blocks and the launch has no tail of light workgroups.
-    const bool pair = CAUSAL && !SPLIT && p.pair_mblocks != 0;
     const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
     const int rem = wg.rem, head = wg.b * p.heads + wg.h;
     const int half = rem % NHALF;                // column half of this workgroup (0 when the columns are not split)
     const int mb_idx = fast_div(rem / NHALF, p.d_n_split);
     const int split = rem / NHALF - mb_idx * n_split;
-    const int njobs = pair ? 2 : 1;
-#pragma clang loop unroll(disable)
-    for (int job = 0; job < njobs; ++job) {
-    if (job) __syncthreads();                    // every wave is done with the LDS tiles of the first query block
-    int mb = mb_idx;
-    if (CAUSAL) mb = (pair && job) ? mb_idx : n_mblk - 1 - mb_idx;     // heaviest query blocks first
+    const int mb = CAUSAL ? n_mblk - 1 - mb_idx : mb_idx;       // heaviest query blocks first
     const int b = wg.b, h = wg.h;
     const int hk = wg.hk;                     // K/V head of this query head
     // ragged sequence lengths are handled as in the full-int8 kernel (zero-filled copies, masked last block, rows past
@@ -405,7 +397,6 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
                         e_seqlen - row0, lane_e);
     if (q_valid && pe->lse != nullptr && lh == 0 && half == 0) pe->lse[((int64_t)eb * e_heads + eh) * e_seqlen + q_row] = lse;
     }
-    }   // job
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

@@ -65,19 +65,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     // L2; give every XCD whole heads so that the K/V tiles of a head are re-read from one L2.
     const int n_mblk = (p.seqlen + kBlockM - 1) / kBlockM;      // the last query block may be partial
     const int n_split = SPLIT ? p.num_splits : 1;
-    // Causal single-pass launches pair query block i with query block n-1-i in one workgroup (heavy one first): every
-    // workgroup then walks the same number of key blocks and the launch has no tail of light workgroups.
-    const bool pair = CAUSAL && !SPLIT && p.pair_mblocks != 0;
     const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
     const int rem = wg.rem, head = wg.b * p.heads + wg.h;
     const int mb_idx = fast_div(rem, p.d_n_split);
     const int split = rem - mb_idx * n_split;
-    const int njobs = pair ? 2 : 1;
-#pragma clang loop unroll(disable)
-    for (int job = 0; job < njobs; ++job) {
-    if (job) __syncthreads();                    // every wave is done with the LDS tiles of the first query block
-    int mb = mb_idx;
-    if (CAUSAL) mb = (pair && job) ? mb_idx : n_mblk - 1 - mb_idx;     // heaviest query blocks first
+    const int mb = CAUSAL ? n_mblk - 1 - mb_idx : mb_idx;       // heaviest query blocks first
     const int b = wg.b, h = wg.h;
     const int hk = wg.hk;                     // K/V head of this query head
 
@@ -584,7 +576,6 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     out_stage_flush<DV>(stage, pe->out + eb * pe->o_sb + eh * pe->o_sh + (int64_t)row0 * pe->o_sn, pe->o_sn, e_seqlen - row0, lane_e);
     if (q_valid && pe->lse != nullptr && lh == 0) pe->lse[((int64_t)eb * e_heads + eh) * e_seqlen + q_row] = lse;
     }
-    }   // job
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

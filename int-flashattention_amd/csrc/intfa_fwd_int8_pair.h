@@ -47,17 +47,11 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     // ---- block -> (head, m-block, split): whole K/V heads per XCD (as in fwd_full_int8_kernel)
     const int n_mblk = (p.seqlen + kBlockM - 1) / kBlockM;
     const int n_split = SPLIT ? p.num_splits : 1;
-    const bool pair = CAUSAL && !SPLIT && p.pair_mblocks != 0;
     const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
     const int rem = wg.rem, head = wg.b * p.heads + wg.h;
     const int mb_idx = fast_div(rem, p.d_n_split);
     const int split = rem - mb_idx * n_split;
-    const int njobs = pair ? 2 : 1;
-#pragma clang loop unroll(disable)
-    for (int job = 0; job < njobs; ++job) {
-    if (job) __syncthreads();                    // every wave is done with the LDS of the first query block
-    int mb = mb_idx;
-    if (CAUSAL) mb = (pair && job) ? mb_idx : n_mblk - 1 - mb_idx;     // heaviest query blocks first
+    const int mb = CAUSAL ? n_mblk - 1 - mb_idx : mb_idx;       // heaviest query blocks first
     const int b = wg.b, h = wg.h;
     const int hk = wg.hk;
 
@@ -405,7 +399,6 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
                          e_seqlen - row0, lane_e);
     if (q_valid && pe->lse != nullptr && lh == 0 && hf == 0) pe->lse[((int64_t)eb * e_heads + eh) * e_seqlen + q_row] = lse;
     }
-    }   // job
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

@@ -32,7 +32,25 @@ inline KParams finish_mapping(const KParams& kp, int grid) {
     k.heads_kv = kp.heads / kp.kv_group;
     const int per_kv = k.per_head * kp.kv_group, units = kp.batch * k.heads_kv;
     k.xcd_whole_wgs = (units / 8) * 8 * per_kv;
+    k.rem_wgs = grid - k.xcd_whole_wgs;
     k.xcd_rem_chunk = ((units % 8) * per_kv) % 8 == 0 ? (units % 8) * per_kv / 8 : 0;
+    // Causal: groups of K/V heads with two rounds of an XCD's workgroup slots (32 compute units; two workgroups each, four at
+    // head_dim 64; four rounds at head_dim 256, one each) whose K and V come to 9 MB at most, since all of a group's heads are read at
+    // once.  Larger groups lose to the 4 MB L2 (half-int8 B8 H32 N2048 d128: 298 us up to 12 MB, 313 us at 48), smaller ones end
+    // unevenly (full-int8 B4 H32 N4096 d64: 390 us with two heads, 349 with eight).
+    const int xcd_units = units / 8, slots = kp.head_dim == 64 ? 256 : 128;
+    const int by_slots = slots / per_kv, by_bytes = (int)(9000000 / ((int64_t)kp.seqlen_k * kp.kv_key_bytes));
+    int run_units = by_slots < by_bytes ? by_slots : by_bytes;
+    run_units = run_units < xcd_units ? run_units : xcd_units;
+    k.run_units = run_units > 1 ? run_units : 1;
+    const int runs = xcd_units / k.run_units > 0 ? xcd_units / k.run_units : 1;
+    k.run_units_last = xcd_units - (runs - 1) * k.run_units;
+    if (k.run_units_last < 1) k.run_units_last = 1;
+    k.run_last_slot = (runs - 1) * k.run_units * per_kv;
+    k.d_run = make_fast_div(k.run_units * per_kv);
+    k.d_run_heads = make_fast_div(k.run_units * kp.kv_group);
+    k.d_run_heads_last = make_fast_div(k.run_units_last * kp.kv_group);
+    k.d_rem_heads = make_fast_div(units % 8 > 0 ? (units % 8) * kp.kv_group : 1);
     k.d_per_kv = make_fast_div(k.per_head * kp.kv_group);
     k.d_heads_kv = make_fast_div(k.heads_kv);
     k.d_per_head = make_fast_div(k.per_head);
@@ -42,11 +60,11 @@ inline KParams finish_mapping(const KParams& kp, int grid) {
     return k;
 }
 
-// One workgroup per (batch, head, 128-row query block, split); causal single-pass launches pair the query blocks.
+// One workgroup per (batch, head, 128-row query block, split).
 // `column_halves`: workgroups per query block (2 where a kernel splits the output columns over two workgroups).
 template <typename K> inline int launch_kernel(K kernel, const KParams& kp, hipStream_t stream, int threads = kThreads,
                                                int column_halves = 1) {
-    const int grid = kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM) * kp.num_splits / (kp.pair_mblocks ? 2 : 1) * column_halves;
+    const int grid = kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM) * kp.num_splits * column_halves;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, finish_mapping(kp, grid));
     return (int)hipGetLastError();
 }

@@ -414,6 +414,7 @@ __device__ __forceinline__ float hide_past(float v, int last, int k_r) {
 // be scheduled into it, and a single s_nop closes the last round before the words can be consumed.
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ v4i requant_p_reference16(const float (&p)[16]) {
     unsigned hb[8];
 #pragma unroll

@@ -29,30 +29,91 @@ __device__ __forceinline__ v8bf pack_p_bf16(const float* e) {
     return r;
 }
 
+// Epilogue of both kernels: a wave's 32 rows, normalised, to the output (16-bit, through LDS: whole lines per store instruction) or,
+// SPLIT, to the split's fp32 partials; the log-sum-exp.
+template <int D, int IO_DT, bool SPLIT>
+__device__ __forceinline__ void f16pv_store(char* smem, const v16f (&o_acc)[D / 32], float m_run, float l_run, bool any_block, int head, int split,
+                                            int row0, int wave, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int DT = D / 32;
+    const KernargPtr pe = kernarg_block();
+    const int e_heads = pe->heads, e_seqlen = pe->seqlen;
+    const int lq = lane & 31, lh = lane >> 5, q_row = row0 + lq;
+    const bool q_valid = q_row < e_seqlen;
+    const int eb = fast_div(head, pe->d_heads), eh = head - eb * e_heads;
+    const float l_tot = half_pair_sum(l_run);
+    // (no key at all - an empty cache entry - gives zeros and lse = -inf instead of 0 / 0)
+    const bool any_key = any_block && m_run > -INFINITY;      // (a causal row above the first key sees nothing)
+    const float inv = any_key ? 1.f / l_tot : 0.f;
+    const float lse = any_key ? m_run + __builtin_log2f(l_tot) : -INFINITY;
+    if (SPLIT) {
+        const int64_t row = ((int64_t)(split * pe->batch + eb) * e_heads + eh) * e_seqlen + q_row;
+        float* op = pe->o_part + row * D;
+        // a row contributes nothing to this split when the split's range is empty for its workgroup, or when every
+        // block of the range lies above the row's diagonal (its wave skipped them: the running max is still -inf)
+        const bool seen = any_block && m_run > -INFINITY;
+        if (q_valid) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4) {
+                    v4f o;
+#pragma unroll
+                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[dt][4 * a4 + b4] * inv : 0.f;
+                    *(v4f*)(op + 32 * dt + 8 * a4 + 4 * lh) = o;
+                }
+            if (lh == 0) pe->lse_part[row] = seen ? lse : -INFINITY;
+        }
+        return;
+    }
+    {
+    // the tiles are dead once every wave is here
+    __syncthreads();
+    // (an opaque copy of the lane index: the staging addresses depend on the lane only and would otherwise be computed
+    // ahead of the main loop and held in registers through it)
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));
+    const int lq_e = lane_e & 31, lh_e = lane_e >> 5;
+    char* stage = smem + wave * OutStage<D>::BYTES;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4) {
+            const int d0 = 32 * dt + 8 * a4 + 4 * lh_e;
+            if (IO_DT == 0) {
+                v4h o;
+#pragma unroll
+                for (int b4 = 0; b4 < 4; ++b4) o[b4] = (_Float16)(any_key ? o_acc[dt][4 * a4 + b4] * inv : 0.f);
+                out_stage_put<D>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
+            } else {
+                v4s o;
+#pragma unroll
+                for (int b4 = 0; b4 < 4; ++b4) o[b4] = f32_to_bf16(any_key ? o_acc[dt][4 * a4 + b4] * inv : 0.f);
+                out_stage_put<D>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
+            }
+        }
+    out_stage_flush<D>(stage, pe->out + eb * pe->o_sb + eh * pe->o_sh + (int64_t)row0 * pe->o_sn, pe->o_sn,
+                        e_seqlen - row0, lane_e);
+    if (q_valid && pe->lse != nullptr && lh == 0) pe->lse[((int64_t)eb * e_heads + eh) * e_seqlen + q_row] = lse;
+    }
+#endif  // __HIP_DEVICE_COMPILE__
+}
+
 // QK_INT8: int8 Q/K with scales (half-int8) or 16-bit Q/K (fp16/bf16 variant).  IO_DT: type of V, P and the output
 // (and of Q/K when !QK_INT8): 0 fp16, 1 bf16.
-// Output columns one workgroup produces.  At head_dim 256 a full-width workgroup needs 128 fp32 output registers per lane:
-// one wave per SIMD and spills.  This kernel can split the columns over two workgroups that each redo Q K^T and the
-// softmax and multiply P with their half of V; the library does not instantiate it at head_dim 256 any more -
-// fwd_f16pv_pair_kernel (intfa_fwd_f16pv_pair.h) divides the work between two waves of one workgroup instead.
-template <int D> struct F16PvGeom {
-    static constexpr int DV = D <= 128 ? D : 128;
-    static constexpr int NHALF = D / DV;
-};
-
-// (16-bit K tiles at head_dim 256 are 32 KiB each: double-buffered beside the V tiles they leave room for one workgroup
-// per compute unit, whatever the register count)
+// Head_dim 64, in grids past two workgroups per compute unit (otherwise, and at head_dim 128, fwd_f16pv_pipe_kernel; head_dim 256:
+// fwd_f16pv_pair_kernel).  Three waves per SIMD hide what the pipeline of the other kernel hides with registers: the
+// instances need 143-168 registers; 33 KiB / 25 KiB of LDS allow it.  The pipelined
+// form needs 187-216, two waves: half-int8 B4 H32 N4096 583 us here, 630 us there.
 template <bool QK_INT8, int D, bool CAUSAL, int IO_DT, bool SPLIT>
-// (head_dim 64: three waves per SIMD - the non-causal instances need 140-146 registers, the masked ones are held to 168
-// and spill 7-9; 33 KiB / 25 KiB of LDS allow it)
-__global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 64 ? 3 : 2)) fwd_f16pv_kernel(const KParams p) {
+__global__ void __launch_bounds__(kThreads, 3) fwd_f16pv_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    static_assert(D == 64, "the registers of head_dim 64");
     constexpr int BN = kBlockN16, NST = BN / 32;
     constexpr int QB = QK_INT8 ? 1 : 2;               // bytes per Q/K element
-    constexpr int DV = F16PvGeom<D>::DV, NHALF = F16PvGeom<D>::NHALF;
-    constexpr int KROW = D * QB, VROW = DV * 2;       // bytes per K row / per V row of this workgroup's columns
+    constexpr int KROW = D * QB, VROW = D * 2;        // bytes per K row / per V row
     constexpr int KS = KROW / 32;                     // MFMA k-steps of S^T (32 bytes of a row each)
-    constexpr int DT = DV / 32;                       // 32-wide output tiles
+    constexpr int DT = D / 32;                        // 32-wide output tiles
     constexpr int KT = BN * KROW, VT = BN * VROW;
     constexpr int KCH = KROW / 16, VCH = VROW / 16;
     constexpr int OFF_KS = 0;
@@ -69,9 +130,8 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
     const int n_split = SPLIT ? p.num_splits : 1;
     const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
     const int rem = wg.rem, head = wg.b * p.heads + wg.h;
-    const int half = rem % NHALF;                // column half of this workgroup (0 when the columns are not split)
-    const int mb_idx = fast_div(rem / NHALF, p.d_n_split);
-    const int split = rem / NHALF - mb_idx * n_split;
+    const int mb_idx = fast_div(rem, p.d_n_split);
+    const int split = rem - mb_idx * n_split;
     const int mb = CAUSAL ? n_mblk - 1 - mb_idx : mb_idx;       // heaviest query blocks first
     const int b = wg.b, h = wg.h;
     const int hk = wg.hk;                     // K/V head of this query head
@@ -106,7 +166,7 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
 
     // ---- global -> LDS copies
     const char* Kg = p.k + b * p.k_sb + hk * p.k_sh;
-    const char* Vg = p.v + b * p.v_sb + hk * p.v_sh + half * DV * 2;
+    const char* Vg = p.v + b * p.v_sb + hk * p.v_sh;
     const v4i k_rsrc = make_rsrc(Kg, (uint32_t)((seqlen_k - 1) * p.k_sn + KROW));
     const v4i v_rsrc = make_rsrc(Vg, (uint32_t)((seqlen_k - 1) * p.v_sn + VROW));
     const uint32_t k_sn = (uint32_t)p.k_sn, v_sn = (uint32_t)p.v_sn;
@@ -255,7 +315,7 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
         }
         const float m_new = m_run;
         // -------- pass 2: P = exp2(x*qsc - m), row sum, cast to the 16-bit type
-        // (head_dim 64: a sum per sub-tile, then their sum - the order of the decode-shaped kernel, whose waves hold a sub-tile each;
+        // (a sum per sub-tile, then their sum - the order of the decode-shaped kernel, whose waves hold a sub-tile each;
         // both give the same bits)
         float lsum = 0.f, lfirst = 0.f;
         v4i pf[NST][2];                                   // B operands: 8 x 16-bit per 16-key step
@@ -264,11 +324,11 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
             if (DIAG && st > gw) continue;
             __builtin_amdgcn_sched_barrier(0);
             float e[16];
-            if (D == 64 && st == 1) lfirst = lsum;
+            if (st == 1) lfirst = lsum;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 e[r] = fast_exp2(fmaf(t[st][r], qsc, -m_new));
-                lsum = r == 0 && (st == 0 || D == 64) ? e[r] : lsum + e[r];
+                lsum = r == 0 ? e[r] : lsum + e[r];
             }
 #pragma unroll
             for (int u = 0; u < 2; ++u)
@@ -277,7 +337,7 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
         }
         {
 #pragma clang fp contract(off)
-            l_run += D == 64 ? lfirst + lsum : lsum;
+            l_run += lfirst + lsum;
         }
         // -------- O^T[d, q] += V^T[d, key] P^T[key, q] (the fp32 accumulators of the MFMAs are the running output)
         __builtin_amdgcn_sched_barrier(0);
@@ -336,67 +396,8 @@ __global__ void __launch_bounds__(kThreads, D > 128 ? (QK_INT8 ? 2 : 1) : (D == 
         }
     }
 
-    // ---- epilogue
-    const KernargPtr pe = kernarg_block();
-    const int e_heads = pe->heads, e_seqlen = pe->seqlen;
-    const int eb = fast_div(head, pe->d_heads), eh = head - eb * e_heads;
-    const float l_tot = half_pair_sum(l_run);
-    // (no key at all - an empty cache entry - gives zeros and lse = -inf instead of 0 / 0)
-    const bool any_key = nb_begin < nb_end && m_run > -INFINITY;      // (a causal row above the first key sees nothing)
-    const float inv = any_key ? 1.f / l_tot : 0.f;
-    const float lse = any_key ? m_run + __builtin_log2f(l_tot) : -INFINITY;
-    if (SPLIT) {
-        const int64_t row = ((int64_t)(split * pe->batch + eb) * e_heads + eh) * e_seqlen + q_row;
-        float* op = pe->o_part + row * D + half * DV;
-        // a row contributes nothing to this split when the split's range is empty for its workgroup, or when every
-        // block of the range lies above the row's diagonal (its wave skipped them: the running max is still -inf)
-        const bool seen = nb_begin < nb_end && m_run > -INFINITY;
-        if (q_valid) {
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int a4 = 0; a4 < 4; ++a4) {
-                    v4f o;
-#pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[dt][4 * a4 + b4] * inv : 0.f;
-                    *(v4f*)(op + 32 * dt + 8 * a4 + 4 * lh) = o;
-                }
-            if (lh == 0 && half == 0) pe->lse_part[row] = seen ? lse : -INFINITY;
-        }
-        return;
-    }
-    {
-    // 16-bit rows go out through LDS (whole lines per store instruction); the tiles are dead once every wave is here
-    static_assert(4 * OutStage<DV>::BYTES <= LDS_BYTES, "output staging fits the tile memory");
-    __syncthreads();
-    // (an opaque copy of the lane index: the staging addresses depend on the lane only and would otherwise be computed
-    // ahead of the main loop and held in registers through it)
-    int lane_e = lane;
-    asm volatile("" : "+v"(lane_e));
-    const int lq_e = lane_e & 31, lh_e = lane_e >> 5;
-    char* stage = smem + wave * OutStage<DV>::BYTES;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int a4 = 0; a4 < 4; ++a4) {
-            const int d0 = 32 * dt + 8 * a4 + 4 * lh_e;
-            if (IO_DT == 0) {
-                v4h o;
-#pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) o[b4] = (_Float16)(any_key ? o_acc[dt][4 * a4 + b4] * inv : 0.f);
-                out_stage_put<DV>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
-            } else {
-                v4s o;
-#pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) o[b4] = f32_to_bf16(any_key ? o_acc[dt][4 * a4 + b4] * inv : 0.f);
-                out_stage_put<DV>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
-            }
-        }
-    const int row0 = mb * kBlockM + wave * 32;
-    out_stage_flush<DV>(stage, pe->out + eb * pe->o_sb + eh * pe->o_sh + (int64_t)row0 * pe->o_sn + half * DV * 2, pe->o_sn,
-                        e_seqlen - row0, lane_e);
-    if (q_valid && pe->lse != nullptr && lh == 0 && half == 0) pe->lse[((int64_t)eb * e_heads + eh) * e_seqlen + q_row] = lse;
-    }
+    static_assert(4 * OutStage<D>::BYTES <= LDS_BYTES, "output staging fits the tile memory");
+    f16pv_store<D, IO_DT, SPLIT>(smem, o_acc, m_run, l_run, nb_begin < nb_end, head, split, mb * kBlockM + wave * 32, wave, lane);
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

@@ -61,10 +61,8 @@ inline KParams finish_mapping(const KParams& kp, int grid) {
 }
 
 // One workgroup per (batch, head, 128-row query block, split).
-// `column_halves`: workgroups per query block (2 where a kernel splits the output columns over two workgroups).
-template <typename K> inline int launch_kernel(K kernel, const KParams& kp, hipStream_t stream, int threads = kThreads,
-                                               int column_halves = 1) {
-    const int grid = kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM) * kp.num_splits * column_halves;
+template <typename K> inline int launch_kernel(K kernel, const KParams& kp, hipStream_t stream, int threads = kThreads) {
+    const int grid = kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM) * kp.num_splits;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, finish_mapping(kp, grid));
     return (int)hipGetLastError();
 }

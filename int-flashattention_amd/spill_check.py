@@ -26,39 +26,67 @@ _EXEC_NARROW = re.compile(r"^\s+(s_and_saveexec_b64|s_or_saveexec_b64|s_and_b64 
 _SPILL = re.compile(r"^\s+(scratch_|buffer_)\w+.*Folded (Spill|Reload)")
 
 
+_BRANCH = re.compile(r"^\s+s_c?branch\w*\s+(\.LBB\d+_\d+)")
+_NO_FALLTHROUGH = ("s_branch", "s_endpgm", "s_setpc_b64")
+
+
 def scan(asm: str) -> List[str]:
-    """Returns one line per suspicious spill / reload in the assembly text of one translation unit."""
+    """Returns one line per suspicious spill / reload in the assembly text of one translation unit.
+
+    Which blocks are entered with a narrowed mask follows the branches, not the order of the text: a block that stands behind an
+    unconditional branch, inside or after a masked region, is entered from wherever its label is named."""
     findings: List[str] = []
     kernel = "?"
-    block: List[tuple] = []          # (line number, text) of the current basic block
-    narrowed_at = 0                    # line of the last exec-narrowing instruction not yet undone (linear order)
+    blocks: List[dict] = []            # basic blocks of the current kernel: label, [(line number, text)], last opcode
 
-    def close_block():
-        restore = next((i for i, (_, t) in enumerate(block) if _EXEC_RESTORE.match(t)), None)
-        if restore is not None:
-            for n, t in block[:restore]:
+    def close_kernel():
+        by_label = {b["label"]: k for k, b in enumerate(blocks) if b["label"]}
+        entry = [0] * len(blocks)      # line of an exec-narrowing instruction that may be in force on entry, 0: none
+        work = list(range(len(blocks)))
+        leaves = [0] * len(blocks)
+        while work:
+            k = work.pop(0)
+            state = entry[k]
+            for n, t in blocks[k]["lines"]:
+                if _EXEC_NARROW.match(t):
+                    state = n
+                elif _EXEC_RESTORE.match(t):
+                    state = 0
+            leaves[k] = state
+            last = blocks[k]["lines"][-1][1] if blocks[k]["lines"] else ""
+            nxt = [by_label[m.group(1)] for m in [_BRANCH.match(last)] if m and m.group(1) in by_label]
+            if not (last.split() and last.split()[0] in _NO_FALLTHROUGH) and k + 1 < len(blocks):
+                nxt.append(k + 1)
+            for j in nxt:
+                if state and not entry[j]:
+                    entry[j] = state
+                    if j not in work:
+                        work.append(j)
+        for k, b in enumerate(blocks):
+            restore = next((i for i, (_, t) in enumerate(b["lines"]) if _EXEC_RESTORE.match(t)), None)
+            state = entry[k]
+            for i, (n, t) in enumerate(b["lines"]):
                 if _SPILL.match(t):
-                    findings.append(f"{kernel}: line {n}: `{t.strip()}` runs before exec is restored at line {block[restore][0]}")
-        block.clear()
+                    if restore is not None and i < restore:
+                        findings.append(f"{kernel}: line {n}: `{t.strip()}` runs before exec is restored at line {b['lines'][restore][0]}")
+                    if state and "Folded Spill" in t:
+                        findings.append(f"{kernel}: line {n}: `{t.strip()}` stores while exec is narrowed (since line {state})")
+                if _EXEC_NARROW.match(t):
+                    state = n
+                elif _EXEC_RESTORE.match(t):
+                    state = 0
+        blocks.clear()
 
     for n, line in enumerate(asm.split("\n"), 1):
         m = _KERNEL.match(line)
         if m:
-            close_block()
-            kernel, narrowed_at = m.group(1), 0
+            close_kernel()
+            kernel = m.group(1)
             continue
-        if _LABEL.match(line):
-            close_block()
-        block.append((n, line))
-        if _EXEC_NARROW.match(line):
-            narrowed_at = n
-        elif _EXEC_RESTORE.match(line):
-            narrowed_at = 0
-        elif narrowed_at and _SPILL.match(line) and "Folded Spill" in line:
-            findings.append(f"{kernel}: line {n}: `{line.strip()}` stores while exec is narrowed (since line {narrowed_at})")
+        if _LABEL.match(line) or not blocks or blocks[-1]["done"]:
+            blocks.append({"label": line.split(":")[0] if _LABEL.match(line) else None, "lines": [], "done": False})
+        blocks[-1]["lines"].append((n, line))
         if _BLOCK_END.match(line):
-            close_block()
-            if line.split()[0] in ("s_endpgm", "s_setpc_b64"):
-                narrowed_at = 0          # nothing falls through: what follows is reached by branches, each with its own mask
-    close_block()
+            blocks[-1]["done"] = True
+    close_kernel()
     return findings

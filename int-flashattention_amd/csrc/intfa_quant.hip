@@ -55,7 +55,7 @@ template <int DT> __device__ __forceinline__ float quotient16(uint16_t xb, RowDi
     return to_f32<DT>(from_f32<DT>(q));
 }
 
-template <int DT> __device__ __forceinline__ void quant_store8(const v4i raw, RowDivisor scale, char* dst) {
+template <int DT> __device__ __forceinline__ v2i quant8(const v4i raw, RowDivisor scale) {
     int out[2];
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
@@ -67,7 +67,7 @@ template <int DT> __device__ __forceinline__ void quant_store8(const v4i raw, Ro
         }
         out[w] = (int)pack4_rne(q[0], q[1], q[2], q[3]);
     }
-    *(v2i*)dst = (v2i){out[0], out[1]};
+    return (v2i){out[0], out[1]};
 }
 
 __device__ __forceinline__ uint32_t amax8(const v4i raw) {
@@ -93,6 +93,17 @@ struct QuantParams {
 // ---- per token: LPR = d / 8 lanes per row, reduction of the row maximum inside those lanes
 constexpr int kRowsInFlight = 8;    // independent 16-byte loads a lane has in flight (HBM latency x bandwidth needs several)
 
+// A workgroup of a streaming launch (per token; maximum and quantisation of large slices) takes up to this many consecutive steps of
+// 256 / LPR rows: 16 KiB of input in one piece, all loads at once, and no further round.  B4 H32 N4096 d128 fp16 (134 MB in, 67 MB
+// out), us: a persistent grid of 2048 workgroups whose eight loads lie 8 MB apart 50.5; the same loads in one 32 KiB piece and no
+// second round 42.0; 16 KiB pieces 37.8; and read and written past the caches (non-temporal: each line is touched once) 33.5,
+// 6.0 TB/s (a copy of the same traffic without arithmetic: 34.7).
+constexpr int kStreamSteps = 4;
+__device__ __forceinline__ void store_stream(v2i v, char* a) {
+    __builtin_nontemporal_store(v, (v2i*)a);
+}
+__device__ __forceinline__ v4i load_stream(const char* a) { return __builtin_nontemporal_load((const v4i*)a); }
+
 // rows are numbered (batch, head, position) in that order; the count fits 31 bits (checked on the host), so the index
 // arithmetic is 32-bit
 __device__ __forceinline__ const char* row_ptr(const QuantParams& p, uint32_t row, int sub, uint32_t* bh_out) {
@@ -102,21 +113,23 @@ __device__ __forceinline__ const char* row_ptr(const QuantParams& p, uint32_t ro
     return p.x + b * p.sb + h * p.sh + n * p.sn + sub * 16;
 }
 
-template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_pertoken_kernel(const QuantParams p) {
+template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_pertoken_kernel(const QuantParams p, int steps) {
     constexpr int RPB = 256 / LPR;                       // rows per workgroup step
     const int sub = threadIdx.x % LPR, rl = threadIdx.x / LPR;
-    const uint32_t step = gridDim.x * RPB, rows = (uint32_t)p.rows;
-    for (uint32_t row0 = blockIdx.x * RPB + rl; row0 < rows; row0 += step * kRowsInFlight) {
-        v4i raw[kRowsInFlight];
+    const uint32_t begin = blockIdx.x * (uint32_t)(RPB * steps), end = begin + RPB * steps;
+    const uint32_t rows = end < (uint32_t)p.rows ? end : (uint32_t)p.rows;
+    for (uint32_t row0 = begin + rl; row0 - rl < rows; row0 += RPB * kStreamSteps) {
+        v4i raw[kStreamSteps];
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
-            const uint32_t row = row0 + u * step;
+        for (int u = 0; u < kStreamSteps; ++u) {
+            const uint32_t row = row0 + u * RPB;
             uint32_t bh;
-            raw[u] = row < rows ? *(const v4i*)row_ptr(p, row, sub, &bh) : (v4i){0, 0, 0, 0};
+            raw[u] = row < rows ? load_stream(row_ptr(p, row, sub, &bh)) : (v4i){0, 0, 0, 0};
         }
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
-            const uint32_t row = row0 + u * step;
+        for (int u = 0; u < kStreamSteps; ++u) {
+            const uint32_t row = row0 + u * RPB;
+            if (row - rl >= rows) break;
             uint32_t m = amax8(raw[u]);
 #pragma unroll
             for (int off = LPR / 2; off > 0; off >>= 1) {
@@ -126,7 +139,7 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_pertoken
             if (row >= rows) continue;
             const uint16_t sbits = from_f32<DT>(to_f32<DT>((uint16_t)m) / 127.0f);
             if (sub == 0) ((uint16_t*)p.scale)[row] = sbits;
-            quant_store8<DT>(raw[u], make_divisor(to_f32<DT>(sbits)), p.q8 + (int64_t)row * p.head_dim + sub * 8);
+            store_stream(quant8<DT>(raw[u], make_divisor(to_f32<DT>(sbits))), p.q8 + (int64_t)row * p.head_dim + sub * 8);
         }
     }
 }
@@ -179,7 +192,7 @@ template <int DT, int LPR> __global__ void __launch_bounds__(kSliceThreads) quan
 #pragma unroll
     for (int u = 0; u < kRowsInFlight; ++u) {
         const int n = rl + u * RPB;
-        if (n < p.seqlen) quant_store8<DT>(raw[u], d, dst + (int64_t)n * p.head_dim);
+        if (n < p.seqlen) *(v2i*)(dst + (int64_t)n * p.head_dim) = quant8<DT>(raw[u], d);
     }
 }
 
@@ -200,15 +213,15 @@ template <int LPR> __global__ void __launch_bounds__(256) quant_slice_amax_kerne
     const char* base = p.x + b * p.sb + h * p.sh + sub * 16;
     const int n_lo = chunk * rows, n_hi = n_lo + rows < p.seqlen ? n_lo + rows : p.seqlen;
     uint32_t m = 0;
-    for (int n0 = n_lo + rl; n0 < n_hi; n0 += RPB * kRowsInFlight) {
-        v4i raw[kRowsInFlight];
+    for (int n0 = n_lo + rl; n0 < n_hi; n0 += RPB * kStreamSteps) {
+        v4i raw[kStreamSteps];
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
+        for (int u = 0; u < kStreamSteps; ++u) {
             const int n = n0 + u * RPB;
-            raw[u] = n < n_hi ? *(const v4i*)(base + (int64_t)n * p.sn) : (v4i){0, 0, 0, 0};
+            raw[u] = n < n_hi ? *(const v4i*)(base + (int64_t)n * p.sn) : (v4i){0, 0, 0, 0};      // (read again below, from the caches if it fits)
         }
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
+        for (int u = 0; u < kStreamSteps; ++u) {
             const uint32_t r = amax8(raw[u]);
             m = m > r ? m : r;
         }
@@ -227,18 +240,14 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_slice_ap
     const char* base = p.x + b * p.sb + h * p.sh + sub * 16;
     char* dst = p.q8 + (int64_t)bh * p.seqlen * p.head_dim + sub * 8;
     const int n_lo = chunk * rows, n_hi = n_lo + rows < p.seqlen ? n_lo + rows : p.seqlen;
-    uint32_t m = 0;
-    for (int i = threadIdx.x; i < parts; i += 256) {
-        const uint32_t a = p.amax[bh * parts + i];
-        m = m > a ? m : a;
-    }
+    const uint32_t m = (int)threadIdx.x < parts ? p.amax[bh * parts + threadIdx.x] : 0u;
     RowDivisor d = {0.f, 0.f};
-    for (int n0 = n_lo + rl; n0 - rl < n_hi; n0 += RPB * kRowsInFlight) {
-        v4i raw[kRowsInFlight];
+    for (int n0 = n_lo + rl; n0 - rl < n_hi; n0 += RPB * kStreamSteps) {
+        v4i raw[kStreamSteps];
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
+        for (int u = 0; u < kStreamSteps; ++u) {
             const int n = n0 + u * RPB;
-            raw[u] = n < n_hi ? *(const v4i*)(base + (int64_t)n * p.sn) : (v4i){0, 0, 0, 0};
+            raw[u] = n < n_hi ? load_stream(base + (int64_t)n * p.sn) : (v4i){0, 0, 0, 0};
         }
         if (n0 - rl == n_lo) {                     // (the first rows are under way)
             const uint16_t sbits = from_f32<DT>(to_f32<DT>((uint16_t)block_max<256>(m)) / 127.0f);
@@ -246,22 +255,35 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_slice_ap
             d = make_divisor(to_f32<DT>(sbits));
         }
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
+        for (int u = 0; u < kStreamSteps; ++u) {
             const int n = n0 + u * RPB;
-            if (n < n_hi) quant_store8<DT>(raw[u], d, dst + (int64_t)n * p.head_dim);
+            if (n < n_hi) store_stream(quant8<DT>(raw[u], d), dst + (int64_t)n * p.head_dim);
         }
     }
 }
 
-// Chunks of a slice: about 8 workgroups per compute unit over all slices, whole steps of `rpb` rows each.
-int slice_chunks(int slices, int seqlen, int rpb) {
-    const int steps = (seqlen + rpb - 1) / rpb, want = (256 * 8 + slices - 1) / slices;
-    return steps < want ? steps : want;
+// Steps of 256 / LPR rows per workgroup of a streaming launch: one while more would leave fewer than eight workgroups per compute
+// unit; more than kStreamSteps, in rounds, where a grid would exceed what a launch may have.
+int stream_steps(int64_t steps) {
+    const int64_t fill = steps / (256 * 8), cap = steps >> 22;
+    const int64_t n = fill < kStreamSteps ? fill : kStreamSteps;
+    return (int)(n < 1 ? 1 : (n > cap ? n : cap + 1));
+}
+
+// Parts of a slice for the maximum: pieces as above, as long as there are no more than one for each thread that reduces them.
+int slice_parts(int slices, int seqlen, int rpb, int* rows) {
+    const int steps = (seqlen + rpb - 1) / rpb;
+    int take = stream_steps((int64_t)steps * slices);
+    if (steps > take * 256) take = (steps + 255) / 256;
+    *rows = take * rpb;
+    return (steps + take - 1) / take;
 }
 
 // ---- per (batch, head, block of rows, channel): fp32 scales, the layout of the V scales of the reference's CUDA
 // kernel (csrc/flash_fwd_kernel_full_qi8.h:156-160).  One workgroup owns one block of rows: column maxima through LDS
-// atomics, then a second sweep over the block (served by the cache) that divides and rounds in fp32.
+// atomics, then the block divided and rounded in fp32 - out of registers when its rows fit the loads a workgroup has in flight
+// (32 KiB: 128 rows of head_dim 128; each line then moves once, past the caches: B4 H32 N4096 d128 41.6 us with two sweeps, 33.3 with one), else in a second
+// sweep served by the cache.
 template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_blockchan_kernel(const QuantParams p, int block, int nblk,
                                                                                          float* scale_out) {
     constexpr int RPB = 256 / LPR;
@@ -274,13 +296,18 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_blockcha
     for (int i = threadIdx.x; i < LPR * 8; i += 256) smax[i] = 0u;
     __syncthreads();
     uint32_t m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int n0 = n_lo + rl; n0 < n_hi; n0 += RPB * kRowsInFlight) {
-        v4i raw[kRowsInFlight];
+    const bool one_sweep = block <= RPB * kRowsInFlight;
+    v4i raw[kRowsInFlight];
+    auto load_rows = [&](int n0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < kRowsInFlight; ++u) {
             const int n = n0 + u * RPB;
-            raw[u] = n < n_hi ? *(const v4i*)(base + (int64_t)n * p.sn) : (v4i){0, 0, 0, 0};
+            const char* a = base + (int64_t)n * p.sn;
+            raw[u] = n >= n_hi ? (v4i){0, 0, 0, 0} : (one_sweep ? load_stream(a) : *(const v4i*)a);
         }
+    };
+    for (int n0 = n_lo + rl; n0 < n_hi; n0 += RPB * kRowsInFlight) {
+        load_rows(n0);
 #pragma unroll
         for (int u = 0; u < kRowsInFlight; ++u)
 #pragma unroll
@@ -309,12 +336,7 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_blockcha
     }
     char* qbase = p.q8 + (int64_t)bh * p.seqlen * p.head_dim + sub * 8;
     for (int n0 = n_lo + rl; n0 < n_hi; n0 += RPB * kRowsInFlight) {
-        v4i raw[kRowsInFlight];
-#pragma unroll
-        for (int u = 0; u < kRowsInFlight; ++u) {
-            const int n = n0 + u * RPB;
-            raw[u] = n < n_hi ? *(const v4i*)(base + (int64_t)n * p.sn) : (v4i){0, 0, 0, 0};
-        }
+        if (!one_sweep) load_rows(n0);
 #pragma unroll
         for (int u = 0; u < kRowsInFlight; ++u) {
             const int n = n0 + u * RPB;
@@ -335,7 +357,7 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_blockcha
                 }
                 out[w2] = (int)pack4_rne(q[0], q[1], q[2], q[3]);
             }
-            *(v2i*)(qbase + (int64_t)n * p.head_dim) = (v2i){out[0], out[1]};
+            store_stream((v2i){out[0], out[1]}, qbase + (int64_t)n * p.head_dim);
         }
     }
 }
@@ -442,7 +464,7 @@ template <int DT, int LPR, bool IS_V> __device__ __forceinline__ void kv_append_
                 *(v2i*)dst = (v2i){out[0], out[1]};
             } else {
                 if (sub == 0) ((uint16_t*)s.scale)[b * s.sb + h * s.sh + pos * s.sn] = sbits;
-                quant_store8<DT>(raw[u], d, dst);
+                *(v2i*)dst = quant8<DT>(raw[u], d);
             }
         }
     }
@@ -474,9 +496,12 @@ int intfa_quant_pertoken(const void* x, int64_t stride_b, int64_t stride_h, int6
     const int rc = check(x, q8, scale, stride_b, stride_h, stride_n, batch, heads, seqlen, head_dim, dtype, &qp);
     if (rc != INTFA_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
-#define INTFA_CALL(LPR) do { const int g = grid_for(qp.rows, 256 / LPR); \
-        if (dtype == INTFA_F16) hipLaunchKernelGGL((quant_pertoken_kernel<0, LPR>), dim3(g), dim3(256), 0, st, qp); \
-        else hipLaunchKernelGGL((quant_pertoken_kernel<1, LPR>), dim3(g), dim3(256), 0, st, qp); } while (0)
+    const int rpb = 256 / (head_dim / 8);
+    const int64_t all_steps = (qp.rows + rpb - 1) / rpb;
+    const int steps = stream_steps(all_steps), g = (int)((all_steps + steps - 1) / steps);
+#define INTFA_CALL(LPR) do { \
+        if (dtype == INTFA_F16) hipLaunchKernelGGL((quant_pertoken_kernel<0, LPR>), dim3(g), dim3(256), 0, st, qp, steps); \
+        else hipLaunchKernelGGL((quant_pertoken_kernel<1, LPR>), dim3(g), dim3(256), 0, st, qp, steps); } while (0)
     INTFA_LPR_SWITCH(head_dim, INTFA_CALL)
 #undef INTFA_CALL
     return (int)hipGetLastError();
@@ -488,7 +513,8 @@ size_t intfa_quant_pertensor_workspace_bytes(int32_t batch, int32_t heads) {
 
 size_t intfa_quant_pertensor_parts_workspace_bytes(int32_t batch, int32_t heads, int32_t seqlen, int32_t head_dim) {
     if (batch <= 0 || heads <= 0 || seqlen <= 0 || head_dim < 16 || head_dim > 256) return 0;
-    return (size_t)batch * heads * slice_chunks(batch * heads, seqlen, 256 / (head_dim / 8)) * sizeof(uint32_t);
+    int rows;
+    return (size_t)batch * heads * slice_parts(batch * heads, seqlen, 256 / (head_dim / 8), &rows) * sizeof(uint32_t);
 }
 
 int intfa_quant_pertensor(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_n, void* q8, void* scale,
@@ -511,16 +537,16 @@ int intfa_quant_pertensor(const void* x, int64_t stride_b, int64_t stride_h, int
         return (int)hipGetLastError();
     }
     const int rpb = 256 / (head_dim / 8);
-    int chunks = slice_chunks(slices, seqlen, rpb);
-    const int rows = ((seqlen + chunks - 1) / chunks + rpb - 1) / rpb * rpb;
-    chunks = (seqlen + rows - 1) / rows;
+    int rows;
+    const int chunks = slice_parts(slices, seqlen, rpb, &rows);
     const int parts = workspace_bytes >= (size_t)slices * chunks * sizeof(uint32_t) ? chunks : 1;
-    const FastDiv d_chunks = make_fast_div(chunks);
+    const int steps = (seqlen + rpb - 1) / rpb, rows2 = stream_steps((int64_t)steps * slices) * rpb, chunks2 = (seqlen + rows2 - 1) / rows2;
+    const FastDiv d_chunks = make_fast_div(chunks), d_chunks2 = make_fast_div(chunks2);
     if (parts < chunks) hipLaunchKernelGGL(quant_clear_kernel, dim3((slices + 255) / 256), dim3(256), 0, st, qp.amax, slices);
 #define INTFA_CALL(LPR) do { \
         hipLaunchKernelGGL((quant_slice_amax_kernel<LPR>), dim3(slices * chunks), dim3(256), 0, st, qp, chunks, rows, parts, d_chunks); \
-        if (dtype == INTFA_F16) hipLaunchKernelGGL((quant_slice_apply_kernel<0, LPR>), dim3(slices * chunks), dim3(256), 0, st, qp, chunks, rows, parts, d_chunks); \
-        else hipLaunchKernelGGL((quant_slice_apply_kernel<1, LPR>), dim3(slices * chunks), dim3(256), 0, st, qp, chunks, rows, parts, d_chunks); } while (0)
+        if (dtype == INTFA_F16) hipLaunchKernelGGL((quant_slice_apply_kernel<0, LPR>), dim3(slices * chunks2), dim3(256), 0, st, qp, chunks2, rows2, parts, d_chunks2); \
+        else hipLaunchKernelGGL((quant_slice_apply_kernel<1, LPR>), dim3(slices * chunks2), dim3(256), 0, st, qp, chunks2, rows2, parts, d_chunks2); } while (0)
     INTFA_LPR_SWITCH(head_dim, INTFA_CALL)
 #undef INTFA_CALL
     return (int)hipGetLastError();

@@ -40,3 +40,18 @@ def test_quant_pertensor_slice_sizes_bit_exact(B, H, N, d, dtype):
     assert rc == 0
     torch.cuda.synchronize()
     assert torch.equal(q8b, q8) and torch.equal(sb, s)
+
+
+# workgroups of one to four steps of rows (8 rows of head_dim 256 each; 2048 workgroups), with a last one of a single row; as one
+# slice for the per-(batch, head) scale the same sizes pass 256 parts of several rounds
+@pytest.mark.parametrize("steps", [1, 2, 3, 5])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_streaming_launch_sizes_bit_exact(steps, dtype):
+    N = 2048 * 8 * steps + 1
+    g = torch.Generator(device=DEV).manual_seed(steps)
+    x = torch.randn((1, 1, N, 256), generator=g, device=DEV).to(dtype)
+    x[0, 0, -1, -1] = 30
+    for fn, ref in ((M.quant_pertoken, O.quant_pertoken), (M.quant_pertensor, O.quant_pertensor)):
+        q8, s = fn(x)
+        ref8, ref_s = ref(x.cpu())
+        assert torch.equal(s.cpu(), ref_s) and torch.equal(q8.cpu(), ref8)

@@ -404,14 +404,15 @@ __device__ __forceinline__ float hide_past(float v, int last, int k_r) {
 }
 
 // The reference's requantisation of P (flash_atten_full_int8.py:49-51) for the 16 probabilities a lane holds of one 32-key
-// sub-tile, in the reference's own fp16 operations: fp16(p) (round to nearest even) * 127 -> fp16, + 0.5 -> fp16,
-// truncating conversion to an integer.  The multiply and the add are the packed fp16 instructions (two values each; kept
-// apart: a fused multiply-add would skip the rounding of the product).  The sixteen truncating conversions write their
-// byte straight into the four packed words (SDWA destination select).  A write with a destination select needs one wait
-// state before the next vector instruction touches that register, and the compiler places wait states for its own
-// instructions only: the conversions are therefore issued word-interleaved (bytes 0 of the four words, then bytes 1, ...),
-// so that three other conversions lie between two writes to one word, each round as ONE asm statement so that nothing can
-// be scheduled into it, and a single s_nop closes the last round before the words can be consumed.
+// sub-tile: fp16(p) (round to nearest even) * 127 -> fp16, + 0.5 -> fp16, truncating conversion to an integer.  The vector pipe
+// bounds the kernels that call this, so the instructions count: 1.75 per value, all but the last packed in pairs.
+//   * Product and sum are one packed fma: it skips the rounding of the product, and the truncated result is the same for
+//     every fp16 number in [0, 1] (exhaustively: tests/test_p_requant_steps.py).
+//   * The truncation is an addition of 1024 with the fp16 rounding mode at "toward zero": the integer lands in the low bits
+//     of the mantissa, and one byte permute packs four of them.  (MODE bits 3:2 round fp16 and fp64 results; the statement
+//     that sets them restores round-to-nearest, which everything else here runs in.)  NaN gives any byte: its row sum is NaN.
+// Before: multiply, add and a converting byte write (SDWA) each, 2.5 per value.  Full-int8, us: d128 B4 H32 N4096 821 -> 793
+// (with the fma alone 845 where the old chain took 863), d64 B4 H32 N1024 50.0 -> 47.0, d256 B16 H16 N1024 257 -> 252.
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
@@ -420,36 +421,19 @@ __device__ __forceinline__ v4i requant_p_reference16(const float (&p)[16]) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         v2h h = __builtin_convertvector((v2f){p[2 * i], p[2 * i + 1]}, v2h);
-        {
-#pragma clang fp contract(off)
-            h = h * (v2h){(_Float16)127.0f, (_Float16)127.0f};
-            h = h + (v2h){(_Float16)0.5f, (_Float16)0.5f};
-        }
+        h = __builtin_elementwise_fma(h, (v2h){(_Float16)127.0f, (_Float16)127.0f}, (v2h){(_Float16)0.5f, (_Float16)0.5f});
         hb[i] = __builtin_bit_cast(unsigned, h);
     }
-    unsigned w0, w1, w2, w3;
-    asm volatile("v_cvt_u16_f16_sdwa %0, %4 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:WORD_0\n\t"
-                 "v_cvt_u16_f16_sdwa %1, %5 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:WORD_0\n\t"
-                 "v_cvt_u16_f16_sdwa %2, %6 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:WORD_0\n\t"
-                 "v_cvt_u16_f16_sdwa %3, %7 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:WORD_0"
-                 : "=&v"(w0), "=&v"(w1), "=&v"(w2), "=&v"(w3) : "v"(hb[0]), "v"(hb[2]), "v"(hb[4]), "v"(hb[6]));
-    asm volatile("v_cvt_u16_f16_sdwa %0, %4 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "v_cvt_u16_f16_sdwa %1, %5 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "v_cvt_u16_f16_sdwa %2, %6 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "v_cvt_u16_f16_sdwa %3, %7 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1"
-                 : "+v"(w0), "+v"(w1), "+v"(w2), "+v"(w3) : "v"(hb[0]), "v"(hb[2]), "v"(hb[4]), "v"(hb[6]));
-    asm volatile("v_cvt_u16_f16_sdwa %0, %4 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0\n\t"
-                 "v_cvt_u16_f16_sdwa %1, %5 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0\n\t"
-                 "v_cvt_u16_f16_sdwa %2, %6 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0\n\t"
-                 "v_cvt_u16_f16_sdwa %3, %7 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0"
-                 : "+v"(w0), "+v"(w1), "+v"(w2), "+v"(w3) : "v"(hb[1]), "v"(hb[3]), "v"(hb[5]), "v"(hb[7]));
-    asm volatile("v_cvt_u16_f16_sdwa %0, %4 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "v_cvt_u16_f16_sdwa %1, %5 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "v_cvt_u16_f16_sdwa %2, %6 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "v_cvt_u16_f16_sdwa %3, %7 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1\n\t"
-                 "s_nop 0"
-                 : "+v"(w0), "+v"(w1), "+v"(w2), "+v"(w3) : "v"(hb[1]), "v"(hb[3]), "v"(hb[5]), "v"(hb[7]));
-    return (v4i){(int)w0, (int)w1, (int)w2, (int)w3};
+    const unsigned k1024 = 0x64006400u;                    // fp16 1024, twice
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3\n\t"
+                 "v_pk_add_f16 %0, %0, %8\n\tv_pk_add_f16 %1, %1, %8\n\tv_pk_add_f16 %2, %2, %8\n\tv_pk_add_f16 %3, %3, %8\n\t"
+                 "v_pk_add_f16 %4, %4, %8\n\tv_pk_add_f16 %5, %5, %8\n\tv_pk_add_f16 %6, %6, %8\n\tv_pk_add_f16 %7, %7, %8\n\t"
+                 "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0"
+                 : "+v"(hb[0]), "+v"(hb[1]), "+v"(hb[2]), "+v"(hb[3]), "+v"(hb[4]), "+v"(hb[5]), "+v"(hb[6]), "+v"(hb[7]) : "s"(k1024));
+    v4i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (int)__builtin_amdgcn_perm(hb[2 * i + 1], hb[2 * i], 0x06040200u);
+    return r;
 }
 
 }  // namespace intfa

@@ -299,7 +299,8 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
     const int cus = num_cus > 0 ? num_cus : 256;
     int64_t slots = 2ll * cus;                                                 // two workgroups per compute unit
     int64_t wgs = (int64_t)p->batch * p->heads * ((p->seqlen + kBlockM - 1) / kBlockM);
-    if (decode_shaped(p->seqlen)) {
+    const bool decode = decode_shaped(p->seqlen);
+    if (decode) {
         wgs = (int64_t)p->batch * p->heads * ((p->seqlen + kDecodeRows - 1) / kDecodeRows);
         // head_dim 256: 96 KiB and more of tiles, one workgroup per compute unit
         if (p->head_dim == 256) slots = cus;
@@ -311,7 +312,29 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
     const int64_t blocks = (seqlen_k + bn - 1) / bn;
     int64_t splits = (slots + wgs - 1) / wgs;
     if (splits > blocks / 4) splits = blocks / 4;                              // keep four key blocks per split
+    // Decode-shaped calls merge inside the launch, so a split costs little (2 us for the first one, then the reading of its partial by
+    // the workgroup that merges) and short ones pay.  Not full-int8: there every split requantises P in a frame of its own, and the
+    // caller would see another 2e-2 of that noise.  Measured, us, one split per four key blocks -> this rule:
+    //   * grids of at most one workgroup per compute unit go down to one step (128 keys) per split, at most 16: fp16 d128 on 8 heads,
+    //     1024 keys 10.6 -> 9.1, half-int8 11.0 -> 9.6.  Past one workgroup per compute unit short splits lose (fp16 d256, 32 heads,
+    //     1024 keys: 8 splits 14.8, 16 splits 24.8).
+    //   * up to four steps (two at head_dim 256) stay one split: fp16 d64, 8 heads, 512 keys 9.0 -> 7.2.
+    //   * the merge reads splits * rows * head_dim floats at 6e-5 us each, a step takes 0.3 us + 2.6e-5 us per byte of K and V: the sum is
+    //     least where splits^2 * rows * head_dim = steps * (5000 + 3/7 bytes).  32 rows: half-int8 d256, 4 K/V heads, 8192 keys 40.5 ->
+    //     34.5; fp16 d128, 8 K/V heads, 8192 keys 27.8 -> 25.
+    const bool decode_f16 = decode && variant != INTFA_VARIANT_FULL_INT8;
+    if (decode_f16) {
+        const int64_t steps = (seqlen_k + 127) / 128;
+        if (steps <= (p->head_dim == 256 ? 2 : 4)) return 1;
+        int64_t few = cus / wgs < steps ? cus / wgs : steps;
+        if (few > 16) few = 16;
+        if (splits < few) splits = few;
+        const int64_t rows = p->seqlen < kDecodeRows ? p->seqlen : kDecodeRows;
+        const int64_t step_bytes = 128ll * p->head_dim * (variant == INTFA_VARIANT_HALF_INT8 ? 3 : 4);
+        while (splits > 1 && splits * splits * rows * p->head_dim > steps * (5000 + step_bytes * 3 / 7)) --splits;
+    }
     if (splits > kMaxSplits) splits = kMaxSplits;
+    if (decode_f16 && splits > 1) splits = (blocks + (blocks + splits - 1) / splits - 1) / ((blocks + splits - 1) / splits);    // no empty split
     return splits < 1 ? 1 : (int)splits;
 }
 

@@ -249,8 +249,8 @@ int run_forward(int variant, const intfa_fwd_params* p, int qk_bytes, int v_byte
     }
     rc = setup_split(p, block_n_for(variant, kp.head_dim), &kp);
     if (rc != INTFA_OK) return rc;
-    // (the decode-shaped kernels merge; the general ones leave it to the merge kernel)
-    const bool merges = decode_kernel_takes(variant, kp);
+    // (the decode-shaped kernels and the general full-int8 one up to head_dim 128 merge; the others leave it to the merge kernel)
+    const bool merges = decode_kernel_takes(variant, kp) || (variant == INTFA_VARIANT_FULL_INT8 && kp.head_dim <= 128);
     if (!merges) kp.ticket = nullptr;
     rc = dispatch(variant, p, kp, false, stream);
     if (rc != INTFA_OK || kp.num_splits <= 1 || kp.ticket != nullptr) return rc;

@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const float l_true = (PROUND == 0) ? l_tot * (1.f / 127.f) : l_tot;
     const float lse = seen ? m_run + __builtin_log2f(l_true) : -INFINITY;
     if (SPLIT) {
-        const SplitPartials part(p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
+        const SplitPartials part(&p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
         if (q_valid) {
 #pragma unroll
             for (int j = 0; j < DTW; ++j) {

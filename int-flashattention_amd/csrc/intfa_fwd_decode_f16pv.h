@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const float inv = seen ? 1.f / l_tot : 0.f;
     const float lse = seen ? m_run + __builtin_log2f(l_tot) : -INFINITY;
     if (SPLIT) {
-        const SplitPartials part(p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
+        const SplitPartials part(&p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
         if (q_valid) {
             if (own_tile) {
 #pragma unroll

@@ -13,6 +13,7 @@
 // integer offsets into ONE array so that operand addresses are a lane register plus an immediate.
 #pragma once
 #include "intfa_device.h"
+#include "intfa_splitkv.h"
 
 namespace intfa {
 
@@ -469,8 +470,15 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 
     // ---- main loop: K/V tiles double-buffered in LDS, one barrier per key block.  The block on the causal
     // diagonal is always the last of the range and gets its own code instance after the loop.
+    // (a ticket per 32 query rows, so per wave; a wave past the last row has none)
+    const int row_blocks = (p.seqlen + 31) / 32, row_block = mb * (kBlockM / 32) + wave;
+    auto open_ticket = [&]() __attribute__((always_inline)) {
+        if (SPLIT && p.ticket != nullptr && lane == 0 && row_block < row_blocks) splitkv_open_tickets(p, head * row_blocks + row_block);
+    };
+    if (nb_begin >= nb_end) open_ticket();
     if (nb_begin < nb_end) {
         issue_loads(nb_begin, 0);
+        open_ticket();
         {
             const uint32_t s0 = load_ks(nb_begin);
             if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(s0);
@@ -521,34 +529,48 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     const bool any_key = nb_begin < nb_end && m_run > -INFINITY;
     const float out_scale = !any_key ? 0.f : (PROUND == 0) ? (vs / l_tot) : (vs / (127.f * l_tot));
     const float l_true = (PROUND == 0) ? l_tot * (1.f / 127.f) : l_tot;
-    const float lse = any_key ? m_run + __builtin_log2f(l_true) : -INFINITY;
-    if (SPLIT) {
-        const int64_t row = ((int64_t)(split * pe->batch + eb) * e_heads + eh) * e_seqlen + q_row;
-        float* op = pe->o_part + row * D;
+    float lse = any_key ? m_run + __builtin_log2f(l_true) : -INFINITY;
+    if constexpr (SPLIT) {
         // a row contributes nothing to this split when the split's range is empty for its workgroup, or when every
         // block of the range lies above the row's diagonal (its wave skipped them: the running max is still -inf)
-        const bool seen = nb_begin < nb_end && m_run > -INFINITY;
+        const int64_t first = ((int64_t)(split * pe->batch + eb) * e_heads + eh) * e_seqlen + (q_row - lq);      // (wave-uniform)
+        const SplitPartials part(pe, D, ((int64_t)__builtin_amdgcn_readfirstlane((int)(first >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)first));
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o_acc[dt][r] = any_key ? o_acc[dt][r] * out_scale : 0.f;
+        const int left = e_seqlen - (q_row - lq), nr = __builtin_amdgcn_readfirstlane(left < 32 ? left : 32);      // rows of this wave
+        const bool tickets = pe->ticket != nullptr;
         if (q_valid) {
+            const WavePartialLayout at(tickets, D, nr, lq, lh);
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int a4 = 0; a4 < 4; ++a4) {
-                    v4f o;
-#pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[dt][4 * a4 + b4] * out_scale : 0.f;
-                    *(v4f*)(op + 32 * dt + 8 * a4 + 4 * lh) = o;
-                }
-            if (lh == 0) pe->lse_part[row] = seen ? lse : -INFINITY;
+                for (int a4 = 0; a4 < 4; ++a4)
+                    part.put(0, D, (int)(at.lane + (uint32_t)(4 * dt + a4) * at.quad),
+                             (v4f){o_acc[dt][4 * a4], o_acc[dt][4 * a4 + 1], o_acc[dt][4 * a4 + 2], o_acc[dt][4 * a4 + 3]});
+            if (lh == 0) part.put_lse(lq, lse);
         }
-        return;
+        // the partials have arrived, and every wave is done with the tiles
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (!tickets || nr <= 0) return;
+        if (!splitkv_last_arrival_wave(pe, head * ((e_seqlen + 31) / 32) + mb * (kBlockM / 32) + wave)) return;
+        // (the weights lie in the part of the tile memory that this wave stages its output in: other waves may be at either)
+        static_assert(OutStage<DV>::BYTES >= 1024, "");
+        lse = splitkv_merge_wave<D>(pe, (float*)(smem + wave * OutStage<DV>::BYTES), o_acc, (uint32_t)((eb * e_heads + eh) * e_seqlen + mb * kBlockM + wave * 32),
+                                    nr, lq, lh);
+        __builtin_amdgcn_wave_barrier();
     }
     if constexpr (!DUMP_S) {
     // 16-bit rows go out through LDS (whole lines per store instruction); the tiles are dead once every wave is here
     static_assert(4 * OutStage<DV>::BYTES <= LDS_BYTES, "output staging fits the tile memory");
     // (the last block's copy slices ran against an empty resource: they fetch nothing but still write zeros into the
     // other tile buffers, asynchronously - every wave awaits its own before the barrier)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    if (!SPLIT) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
     // (an opaque copy of the lane index: the staging addresses depend on the lane only and would otherwise be computed
     // ahead of the main loop and held in registers through it)
     int lane_e = lane;
@@ -563,12 +585,12 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             if (OUT_DT == 0) {
                 v4h o;
 #pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) o[b4] = (_Float16)(any_key ? o_acc[dt][4 * a4 + b4] * out_scale : 0.f);
+                for (int b4 = 0; b4 < 4; ++b4) o[b4] = (_Float16)(SPLIT ? o_acc[dt][4 * a4 + b4] : any_key ? o_acc[dt][4 * a4 + b4] * out_scale : 0.f);
                 out_stage_put<DV>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
             } else {
                 v4s o;
 #pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) o[b4] = f32_to_bf16(any_key ? o_acc[dt][4 * a4 + b4] * out_scale : 0.f);
+                for (int b4 = 0; b4 < 4; ++b4) o[b4] = f32_to_bf16(SPLIT ? o_acc[dt][4 * a4 + b4] : any_key ? o_acc[dt][4 * a4 + b4] * out_scale : 0.f);
                 out_stage_put<DV>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
             }
         }

@@ -27,11 +27,12 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 struct SplitPartials {
     BufferRsrc o, l;
     uint32_t rows;                             // batch * heads * seqlen: rows of one split
-    __device__ __forceinline__ explicit SplitPartials(const KParams& p, int D, int64_t first) {
-        rows = (uint32_t)(p.batch * p.heads) * (uint32_t)p.seqlen;
-        const int64_t left = (int64_t)rows * p.num_splits - first, ob = left * D * 4, lb = left * 4;
-        o = __builtin_amdgcn_make_buffer_rsrc(p.o_part + first * D, 0, (int)(uint32_t)(ob < 0xffffffffll ? ob : 0xffffffffll), 0x00020000);
-        l = __builtin_amdgcn_make_buffer_rsrc(p.lse_part + first, 0, (int)(uint32_t)(lb < 0xffffffffll ? lb : 0xffffffffll), 0x00020000);
+    // (P: KParams pointer, or the kernel-argument pointer of the epilogues)
+    template <typename P> __device__ __forceinline__ explicit SplitPartials(P p, int D, int64_t first) {
+        rows = (uint32_t)(p->batch * p->heads) * (uint32_t)p->seqlen;
+        const int64_t left = (int64_t)rows * p->num_splits - first, ob = left * D * 4, lb = left * 4;
+        o = __builtin_amdgcn_make_buffer_rsrc(p->o_part + first * D, 0, (int)(uint32_t)(ob < 0xffffffffll ? ob : 0xffffffffll), 0x00020000);
+        l = __builtin_amdgcn_make_buffer_rsrc(p->lse_part + first, 0, (int)(uint32_t)(lb < 0xffffffffll ? lb : 0xffffffffll), 0x00020000);
     }
     __device__ __forceinline__ void put(uint32_t row, int D, int col, v4f x) const {
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, x), o, (row * (uint32_t)D + (uint32_t)col) * 4u, 0, kSplitAux);
@@ -85,6 +86,96 @@ __device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* sme
     return __builtin_amdgcn_readfirstlane(*(const int*)smem) != 0;
 }
 
+// ---- The same for the general full-int8 kernel, whose waves own 32 query rows each: a ticket per wave and no barrier.  The wave
+// that arrives last reads the partials in the layout of its accumulators, so the row statistics are one value per lane.
+// Instead of a second launch of splitkv_combine_kernel, whose arithmetic and order of splits it keeps (the same bits, whichever
+// wave is last), us: causal chunk B2 H32/8 Nq512 Nk7680 d128 (2 splits) 113 -> 105.5, B4 H12/3 Nq300 Nk3000 (4) 47 -> 43.4, d64 H16/4
+// Nq600 Nk4000 (7) 35.4 -> 31.1.  Not at head_dim 256, whose rows are spread over two waves.
+template <typename P> __device__ __forceinline__ bool splitkv_last_arrival_wave(P p, int group) {
+    unsigned last = 0;                                     // (after the wave's partials have been acknowledged)
+    if ((threadIdx.x & 63) == 0) {
+        uint64_t* t = p->ticket + group;
+        const uint64_t before = __hip_atomic_fetch_add(t, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = before == (p->epoch | (uint64_t)(p->num_splits - 1));
+        if (last) __hip_atomic_store(t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return __builtin_amdgcn_readfirstlane(last) != 0;
+}
+// Offset (floats) of a lane's four columns 8 c + 4 lh .. of accumulator quad c inside its wave's block of `nr` rows.  With tickets a
+// quad of the wave is one contiguous piece (rows side by side, 16 bytes each): a piece per row wrote and read 32 bytes of every
+// line (d64 B3 H16 Nq256 Nk2500 40 us).  Without, rows as splitkv_combine_kernel reads them.
+struct WavePartialLayout {
+    uint32_t lane, quad;
+    __device__ __forceinline__ WavePartialLayout(bool tickets, int D, int nr, int row, int lh) {
+        lane = tickets ? (uint32_t)(lh * nr + row) * 4u : (uint32_t)(row * D + 4 * lh);
+        quad = tickets ? 8u * (uint32_t)nr : 8u;
+    }
+};
+// acc[dt][4 a4 + b4], quad 4 dt + a4: the merged row.  `block`: first row of the wave's block of nr rows on the row axis of one split; `w`: 1 KiB
+// of LDS of this wave.  Returns the merged lse.  The partial of the next split is on its way while one is added, half a row at
+// a time.  (The wave's own partial is read back like the others: kept in registers beside sum and loads it spills 100 of them.)
+template <int D, typename P>
+__device__ __forceinline__ float splitkv_merge_wave(P p, float* w, float (&acc)[D / 32][16], uint32_t block, int nr, int lq, int lh) {
+    constexpr int DT = D / 32, H = DT / 2;
+    const SplitPartials part(p, D, 0);
+    const int ns = p->num_splits, rl = lq < nr ? lq : nr - 1;
+    const WavePartialLayout at(true, D, nr, rl, lh);
+    v4f x[DT][4];
+    auto request = [&](int s, int half) __attribute__((always_inline)) {
+        const uint32_t base = ((uint32_t)s * part.rows + block) * (uint32_t)D + at.lane;
+#pragma unroll
+        for (int dt = half * H; dt < half * H + H; ++dt)
+#pragma unroll
+            for (int a4 = 0; a4 < 4; ++a4) x[dt][a4] = part.get(0, D, (int)(base + (uint32_t)(4 * dt + a4) * at.quad));
+    };
+    request(0, 0);
+    request(0, 1);
+    float l[8];
+    auto load8 = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) l[u] = part.get_lse((uint32_t)(s0 + u < ns ? s0 + u : ns - 1) * part.rows + block + (uint32_t)rl);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) l[u] = s0 + u >= ns ? -INFINITY : l[u];
+    };
+    float mx = -INFINITY, sum = 0.f;
+    for (int s0 = 0; s0 < ns; s0 += 8) {
+        load8(s0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mx = fmaxf(mx, l[u]);
+    }
+    const bool empty = mx == -INFINITY;
+    if (empty) mx = 0.f;
+    for (int s0 = 0; s0 < ns; s0 += 8) {
+        if (ns > 8) load8(s0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum += fast_exp2(l[u] - mx);
+    }
+    const float lse = empty ? -INFINITY : __builtin_log2f(sum) + mx;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+    for (int s0 = 0; s0 < ns; s0 += 8) {
+        if (ns > 8) load8(s0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) w[u * 32 + lq] = empty ? 0.f : fast_exp2(l[u] - lse);       // (both halves of the wave write the same)
+        const int s_end = s0 + 8 < ns ? s0 + 8 : ns;
+        for (int s = s0; s < s_end; ++s) {
+            const float ws = w[(s - s0) * 32 + lq];
+            const int s_next = s + 1;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+#pragma unroll
+                for (int dt = half * H; dt < half * H + H; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[dt][r] = fmaf(ws, x[dt][r >> 2][r & 3], acc[dt][r]);
+                if (s_next < ns) request(s_next, half);
+            }
+        }
+    }
+    return lse;
+}
+
 // Reductions over eight consecutive lanes (quad_perm 1,0,3,2 / 2,3,0,1, then the mirrored half row).
 template <typename F> __device__ __forceinline__ float reduce8(float x, F op) {
     x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true)));
@@ -102,7 +193,7 @@ constexpr int kMergeLds = 16 + 32 * kMaxSplits * 4 + 256 * 16;
 template <int D, int OUT_DT>
 __device__ __forceinline__ void splitkv_merge_rows(const KParams& p, char* smem, int b, int h, int row0, int nrows) {
     constexpr int LPR = D / 4, RP = 256 / LPR, KL = kMaxSplits / 8, U = 4;
-    const SplitPartials part(p, D, 0);
+    const SplitPartials part(&p, D, 0);
     const int ns = p.num_splits, tid = threadIdx.x;
     float* w = (float*)(smem + 16);                        // [split][32]
     v4f* red = (v4f*)(smem + 16 + 32 * kMaxSplits * 4);

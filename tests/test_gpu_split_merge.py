@@ -85,6 +85,30 @@ def test_merge_in_the_kernel_equals_the_merge_launch(variant, D, Nq, Nk, splits)
         close(lse, want_lse)
 
 
+# the general full-int8 kernel, a ticket per 32-row wave: more than 64 rows, a last query block with one, two and four waves of
+# rows; the fewest splits, an odd number, the most, more than there are blocks; causal rows that some splits do not see
+@pytest.mark.parametrize("D,Nq,Nk,splits,causal", [
+    (128, 65, 1024, 2, 0), (128, 128, 8200, 64, 0), (128, 161, 700, 9, 1), (128, 512, 2048, 2, 1), (64, 129, 300, 3, 0), (64, 250, 3001, 5, 1),
+])
+def test_merge_in_the_general_kernel_equals_the_merge_launch(D, Nq, Nk, splits, causal):
+    lib = _capi.load()
+    p, out, lse, keep = problem("full", 2, 3, Nq, Nk, D, splits + Nq, lens=[Nk, max(1, Nk // 3)])
+    p.num_splits, p.causal = splits, causal
+    small, need = lib.intfa_fwd_workspace_bytes(ctypes.byref(p)), lib.intfa_fwd_merge_workspace_bytes(ctypes.byref(p))
+    ws = torch.empty((need,), dtype=torch.uint8, device=DEV)
+    call("full", p, ws, small)
+    torch.cuda.synchronize()
+    want, want_lse = out.clone(), lse.clone()
+    for fill in (0, 255, None, 1):
+        if fill is not None:
+            ws.fill_(fill)
+        out.fill_(float("nan"))
+        lse.fill_(float("nan"))
+        call("full", p, ws, need)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(lse, want_lse)          # the same sums in the same order
+
+
 def test_merge_replays_from_a_graph_beside_other_calls():
     lib = _capi.load()
     p, out, lse, keep = problem("half", 1, 4, 4, 4096, 128, 3)

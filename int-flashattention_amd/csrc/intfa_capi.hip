@@ -192,7 +192,17 @@ bool decode_kernel_takes(int variant, const KParams& kp) {
     return (decode_shaped(kp.seqlen) || small) && !(variant == INTFA_VARIANT_FULL_INT8 && kp.vs_sub == 2);
 }
 
-int dispatch(int variant, const intfa_fwd_params* p, const KParams& kp, bool dump_s, hipStream_t stream) {
+// K and V of a decode-shaped call are loaded past the caches (non-temporal) when one workgroup alone reads each tile and the
+// caches could not keep them for the next pass anyway: 128 MiB and more, half of the last-level cache, which other layers' K and V
+// share.  Measured, three sets of inputs in turn, us, plain -> non-temporal: fp16 B32 H32 Nk4096 d128 (2.1 GB) 354 -> 306 (6.1 ->
+// 7.0 TB/s), full-int8 B16 H32/8 Nk8192 (268 MB) 53.9 -> 47.2, 134 MB 29.9 -> 28.8, 101 MB 31.6 - 32.3 -> 31.7 - 32.5; 67 MB, which the
+// cache keeps, 17.8 -> 19.7.  An instance of its own: a choice at run time inside the kernel cost the small calls 2 - 3 %.
+constexpr int64_t kStreamKvBytes = 128ll << 20;
+bool streams_kv(const KParams& kp) {
+    return kp.seqlen <= kDecodeRows && kp.kv_group == 1 && (int64_t)kp.batch * kp.heads * kp.seqlen_k * kp.kv_key_bytes >= kStreamKvBytes;
+}
+
+int dispatch(int variant, const intfa_fwd_params* p, KParams kp, bool dump_s, hipStream_t stream) {
     const bool vblk = variant == INTFA_VARIANT_FULL_INT8 && !dump_s && kp.vs_g > 0;
     LaunchSel sel;
     sel.causal = kp.causal != 0;
@@ -204,6 +214,7 @@ int dispatch(int variant, const intfa_fwd_params* p, const KParams& kp, bool dum
     if (vblk && kp.vs_sub == 2) {
         if (d == 128) return launch_full_int8_vblk64_d128(kp, sel, stream);
     } else if (!dump_s && decode_kernel_takes(variant, kp)) {
+        kp.stream_kv = streams_kv(kp);
         if (variant == INTFA_VARIANT_FULL_INT8) {
             if (d == 64) return launch_decode_full_int8_d64(kp, sel, stream);
             if (d == 128) return launch_decode_full_int8_d128(kp, sel, stream);

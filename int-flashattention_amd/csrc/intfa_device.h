@@ -81,6 +81,7 @@ struct KParams {
     int32_t run_units, run_units_last, run_last_slot;      // run_last_slot: first slot of the last group
     int32_t rem_wgs;                                       // workgroups of the K/V heads that are not dealt whole
     int32_t kv_key_bytes;                                  // bytes of one key's K and V rows
+    int32_t stream_kv;                                     // decode-shaped kernels: K and V tiles are loaded non-temporally
     FastDiv d_run, d_run_heads, d_run_heads_last, d_rem_heads;
 };
 
@@ -317,22 +318,25 @@ __device__ __forceinline__ v4i make_rsrc(const void* base, uint32_t bytes) {
 // entry for it and ignores it.  Nothing the compiler generates in these kernels reads M0 (no LDS-DMA builtins, GWS,
 // relative moves or interpolation), and every copy sets it afresh.  tile_off and row_stride must be wave-uniform values
 // the compiler can see as such (kernel arguments, readfirstlane results): they end up in scalar operands.
-template <int ROW_BYTES, int SWZ, int ROWS>
+// NT: non-temporal, for tiles that nothing reads again.
+template <int ROW_BYTES, int SWZ, int ROWS, bool NT = false>
 __device__ __forceinline__ void issue_tile_part(v4i rsrc, uint32_t tile_off, uint32_t row_stride, uint32_t lds_tile,
                                                 int wave, const TileLoadLane<ROW_BYTES, SWZ, ROWS>& ln, int it) {
     using T = TileLoadLane<ROW_BYTES, SWZ, ROWS>;
     const int i = it * 4 + wave;                     // wave-uniform instruction index
     const uint32_t m0v = lds_tile + (uint32_t)i * 1024u;
     const uint32_t soff = tile_off + (uint32_t)(i * T::RPI) * row_stride;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    if (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :: "s"(m0v), "v"(ln.off[it % T::NV]), "s"(rsrc), "s"(soff) : "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :: "s"(m0v), "v"(ln.off[it % T::NV]), "s"(rsrc), "s"(soff) : "memory");
 }
-template <int ROW_BYTES, int SWZ, int ROWS>
+template <int ROW_BYTES, int SWZ, int ROWS, bool NT = false>
 __device__ __forceinline__ void issue_tile_load(v4i rsrc, uint32_t tile_off, uint32_t row_stride, uint32_t lds_tile,
                                                 int wave, const TileLoadLane<ROW_BYTES, SWZ, ROWS>& ln) {
     using T = TileLoadLane<ROW_BYTES, SWZ, ROWS>;
 #pragma unroll
-    for (int it = 0; it < T::NINST / 4; ++it) issue_tile_part<ROW_BYTES, SWZ, ROWS>(rsrc, tile_off, row_stride, lds_tile, wave, ln, it);
+    for (int it = 0; it < T::NINST / 4; ++it) issue_tile_part<ROW_BYTES, SWZ, ROWS, NT>(rsrc, tile_off, row_stride, lds_tile, wave, ln, it);
 }
 
 // ---- 16-bit output rows through LDS.  In the accumulator layout a lane holds four consecutive columns of ONE row per

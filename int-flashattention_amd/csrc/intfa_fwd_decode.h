@@ -28,7 +28,7 @@
 namespace intfa {
 
 // Head_dim 128: one 128-key block per step, the block of the general kernel.  Head dims 64 and 256: two 64-key blocks.
-template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK>
+template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK, bool STREAM /* K, V tiles non-temporal: KParams::stream_kv */>
 __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_int8_kernel(const KParams p) {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
@@ -108,8 +108,8 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const auto v_lane = tile_load_lane<D, SWZ_V8, BN>(v_sn, wave, lane);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<D, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
-        issue_tile_load<D, SWZ_V8, BN>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        issue_tile_load<D, SWZ_K, BN, STREAM>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
+        issue_tile_load<D, SWZ_V8, BN, STREAM>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
     };
     // k_scale of a block: thread t < 128 fetches the scale of key t; converted to fp32 when stored to LDS
     const KScaleSource ks_src(p, b, hk, seqlen_k);

@@ -32,7 +32,7 @@ namespace intfa {
 
 // QK_INT8: int8 Q/K with per-token scales (half-int8) or 16-bit Q/K.  IO_DT: type of V, P and the output (and of Q/K
 // when !QK_INT8): 0 fp16, 1 bf16.  The causal mask is a run-time switch here (p.causal).
-template <bool QK_INT8, int D, int IO_DT, bool SPLIT>
+template <bool QK_INT8, int D, int IO_DT, bool SPLIT, bool STREAM /* K, V tiles non-temporal: KParams::stream_kv */>
 __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8) ? 3 : 2) fwd_decode_f16pv_kernel(const KParams p) {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128 and 256");
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
@@ -116,8 +116,8 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const auto v_lane = tile_load_lane<VROW, SWZ_V16, BN>(v_sn, wave, lane);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<KROW, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
-        issue_tile_load<VROW, SWZ_V16, BN>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        issue_tile_load<KROW, SWZ_K, BN, STREAM>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
+        issue_tile_load<VROW, SWZ_V16, BN, STREAM>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
     };
     // k_scale of a step: thread t < 128 fetches the scale of key t; converted to fp32 when stored to LDS
     const KScaleSource ks_src(p, b, hk, seqlen_k);

@@ -1,0 +1,63 @@
+"""What lies behind the causal mask must not be seen: a V row that is not finite, as the padding behind a prompt may hold, leaves the rows
+alone whose keys end before it.  The kernels multiply P = 0 with the hidden keys of a 32-key sub-tile that some row of a 32-row group
+does see, and with no others; the eight-wave kernel of head_dim 256 does so for the 64-key blocks that a 128-row group sees."""
+import pytest
+import torch
+
+import int_flashattention_amd as M
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+NAN = float("nan")
+
+
+def inputs(variant, H, Nq, Nk, D, dt, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    q, k, v = (torch.randn((1, H, n, D), generator=g, device=DEV).to(dt) for n in (Nq, Nk, Nk))
+    if variant == "fp":
+        return q, k, v
+    (q8, qs), (k8, ks) = M.quant_pertoken(q), M.quant_pertoken(k)
+    return q8, k8, v, qs, ks
+
+
+def call(variant, args, v, sm, **kw):
+    if variant == "fp":
+        return M.attention(args[0], args[1], v, True, sm, **kw)
+    return M.attention_int8(args[0], args[1], v, args[3], args[4], True, sm, **kw)
+
+
+# One head (times reps) per hidden position: about twenty at 300 keys, forty at 600.  Head_dim 128 is the pipelined kernel from 65 rows on;
+# head_dim 64 the pipelined one past 512 workgroups of 32 rows (N 600), the one with three waves per SIMD past 512 of 128 rows (three times the
+# heads); head_dim 256 the decode-shaped and the eight-wave kernel.  More keys than queries by a part of a sub-tile, by one and by two
+# blocks; split passes
+@pytest.mark.parametrize("variant", ["half", "fp"])
+@pytest.mark.parametrize("D,reps,Nq,Nk,splits", [
+    (128, 1, 300, 300, 1), (128, 1, 384, 384, 1), (128, 1, 129, 200, 1), (128, 1, 260, 324, 1), (128, 1, 256, 384, 1), (128, 1, 330, 330, 3),
+    (64, 1, 600, 600, 1), (64, 1, 576, 640, 1), (64, 1, 600, 600, 2), (64, 3, 600, 600, 1), (256, 1, 300, 300, 1), (256, 2, 300, 300, 1),
+])
+def test_non_finite_values_behind_the_mask_reach_no_row_before_them(variant, D, reps, Nq, Nk, splits):
+    off, sm, dt = Nk - Nq, D ** -0.5, torch.bfloat16 if Nq % 2 else torch.float16
+    # one hidden position per head: edges of sub-tiles and blocks, and keys in between
+    at = sorted({t for s in range(0, Nk, 64) for t in (s, s + 31, s + 32, s + 63) if off < t < Nk} | {Nk - 1})
+    H = len(at) * reps
+    args = inputs(variant, H, Nq, Nk, D, dt, Nq + Nk + D)
+    v = args[2]
+    clean = call(variant, args, v, sm, num_splits=splits)
+    bad = v.clone()
+    for h in range(H):
+        bad[0, h, at[h % len(at)]] = NAN if h % 2 else float("inf")
+    got = call(variant, args, bad, sm, num_splits=splits)
+    torch.cuda.synchronize()
+    rows = torch.arange(Nq)
+    for h in range(H):
+        t = at[h % len(at)]
+        if D == 256 and Nq > 64:
+            safe = (rows // 128 * 128 + 127 + off) // 64 < t // 64
+        else:
+            safe = (rows // 32 * 32 + 31 + off) // 32 < t // 32
+        sees = rows + off >= t
+        o, c = got[0, h].cpu(), clean[0, h].cpu()
+        assert torch.equal(o[safe], c[safe]), (t, rows[safe][(o[safe] != c[safe]).any(-1)])
+        assert not torch.isfinite(o[sees]).any(), t
+        assert safe.any() or t <= off + 190
+

@@ -156,6 +156,7 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     // the smallest and this lane's own last visible key
     const int first_lim = p.causal ? (fold ? 0 : mb * kDecodeRows) + causal_off : 0x3fffffff;
     const int row_lim = p.causal ? (fold ? q_row % fold : q_row) + causal_off : 0x3fffffff;
+    const int last_lim = p.causal ? (fold ? fold : mb * kDecodeRows + kDecodeRows) - 1 + causal_off : 0x3fffffff;   // ... of the last row
     const bool blk_a = NBS == 1 || wave < 2;          // this wave's keys belong to the first block of a step
     // head_dim 64, where fwd_f16pv_kernel could have taken the call (more than kDecodeMaxRows query rows), its lazy frame: it follows a row's maximum when that exceeds it by more than
     // kFrameSlack in some row of the 32, and in the blocks that kernel masks (of its 128-row query blocks): the causal
@@ -269,6 +270,18 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
             v4i pall[NG];
 #pragma unroll
             for (int g = 0; g < NG; ++g) pall[g] = *(const v4i*)(smem + xp_rd + 1024 * g);
+            if (tail) {
+                // sub-tiles past the last key that any of the rows sees (the second block of a step may lie past the range): P is
+                // zero there, but zero times a V that is not finite (what a prompt's padding may hold) is not
+                asm volatile("");
+                const int seen = (last_lim < key_end - 1 ? last_lim : key_end - 1) - key0;
+#pragma unroll
+                for (int g = 2; g < NG; ++g)
+                    if (32 * (g / 2) > seen) {
+#pragma unroll
+                        for (int j = 0; j < DTW; ++j) vf[j][g] = (v4i){0, 0, 0, 0};
+                    }
+            }
 #pragma unroll
             for (int j = 0; j < DTW; ++j) {
 #pragma unroll

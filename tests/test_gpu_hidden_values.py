@@ -27,13 +27,15 @@ def call(variant, args, v, sm, **kw):
 
 
 # One head (times reps) per hidden position: about twenty at 300 keys, forty at 600.  Head_dim 128 is the pipelined kernel from 65 rows on;
-# head_dim 64 the pipelined one past 512 workgroups of 32 rows (N 600), the one with three waves per SIMD past 512 of 128 rows (three times the
-# heads); head_dim 256 the decode-shaped and the eight-wave kernel.  More keys than queries by a part of a sub-tile, by one and by two
-# blocks; split passes
+# head_dim 64 the decode-shaped kernel up to 512 workgroups of 32 rows (N 320), the pipelined one (N 600), the one with three waves per SIMD
+# past 512 workgroups of 128 rows (N 600, three times the heads); head_dim 256 the decode-shaped and the eight-wave kernel.  More keys than
+# queries by a part of a sub-tile, by one and by two blocks; split passes
 @pytest.mark.parametrize("variant", ["half", "fp"])
 @pytest.mark.parametrize("D,reps,Nq,Nk,splits", [
     (128, 1, 300, 300, 1), (128, 1, 384, 384, 1), (128, 1, 129, 200, 1), (128, 1, 260, 324, 1), (128, 1, 256, 384, 1), (128, 1, 330, 330, 3),
+    (64, 1, 320, 320, 1), (64, 1, 200, 271, 1), (64, 1, 256, 320, 1), (64, 1, 64, 100, 2),
     (64, 1, 600, 600, 1), (64, 1, 576, 640, 1), (64, 1, 600, 600, 2), (64, 3, 600, 600, 1), (256, 1, 300, 300, 1), (256, 2, 300, 300, 1),
+    (64, 1, 64, 612, 1), (128, 1, 64, 612, 1), (256, 1, 64, 612, 1),
 ])
 def test_non_finite_values_behind_the_mask_reach_no_row_before_them(variant, D, reps, Nq, Nk, splits):
     off, sm, dt = Nk - Nq, D ** -0.5, torch.bfloat16 if Nq % 2 else torch.float16

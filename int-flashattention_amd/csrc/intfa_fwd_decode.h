@@ -124,13 +124,13 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const int vs_i = NV > 128 ? tid : (vs_thread ? tid - 128 : 0);
     const int vs_blk0 = NV > 128 ? 0 : vs_i / D;              // block (inside the step) of the thread's first value
     const float* Vsg = (const float*)p.v_scale + (b * p.vs_sb + hk * p.vs_sh + vs_i % D);
-    const int vs_last_row = VBLK ? ((p.seqlen_k + BNB - 1) / BNB - 1) / p.vs_g : 0;
-    // (a step's second block may lie past the end of the sequence: its keys are hidden, any scale row serves)
+    // (a step's second block may lie past the range: its P8 are zero, and the scales of the range's last block serve - not its own, which
+    // lie behind the mask and need not be finite)
     auto load_vs = [&](int nb, int j) __attribute__((always_inline)) -> float {
         if (!VBLK) return 0.f;
-        const int blk = nb + vs_blk0 + j;
-        int row = p.vs_g == 1 ? blk : blk / p.vs_g;
-        row = row < vs_last_row ? row : vs_last_row;
+        int blk = nb + vs_blk0 + j;
+        blk = blk < nb_end ? blk : nb_end - 1;
+        const int row = p.vs_g == 1 ? blk : blk / p.vs_g;
         return Vsg[(int64_t)row * p.vs_sblk];
     };
 

@@ -1,6 +1,7 @@
-"""What lies behind the causal mask must not be seen: a V row that is not finite, as the padding behind a prompt may hold, leaves the rows
-alone whose keys end before it.  The kernels multiply P = 0 with the hidden keys of a 32-key sub-tile that some row of a 32-row group
-does see, and with no others; the eight-wave kernel of head_dim 256 does so for the 64-key blocks that a 128-row group sees."""
+"""What lies behind the causal mask must not be seen: a V row (or the scale row of a V block) that is not finite, as the padding behind a
+prompt may hold, leaves the rows alone whose keys end before it.  The kernels multiply P = 0 with the hidden keys of a 32-key sub-tile
+(of a key block, for the scales) that some row of a 32-row group does see, and with no others; the eight-wave kernels of head_dim 256 do so for
+the 64-key blocks that a 128-row group sees."""
 import pytest
 import torch
 
@@ -63,3 +64,49 @@ def test_non_finite_values_behind_the_mask_reach_no_row_before_them(variant, D, 
         assert not torch.isfinite(o[sees]).any(), t
         assert safe.any() or t <= off + 190
 
+
+# The scales of a V block behind the mask; head_dim 64 and 256 take two blocks per step in the decode-shaped kernel (reps 1), the other grids
+# run the general kernels
+@pytest.mark.parametrize("D,reps,Nq,Nk,vsb", [
+    (64, 1, 320, 320, 64), (64, 1, 200, 456, 128), (64, 1, 60, 450, 64), (64, 16, 320, 320, 64), (128, 1, 400, 400, 128), (128, 16, 400, 400, 128),
+    (256, 1, 256, 320, 64), (256, 1, 300, 300, 64), (256, 16, 256, 320, 64),
+])
+def test_non_finite_v_scales_behind_the_mask_reach_no_row_before_them(D, reps, Nq, Nk, vsb):
+    off, sm = Nk - Nq, D ** -0.5
+    first = [s for s in range(vsb, Nk, vsb) if s > off]
+    H = len(first) * reps
+    q8, k8, v, qs, ks = inputs("half", H, Nq, Nk, D, torch.float16, D + Nq)
+    v8, vs = M.quant_perblock_channel(v, vsb)
+    run = lambda s: M.attention_full_int8(q8, k8, v8, qs, ks, s, True, sm, v_scale_block=vsb)
+    clean = run(vs)
+    bad = vs.clone()
+    for h in range(H):
+        bad[0, h, first[h % len(first)] // vsb] = NAN
+    got = run(bad)
+    torch.cuda.synchronize()
+    rows = torch.arange(Nq)
+    group = 128 if D == 256 else 32
+    for h in range(H):
+        s = first[h % len(first)]
+        safe = rows // group * group + group - 1 + off < s
+        o, c = got[0, h].cpu(), clean[0, h].cpu()
+        assert torch.equal(o[safe], c[safe]), (s, rows[safe][(o[safe] != c[safe]).any(-1)])
+        assert not torch.isfinite(o[rows + off >= s]).any(), s
+
+
+# an odd number of 64-key blocks per entry: the second block of the last step is past the entry's length
+@pytest.mark.parametrize("D,Nq", [(64, 1), (64, 100), (256, 1), (256, 100)])
+def test_scale_rows_past_an_entrys_length_are_not_used(D, Nq):
+    lens, Nk, vsb = [64, 180], 384, 64
+    g = torch.Generator(device=DEV).manual_seed(D + Nq)
+    q, k, v = (torch.randn((2, 2, n, D), generator=g, device=DEV).half() for n in (Nq, Nk, Nk))
+    (q8, qs), (k8, ks), (v8, vs) = M.quant_pertoken(q), M.quant_pertoken(k), M.quant_perblock_channel(v, vsb)
+    run = lambda s: M.attention_full_int8(q8, k8, v8, qs, ks, s, False, D ** -0.5, v_scale_block=vsb,
+                                          seqlens_k=torch.tensor(lens, dtype=torch.int32, device=DEV))
+    clean = run(vs)
+    bad = vs.clone()
+    for b, n in enumerate(lens):
+        bad[b, :, -(-n // vsb):] = NAN
+    got = run(bad)
+    torch.cuda.synchronize()
+    assert torch.equal(got, clean) and torch.isfinite(got).all()

@@ -150,9 +150,9 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     const bool vs_thread = VBLK && wave >= 2 && (wave - 2) * 64 < DV;   // threads 128 .. 128 + DV - 1: one channel each
     // (these scales are fp32 whatever the type of the per-token scales, as in the reference's kernel)
     const float* Vsg = (const float*)p.v_scale + (b * p.vs_sb + hk * p.vs_sh + (vs_thread ? vs_c : 0));
-    // (VBLK == 2: scale rows 2 nb and 2 nb + 1; the second one does not exist when the sequence ends inside the block's
-    // first half - its keys are masked, any row serves)
-    const int vs_last_row = VBLK == 2 ? (p.seqlen_k + 63) / 64 - 1 : 0;
+    // (VBLK == 2: scale rows 2 nb and 2 nb + 1; when the entry's keys end inside the block's first half the second one does not exist or
+    // lies past its length and need not be finite: the first one serves, P8 is zero there)
+    const int vs_last_row = VBLK == 2 ? (seqlen_k + 63) / 64 - 1 : 0;
     auto load_vs = [&](int nb, int sub) __attribute__((always_inline)) -> float {
         if (!VBLK) return 0.f;
         int row = p.vs_g == 1 ? nb : nb / p.vs_g;

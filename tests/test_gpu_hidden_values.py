@@ -94,8 +94,9 @@ def test_non_finite_v_scales_behind_the_mask_reach_no_row_before_them(D, reps, N
         assert not torch.isfinite(o[rows + off >= s]).any(), s
 
 
-# an odd number of 64-key blocks per entry: the second block of the last step is past the entry's length
-@pytest.mark.parametrize("D,Nq", [(64, 1), (64, 100), (256, 1), (256, 100)])
+# an odd number of 64-key blocks per entry: the second block of the last step (head_dim 128: the second scale row of the last block) is past
+# the entry's length
+@pytest.mark.parametrize("D,Nq", [(64, 1), (64, 100), (256, 1), (256, 100), (128, 1), (128, 100)])
 def test_scale_rows_past_an_entrys_length_are_not_used(D, Nq):
     lens, Nk, vsb = [64, 180], 384, 64
     g = torch.Generator(device=DEV).manual_seed(D + Nq)

@@ -12,7 +12,10 @@ namespace intfa {
 // pass itself.  Instead every workgroup publishes its partial and takes a ticket of its query block; the one that draws the
 // last ticket merges the block while the other workgroups of the launch still run.
 //   * Partials are written and read at agent scope (sc1: past the L2 of the XCD, which is not coherent with the seven
-//     others); the ticket is an atomic at the same scope, drawn after the writes have been acknowledged.
+//     others): each access is what an atomic one at that scope compiles to, so the caches need no write-back and no invalidation.  The
+//     ticket is an atomic at the same scope, drawn after the writes have been acknowledged; the merge's loads are held behind it by
+//     a fence that orders the compiler and the wave's own issue only (at agent scope it would invalidate the L1 in front of the merge:
+//     decoding steps and chunks 1 - 4 % slower, half-int8 drafts d64 14.2 -> 14.8 us, causal chunk 109 -> 112).
 //   * A ticket word is the launch's epoch (upper 56 bits, never the same twice in a process) and the arrivals so far.  The
 //     workspace is not cleared: every workgroup of the block looks at the word when it starts and exchanges anything that
 //     is not of this epoch for (epoch, 0) - under the first tiles' way from HBM, so that the arrival itself is one atomic add
@@ -83,7 +86,9 @@ __device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* sme
         *(int*)smem = last;
     }
     __syncthreads();
-    return __builtin_amdgcn_readfirstlane(*(const int*)smem) != 0;
+    const bool last = __builtin_amdgcn_readfirstlane(*(const int*)smem) != 0;
+    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return last;
 }
 
 // ---- The same for the general full-int8 kernel, whose waves own 32 query rows each: a ticket per wave and no barrier.  The wave
@@ -92,14 +97,16 @@ __device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* sme
 // wave is last), us: causal chunk B2 H32/8 Nq512 Nk7680 d128 (2 splits) 113 -> 105.5, B4 H12/3 Nq300 Nk3000 (4) 47 -> 43.4, d64 H16/4
 // Nq600 Nk4000 (7) 35.4 -> 31.1.  Not at head_dim 256, whose rows are spread over two waves.
 template <typename P> __device__ __forceinline__ bool splitkv_last_arrival_wave(P p, int group) {
-    unsigned last = 0;                                     // (after the wave's partials have been acknowledged)
+    unsigned drew_last = 0;                                // (after the wave's partials have been acknowledged)
     if ((threadIdx.x & 63) == 0) {
         uint64_t* t = p->ticket + group;
         const uint64_t before = __hip_atomic_fetch_add(t, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = before == (p->epoch | (uint64_t)(p->num_splits - 1));
-        if (last) __hip_atomic_store(t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        drew_last = before == (p->epoch | (uint64_t)(p->num_splits - 1));
+        if (drew_last) __hip_atomic_store(t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    return __builtin_amdgcn_readfirstlane(last) != 0;
+    const bool last = __builtin_amdgcn_readfirstlane(drew_last) != 0;
+    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return last;
 }
 // Offset (floats) of a lane's four columns 8 c + 4 lh .. of accumulator quad c inside its wave's block of `nr` rows.  With tickets a
 // quad of the wave is one contiguous piece (rows side by side, 16 bytes each): a piece per row wrote and read 32 bytes of every

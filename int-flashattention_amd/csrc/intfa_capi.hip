@@ -114,6 +114,7 @@ int make_kparams(const intfa_fwd_params* p, int qk_bytes, int v_bytes, bool need
     k.kv_key_bytes = p->head_dim * (qk_bytes + v_bytes);
     k.num_splits = 1; k.blocks_per_split = p->seqlen;   // single pass: never the limit
     k.qk_scale_log2 = p->sm_scale * 1.44269504f;      // flash_atten_full_int8.py:156-157
+    if (k.qk_scale_log2 == 0.f) k.qk_scale_log2 = 0x1p-126f;      // (as load_q_scale_log2: the scores of hidden keys are -infinity)
     *kp = k;
     return INTFA_OK;
 }

@@ -214,9 +214,12 @@ __device__ __forceinline__ void load_q8_fragments(v4i (&qreg)[KS], const KParams
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qreg[ks] = *(const v4i*)(qrow + ks * 32 + lh * 16);
 }
-// q_scale of query row q_ld times sm_scale * log2(e): the factor between S * k_scale and the exponent of exp2.
+// q_scale of query row q_ld times sm_scale * log2(e): the factor between S * k_scale and the exponent of exp2.  Never zero: the scores
+// of hidden keys are -infinity, and a row of zeros (scale zero, as padding has) must not make NaN of them.  The smallest normal number
+// gives a row's visible keys the same exponent as zero would.
 __device__ __forceinline__ float load_q_scale_log2(const KParams& p, int b, int h, int q_ld) {
-    return load_scale(p.q_scale, b * p.qs_sb + h * p.qs_sh + (int64_t)q_ld * p.qs_sn, p.scale_dtype) * p.qk_scale_log2;
+    const float c = load_scale(p.q_scale, b * p.qs_sb + h * p.qs_sh + (int64_t)q_ld * p.qs_sn, p.scale_dtype) * p.qk_scale_log2;
+    return c == 0.f ? 0x1p-126f : c;
 }
 
 // k_scale of the keys of one (batch, K/V head): fetched as raw bits (one key per thread, ahead of the block that uses

@@ -155,8 +155,7 @@ __global__ void __launch_bounds__(kThreads, 3) fwd_f16pv_kernel(const KParams p)
         for (int ks = 0; ks < KS; ++ks) qreg[ks] = *(const v4i*)(qrow + ks * 32 + lh * 16);
     }
     // exponent scale of this lane's row: q_scale * sm_scale * log2(e) (int8 Q K^T) or sm_scale * log2(e)
-    const float qsc = QK_INT8 ? load_scale(p.q_scale, b * p.qs_sb + h * p.qs_sh + (int64_t)q_ld * p.qs_sn, p.scale_dtype) * p.qk_scale_log2
-                              : p.qk_scale_log2;
+    const float qsc = QK_INT8 ? load_q_scale_log2(p, b, h, q_ld) : p.qk_scale_log2;
     float m_run = -INFINITY, l_run = 0.f;
     v16f o_acc[DT];
 #pragma unroll

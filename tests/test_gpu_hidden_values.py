@@ -111,3 +111,34 @@ def test_scale_rows_past_an_entrys_length_are_not_used(D, Nq):
     got = run(bad)
     torch.cuda.synchronize()
     assert torch.equal(got, clean) and torch.isfinite(got).all()
+
+
+# Hidden keys of a row whose scores are all zero: a query row of zeros has the scale zero, sm_scale may be zero.  Every key that the row sees
+# weighs the same: the output is the mean of its values.  reps: the decode-shaped and the general kernels; ragged ends and the causal diagonal
+@pytest.mark.parametrize("variant", ["full", "half", "fp"])
+@pytest.mark.parametrize("D,reps,Nq,Nk,splits", [(64, 1, 100, 100, 1), (64, 150, 100, 100, 1), (64, 20, 600, 600, 1), (64, 1, 5, 300, 3),
+                                                 (128, 1, 100, 100, 1), (128, 150, 100, 231, 1), (128, 2, 300, 300, 2), (128, 1, 5, 300, 3),
+                                                 (256, 1, 100, 100, 1), (256, 80, 100, 100, 1)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_hidden_keys_of_a_row_without_scores(variant, D, reps, Nq, Nk, splits, causal):
+    g = torch.Generator(device=DEV).manual_seed(D + Nq)
+    q, k, v = (torch.randn((1, reps, n, D), generator=g, device=DEV).half() for n in (Nq, Nk, Nk))
+    zero = [0, Nq // 2, Nq - 1]
+    q[:, :, zero] = 0
+    def run(sm):
+        if variant == "fp":
+            return M.attention(q, k, v, causal, sm, num_splits=splits)
+        (q8, qs), (k8, ks) = M.quant_pertoken(q), M.quant_pertoken(k)
+        if variant == "half":
+            return M.attention_int8(q8, k8, v, qs, ks, causal, sm, num_splits=splits)
+        v8, vs = M.quant_pertensor(v)
+        return M.attention_full_int8(q8, k8, v8, qs, ks, vs, causal, sm, num_splits=splits)
+    some, flat = run(D ** -0.5), run(0.0)
+    torch.cuda.synchronize()
+    assert torch.isfinite(some).all()
+    # P is the same for every key: only V's int8 rounding (full) and the 16-bit output are left
+    tol = 2e-3 + (v.abs().max().item() / 127 / 2 if variant == "full" else 0)
+    for rows, out in ((zero, some), (range(0, Nq, 7), flat)):
+        for r in rows:
+            n = r + 1 + Nk - Nq if causal else Nk
+            assert (out[0, :, r].float() - v[0, :, :n].float().mean(1)).abs().max().item() <= tol, (r, n)

@@ -6,6 +6,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 from test_gpu_parity import DEV, MAX_ABS, MEAN_REL, assert_same_rounding, gpu, max_abs, mean_rel
 
 pytestmark = pytest.mark.gpu
@@ -87,13 +88,14 @@ def test_decode_blocked_v_scales_bf16_and_strided_cache():
 
 
 def test_decode_kernel_agrees_with_the_general_kernel():
-    """65 query rows run the general kernel, the first 64 of them alone the decode kernel: same rows, same block maxima,
+    """65 query rows of many heads run the general kernel, the first 64 of them alone the decode kernel: same rows, same block maxima,
     same P8 and the same int32 sums, so the outputs differ only through the order of the fp32 row-sum additions."""
     x = decode_inputs(1, 2, 2, 65, 1500, 128, seed=93)
     sm = 128 ** -0.5
     k8, v8, ks, vs = gpu(x["k8"], x["v8"], x["ks"], x["vs"])
     q8, qs = gpu(x["q8"], x["qs"])
-    general = M.attention_full_int8(q8, k8, v8, qs, ks, vs, False, sm, p_round="rne")
+    many = repeated(repetitions(1, 2, 65), q8, k8, v8, qs, ks, vs)
+    general = first_heads(M.attention_full_int8(*many, False, sm, p_round="rne"), 2)
     decode = M.attention_full_int8(q8[:, :, :64].contiguous(), k8, v8, qs[:, :, :64].contiguous(), ks, vs, False, sm, p_round="rne")
     torch.cuda.synchronize()
     assert max_abs(decode, general[:, :, :64]) <= 1e-3 and mean_rel(decode, general[:, :, :64]) <= 1e-5
@@ -304,15 +306,16 @@ def test_decode_head_dim_256_matches_oracle(B, H, H_kv, Nq, Nk, causal, p_round)
 
 @pytest.mark.parametrize("causal", [False, True])
 def test_decode_head_dim_256_agrees_with_the_general_kernel(causal):
-    """65 query rows run the eight-wave general kernel, 64 of them alone the decode kernel: the same blocks, maxima, P8
-    and int32 sums; only the row sums are added in another order."""
+    """65 query rows of many heads run the eight-wave general kernel, 64 of them alone the decode kernel: the same blocks, maxima,
+    P8 and int32 sums; only the row sums are added in another order."""
     D = 256
     x = decode_inputs(1, 2, 2, 65, 1500, D, seed=111)
     sm = D ** -0.5
     k8, v8, ks, vs = gpu(x["k8"], x["v8"], x["ks"], x["vs"])
     q8, qs = gpu(x["q8"], x["qs"])
     rows = slice(1, 65) if causal else slice(0, 64)          # the mask is aligned to the end of the cache
-    general = M.attention_full_int8(q8, k8, v8, qs, ks, vs, causal, sm, p_round="rne")
+    many = repeated(repetitions(1, 2, 65), q8, k8, v8, qs, ks, vs)
+    general = first_heads(M.attention_full_int8(*many, causal, sm, p_round="rne"), 2)
     decode = M.attention_full_int8(q8[:, :, rows].contiguous(), k8, v8, qs[:, :, rows].contiguous(), ks, vs, causal, sm, p_round="rne")
     torch.cuda.synchronize()
     assert max_abs(decode, general[:, :, rows]) <= 1e-3 and mean_rel(decode, general[:, :, rows]) <= 1e-5

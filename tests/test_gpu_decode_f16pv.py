@@ -12,6 +12,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -114,7 +115,7 @@ def test_decode_matches_oracle(B, H, H_kv, Nq, Nk, D, causal, variant, dtype):
 @pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("causal", [False, True])
 def test_decode_kernel_agrees_with_the_general_kernel(variant, D, causal):
-    """65 query rows run the general kernel, 64 of them alone the decode kernel.  At head_dim 256 both take the same block
+    """65 query rows of many heads run the general kernel, 64 of them alone the decode kernel.  At head_dim 256 both take the same block
     maxima, the same 16-bit P and the same MFMA steps per block, so a row's result differs only through the order of the
     fp32 row-sum additions (one rounding of the 16-bit output now and then).  At head_dim <= 128 the general kernel takes
     exp2 against a reference point that lags the running maximum (it rescales the output only when a row's maximum rises by
@@ -123,7 +124,7 @@ def test_decode_kernel_agrees_with_the_general_kernel(variant, D, causal):
     With the mask the 64 rows are the LAST 64 of the 65 (the mask is aligned to the end of the cache)."""
     q, k, v = inputs(1, 2, 2, 65, 1500, D, seed=3100 + D)
     sm = D ** -0.5
-    general, lg = run(variant, q, k, v, causal, sm, return_lse=True)
+    general, lg = (first_heads(t, 2) for t in run(variant, *repeated(repetitions(1, 2, 65), q, k, v), causal, sm, return_lse=True))
     rows = slice(1, 65) if causal else slice(0, 64)
     decode, ld = run(variant, q[:, :, rows].contiguous(), k, v, causal, sm, return_lse=True)
     assert max_abs(decode, general[:, :, rows]) <= 1e-3 and mean_rel(decode, general[:, :, rows]) <= (2e-5 if D == 256 else 6e-4)

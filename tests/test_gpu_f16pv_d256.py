@@ -1,5 +1,6 @@
 """Half-int8 and fp16/bf16 attention at head_dim 256: the eight-wave kernel in which two waves share 32 query rows
-(each computes the softmax of half of a 64-key block and the output of half of the columns).
+(each computes the softmax of half of a 64-key block and the output of half of the columns), and the decode-shaped kernel, which
+takes few query rows and small grids.
 
 No P requantisation on these paths: against the oracle (flash_atten_int8.py:9-66, flash_atten_fp.py:9-60 restated with
 the kernel's 64-key block) the only differences are the fp32 summation order inside the MFMA, the hardware exp2 and where
@@ -11,6 +12,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -71,8 +73,8 @@ def repeat_kv(t, g):
 SHAPES = [
     # B, H, Nq, Nk, causal
     (1, 2, 128, 128, False),      # one query block, two key blocks
-    (2, 3, 384, 384, True),       # paired query blocks (one left over), diagonal blocks
-    (1, 2, 512, 512, True),       # paired query blocks, even count
+    (2, 3, 384, 384, True),       # three query blocks, diagonal blocks
+    (1, 2, 512, 512, True),
     (1, 2, 300, 300, False),      # ragged rows and keys
     (1, 2, 641, 641, True),
     (1, 2, 1, 700, False),        # one query row against a cache
@@ -87,9 +89,21 @@ SHAPES = [
 @pytest.mark.parametrize("variant", ["half", "fp"])
 @pytest.mark.parametrize("B,H,Nq,Nk,causal", SHAPES)
 def test_matches_oracle(B, H, Nq, Nk, causal, variant, dtype):
+    check_against_oracle(B, H, Nq, Nk, causal, variant, dtype)
+
+
+# the single passes above are small grids, the decode-shaped kernel's: the same among as many heads as the eight-wave kernel takes
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("variant", ["half", "fp"])
+@pytest.mark.parametrize("B,H,Nq,Nk,causal", [c for c in SHAPES if c[2] > 64])
+def test_eight_wave_kernel_matches_oracle(B, H, Nq, Nk, causal, variant, dtype):
+    check_against_oracle(B, H, Nq, Nk, causal, variant, dtype, reps=repetitions(B, H, Nq))
+
+
+def check_against_oracle(B, H, Nq, Nk, causal, variant, dtype, reps=1):
     q, k, v = inputs(B, H, Nq, Nk, seed=2560 + Nq + Nk, dtype=dtype)
     sm = D ** -0.5
-    o, lse = run(variant, q, k, v, causal, sm, return_lse=True)
+    o, lse = (first_heads(t, H) for t in run(variant, *repeated(reps, q, k, v), causal, sm, return_lse=True))
     assert o.dtype == dtype and o.shape == (B, H, Nq, D) and torch.isfinite(o).all()
     ref, lse_ref = oracle(variant, q, k, v, causal, sm, return_lse=True)
     ma, mr = bounds(dtype)

@@ -18,6 +18,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -40,15 +41,17 @@ def rising_inputs(B, H, Nq, Nk, D, bn, seed, growth=1.6, dtype=torch.float16):
 
 CASES = [
     # D, Nq, Nk, causal, splits, v_scale_block
-    (128, 256, 512, False, 1, None),        # headline kernel, 4 key blocks
-    (128, 256, 512, True, 1, None),         # causal (rows see 2 - 4 blocks), paired query blocks
-    (128, 128, 640, False, 2, None),        # split-KV: 3 + 2 blocks
+    # (four heads in all: the single-pass cases are small grids and run the decode-shaped kernel, which has no hand-written update; the
+    # general kernels run them in the test behind this one, among more heads)
+    (128, 256, 512, False, 1, None),        # 4 key blocks
+    (128, 256, 512, True, 1, None),         # causal (rows see 2 - 4 blocks)
+    (128, 128, 640, False, 2, None),        # split-KV, the general kernel: 3 + 2 blocks
     (64, 256, 384, False, 1, None),
     (128, 256, 512, False, 1, 128),         # per-block, per-channel V scales
-    (128, 256, 512, False, 1, 64),          # 64-key V scale rows: two chains per block
-    (256, 256, 256, False, 1, None),        # wave-pair kernel, 64-key blocks
+    (128, 256, 512, False, 1, 64),          # 64-key V scale rows: two chains per block of the general kernel
+    (256, 256, 256, False, 1, None),        # 64-key blocks
     (256, 128, 320, True, 1, None),
-    (128, 8, 512, False, 1, None),          # decode-shaped kernel
+    (128, 8, 512, False, 1, None),          # few query rows
     (64, 40, 384, False, 1, None),
 ]
 
@@ -56,6 +59,19 @@ CASES = [
 @pytest.mark.parametrize("p_round", ["rne", "reference"])
 @pytest.mark.parametrize("D,Nq,Nk,causal,splits,vsb", CASES)
 def test_rescale_factor_reaches_the_first_accumulator_update(D, Nq, Nk, causal, splits, vsb, p_round):
+    check_rescale_factor(D, Nq, Nk, causal, splits, vsb, p_round)
+
+
+# the headline kernel, its head_dim 64 form and the wave-pair kernel; the blocked-scale instances of each, masked and not
+@pytest.mark.parametrize("p_round", ["rne", "reference"])
+@pytest.mark.parametrize("D,Nq,Nk,causal,splits,vsb", [c for c in CASES if c[1] > 64 and c[4] == 1 and c[5] != 64] + [
+    (64, 256, 384, True, 1, None), (64, 256, 384, False, 1, 64), (64, 256, 384, True, 1, 128), (128, 256, 512, True, 1, 128),
+    (256, 256, 256, False, 1, 64), (256, 128, 320, True, 1, 128)])
+def test_rescale_factor_reaches_the_first_accumulator_update_of_the_general_kernels(D, Nq, Nk, causal, splits, vsb, p_round):
+    check_rescale_factor(D, Nq, Nk, causal, splits, vsb, p_round, reps=repetitions(2, 2, Nq))
+
+
+def check_rescale_factor(D, Nq, Nk, causal, splits, vsb, p_round, reps=1):
     B, H = 2, 2
     bn = M.block_n("full", D)
     q, k, v = rising_inputs(B, H, Nq, Nk, D, bn, seed=1000 + D + Nq + Nk)
@@ -68,10 +84,10 @@ def test_rescale_factor_reaches_the_first_accumulator_update(D, Nq, Nk, causal, 
     sm = D ** -0.5
     rq = O.p_requant_reference if p_round == "reference" else O.p_requant_rne
     kw = {} if vsb is None else {"v_scale_block": vsb}
-    got, lse = M.attention_full_int8(*gpu(q8, k8, v8, qs, ks, vs), causal, sm, num_splits=splits, p_round=p_round,
+    got, lse = M.attention_full_int8(*repeated(reps, *gpu(q8, k8, v8, qs, ks, vs)), causal, sm, num_splits=splits, p_round=p_round,
                                      return_lse=True, **kw)
     torch.cuda.synchronize()
-    got = got.float().cpu()
+    got, lse = first_heads(got, H).float().cpu(), first_heads(lse, H)
     if splits > 1:
         ref = O.attention_full_int8_splitkv(q8, k8, v8, qs, ks, vs, causal, sm, splits, block_n=bn, p_requant=rq)
     else:
@@ -115,6 +131,16 @@ def identity_v(B, H, Nk, D, shift):
 @pytest.mark.parametrize("D,Nq,Nk", [(128, 128, 128), (128, 384, 128), (64, 256, 64), (256, 128, 64), (128, 16, 128), (64, 33, 64)])
 @pytest.mark.parametrize("pattern", ["powers_of_two", "random"])
 def test_reference_rounding_packs_every_byte(D, Nq, Nk, pattern):
+    check_packed_bytes(D, Nq, Nk, pattern)
+
+
+@pytest.mark.parametrize("D,Nq,Nk", [(128, 128, 128), (128, 384, 128), (64, 256, 64), (256, 128, 64)])
+@pytest.mark.parametrize("pattern", ["powers_of_two", "random"])
+def test_reference_rounding_packs_every_byte_in_the_general_kernels(D, Nq, Nk, pattern):
+    check_packed_bytes(D, Nq, Nk, pattern, reps=repetitions(1, 2, Nq))
+
+
+def check_packed_bytes(D, Nq, Nk, pattern, reps=1):
     """One key block, V = identity (shifted to reach the keys beyond head_dim): P8 read back from the output."""
     B, H = 1, 2
     bn = M.block_n("full", D)
@@ -140,7 +166,7 @@ def test_reference_rounding_packs_every_byte(D, Nq, Nk, pattern):
     ref_rows = torch.zeros((B, H, Nq, Nk))
     for shift in range(0, Nk, D):
         v8 = identity_v(B, H, Nk, D, shift)
-        got = M.attention_full_int8(*gpu(q8, k8, v8, qs, ks, vs), False, sm, p_round="reference")
+        got = first_heads(M.attention_full_int8(*repeated(reps, *gpu(q8, k8, v8, qs, ks, vs)), False, sm, p_round="reference"), H)
         torch.cuda.synchronize()
         ref = O.attention_full_int8(q8, k8, v8, qs, ks, vs, False, sm, block_n=bn, p_requant=O.p_requant_reference)
         ncol = min(Nk - shift, D)

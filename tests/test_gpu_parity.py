@@ -13,6 +13,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -85,7 +86,7 @@ def test_qk_int32_extreme_values():
     (1, 2, 1024, 128, False),
     (1, 2, 256, 256, False),       # head_dim 256 runs with 64-key blocks
     (2, 2, 384, 256, True),
-    (1, 2, 512, 256, True),        # four query blocks: two per workgroup
+    (1, 2, 512, 256, True),        # four query blocks of 128 rows
 ])
 @pytest.mark.parametrize("p_round", ["rne", "reference"])
 def test_full_int8_matches_oracle(B, H, N, D, causal, p_round):
@@ -104,6 +105,32 @@ def test_full_int8_matches_oracle(B, H, N, D, causal, p_round):
     assert_same_rounding(o, same)
     exact = O.attention_exact(x["q"], x["k"], x["v"], causal, sm)
     assert max_abs(o, exact) <= 6e-2                        # quantisation error itself, reported by the bench
+
+
+# The single passes of a few heads in this file are small grids, which the decode-shaped kernels take; here the same arithmetic runs in the
+# general kernels (other lengths, masks and options: test_gpu_random_shapes.py)
+@pytest.mark.parametrize("B,H,N,D,causal", [(1, 4, 256, 64, False), (2, 3, 333, 64, True), (1, 4, 671, 128, False), (1, 2, 512, 128, True),
+                                            (1, 2, 200, 128, True), (2, 2, 384, 256, True), (1, 2, 130, 256, False)])
+@pytest.mark.parametrize("variant", ["full-rne", "full-reference", "half", "fp"])
+def test_general_kernels_match_oracle(variant, B, H, N, D, causal):
+    x = quantised(B, H, N, D, seed=12)
+    sm = D ** -0.5
+    bn = M.block_n(variant.split("-")[0], D)
+    # (head_dim 64 of the 16-bit P V: past the grids of the pipelined kernel as well)
+    many = lambda *names: gpu(*repeated(repetitions(B, H, N, rows=128 if D == 64 else 32), *(x[n] for n in names)))
+    if variant.startswith("full"):
+        p_round = variant.split("-")[1]
+        names = ("q8", "k8", "v8", "qs", "ks", "vs")
+        o, lse = M.attention_full_int8(*many(*names), causal, sm, p_round=p_round, return_lse=True)
+        ref, lse_ref = O.attention_full_int8(*(x[n] for n in names), causal, sm, block_n=bn, return_lse=True,
+                                             p_requant=O.p_requant_rne if p_round == "rne" else O.p_requant_reference)
+        assert_same_rounding(first_heads(o, H), ref)
+    else:
+        names = ("q8", "k8", "v", "qs", "ks") if variant == "half" else ("q", "k", "v")
+        o, lse = (M.attention_int8 if variant == "half" else M.attention)(*many(*names), causal, sm, return_lse=True)
+        ref, lse_ref = (O.attention_int8 if variant == "half" else O.attention_fp)(*(x[n] for n in names), causal, sm, block_n=bn, return_lse=True)
+        assert max_abs(first_heads(o, H), ref) <= 2e-3 and mean_rel(first_heads(o, H), ref) <= 3e-4
+    assert (first_heads(lse, H).cpu() - lse_ref).abs().max().item() <= 2e-3
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])

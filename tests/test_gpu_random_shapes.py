@@ -3,7 +3,8 @@ oracle.  The fixed-shape tests pin named cases; these draw the combinations nobo
 query and key lengths on either side of every tile size, grouped K/V heads, per-batch cache lengths, both P roundings,
 all output and scale types, blocked V scales, split counts, the causal mask with more or fewer queries than keys.  A case
 is a pure function of its seed (printed in the test id).  Outputs, every row's log-sum-exp and the rows that see no key
-are checked.
+are checked.  Single passes of this size are small grids, which the decode-shaped kernels take: the tests named "general" repeat the
+heads until the general kernels do.
 
 Bounds (mean-rel = mean|a-b| / mean|b|):
   full-int8, single pass, against the oracle at the kernel's key block and rounding: fp16 out max-abs 2e-2 / mean-rel
@@ -23,6 +24,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -88,7 +90,20 @@ def full_int8_case(seed):
 
 @pytest.mark.parametrize("seed", range(1000, 1090))
 def test_full_int8_random_case(seed):
-    c = full_int8_case(seed)
+    check_full_int8_case(full_int8_case(seed), seed)
+
+
+@pytest.mark.parametrize("seed", range(3000, 3060))
+def test_full_int8_random_case_of_the_general_kernels(seed):
+    """A single pass over more than 64 query rows, with its heads repeated past the grids that the decode-shaped kernels take; two of three
+    with blocked V scales."""
+    c = next(c for c in (full_int8_case(100 * seed + i) for i in range(100)) if c["Nq"] > 64)
+    c["splits"] = 1
+    c["vb"] = (1 + seed % 2) * c["bn"] if seed % 3 else None
+    check_full_int8_case(c, seed, reps=repetitions(c["B"], c["Hkv"] * c["g"], c["Nq"]))
+
+
+def check_full_int8_case(c, seed, reps=1):
     B, Hkv, g, Nq, Nk, D, vb = c["B"], c["Hkv"], c["g"], c["Nq"], c["Nk"], c["D"], c["vb"]
     gen = torch.Generator().manual_seed(seed)
     q = torch.randn((B, Hkv * g, Nq, D), generator=gen).half()
@@ -105,8 +120,9 @@ def test_full_int8_random_case(seed):
         kw["v_scale_block"] = vb
     if c["lens"]:
         kw["seqlens_k"] = torch.tensor(c["lens"], dtype=torch.int32, device=DEV)
-    o, lse = M.attention_full_int8(q8.to(DEV), k8.to(DEV), v8.to(DEV), qs.to(DEV), ks.to(DEV), vs.to(DEV), c["causal"], c["sm"], **kw)
+    o, lse = M.attention_full_int8(*(t.to(DEV) for t in repeated(reps, q8, k8, v8, qs, ks, vs)), c["causal"], c["sm"], **kw)
     torch.cuda.synchronize()
+    o, lse = first_heads(o, Hkv * g), first_heads(lse, Hkv * g)
     rq = O.p_requant_rne if c["pr"] == "rne" else O.p_requant_reference
     rep = lambda t: t.repeat_interleave(g, dim=1)
     for b in range(B):
@@ -157,7 +173,18 @@ def f16pv_case(seed):
 
 @pytest.mark.parametrize("seed", range(2000, 2090))
 def test_half_int8_and_fp_random_case(seed):
-    c = f16pv_case(seed)
+    check_half_int8_and_fp_case(f16pv_case(seed), seed)
+
+
+@pytest.mark.parametrize("seed", range(4000, 4040))
+def test_half_int8_and_fp_random_case_of_the_general_kernels(seed):
+    """As above; head_dim 64 past the pipelined kernel's grids too in every other case (head_dim 128 has no decode-shaped form past 64 rows)."""
+    c = next(c for c in (f16pv_case(100 * seed + i) for i in range(100)) if c["Nq"] > 64 and c["D"] != 128)
+    c["splits"] = 1
+    check_half_int8_and_fp_case(c, seed, reps=repetitions(c["B"], c["Hkv"] * c["g"], c["Nq"], rows=128 if seed % 2 else 32))
+
+
+def check_half_int8_and_fp_case(c, seed, reps=1):
     B, Hkv, g, Nq, Nk, D, dt = c["B"], c["Hkv"], c["g"], c["Nq"], c["Nk"], c["D"], c["dt"]
     gen = torch.Generator().manual_seed(seed)
     q = torch.randn((B, Hkv * g, Nq, D), generator=gen).to(dt)
@@ -170,10 +197,11 @@ def test_half_int8_and_fp_random_case(seed):
         q8, qs = O.quant_pertoken(q)
         k8, ks = O.quant_pertoken(k)
         qs, ks = qs.to(c["sdt"]), ks.to(c["sdt"])
-        o, lse = M.attention_int8(q8.to(DEV), k8.to(DEV), v.to(DEV), qs.to(DEV), ks.to(DEV), c["causal"], c["sm"], **kw)
+        o, lse = M.attention_int8(*(t.to(DEV) for t in repeated(reps, q8, k8, v, qs, ks)), c["causal"], c["sm"], **kw)
     else:
-        o, lse = M.attention(q.to(DEV), k.to(DEV), v.to(DEV), c["causal"], c["sm"], **kw)
+        o, lse = M.attention(*(t.to(DEV) for t in repeated(reps, q, k, v)), c["causal"], c["sm"], **kw)
     torch.cuda.synchronize()
+    o, lse = first_heads(o, Hkv * g), first_heads(lse, Hkv * g)
     rep = lambda t: t.repeat_interleave(g, dim=1)
     for b in range(B):
         n = c["lens"][b] if c["lens"] else Nk

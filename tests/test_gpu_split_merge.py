@@ -50,6 +50,26 @@ def call(variant, p, ws, nbytes):
     assert fn(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
 
 
+# (here for `problem`) rows behind the last one of a ragged length: every kernel writes its valid rows only, also where a head's rows are
+# followed by room and not by the next head.  1 head: the decode-shaped kernels; past 512 workgroups: the general ones; 2 splits: the merges
+@pytest.mark.parametrize("variant,D,H,splits", [("full", 64, 1, 1), ("full", 128, 1, 1), ("full", 256, 1, 1), ("half", 64, 1, 1), ("fp", 256, 1, 1),
+                                                ("full", 64, 110, 1), ("full", 128, 110, 1), ("full", 256, 110, 1), ("half", 64, 110, 1),
+                                                ("fp", 64, 300, 1), ("half", 128, 3, 1), ("fp", 128, 3, 1), ("half", 256, 110, 1), ("fp", 256, 110, 1),
+                                                ("full", 128, 2, 2), ("full", 256, 2, 2), ("half", 128, 2, 2)])
+def test_rows_behind_the_last_one_are_not_written(variant, D, H, splits):
+    lib, N, room = _capi.load(), 130, 256
+    p, out, _, keep = problem(variant, 1, H, N, N, D, D + H)
+    p.num_splits = splits
+    ws = torch.empty((max(16, lib.intfa_fwd_merge_workspace_bytes(ctypes.byref(p))),), dtype=torch.uint8, device=DEV)
+    call(variant, p, ws, ws.numel())
+    big = torch.full((1, H, room, D), 7.0, dtype=torch.float16, device=DEV)
+    p.out = big.data_ptr()
+    p.o_stride_b, p.o_stride_h, p.o_stride_n, _ = big.stride()
+    call(variant, p, ws, ws.numel())
+    torch.cuda.synchronize()
+    assert torch.equal(big[:, :, :N], out) and (big[:, :, N:] == 7.0).all()
+
+
 def close(a, b):
     assert torch.equal(torch.isfinite(a), torch.isfinite(b))
     f = torch.isfinite(b)

@@ -7,6 +7,7 @@ import torch
 
 import intfa_oracle as O
 import int_flashattention_amd as M
+from many_heads import first_heads, repeated, repetitions
 from test_gpu_parity import DEV, MAX_ABS, MEAN_REL, assert_same_rounding, gpu, max_abs, mean_rel
 
 pytestmark = pytest.mark.gpu
@@ -47,14 +48,16 @@ def test_quant_perblock_channel_strided_input():
     assert torch.equal(q.cpu(), q_ref) and torch.equal(s.cpu(), s_ref)
 
 
-@pytest.mark.parametrize("B,H,N,D,causal,mult", [
+# (these are small grids, which the decode-shaped kernel takes unless head_dim 128 has 64-key scale rows; the second test below runs them in
+# the general kernels)
+SHAPES = [
     (1, 2, 512, 128, False, 1),
     (2, 2, 384, 64, True, 1),
     (1, 2, 512, 128, True, 2),         # one scale row per two key blocks of the kernel
-    (1, 2, 256, 256, False, 1),        # head_dim 256: 64-key blocks, column halves
+    (1, 2, 256, 256, False, 1),        # head_dim 256: 64-key blocks
     (1, 2, 320, 256, True, 2),
-    (1, 2, 384, 256, True, 1),         # three query blocks: one per workgroup, heaviest first
-    (2, 3, 512, 256, True, 1),         # four query blocks: paired in one workgroup
+    (1, 2, 384, 256, True, 1),         # three query blocks of 128 rows
+    (2, 3, 512, 256, True, 1),         # four query blocks
     (1, 3, 300, 128, False, 1),        # ragged length: the last scale row covers 44 keys
     (1, 2, 97, 64, True, 1),
     # 64-key scale rows under the 128-key block: the granularity of the reference's CUDA kernel (kBlockN = 64 at
@@ -65,16 +68,32 @@ def test_quant_perblock_channel_strided_input():
     (1, 2, 200, 128, False, 0.5),      # the last block's second half holds 8 keys
     (1, 2, 160, 64, False, 1),         # head_dim 64: a scale row per 64-key block is the kernel's own block
     (1, 2, 40, 128, True, 0.5),        # few query rows (the decode-shaped kernel has no 64-key rows: the general one runs)
-])
+]
+
+
+@pytest.mark.parametrize("B,H,N,D,causal,mult", SHAPES)
 @pytest.mark.parametrize("p_round", ["rne", "reference"])
 def test_blocked_v_scale_matches_oracle(B, H, N, D, causal, mult, p_round):
+    check_against_oracle(B, H, N, D, causal, mult, p_round)
+
+
+# (the last four: more key blocks per row)
+@pytest.mark.parametrize("B,H,N,D,causal,mult", [c for c in SHAPES if c[2] > 64 and not (c[3] == 128 and c[5] == 0.5)] + [
+    (1, 2, 512, 64, False, 2), (1, 1, 700, 64, True, 1), (1, 1, 700, 128, True, 1), (1, 1, 700, 256, True, 1)])
+@pytest.mark.parametrize("p_round", ["rne", "reference"])
+def test_blocked_v_scale_of_the_general_kernels_matches_oracle(B, H, N, D, causal, mult, p_round):
+    check_against_oracle(B, H, N, D, causal, mult, p_round, reps=repetitions(B, H, N))
+
+
+def check_against_oracle(B, H, N, D, causal, mult, p_round, reps=1):
     bn = M.block_n("full", D)
     vsb = int(bn * mult)
     x = blocked_inputs(B, H, N, D, 80, vsb)
     sm = D ** -0.5
-    o, lse = M.attention_full_int8(*gpu(x["q8"], x["k8"], x["v8"], x["qs"], x["ks"], x["vs"]), causal, sm, p_round=p_round,
+    o, lse = M.attention_full_int8(*repeated(reps, *gpu(x["q8"], x["k8"], x["v8"], x["qs"], x["ks"], x["vs"])), causal, sm, p_round=p_round,
                                    v_scale_block=vsb, return_lse=True)
     torch.cuda.synchronize()
+    o, lse = first_heads(o, H), first_heads(lse, H)
     assert o.dtype == torch.float16 and o.shape == (B, H, N, D)
     ref, lse_ref = O.attention_full_int8(x["q8"], x["k8"], x["v8"], x["qs"], x["ks"], x["vs"], causal, sm, block_n=bn,
                                          v_scale_block=vsb, return_lse=True)

@@ -183,7 +183,6 @@ int launch_combine(const intfa_fwd_params* p, const KParams& kp, hipStream_t str
 // Not half-int8 and fp16 at head_dim 128: there two of the four waves have no share of Q K^T, the gain ends at 10 %, and the
 // kernels differ in the rounding of P.  Everywhere else both kernels give the same bits, so that an output does not depend on how
 // many heads and batch entries it is computed with.
-constexpr int kComputeUnits = 256;
 bool decode_shaped(int seqlen) { return seqlen <= kDecodeMaxRows; }
 // (scale rows of 64 keys under the 128-key block: the decode kernel has one scale row per block)
 bool decode_kernel_takes(int variant, const KParams& kp) {
@@ -308,7 +307,7 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
     if (p->batch <= 0 || p->heads <= 0) return INTFA_ERR_SHAPE;
     if (p->seqlen <= 0 || p->seqlen_k < 0) return INTFA_ERR_SEQLEN;
     if (p->head_dim != 64 && p->head_dim != 128 && p->head_dim != 256) return INTFA_ERR_HEAD_DIM;
-    const int cus = num_cus > 0 ? num_cus : 256;
+    const int cus = num_cus > 0 ? num_cus : kComputeUnits;
     int64_t slots = 2ll * cus;                                                 // two workgroups per compute unit
     int64_t wgs = (int64_t)p->batch * p->heads * ((p->seqlen + kBlockM - 1) / kBlockM);
     const bool decode = decode_shaped(p->seqlen);

@@ -5,6 +5,11 @@
 
 namespace intfa {
 
+// The MI355X as one device: 8 XCDs of 32 compute units.  The mapping of workgroups to XCDs and the lines between kernels are laid out for
+// it; on a partition of the card with fewer of either, the lines lie too high and the order is less even, with the same results.
+// (intfa_fwd_suggest_splits takes the device's number from its caller, because a split count may change the results.)
+constexpr int kXcds = 8, kCusPerXcd = 32, kComputeUnits = kXcds * kCusPerXcd;
+
 constexpr int kDecodeMaxRows = 64;    // most query rows per head of a decode-shaped call
 constexpr int kDecodeRows = 32;       // query rows per workgroup of the decode-shaped kernel (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h)
 
@@ -31,14 +36,14 @@ inline KParams finish_mapping(const KParams& kp, int grid) {
     k.per_head = grid / (kp.batch * kp.heads);
     k.heads_kv = kp.heads / kp.kv_group;
     const int per_kv = k.per_head * kp.kv_group, units = kp.batch * k.heads_kv;
-    k.xcd_whole_wgs = (units / 8) * 8 * per_kv;
+    k.xcd_whole_wgs = (units / kXcds) * kXcds * per_kv;
     k.rem_wgs = grid - k.xcd_whole_wgs;
-    k.xcd_rem_chunk = ((units % 8) * per_kv) % 8 == 0 ? (units % 8) * per_kv / 8 : 0;
+    k.xcd_rem_chunk = ((units % kXcds) * per_kv) % kXcds == 0 ? (units % kXcds) * per_kv / kXcds : 0;
     // Causal: groups of K/V heads with two rounds of an XCD's workgroup slots (32 compute units; two workgroups each, four at
     // head_dim 64; four rounds at head_dim 256, one each) whose K and V come to 9 MB at most, since all of a group's heads are read at
     // once.  Larger groups lose to the 4 MB L2 (half-int8 B8 H32 N2048 d128: 298 us up to 12 MB, 313 us at 48), smaller ones end
     // unevenly (full-int8 B4 H32 N4096 d64: 390 us with two heads, 349 with eight).
-    const int xcd_units = units / 8, slots = kp.head_dim == 64 ? 256 : 128;
+    const int xcd_units = units / kXcds, slots = 2 * kCusPerXcd * (kp.head_dim == 64 ? 4 : 2);
     const int by_slots = slots / per_kv, by_bytes = (int)(9000000 / ((int64_t)kp.seqlen_k * kp.kv_key_bytes));
     int run_units = by_slots < by_bytes ? by_slots : by_bytes;
     run_units = run_units < xcd_units ? run_units : xcd_units;
@@ -50,7 +55,7 @@ inline KParams finish_mapping(const KParams& kp, int grid) {
     k.d_run = make_fast_div(k.run_units * per_kv);
     k.d_run_heads = make_fast_div(k.run_units * kp.kv_group);
     k.d_run_heads_last = make_fast_div(k.run_units_last * kp.kv_group);
-    k.d_rem_heads = make_fast_div(units % 8 > 0 ? (units % 8) * kp.kv_group : 1);
+    k.d_rem_heads = make_fast_div(units % kXcds > 0 ? (units % kXcds) * kp.kv_group : 1);
     k.d_per_kv = make_fast_div(k.per_head * kp.kv_group);
     k.d_heads_kv = make_fast_div(k.heads_kv);
     k.d_per_head = make_fast_div(k.per_head);

@@ -265,7 +265,7 @@ template <int DT, int LPR> __global__ void __launch_bounds__(256) quant_slice_ap
 // Steps of 256 / LPR rows per workgroup of a streaming launch: one while more would leave fewer than eight workgroups per compute
 // unit; more than kStreamSteps, in rounds, where a grid would exceed what a launch may have.
 int stream_steps(int64_t steps) {
-    const int64_t fill = steps / (256 * 8), cap = steps >> 22;
+    const int64_t fill = steps / (kComputeUnits * 8), cap = steps >> 22;
     const int64_t n = fill < kStreamSteps ? fill : kStreamSteps;
     return (int)(n < 1 ? 1 : (n > cap ? n : cap + 1));
 }

@@ -97,7 +97,9 @@ constexpr int kRowsInFlight = 8;    // independent 16-byte loads a lane has in f
 // 256 / LPR rows: 16 KiB of input in one piece, all loads at once, and no further round.  B4 H32 N4096 d128 fp16 (134 MB in, 67 MB
 // out), us: a persistent grid of 2048 workgroups whose eight loads lie 8 MB apart 50.5; the same loads in one 32 KiB piece and no
 // second round 42.0; 16 KiB pieces 37.8; and read and written past the caches (non-temporal: each line is touched once) 33.5,
-// 6.0 TB/s (a copy of the same traffic without arithmetic: 34.7).
+// 6.0 TB/s (a copy of the same traffic without arithmetic: 34.7).  What reads the int8 rows next does not miss the caches: Q, K, V written by
+// a kernel, quantised and attended, non-temporal against plain, us: B1 H8 N250 d64 20.6 / 20.3, B1 H16 N512 d128 30.6 / 30.4, B1 H32 N1024
+// 51.9 / 52.3, N2048 86.9 / 90.5, N4096 191 / 195 (causal), B4 H32 N4096 1035 / 1057.
 constexpr int kStreamSteps = 4;
 __device__ __forceinline__ void store_stream(v2i v, char* a) {
     __builtin_nontemporal_store(v, (v2i*)a);

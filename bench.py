@@ -108,9 +108,9 @@ WORKLOADS = {
 # them, NOT measured in the run that prints them (counters need the profiler); workloads without a profile report None.
 MEASURED_TRAFFIC_BYTES = {
     # FETCH_SIZE x 1.9997 + WRITE_SIZE x 1.0 (KiB per dispatch, factors from a 256 MiB copy): 194.3 MiB read + 128 MiB written
-    "full_int8_B4_H32_N4096_d128": (337941156, "profiles/fwd_full_int8_d128_B4_H32_N4096.txt"),
+    "full_int8_B4_H32_N4096_d128": (337920763, "profiles/fwd_full_int8_d128_B4_H32_N4096.txt"),
     # FETCH_SIZE x 1.9998 + WRITE_SIZE 256 x 1.0: 1032.2 MiB read + 0.25 MiB written (algorithmic: 1082523648)
-    "full_int8_decode_B32_H32_Nq1_Nk4096_d128": (1082595402, "profiles/fwd_decode_full_int8_d128_B32_H32_Nq1_Nk4096.txt"),
+    "full_int8_decode_B32_H32_Nq1_Nk4096_d128": (1082598465, "profiles/fwd_decode_full_int8_d128_B32_H32_Nq1_Nk4096.txt"),
 }
 
 
@@ -204,7 +204,7 @@ def bench_quant(args, variant, x, B, H, N, D, dt):
                         "frac": alg_bytes / (kern_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
                         "kernel": {"quant_token": "quant_pertoken_kernel", "quant_block": "quant_blockchan_kernel",
                                    "quant_tensor": "quant_slice_amax_kernel + quant_slice_apply_kernel",
-                                   "quant_append": "kv_append_kernel (keys) + kv_append_kernel (values)"}[variant],
+                                   "quant_append": "kv_append_kernel (keys and values)"}[variant],
                         "avg_launch_ms": kern_ms, "median_launch_ms": statistics.median(per_launch_ms)},
            "peak_check": device_peak_check(torch, x.device), "device_spinup": spin}
     print(json.dumps(out))
@@ -382,7 +382,9 @@ def main():
         peak_model, dtype_s = "half of the ops at the int8 rate (5033 T), half at the fp16 rate (2517 T)", "int8+f16"
     else:
         peak, peak_model, dtype_s = FP16_PEAK_TFLOPS, "256 CU x 2.4 GHz x 4096 fp16 flops/clk/CU", "f16"
-    kernel_name = "fwd_full_int8_kernel" if variant == "full" else "fwd_f16pv_kernel"
+    # (the kernels that these workloads run; which one a call runs also depends on its grid)
+    kernel_name = {64: "fwd_full_int8_kernel", 128: "fwd_full_int8_kernel", 256: "fwd_full_int8_pair_kernel"}[D] if variant == "full" else \
+                  {64: "fwd_f16pv_kernel", 128: "fwd_f16pv_pipe_kernel", 256: "fwd_f16pv_pair_kernel"}[D]
     out = {
         "metric": "attention fwd TOPS + % int8 MFMA peak, B4 H32 N4096 d128 full-int8",
         "value": value, "unit": "TOPS", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
@@ -401,7 +403,7 @@ def main():
                      "frac": achieved / peak, "traffic": traffic_of(args.workload)[0], "traffic_source": traffic_of(args.workload)[1],
                      "kernel": kernel_name, "avg_launch_ms": kern_ms, "median_launch_ms": kern_med_ms,
                      "achieved_at_median": ops / (kern_med_ms * 1e-3) / 1e12, "peak_model": peak_model,
-                     "launch_includes": "forward kernel" + (" + split-KV combine kernel" if splits != 1 else "")},
+                     "launch_includes": "forward kernel" + (", which merges the split-KV partials" if splits != 1 else "")},
         "peak_check": device_peak_check(torch, dev),
         "device_spinup": spin,
     }
@@ -428,7 +430,7 @@ def main():
         out["roofline"] = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
                            "traffic": traffic_of(args.workload)[0], "traffic_source": traffic_of(args.workload)[1],
                            "kernel": "fwd_decode_full_int8_kernel" if variant == "full" else "fwd_decode_f16pv_kernel", "avg_launch_ms": kern_ms, "median_launch_ms": kern_med_ms,
-                           "launch_includes": "forward kernel" + (" + split-KV combine kernel" if splits != 1 else "")}
+                           "launch_includes": "forward kernel" + (", which merges the split-KV partials" if splits != 1 else "")}
         if other_round is not None:         # the same bytes over the other rounding's launch time
             g_o = alg_bytes / (other_round["avg_launch_ms"] * 1e-3) / 1e9
             out["roofline_" + other_round["p_round"] + "_rounding"].update(

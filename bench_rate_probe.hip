@@ -15,10 +15,10 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 enum Kind { ADD, MUL, FMA, MOV, SUB_INLINE, ADD_SGPR, CVT_I32, MAX3, MAX, CVT_PK_U8, CVT_PK_F16, PK_MUL_F16, PK_ADD_F16,
-            CVT_U16_SDWA, DOT2, PERM, FMA_MIX, LDEXP, XOR, LSHL, EXP, RCP, FMA_F16, NKIND };
+            PK_FMA_F16, DOT2, PERM, FMA_MIX, LDEXP, XOR, LSHL, EXP, RCP, FMA_F16, NKIND };
 static const char* kind_name[NKIND] = {"v_add_f32", "v_mul_f32", "v_fma_f32", "v_mov_b32", "v_sub_f32 (inline constant)",
     "v_add_f32 (SGPR operand)", "v_cvt_f32_i32", "v_max3_f32", "v_max_f32", "v_cvt_pk_u8_f32", "v_cvt_pk_f16_f32", "v_pk_mul_f16",
-    "v_pk_add_f16", "v_cvt_u16_f16 (SDWA byte write)", "v_dot2_f32_f16", "v_perm_b32", "v_fma_mix_f32", "v_ldexp_f32", "v_xor_b32",
+    "v_pk_add_f16", "v_pk_fma_f16", "v_dot2_f32_f16", "v_perm_b32", "v_fma_mix_f32", "v_ldexp_f32", "v_xor_b32",
     "v_lshlrev_b32", "v_exp_f32", "v_rcp_f32", "v_fma_f16"};
 
 template <int K> __device__ __forceinline__ void emit(float& x, float a, float b) {
@@ -35,7 +35,7 @@ template <int K> __device__ __forceinline__ void emit(float& x, float a, float b
     if (K == CVT_PK_F16) asm volatile("v_cvt_pk_f16_f32 %0, %0, %1" : "+v"(x) : "v"(a), "v"(b));
     if (K == PK_MUL_F16) asm volatile("v_pk_mul_f16 %0, %0, %1" : "+v"(x) : "v"(a), "v"(b));
     if (K == PK_ADD_F16) asm volatile("v_pk_add_f16 %0, %0, %1" : "+v"(x) : "v"(a), "v"(b));
-    if (K == CVT_U16_SDWA) asm volatile("v_cvt_u16_f16_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_1" : "+v"(x) : "v"(a), "v"(b));
+    if (K == PK_FMA_F16) asm volatile("v_pk_fma_f16 %0, %0, %1, %2" : "+v"(x) : "v"(a), "v"(b));
     if (K == DOT2) asm volatile("v_dot2_f32_f16 %0, %1, %2, %0" : "+v"(x) : "v"(a), "v"(b));
     if (K == PERM) asm volatile("v_perm_b32 %0, %0, %1, %2" : "+v"(x) : "v"(a), "v"(b));
     if (K == FMA_MIX) asm volatile("v_fma_mix_f32 %0, %0, %1, %2" : "+v"(x) : "v"(a), "v"(b));
@@ -119,7 +119,7 @@ int main() {
     if (hipMalloc(&g_out, 256 * 16 * 64 * 4) != hipSuccess) { printf("no GPU\n"); return 1; }
     printf("A. one kind, 64 independent instructions per trip: SIMD ns per instruction at 1 / 2 / 4 waves per SIMD\n");
     alone<ADD>(); alone<MUL>(); alone<FMA>(); alone<MOV>(); alone<SUB_INLINE>(); alone<ADD_SGPR>(); alone<CVT_I32>(); alone<MAX3>();
-    alone<MAX>(); alone<CVT_PK_U8>(); alone<CVT_PK_F16>(); alone<PK_MUL_F16>(); alone<PK_ADD_F16>(); alone<CVT_U16_SDWA>(); alone<DOT2>();
+    alone<MAX>(); alone<CVT_PK_U8>(); alone<CVT_PK_F16>(); alone<PK_MUL_F16>(); alone<PK_ADD_F16>(); alone<PK_FMA_F16>(); alone<DOT2>();
     alone<PERM>(); alone<FMA_MIX>(); alone<LDEXP>(); alone<XOR>(); alone<LSHL>(); alone<EXP>(); alone<RCP>(); alone<FMA_F16>();
     printf("B. two kinds alternating, two waves per SIMD: SIMD ns per PAIR\n");
     pair<CVT_I32, ADD>(); pair<CVT_I32, FMA>(); pair<MAX3, MUL>(); pair<CVT_PK_U8, ADD>(); pair<CVT_I32, CVT_PK_U8>(); pair<ADD, MUL>();

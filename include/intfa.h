@@ -101,7 +101,15 @@ typedef struct intfa_fwd_params {
     int32_t causal;           /* 0 / 1.  Query row i sees keys 0 .. i + (seqlen_k - seqlen): with equal lengths the reference's
                                  mask (flash_atten_full_int8.py:39-43); with more keys than queries (a chunk of new tokens
                                  against a cache) the mask is aligned to the bottom right corner as in the reference's CUDA
-                                 tree (csrc/mask.h:53,172).  A row that sees no key (fewer keys than queries) gives zeros. */
+                                 tree (csrc/mask.h:53,172).  A row that sees no key (fewer keys than queries) gives zeros.
+                                 Hidden keys have no part in a row's result as long as V (and blocked V scales) are finite.
+                                 A value that is not finite, for instance in the padding behind a prompt, reaches rows in
+                                 front of it only inside a tile: the 32 rows computed together share the 32-key range of
+                                 their last key (rows at most 31 before the value with equal lengths, 62 otherwise).
+                                 Head_dim 256 with a 16-bit V on large grids: 128 rows share their last 64-key block (127,
+                                 190).  Blocked V scales: the rows computed together (32; 128 for large grids at head_dim 256)
+                                 share the key block of their last key, at head_dim 128 with v_scale_block = 64 the
+                                 128-key block. */
     float   sm_scale;
     int32_t p_round;          /* INTFA_PROUND_* (full-int8 only) */
 
@@ -142,7 +150,7 @@ typedef struct intfa_fwd_params {
                                  key/value cache filled to different lengths; the counterpart of the reference's
                                  seqused_k and of cu_seqlens_k used as lengths, csrc/flash.h:95-99,149-151,
                                  csrc/block_info.h:21-22).  k, v and k_scale keep their seqlen_k-row layout; rows past a
-                                 batch entry's length are not read.  An entry with no key gives zeros (lse = -inf).
+                                 batch entry's length are not read, nor scale rows of v_scale past it.  An entry with no key gives zeros (lse = -inf).
                                  NULL = every entry has seqlen_k keys.  With causal the mask of an entry is aligned to
                                  its own length. */
     int32_t causal_rows;      /* 0, or the number of query positions when the row axis holds several query heads of one
@@ -172,8 +180,11 @@ int intfa_fwd_block_n(int variant, int head_dim);
 /* A split count for the problem in *p (its num_splits and workspace members are ignored): 1 when the single-pass grid
  * already fills the GPU, otherwise enough splits to reach about two workgroups per compute unit while leaving every split
  * at least four key blocks (decode-shaped half-int8 and fp16 calls that stay within one workgroup per compute unit: at
- * least 128 keys, up to 16 splits; fewer where merging many query rows would take longer than the splits save); the
- * counterpart of the heuristic that lives in the reference's absent flash_api.cpp
+ * least 128 keys, up to 16 splits; fewer where merging many query rows would take longer than the splits save).  The count is
+ * a choice for speed that may differ between versions of the library, and the results depend on it: P is rounded in the
+ * frame of each split's running maximum (full-int8: to int8, about 2e-2 of the output between counts; half-int8 and fp16: to
+ * 16 bits, about one rounding of the 16-bit output), with no count closer to exact attention than another.  A caller who
+ * needs the same bits passes the count.  The counterpart of the heuristic that lives in the reference's absent flash_api.cpp
  * (csrc/flash_fwd_launch_template.h:193-253 only consumes it).  variant: INTFA_VARIANT_*; num_cus: compute units of
  * the device, 0 = 256 (MI355X).  Negative INTFA_ERR_* for a rejected block. */
 int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus);

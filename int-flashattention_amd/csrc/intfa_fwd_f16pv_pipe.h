@@ -2,11 +2,14 @@
 // in grids that leave a SIMD two waves.
 //
 // What bounds the kernel: a block's Q K^T, softmax and P V in turn leave the matrix pipe idle during the softmax and the vector pipe
-// during the products, and with two waves per SIMD the other wave fills only part of that (matrix pipe busy 47 % of the cycles at fp16
-// B4 H32 N4096).  Here every MFMA of block n+1's Q K^T and of block n-1's P V is followed by its share of block n's softmax: 2.07 M
-// cycles become 1.70 M per XCD.  Large launches then meet the power limit of the card (1.86 GHz before, 1.62 GHz now), so the time
-// falls by less than the cycles; short ones keep the clock.  B4 H32 d128, us, before -> with the pipeline: N4096 fp16 1106 -> 1038,
-// causal 608 -> 563, half-int8 969 -> 929; N512 fp16 causal 27.6 -> 21.0, half-int8 30.3 -> 21.0, causal 30.1 -> 18.5.
+// during the products, and with two waves per SIMD the other wave fills only part of that.  Here every MFMA of block n+1's Q K^T and of
+// block n-1's P V is followed by its share of block n's softmax.  By the counters, before -> with the pipeline: fp16 B4 H32 N4096 d128
+// 2.09 M -> 1.74 M clocks, matrix pipe busy 50 -> 60 % of them; half-int8 1.87 M -> 1.72 M, 42 -> 46 %.  The card lowers its clock under
+// that load (1.86 -> 1.63 GHz, 1.90 -> 1.81), so the time falls by less than the clocks.  Causal half-int8 B8 H32 N2048 keeps 2.03 GHz and has neither
+// pipe full (matrix 35 %, 30 % of the waves' time in waits): its workgroups are 17 key blocks long on average and fill and drain the
+// pipeline each for itself, 2120 clocks per wave and block where the non-causal launch takes 1670.
+// B4 H32 d128, us, before -> with the pipeline: N4096 fp16 1106 -> 1038, causal 608 -> 563, half-int8 969 -> 929; N512 fp16 causal
+// 27.6 -> 21.0, half-int8 30.3 -> 21.0, causal 30.1 -> 18.5.
 // (Two row blocks per wave at one wave per SIMD halve the LDS reads per MFMA: fp16 N4096 another 6 %, but half-int8, whose dequantisation
 // fills the issue slots, loses 15 %, and every grid of fewer than some hundred workgroups loses; not kept.)
 #pragma once

@@ -272,7 +272,8 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
             for (int g = 0; g < NG; ++g) pall[g] = *(const v4i*)(smem + xp_rd + 1024 * g);
             if (tail) {
                 // sub-tiles past the last key that any of the rows sees (the second block of a step may lie past the range): P is
-                // zero there, but zero times a V that is not finite (what a prompt's padding may hold) is not
+                // zero there, but zero times a V that is not finite (what a prompt's padding may hold) is not.  (fp16 B1 H16 N1000 causal d64
+                // 13.3 -> 13.5 us; a masked copy of the loop below that skips their MFMAs: 13.8)
                 asm volatile("");
                 const int seen = (last_lim < key_end - 1 ? last_lim : key_end - 1) - key0;
 #pragma unroll

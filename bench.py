@@ -5,7 +5,7 @@ Prints ONE JSON line.  `value` is whole-job throughput in TOPS with the work mod
 ops = 4*B*H*N^2*d (x0.5 causal; benchmark.py:90-93), inputs resident in HBM before the timed region.
 `roofline` prices the forward kernel against the dense int8 MFMA peak from per-launch HIP-event times;
 `cpu_baseline` times the CPU oracle (a port of the reference's quantised arithmetic) on a bounded sample of the
-same workload - one (batch, head) slice - on this box's host cores.
+same workload - one (batch, head) slice - on the host's cores.
 """
 import argparse
 import json
@@ -71,7 +71,7 @@ WORKLOADS = {
     "full_int8_B16_H16_N1024_d256_bf16": dict(variant="full", B=16, H=16, N=1024, D=256, causal=False, splits=1,
                                               dtype="bfloat16", std=0.5),
     # the grid of the reference's own benchmark script (benchmark.py:23-45: BATCH, N_HEADS, HEAD_DIM = 4, 32, 64, N_CTX = 2^10 ..
-    # 2^14, non-causal, providers full-int8 / int8 / fp16), with this build's input recipe
+    # 2^14, non-causal, providers full-int8 / int8 / fp16), with this file's input recipe
     "full_int8_B4_H32_N1024_d64": dict(variant="full", B=4, H=32, N=1024, D=64, causal=False, splits=1),
     "full_int8_B4_H32_N4096_d64": dict(variant="full", B=4, H=32, N=4096, D=64, causal=False, splits=1),
     "full_int8_B4_H32_N16384_d64": dict(variant="full", B=4, H=32, N=16384, D=64, causal=False, splits=1),
@@ -211,7 +211,7 @@ def bench_quant(args, variant, x, B, H, N, D, dt):
 
 
 def device_spinup(torch, step, ms):
-    """The GPU's clock needs some tens of milliseconds of sustained load to leave its idle state: on these boxes the
+    """The GPU's clock needs some tens of milliseconds of sustained load to leave its idle state: the
     launch time of the headline kernel falls from 1.1 ms to its steady 0.85 ms over the first ~30 launches of a process,
     whatever ran before.  Five warm-up steps do not cover that, so the workload is run untimed for `ms` milliseconds
     first; the warm-up steps and the timed steps follow as the flags say."""
@@ -253,7 +253,7 @@ def main():
                          "HBM traffic that calibrates FETCH_SIZE / WRITE_SIZE when the run is under rocprofv3 --pmc")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py: this build measures one GPU only (every (batch, head) is independent; there is no "
+        print("bench.py: one GPU only is measured (every (batch, head) is independent; there is no "
               "multi-GPU path to time). Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
 

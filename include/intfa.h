@@ -263,7 +263,7 @@ int intfa_quant_perblock_channel(const void* x, int64_t stride_b, int64_t stride
 
 /* Appends new keys (and values) to an int8 K/V cache: the counterpart, for the quantised cache this library reads, of
  * the copy the reference's cache kernel makes of knew/vnew before it attends (csrc/flash_fwd_kernel.h:690-790,
- * Append_KV; csrc/flash.h:104-112; rotary embedding and paged caches are not part of this build).  For batch entry b the
+ * Append_KV; csrc/flash.h:104-112; rotary embedding and paged caches are not part of this library).  For batch entry b the
  * rows go to positions len_b .. len_b + seqlen_new - 1 of the cache, len_b = seqlens_k[b] (device memory, clamped to
  * [0, seqlen_cache]) or seqlen_filled when seqlens_k is NULL; rows that would land at or past seqlen_cache are dropped.
  * The lengths themselves are the caller's to advance (a forward call with seqlens_k = len + seqlen_new then sees them).

@@ -4,7 +4,7 @@
 // What bounds it: a decoding step launches kernels of 2 - 10 us each, so the host has to get from the Python call to the
 // launch in about the same time.  The same steps written in Python over ctypes (attribute accesses on tensors, one setattr
 // per field, a device context manager, record_stream through the dispatcher) took 28 - 32 us per attention call and 15 - 18 us
-// per quantiser call on the GPU boxes; here the tensors are read through their C++ objects and the arguments arrive by
+// per quantiser call; here the tensors are read through their C++ objects and the arguments arrive by
 // vectorcall, without a binding layer in between.
 //
 // Functions take positional arguments only (the keyword interface and its defaults live in the Python modules).

@@ -6,7 +6,7 @@ Tolerances: max-abs 2e-2 / mean-rel 1e-2 against the reference's quantised arith
 P rounding and the kernel's key-block length); far tighter against the oracle evaluated with the kernel's own rounding.
 
 Split-KV has no counterpart in the reference's int8 kernels (csrc/kernel_traits.h:199 leaves it open), so its
-"reference arithmetic" is a definition of this build: the oracle evaluated over the same key ranges and merged by the
+"reference arithmetic" is a definition of this package: the oracle evaluated over the same key ranges and merged by the
 reference's combine formula (csrc/flash_fwd_kernel.h:1212-1283).  A split restarts the running maximum, so its P8 are
 quantised in another frame than the single pass's: the two results differ by about the quantisation noise of P itself
 (both are equally far from exact attention).  The tests pin exactly that: the split result is within the stated bounds

@@ -125,11 +125,11 @@ size_t workspace_bytes_for(const intfa_fwd_params* p) {
     return rows * (size_t)p->head_dim * sizeof(float) + rows * sizeof(float);
 }
 
-// One 8-byte arrival word per query block of at least kDecodeRows rows, behind the partials.
+// One arrival word per query block of at least 16 rows (kTicketStride apart), behind the partials.
 size_t ticket_offset(const intfa_fwd_params* p) { return (workspace_bytes_for(p) + 7) & ~(size_t)7; }
 size_t merge_workspace_bytes_for(const intfa_fwd_params* p) {
     if (workspace_bytes_for(p) == 0) return 0;
-    return ticket_offset(p) + (size_t)p->batch * p->heads * ((p->seqlen + kDecodeRows - 1) / kDecodeRows) * sizeof(uint64_t);
+    return ticket_offset(p) + (size_t)p->batch * p->heads * ((p->seqlen + 15) / 16) * kTicketStride * sizeof(uint64_t);
 }
 
 // Epochs of the launches that merge their splits themselves: 56 bits in the upper bits of the word, counted from a random
@@ -171,11 +171,10 @@ int launch_combine(const intfa_fwd_params* p, const KParams& kp, hipStream_t str
     return e == hipSuccess ? INTFA_OK : (int)e;
 }
 
-// The pass runs a kernel whose four waves share the keys of a block and own 32 query rows together, instead of 32 each
-// (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h), where the latter would leave waves without rows or compute units without a
-// workgroup:
-//   * few query rows per head (decoding against a cache), at any size;
-//   * small problems in a single pass: four times the workgroups, each walking its keys in a fraction of the time, as
+// The pass runs a kernel whose waves share the keys of a block and own 16 or 32 query rows together, instead of 32 each, where the latter
+// would leave waves without rows or compute units without a workgroup:
+//   * few query rows per head (decoding against a cache), at any size: intfa_fwd_decode_wide.h;
+//   * small problems in a single pass (intfa_fwd_decode.h, intfa_fwd_decode_f16pv.h): four times the workgroups, each walking its keys in a fraction of the time, as
 //     long as all of them are resident at once.  That is two per compute unit at head_dim 64 and for full-int8 at head_dim 128,
 //     one at head_dim 256 (a workgroup fills the LDS).  Measured around the line (general -> this, us): full-int8 d128
 //     causal B1 H16 N1024 22.7 -> 17.4, B3 H32 N256 (768 workgroups) 10.8 -> 12.8; full-int8 d256 B1 H8 N1024 31.5 -> 20.3,
@@ -196,7 +195,7 @@ bool decode_kernel_takes(int variant, const KParams& kp) {
 // caches could not keep them for the next pass anyway: 128 MiB and more, half of the last-level cache, which other layers' K and V
 // share.  Measured, three sets of inputs in turn, us, plain -> non-temporal: fp16 B32 H32 Nk4096 d128 (2.1 GB) 354 -> 306 (6.1 ->
 // 7.0 TB/s), full-int8 B16 H32/8 Nk8192 (268 MB) 53.9 -> 47.2, 134 MB 29.9 -> 28.8, 101 MB 31.6 - 32.3 -> 31.7 - 32.5; 67 MB, which the
-// cache keeps, 17.8 -> 19.7.  An instance of its own: a choice at run time inside the kernel cost the small calls 2 - 3 %.
+// cache keeps, 17.8 -> 19.7.
 constexpr int64_t kStreamKvBytes = 128ll << 20;
 bool streams_kv(const KParams& kp) {
     return kp.seqlen <= kDecodeRows && kp.kv_group == 1 && (int64_t)kp.batch * kp.heads * kp.seqlen_k * kp.kv_key_bytes >= kStreamKvBytes;
@@ -210,6 +209,13 @@ int dispatch(int variant, const intfa_fwd_params* p, KParams kp, bool dump_s, hi
     sel.p_round = p->p_round == INTFA_PROUND_REFERENCE ? 1 : 0;
     sel.split = kp.num_splits > 1;
     sel.dump_s = dump_s;
+    sel.wide = decode_shaped(kp.seqlen);
+    const int64_t wgs = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kDecodeRows - 1) / kDecodeRows) * kp.num_splits;
+    // The decode-shaped kernels' forms, which give the same bits.  Rows past the 16th go to a workgroup of their own while both find a compute
+    // unit to themselves (half-int8 d64, 20 rows, 256 keys 6.0 -> 5.3 us; K and V then come from the L2 twice).  Half steps: two
+    // workgroups per compute unit instead of one (WideGeom).
+    sel.row_tiles = kp.seqlen <= 16 || (2 * wgs <= kComputeUnits && !streams_kv(kp)) ? 1 : 2;
+    sel.half_steps = wgs > kComputeUnits;
     const int d = kp.head_dim;
     if (vblk && kp.vs_sub == 2) {
         if (d == 128) return launch_full_int8_vblk64_d128(kp, sel, stream);
@@ -313,15 +319,18 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
     const bool decode = decode_shaped(p->seqlen);
     if (decode) {
         wgs = (int64_t)p->batch * p->heads * ((p->seqlen + kDecodeRows - 1) / kDecodeRows);
-        // head_dim 256: 96 KiB and more of tiles, one workgroup per compute unit
-        if (p->head_dim == 256) slots = cus;
+        // head_dim 256 with 16-bit V: 96 KiB and more of tiles, one workgroup per compute unit
+        if (p->head_dim == 256 && variant != INTFA_VARIANT_FULL_INT8) slots = cus;
     }
     else if (p->head_dim == 256) wgs *= 2;     // full-int8: eight-wave workgroups, one per compute unit; the others: column halves
     if (wgs * 5 >= slots * 4) return 1;                                        // at least 80 % of the slots are used anyway
     const int seqlen_k = p->seqlen_k > 0 ? p->seqlen_k : p->seqlen;
     const int bn = block_n_for(variant, p->head_dim);
     const int64_t blocks = (seqlen_k + bn - 1) / bn;
-    int64_t splits = (slots + wgs - 1) / wgs;
+    // (decode-shaped workgroups are equal in work, so one that starts in a second round doubles the time: full-int8 d128, 36 heads, 16363 keys,
+    // 15 splits on 512 slots 42 us, 14 splits 31)
+    int64_t splits = decode ? slots / wgs : (slots + wgs - 1) / wgs;
+    if (splits < 1) splits = 1;
     if (splits > blocks / 4) splits = blocks / 4;                              // keep four key blocks per split
     // Decode-shaped calls merge inside the launch, so a split costs little (2 us for the first one, then the reading of its partial by
     // the workgroup that merges) and short ones pay.  Not full-int8: there every split requantises P in a frame of its own, and the

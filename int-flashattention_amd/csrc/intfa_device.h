@@ -28,6 +28,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 
@@ -92,6 +93,27 @@ __device__ __forceinline__ KernargPtr kernarg_block() {
     KernargPtr pe = (KernargPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(pe));       // opaque: the fields are loaded where they are used, not held since the prologue
     return pe;
+}
+// Requests every 64-byte line of the kernel's argument block in one go.  The block is cold in each launch, and a workgroup's prologue
+// reads it in three or four places that depend on one another: each would be a trip to memory of its own, ahead of the first tile load.
+// The statement passes the workgroup's number through, on which everything else depends.  (Not a volatile one: the compiler would take it
+// for a possible write to memory and load what follows through the vector unit.)
+__device__ __forceinline__ int block_after_kernargs() {
+    int bid = blockIdx.x;
+    typedef const __attribute__((address_space(4))) int* Words;
+    const Words w = (Words)__builtin_amdgcn_kernarg_segment_ptr();
+    static_assert((sizeof(KParams) - 1) / 64 == 7, "the statement names a word of each line");
+    asm("" : "+s"(bid) : "s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[48]), "s"(w[64]), "s"(w[80]), "s"(w[96]), "s"(w[112]));
+    return bid;
+}
+// A scale as its bits, and their conversion: the request does not wait for the value, so it can stand ahead of work that hides it.
+__device__ __forceinline__ uint32_t load_scale_bits(const char* base, int64_t idx, int dtype) {
+    if (dtype == 2) return ((const uint32_t*)base)[idx];
+    return ((const uint16_t*)base)[idx];
+}
+__device__ __forceinline__ float cvt_scale_bits(uint32_t raw, int dtype) {
+    if (dtype == 0) return (float)__builtin_bit_cast(_Float16, (uint16_t)raw);
+    return __builtin_bit_cast(float, dtype == 1 ? raw << 16 : raw);
 }
 __device__ __forceinline__ float load_scale(const char* base, int64_t idx, int dtype) {
     if (dtype == 0) return (float)((const _Float16*)base)[idx];
@@ -217,9 +239,15 @@ __device__ __forceinline__ void load_q8_fragments(v4i (&qreg)[KS], const KParams
 // q_scale of query row q_ld times sm_scale * log2(e): the factor between S * k_scale and the exponent of exp2.  Never zero: the scores
 // of hidden keys are -infinity, and a row of zeros (scale zero, as padding has) must not make NaN of them.  The smallest normal number
 // gives a row's visible keys the same exponent as zero would.
-__device__ __forceinline__ float load_q_scale_log2(const KParams& p, int b, int h, int q_ld) {
-    const float c = load_scale(p.q_scale, b * p.qs_sb + h * p.qs_sh + (int64_t)q_ld * p.qs_sn, p.scale_dtype) * p.qk_scale_log2;
+__device__ __forceinline__ uint32_t load_q_scale_bits(const KParams& p, int b, int h, int q_ld) {
+    return load_scale_bits(p.q_scale, b * p.qs_sb + h * p.qs_sh + (int64_t)q_ld * p.qs_sn, p.scale_dtype);
+}
+__device__ __forceinline__ float q_scale_log2(const KParams& p, uint32_t bits) {
+    const float c = cvt_scale_bits(bits, p.scale_dtype) * p.qk_scale_log2;
     return c == 0.f ? 0x1p-126f : c;
+}
+__device__ __forceinline__ float load_q_scale_log2(const KParams& p, int b, int h, int q_ld) {
+    return q_scale_log2(p, load_q_scale_bits(p, b, h, q_ld));
 }
 
 // k_scale of the keys of one (batch, K/V head): fetched as raw bits (one key per thread, ahead of the block that uses
@@ -316,23 +344,25 @@ __device__ __forceinline__ v4i make_rsrc(const void* base, uint32_t bytes) {
     r[3] = 0x00020000;
     return r;
 }
-// Issues wave instruction number `it` (0 .. NINST/4 - 1) of this wave's share of one tile copy.
+// One wave instruction of a copy: 64 x 16 bytes from the resource at soff + the lane's offset to 1 KiB of LDS.
 // The statement overwrites M0 and cannot say so: the compiler keeps M0 reserved on this target, warns about a clobber
 // entry for it and ignores it.  Nothing the compiler generates in these kernels reads M0 (no LDS-DMA builtins, GWS,
-// relative moves or interpolation), and every copy sets it afresh.  tile_off and row_stride must be wave-uniform values
+// relative moves or interpolation), and every copy sets it afresh.  soff and lds must be wave-uniform values
 // the compiler can see as such (kernel arguments, readfirstlane results): they end up in scalar operands.
 // NT: non-temporal, for tiles that nothing reads again.
+template <bool NT> __device__ __forceinline__ void issue_copy_1k(v4i rsrc, uint32_t lane_off, uint32_t soff, uint32_t lds) {
+    if (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :: "s"(lds), "v"(lane_off), "s"(rsrc), "s"(soff) : "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds), "v"(lane_off), "s"(rsrc), "s"(soff) : "memory");
+}
+// Issues wave instruction number `it` (0 .. NINST/4 - 1) of this wave's share of one tile copy.
 template <int ROW_BYTES, int SWZ, int ROWS, bool NT = false>
 __device__ __forceinline__ void issue_tile_part(v4i rsrc, uint32_t tile_off, uint32_t row_stride, uint32_t lds_tile,
                                                 int wave, const TileLoadLane<ROW_BYTES, SWZ, ROWS>& ln, int it) {
     using T = TileLoadLane<ROW_BYTES, SWZ, ROWS>;
     const int i = it * 4 + wave;                     // wave-uniform instruction index
-    const uint32_t m0v = lds_tile + (uint32_t)i * 1024u;
-    const uint32_t soff = tile_off + (uint32_t)(i * T::RPI) * row_stride;
-    if (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                 :: "s"(m0v), "v"(ln.off[it % T::NV]), "s"(rsrc), "s"(soff) : "memory");
-    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(m0v), "v"(ln.off[it % T::NV]), "s"(rsrc), "s"(soff) : "memory");
+    issue_copy_1k<NT>(rsrc, ln.off[it % T::NV], tile_off + (uint32_t)(i * T::RPI) * row_stride, lds_tile + (uint32_t)i * 1024u);
 }
 template <int ROW_BYTES, int SWZ, int ROWS, bool NT = false>
 __device__ __forceinline__ void issue_tile_load(v4i rsrc, uint32_t tile_off, uint32_t row_stride, uint32_t lds_tile,
@@ -423,6 +453,27 @@ __device__ __forceinline__ float hide_past(float v, int last, int k_r) {
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+// (the same for the 4 NT probabilities of the decode-shaped kernels' lanes: four consecutive keys of NT tiles, four bytes each)
+template <int NT> __device__ __forceinline__ void requant_p_reference(const float (&p)[4 * NT], uint32_t (&out)[NT]) {
+    unsigned hb[2 * NT];
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) {
+        v2h h = __builtin_convertvector((v2f){p[2 * i], p[2 * i + 1]}, v2h);
+        h = __builtin_elementwise_fma(h, (v2h){(_Float16)127.0f, (_Float16)127.0f}, (v2h){(_Float16)0.5f, (_Float16)0.5f});
+        hb[i] = __builtin_bit_cast(unsigned, h);
+    }
+    const unsigned k1024 = 0x64006400u;                    // fp16 1024, twice
+    static_assert(NT == 1 || NT == 2, "four or eight probabilities");
+    if constexpr (NT == 1)
+        asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3\n\tv_pk_add_f16 %0, %0, %2\n\tv_pk_add_f16 %1, %1, %2\n\t"
+                     "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" : "+v"(hb[0]), "+v"(hb[1]) : "s"(k1024));
+    else
+        asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3\n\tv_pk_add_f16 %0, %0, %4\n\tv_pk_add_f16 %1, %1, %4\n\t"
+                     "v_pk_add_f16 %2, %2, %4\n\tv_pk_add_f16 %3, %3, %4\n\ts_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0"
+                     : "+v"(hb[0]), "+v"(hb[1]), "+v"(hb[2]), "+v"(hb[3]) : "s"(k1024));
+#pragma unroll
+    for (int t = 0; t < NT; ++t) out[t] = __builtin_amdgcn_perm(hb[2 * t + 1], hb[2 * t], 0x06040200u);
+}
 __device__ __forceinline__ v4i requant_p_reference16(const float (&p)[16]) {
     unsigned hb[8];
 #pragma unroll

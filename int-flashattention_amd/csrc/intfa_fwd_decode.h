@@ -1,10 +1,10 @@
-// Full-int8 forward for few query rows per head (decoding against a key/value cache, Nq << Nk).
+// Full-int8 forward whose waves share the keys: for small single-pass problems (decode_kernel_takes, intfa_capi.hip) the kernel of this file,
+// for few query rows per head the one of intfa_fwd_decode_wide.h behind the same name.
 //
 // Same arithmetic as fwd_full_int8_kernel (flash_atten_full_int8.py:9-71 per 128-key block: int32 S, dequantise, running
 // max, P = exp2(X c - m), P requantised with the fixed scale 127, int32 P V, fp32 accumulator), other division of labour.
-// The general kernel gives each of its four waves 32 query rows; with one or a few query rows three of them would redo
-// the first one's work on padding while the pass is bound by streaming K and V from HBM.  Here one workgroup owns 32
-// query rows and its four waves share every key block:
+// The general kernel gives each of its four waves 32 query rows; a small problem then leaves compute units without a workgroup.
+// Here one workgroup owns 32 query rows and its four waves share every key block:
 //   * wave w computes S^T for keys 32w .. 32w+31 of the block (KS MFMAs), dequantises and takes the partial row maxima;
 //   * the partial maxima meet in LDS (barrier), every wave then holds the block's row maximum;
 //   * wave w exponentiates and requantises its 32 keys and publishes its P8 fragment and row sums in LDS (barrier);
@@ -13,7 +13,7 @@
 // The int32 sums run over the same 128 keys as in the general kernel, and the waves exchange the row sums of their keys with
 // the P8 fragments and add them in that kernel's order: the results are the same bits, and which of the two runs may depend on
 // the number of heads and batch entries.  K/V tiles are double-buffered in LDS and the whole next tile is requested at the
-// start of a block (the data comes from HBM, not from a cache shared with other query blocks).
+// start of a block.
 // Head dims 64 and 256: the general kernels' key block is 64 there (the reference admits no key block longer than head_dim,
 // flash_atten_full_int8.py:88; at 256 registers set the limit), so a 128-key step of this
 // kernel covers TWO blocks A (waves 0, 1) and B (waves 2, 3): after the one exchange of partial maxima every wave knows
@@ -23,12 +23,12 @@
 #pragma once
 #include "intfa_device.h"
 #include "intfa_launch.h"
-#include "intfa_splitkv.h"
+#include "intfa_fwd_decode_wide.h"
 
 namespace intfa {
 
 // Head_dim 128: one 128-key block per step, the block of the general kernel.  Head dims 64 and 256: two 64-key blocks.
-template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK, bool STREAM /* K, V tiles non-temporal: KParams::stream_kv */>
+template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool VBLK>
 __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_int8_kernel(const KParams p) {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
@@ -58,39 +58,24 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lq = lane & 31, lh = lane >> 5;
 
-    // ---- block -> (head, 32-row query block, split); whole K/V heads go to one XCD as in the general kernel
+    // ---- block -> (head, 32-row query block); whole K/V heads go to one XCD as in the general kernel
     const int n_mblk = (p.seqlen + kDecodeRows - 1) / kDecodeRows;
-    const int n_split = SPLIT ? p.num_splits : 1;
-    const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
-    const int rem = wg.rem, head = wg.b * p.heads + wg.h;
-    const int mb_idx = fast_div(rem, p.d_n_split), split = rem - mb_idx * n_split;
-    const int mb = p.causal ? n_mblk - 1 - mb_idx : mb_idx;     // heaviest query blocks first
-    const int b = wg.b, h = wg.h;
-    const int hk = wg.hk;
+    const WorkgroupJob wg = deal_workgroup(p, block_after_kernargs());
+    const int mb = p.causal ? n_mblk - 1 - wg.rem : wg.rem;     // heaviest query blocks first
+    const int b = wg.b, h = wg.h, hk = wg.hk;
 
     const int seqlen_k = keys_of_batch(p, b);
     // causal: row i sees keys 0 .. i + causal_off (mask aligned to the bottom right corner as in the general kernels: a few
     // new tokens against a cache); blocks past the last row's limit are not visited
-    // (causal_rows: the rows hold several query heads of one K/V group, causal_rows positions each; a row's position is
-    // then row % causal_rows and a 32-row block can hold every position)
-    const int fold = p.causal_rows;
-    const int causal_off = seqlen_k - (fold ? fold : p.seqlen);
-    // (a split takes blocks_per_split blocks of the whole key range, masked or not: every row of a decode-shaped problem
-    // sees nearly all keys)
-    const KeyBlocks kb = key_block_range<BNB>(seqlen_k, p.causal != 0, fold ? fold : mb * kDecodeRows + kDecodeRows, causal_off, SPLIT,
-                                             n_split, split, false, p.blocks_per_split);
+    const int causal_off = seqlen_k - p.seqlen;
+    const KeyBlocks kb = key_block_range<BNB>(seqlen_k, p.causal != 0, mb * kDecodeRows + kDecodeRows, causal_off, false, 1, 0, false, 0);
     const int nb_begin = kb.begin, nb_end = kb.end;         // in blocks of BNB keys
     const int key_end = nb_end * BNB < seqlen_k ? nb_end * BNB : seqlen_k;      // one past the last key of the range
     const int q_row = mb * kDecodeRows + lq;
     const bool q_valid = q_row < p.seqlen;
     const int q_ld = q_valid ? q_row : p.seqlen - 1;
 
-    // ---- Q fragment (B operand of S^T = K Q^T), the same 32 rows in every wave
-    v4i qreg[KS];
-    load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);
-    const float qsc = load_q_scale_log2(p, b, h, q_ld);
-
-    float m_run = -INFINITY, l_run = 0.f;
+    float qsc = 0.f, m_run = -INFINITY, l_run = 0.f;
     float l_odd = 0.f;                           // head_dim 256: row sums of the odd sub-tiles (a wave of its own in that general kernel)
     float o_acc[DTW][16];
 #pragma unroll
@@ -108,9 +93,17 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const auto v_lane = tile_load_lane<D, SWZ_V8, BN>(v_sn, wave, lane);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<D, SWZ_K, BN, STREAM>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
-        issue_tile_load<D, SWZ_V8, BN, STREAM>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        issue_tile_load<D, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
+        issue_tile_load<D, SWZ_V8, BN>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
     };
+    // The first tiles are requested ahead of everything else: Q, the scales and the lane offsets below arrive or are computed under
+    // their way from HBM.
+    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    // ---- Q fragment (B operand of S^T = K Q^T), the same 32 rows in every wave
+    v4i qreg[KS];
+    load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);
+    const uint32_t q_scale_bits = load_q_scale_bits(p, b, h, q_ld);
+    const uint32_t v_scale_bits = VBLK ? 0u : load_scale_bits(p.v_scale, b * p.vs_sb + hk * p.vs_sh, p.scale_dtype);
     // k_scale of a block: thread t < 128 fetches the scale of key t; converted to fp32 when stored to LDS
     const KScaleSource ks_src(p, b, hk, seqlen_k);
     auto load_ks = [&](int nb) __attribute__((always_inline)) -> uint32_t { return ks_src.load(nb * BNB + (tid & (BN - 1))); };
@@ -164,8 +157,8 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     // nothing (the same instruction stream for every wave; a run-time "owns a tile" test around the V fragments and the
     // accumulator update costs the owners a hundred register copies per step)
     // the last visible key of the first row of this query block, and of the lane's row
-    const int first_lim = p.causal ? (fold ? 0 : mb * kDecodeRows) + causal_off : 0x3fffffff;
-    const int row_lim = p.causal ? (fold ? q_row % fold : q_row) + causal_off : 0x3fffffff;
+    const int first_lim = p.causal ? mb * kDecodeRows + causal_off : 0x3fffffff;
+    const int row_lim = p.causal ? q_row + causal_off : 0x3fffffff;
     const bool blk_a = NBS == 1 || wave < 2;                          // this wave's keys belong to the first block of a step
 
     auto step = [&](auto buf_tag, int nb) __attribute__((always_inline)) {
@@ -319,14 +312,13 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
         }
     };
 
-    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
-    if (SPLIT && p.ticket != nullptr && tid == 0) splitkv_open_tickets(p, (b * p.heads + h) * n_mblk + mb);
     if (nb_begin < nb_end) {
         if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(load_ks(nb_begin));
         if (vs_thread) {
 #pragma unroll
             for (int j = 0; j < VPT; ++j) *(float*)(smem + vs_wr + j * kThreads * 4) = load_vs(nb_begin, j);
         }
+        qsc = q_scale_log2(p, q_scale_bits);
         int nb = nb_begin;
         while (true) {
             if (nb >= nb_end) break;
@@ -340,36 +332,13 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 
     // ---- epilogue: every wave scales and stores its own output columns
     const float l_tot = half_pair_sum(l_run) + (D == 256 ? half_pair_sum(l_odd) : 0.f);      // units of 1/127 when PROUND == 0
-    const float vs = VBLK ? 1.f : load_scale(p.v_scale, b * p.vs_sb + hk * p.vs_sh, p.scale_dtype);
+    const float vs = VBLK ? 1.f : cvt_scale_bits(v_scale_bits, p.scale_dtype);
     // false: an empty split range, an empty cache entry, or a causal row above the first key (zeros, lse = -inf; such a
     // row's accumulators hold NaN from exp2(-inf - -inf), hence the selects below)
     const bool seen = nb_begin < nb_end && m_run > -INFINITY;
     const float out_scale = !seen ? 0.f : (PROUND == 0) ? (vs / l_tot) : (vs / (127.f * l_tot));
     const float l_true = (PROUND == 0) ? l_tot * (1.f / 127.f) : l_tot;
     const float lse = seen ? m_run + __builtin_log2f(l_true) : -INFINITY;
-    if (SPLIT) {
-        const SplitPartials part(&p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
-        if (q_valid) {
-#pragma unroll
-            for (int j = 0; j < DTW; ++j) {
-                const int dt = wave + 4 * j;
-                if (dt >= DT) continue;
-#pragma unroll
-                for (int a4 = 0; a4 < 4; ++a4) {
-                    v4f o;
-#pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * out_scale : 0.f;
-                    part.put(lq, D, 32 * dt + 8 * a4 + 4 * lh, o);
-                }
-            }
-            if (wave == 0 && lh == 0) part.put_lse(lq, seen ? lse : -INFINITY);
-        }
-        if (p.ticket == nullptr || !splitkv_last_arrival(p, smem, (b * p.heads + h) * n_mblk + mb)) return;
-        static_assert(kMergeLds <= LDS_BYTES, "the merge fits the tile memory");
-        const int row0 = mb * kDecodeRows;
-        splitkv_merge_rows<D, OUT_DT>(p, smem, b, h, row0, p.seqlen - row0 < kDecodeRows ? p.seqlen - row0 : kDecodeRows);
-        return;
-    }
     if (!q_valid) return;
     char* orow = p.out + b * p.o_sb + h * p.o_sh + (int64_t)q_row * p.o_sn;
 #pragma unroll
@@ -394,6 +363,14 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     }
     if (p.lse != nullptr && wave == 0 && lh == 0) p.lse[((int64_t)b * p.heads + h) * p.seqlen + q_row] = lse;
 #endif  // __HIP_DEVICE_COMPILE__
+}
+
+// Few query rows per head, split or not: intfa_fwd_decode_wide.h.
+template <int D, class /* WideRows */ R, int OUT_DT, int PROUND, bool VBLK>
+__global__ void __launch_bounds__(kWideThreads, (D == 128 && !R::half_steps) || (D == 256 && VBLK && R::tiles == 2) ? 2 : 4) fwd_decode_full_int8_kernel(const KParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    decode_wide<D, true, true, OUT_DT, PROUND, VBLK, R>(p);
+#endif
 }
 
 }  // namespace intfa

@@ -1,4 +1,5 @@
-// Half-int8 and fp16/bf16 forward for few query rows per head (decoding against a key/value cache, Nq << Nk).
+// Half-int8 and fp16/bf16 forward whose waves share the keys: for small single-pass problems at head_dim 64 and 256 (decode_kernel_takes,
+// intfa_capi.hip) the kernel of this file, for few query rows per head the one of intfa_fwd_decode_wide.h behind the same name.
 //
 // Same arithmetic as fwd_f16pv_kernel (flash_atten_int8.py:9-66, flash_atten_fp.py:9-60 per 64-key block: S, running
 // max, P = exp2(S c - m) cast to V's 16-bit type, fp32 accumulator scaled by alpha and P V added on top), other division
@@ -12,29 +13,24 @@
 //   * wave w exponentiates its 32 keys against its block's maximum, casts to 16 bits and publishes two MFMA operands
 //     in LDS (barrier);
 //   * waves 0 and 1 own 32 output columns each: O = (O alpha_A + P_A V_A) alpha_B + P_B V_B with all eight operands.
-// Head_dim 128 and 256: a step is ONE 64-key block.  Waves 0 and 1 compute S^T and P for its two 32-key sub-tiles,
-// waves 2 and 3 only pass the barriers in that phase (the pass is bound by the stream of K and V, not by the arithmetic),
-// every wave owns one (two at head_dim 256) 32-column output tile.  The smaller step is what the stream wants there: 24
-// to 32 KiB of tiles per step let two or three workgroups share a compute unit at head_dim 128 (6.0 TB/s of K+V against
-// 5.4 - 5.9 with 128-key steps and one workgroup), and at head_dim 256 two steps of 128 keys would not fit the LDS.
-// In calls that the general kernels could have taken, at head_dim 64 and 256, every block is evaluated with the same frame, the same P, the same order of MFMA steps and of the row
-// sums as in the general kernels, so that the results are the same bits and which of the two runs may depend on the number of
-// heads and batch entries.  (At head_dim 128 and in decode-shaped calls the frame is the running maximum of every block,
-// which moves P's 16-bit rounding against the general kernel's lazy frame.)  K/V tiles of a step are
-// double-buffered in LDS and the whole next step is requested at the start of a step.
+// Head_dim 256: a step is ONE 64-key block (two steps of 128 keys would not fit the LDS).  Waves 0 and 1 compute S^T and P for its two
+// 32-key sub-tiles, waves 2 and 3 only pass the barriers in that phase, every wave owns two 32-column output tiles.
+// Every block is evaluated with the same frame, the same P, the same order of MFMA steps and of the row sums as in the general
+// kernels, so that the results are the same bits and which of the two runs may depend on the number of heads and batch entries.
+// K/V tiles of a step are double-buffered in LDS and the whole next step is requested at the start of a step.
 #pragma once
 #include "intfa_device.h"
 #include "intfa_launch.h"
-#include "intfa_splitkv.h"
+#include "intfa_fwd_decode_wide.h"
 #include "intfa_fwd_f16pv.h"
 
 namespace intfa {
 
 // QK_INT8: int8 Q/K with per-token scales (half-int8) or 16-bit Q/K.  IO_DT: type of V, P and the output (and of Q/K
 // when !QK_INT8): 0 fp16, 1 bf16.  The causal mask is a run-time switch here (p.causal).
-template <bool QK_INT8, int D, int IO_DT, bool SPLIT, bool STREAM /* K, V tiles non-temporal: KParams::stream_kv */>
-__global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8) ? 3 : 2) fwd_decode_f16pv_kernel(const KParams p) {
-    static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128 and 256");
+template <bool QK_INT8, int D, int IO_DT>
+__global__ void __launch_bounds__(kThreads, D == 256 ? 1 : 2) fwd_decode_f16pv_kernel(const KParams p) {
+    static_assert(D == 64 || D == 256, "head dims 64 and 256");
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
     constexpr int BNB = kBlockN16;                    // key block of the arithmetic
     constexpr int NBS = D <= 64 ? 2 : 1;              // key blocks per step
@@ -65,41 +61,23 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lq = lane & 31, lh = lane >> 5;
 
-    // ---- block -> (head, 32-row query block, split)
+    // ---- block -> (head, 32-row query block)
     const int n_mblk = (p.seqlen + kDecodeRows - 1) / kDecodeRows;
-    const int n_split = SPLIT ? p.num_splits : 1;
-    const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
-    const int rem = wg.rem, head = wg.b * p.heads + wg.h;
-    const int mb_idx = fast_div(rem, p.d_n_split), split = rem - mb_idx * n_split;
-    const int mb = p.causal ? n_mblk - 1 - mb_idx : mb_idx;     // heaviest query blocks first
-    const int b = wg.b, h = wg.h;
-    const int hk = wg.hk;
+    const WorkgroupJob wg = deal_workgroup(p, block_after_kernargs());
+    const int mb = p.causal ? n_mblk - 1 - wg.rem : wg.rem;     // heaviest query blocks first
+    const int b = wg.b, h = wg.h, hk = wg.hk;
 
     const int seqlen_k = keys_of_batch(p, b);
     // causal: the row at position i sees keys 0 .. i + causal_off (mask aligned to the bottom right corner)
-    // (causal_rows: the rows hold several query heads of one K/V group, causal_rows positions each)
-    const int fold = p.causal_rows;
-    const int causal_off = seqlen_k - (fold ? fold : p.seqlen);
-    // (a split takes blocks_per_split 64-key blocks of the whole key range: every row of a decode-shaped problem sees
-    // nearly all keys)
-    const KeyBlocks kb = key_block_range<BNB>(seqlen_k, p.causal != 0, fold ? fold : mb * kDecodeRows + kDecodeRows, causal_off, SPLIT,
-                                              n_split, split, false, p.blocks_per_split);
+    const int causal_off = seqlen_k - p.seqlen;
+    const KeyBlocks kb = key_block_range<BNB>(seqlen_k, p.causal != 0, mb * kDecodeRows + kDecodeRows, causal_off, false, 1, 0, false, 0);
     const int nb_begin = kb.begin, nb_end = kb.end;
     const int key_end = nb_end * BNB < seqlen_k ? nb_end * BNB : seqlen_k;      // one past the last key of the range
     const int q_row = mb * kDecodeRows + lq;
     const bool q_valid = q_row < p.seqlen;
     const int q_ld = q_valid ? q_row : p.seqlen - 1;
 
-    // ---- Q fragments (B operand of S^T = K Q^T), the same 32 rows in every wave
-    v4i qreg[KS];
-    {
-        const char* qrow = p.q + b * p.q_sb + h * p.q_sh + (int64_t)q_ld * p.q_sn;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qreg[ks] = *(const v4i*)(qrow + ks * 32 + lh * 16);
-    }
-    const float qsc = QK_INT8 ? load_q_scale_log2(p, b, h, q_ld) : p.qk_scale_log2;
-
-    float m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only (head_dim 64: all keys)
+    float qsc = p.qk_scale_log2, m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only (head_dim 64: all keys)
     v16f o_acc[DTW];
 #pragma unroll
     for (int j = 0; j < DTW; ++j)
@@ -116,9 +94,20 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const auto v_lane = tile_load_lane<VROW, SWZ_V16, BN>(v_sn, wave, lane);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<KROW, SWZ_K, BN, STREAM>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
-        issue_tile_load<VROW, SWZ_V16, BN, STREAM>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        issue_tile_load<KROW, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
+        issue_tile_load<VROW, SWZ_V16, BN>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
     };
+    // The first tiles are requested ahead of everything else: Q, the scales and the lane offsets below arrive or are computed under
+    // their way from HBM.
+    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    // ---- Q fragments (B operand of S^T = K Q^T), the same 32 rows in every wave
+    v4i qreg[KS];
+    {
+        const char* qrow = p.q + b * p.q_sb + h * p.q_sh + (int64_t)q_ld * p.q_sn;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) qreg[ks] = *(const v4i*)(qrow + ks * 32 + lh * 16);
+    }
+    const uint32_t q_scale_bits = QK_INT8 ? load_q_scale_bits(p, b, h, q_ld) : 0u;
     // k_scale of a step: thread t < 128 fetches the scale of key t; converted to fp32 when stored to LDS
     const KScaleSource ks_src(p, b, hk, seqlen_k);
     const bool ks_wave = wave < BN / 64;              // threads 0 .. BN-1 fetch one k_scale each (a scalar test: see fwd_full_int8_kernel)
@@ -154,14 +143,14 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const uint32_t xp_rd = OFF_XP + 16 * lane;                       // + 1024 per MFMA step
     const uint32_t xs_rd = OFF_XS + 16 * lane, xs_wr = xs_rd + 4 * wave;
     // the smallest and this lane's own last visible key
-    const int first_lim = p.causal ? (fold ? 0 : mb * kDecodeRows) + causal_off : 0x3fffffff;
-    const int row_lim = p.causal ? (fold ? q_row % fold : q_row) + causal_off : 0x3fffffff;
-    const int last_lim = p.causal ? (fold ? fold : mb * kDecodeRows + kDecodeRows) - 1 + causal_off : 0x3fffffff;   // ... of the last row
+    const int first_lim = p.causal ? mb * kDecodeRows + causal_off : 0x3fffffff;
+    const int row_lim = p.causal ? q_row + causal_off : 0x3fffffff;
+    const int last_lim = p.causal ? mb * kDecodeRows + kDecodeRows - 1 + causal_off : 0x3fffffff;   // ... of the last row
     const bool blk_a = NBS == 1 || wave < 2;          // this wave's keys belong to the first block of a step
-    // head_dim 64, where fwd_f16pv_kernel could have taken the call (more than kDecodeMaxRows query rows), its lazy frame: it follows a row's maximum when that exceeds it by more than
+    // head_dim 64: the lazy frame of fwd_f16pv_kernel: it follows a row's maximum when that exceeds it by more than
     // kFrameSlack in some row of the 32, and in the blocks that kernel masks (of its 128-row query blocks): the causal
     // diagonal's, or the ragged last one
-    const int masked_first = p.seqlen <= kDecodeMaxRows ? 0 : p.causal ? ((mb * kDecodeRows / kBlockM) * kBlockM + causal_off + 1) / BNB : seqlen_k / BNB;
+    const int masked_first = p.causal ? ((mb * kDecodeRows / kBlockM) * kBlockM + causal_off + 1) / BNB : seqlen_k / BNB;
     auto frame = [&](float m, float mxs, int blk) __attribute__((always_inline)) -> float {
         const bool move = blk >= masked_first || __builtin_amdgcn_ballot_w64(mxs > m + kFrameSlack) != 0;
         return move ? fmaxf(m, mxs) : m;
@@ -314,13 +303,12 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
         if (QK_INT8 && more && ks_wave) *(float*)(smem + ks_wr + (BUF ^ 1) * BN * 4) = cvt_ks(ks_next);
     };
 
-    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
-    if (SPLIT && p.ticket != nullptr && tid == 0) splitkv_open_tickets(p, (b * p.heads + h) * n_mblk + mb);
     if (nb_begin < nb_end) {
         if (QK_INT8) {
             const uint32_t s0 = load_ks(nb_begin);
             if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(s0);
         }
+        if (QK_INT8) qsc = q_scale_log2(p, q_scale_bits);
         int nb = nb_begin;
         while (true) {
             step(BoolTag<false>{}, nb);
@@ -346,28 +334,6 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     const bool seen = nb_begin < nb_end && m_run > -INFINITY;
     const float inv = seen ? 1.f / l_tot : 0.f;
     const float lse = seen ? m_run + __builtin_log2f(l_tot) : -INFINITY;
-    if (SPLIT) {
-        const SplitPartials part(&p, D, ((int64_t)(split * p.batch + b) * p.heads + h) * p.seqlen + mb * kDecodeRows);
-        if (q_valid) {
-            if (own_tile) {
-#pragma unroll
-                for (int j = 0; j < DTW; ++j)
-#pragma unroll
-                    for (int a4 = 0; a4 < 4; ++a4) {
-                        v4f o;
-#pragma unroll
-                        for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * inv : 0.f;
-                        part.put(lq, D, 32 * (wave + 4 * j) + 8 * a4 + 4 * lh, o);
-                    }
-            }
-            if (wave == 0 && lh == 0) part.put_lse(lq, seen ? lse : -INFINITY);
-        }
-        if (p.ticket == nullptr || !splitkv_last_arrival(p, smem, (b * p.heads + h) * n_mblk + mb)) return;
-        static_assert(kMergeLds <= LDS_BYTES, "the merge fits the tile memory");
-        const int row0 = mb * kDecodeRows;
-        splitkv_merge_rows<D, IO_DT>(p, smem, b, h, row0, p.seqlen - row0 < kDecodeRows ? p.seqlen - row0 : kDecodeRows);
-        return;
-    }
     if (!q_valid) return;
     char* orow = p.out + b * p.o_sb + h * p.o_sh + (int64_t)q_row * p.o_sn;
     if (own_tile) {
@@ -391,6 +357,14 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : (D == 128 && QK_INT8)
     }
     if (p.lse != nullptr && wave == 0 && lh == 0) p.lse[((int64_t)b * p.heads + h) * p.seqlen + q_row] = lse;
 #endif  // __HIP_DEVICE_COMPILE__
+}
+
+// Few query rows per head, split or not: intfa_fwd_decode_wide.h
+template <bool QK_INT8, int D, class /* WideRows */ R, int IO_DT>
+__global__ void __launch_bounds__(kWideThreads, D == 256 ? 2 : 4) fwd_decode_f16pv_kernel(const KParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    decode_wide<D, QK_INT8, false, IO_DT, 0, false, R>(p);
+#endif
 }
 
 }  // namespace intfa

@@ -20,6 +20,9 @@ struct LaunchSel {
     int p_round;     // full-int8 only
     bool split;      // write split-KV partials instead of the output
     bool dump_s;     // full-int8 only: export int32 S and stop
+    bool wide;       // decode-shaped kernels: few query rows per head (intfa_fwd_decode_wide.h)
+    int row_tiles;   // ... tiles of 16 query rows per workgroup
+    bool half_steps; // ... in more workgroups than compute units
 };
 
 inline FastDiv make_fast_div(int d) {

@@ -21,6 +21,9 @@ namespace intfa {
 //     is not of this epoch for (epoch, 0) - under the first tiles' way from HBM, so that the arrival itself is one atomic add
 //     (a compare-and-swap loop there, with all splits of a block arriving together, cost 5 us with eight of them).  The last
 //     arrival stores zero, so the replays of a captured graph, whose epoch is a constant, find no word of an earlier one.
+//   * Each word has 256 bytes to itself: atomics on one line follow one another at some 80 ns, and the words of eight heads side by side
+//     made 32 splits of each wait 2.5 - 3.2 us for their tickets (0.5 - 0.6 alone).
+constexpr int kTicketStride = 32;              // words
 constexpr int kSplitAux = 16;                  // sc1 in the cache-policy operand of the buffer intrinsics
 typedef __amdgpu_buffer_rsrc_t BufferRsrc;
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -67,21 +70,35 @@ template <int OUT_DT> __device__ __forceinline__ void store_out4(char* dst, v4f 
 
 // Thread 0, at the start: the ticket word of query block `group` becomes this epoch's.
 __device__ __forceinline__ void splitkv_open_tickets(const KParams& p, int group) {
-    uint64_t* t = p.ticket + group;
+    uint64_t* t = p.ticket + group * kTicketStride;
     uint64_t seen = __hip_atomic_load(t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if ((seen ^ p.epoch) >= 256u)
         __hip_atomic_compare_exchange_strong(t, &seen, p.epoch, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The same in two halves, for a kernel that has something to do under the look's way to memory and back: thread 0 looks at the word early ...
+__device__ __forceinline__ uint64_t splitkv_look_at_tickets(const KParams& p, int group) {
+    uint64_t seen = 0;
+    if (p.ticket != nullptr && threadIdx.x == 0) seen = __hip_atomic_load(p.ticket + group * kTicketStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return seen;
+}
+// ... and exchanges it before its own arrival (one that was exchanged by another workgroup since is left alone).
+__device__ __forceinline__ void splitkv_open_tickets(KernargPtr p, int group, uint64_t seen) {
+    uint64_t* const t = p->ticket;
+    const uint64_t epoch = p->epoch;
+    if (t != nullptr && threadIdx.x == 0 && (seen ^ epoch) >= 256u)
+        __hip_atomic_compare_exchange_strong(t + group * kTicketStride, &seen, epoch, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Takes this workgroup's ticket of query block `group`; true for the last of the block's num_splits workgroups.
 // Called by every thread of the workgroup after its stores; `smem` is free (16 bytes of it are used).
-__device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* smem, int group) {
+template <typename P> __device__ __forceinline__ bool splitkv_last_arrival(P p, char* smem, int group) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's partials have reached the point of coherence
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint64_t* t = p.ticket + group;
+        uint64_t* t = p->ticket + group * kTicketStride;
         const uint64_t before = __hip_atomic_fetch_add(t, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool last = before == (p.epoch | (uint64_t)(p.num_splits - 1));
+        const bool last = before == (p->epoch | (uint64_t)(p->num_splits - 1));
         if (last) __hip_atomic_store(t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         *(int*)smem = last;
     }
@@ -90,6 +107,7 @@ __device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* sme
     if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     return last;
 }
+__device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* smem, int group) { return splitkv_last_arrival(&p, smem, group); }
 
 // ---- The same for the general full-int8 kernel, whose waves own 32 query rows each: a ticket per wave and no barrier.  The wave
 // that arrives last reads the partials in the layout of its accumulators, so the row statistics are one value per lane.
@@ -99,7 +117,7 @@ __device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* sme
 template <typename P> __device__ __forceinline__ bool splitkv_last_arrival_wave(P p, int group) {
     unsigned drew_last = 0;                                // (after the wave's partials have been acknowledged)
     if ((threadIdx.x & 63) == 0) {
-        uint64_t* t = p->ticket + group;
+        uint64_t* t = p->ticket + group * kTicketStride;
         const uint64_t before = __hip_atomic_fetch_add(t, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         drew_last = before == (p->epoch | (uint64_t)(p->num_splits - 1));
         if (drew_last) __hip_atomic_store(t, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -183,93 +201,111 @@ __device__ __forceinline__ float splitkv_merge_wave(P p, float* w, float (&acc)[
     return lse;
 }
 
-// Reductions over eight consecutive lanes (quad_perm 1,0,3,2 / 2,3,0,1, then the mirrored half row).
-template <typename F> __device__ __forceinline__ float reduce8(float x, F op) {
+// The four lanes l, l ^ 16, l ^ 32, l ^ 48; the sixteen lanes of a row of 16; all lanes of the wave.
+template <typename F> __device__ __forceinline__ float reduce_row_lanes(float x, F op) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const float y = op(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1]));
+    const unsigned w = __builtin_bit_cast(unsigned, y);
+    const auto c = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return op(__builtin_bit_cast(float, (unsigned)c[0]), __builtin_bit_cast(float, (unsigned)c[1]));
+}
+template <typename F> __device__ __forceinline__ float reduce_wave(float x, F op) {      // (quad_perm 1,0,3,2 / 2,3,0,1, the mirrored half row, the mirrored row)
     x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true)));
     x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true)));
-    return op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true)));
+    x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x141, 0xf, 0xf, true)));
+    x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x140, 0xf, 0xf, true)));
+    return reduce_row_lanes(x, op);
 }
 
-// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; 256 threads.
-// LDS: kMergeLds bytes of `smem`.  Eight lanes per row read the row's log-sum-exps (all in flight at once) and leave the
-// weights in LDS; then D / 4 lanes take a row, four columns each, 256 / (D / 4) rows side by side.  With fewer rows than that the
-// idle threads share the splits of a row and their sums are added in LDS.  Everything that can be requested before the
-// weights are known is: this runs once, at the end of a block, and its time is a chain of latencies.
-constexpr int kMaxSplits = 64;
-constexpr int kMergeLds = 16 + 32 * kMaxSplits * 4 + 256 * 16;
+// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; kMergeWaves waves, kMergeLds bytes of `smem`.
+// This runs once, at the end of a query block, and its time is a chain of latencies: a wave takes a row, its lanes the row's log-sum-exps
+// (lane s that of split s), which make the weights without a word of LDS, and the partials of the first splits are on their way
+// meanwhile, four columns per lane.  With fewer rows than waves the waves of a row share its splits and meet in LDS.
+constexpr int kMaxSplits = 64;                           // the lanes of a wave
+constexpr int kMergeWaves = 8;
+constexpr int kMergeLds = kMergeWaves * 64 * 16;
 template <int D, int OUT_DT>
-__device__ __forceinline__ void splitkv_merge_rows(const KParams& p, char* smem, int b, int h, int row0, int nrows) {
-    constexpr int LPR = D / 4, RP = 256 / LPR, KL = kMaxSplits / 8, U = 4;
-    const SplitPartials part(&p, D, 0);
-    const int ns = p.num_splits, tid = threadIdx.x;
-    float* w = (float*)(smem + 16);                        // [split][32]
-    v4f* red = (v4f*)(smem + 16 + 32 * kMaxSplits * 4);
-    const uint32_t base = (uint32_t)(b * p.heads + h) * (uint32_t)p.seqlen + (uint32_t)row0;
-    // rows side by side: a power of two; G threads share one (row, columns)
-    int rs_log = 0;
-    while ((1 << rs_log) < nrows && (1 << rs_log) < RP) ++rs_log;
-    const int rs = 1 << rs_log, G = RP >> rs_log;
-    const int slot = tid / LPR, col = (tid % LPR) * 4, g = slot >> rs_log, r_first = slot & (rs - 1);
-    const int wr = tid >> 3, wj = tid & 7;
-    const uint32_t wrow = base + (wr < nrows ? wr : nrows - 1);
-    float lse[KL];
-#pragma unroll
-    for (int k = 0; k < KL; ++k) {
-        const int s = 8 * k + wj;
-        lse[k] = part.get_lse((uint32_t)(s < ns ? s : ns - 1) * part.rows + wrow);
-    }
-    v4f x[U];
-    auto request = [&](int r, int s0) __attribute__((always_inline)) {
+__device__ __forceinline__ void splitkv_merge_rows(KernargPtr p, char* smem, int b, int h, int row0, int nrows) {
+    constexpr int LPR = D / 4, SUBS = 64 / LPR, U = 4;
+    const SplitPartials part(p, D, 0);
+    const int ns = p->num_splits, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int rs_log = 0;                                      // rows side by side: a power of two; G waves share one
+    while ((1 << rs_log) < nrows && (1 << rs_log) < kMergeWaves) ++rs_log;
+    const int rs = 1 << rs_log, G = kMergeWaves >> rs_log, g = wave >> rs_log;
+    const int sub = lane / LPR, col = (lane % LPR) * 4, s_first = g * SUBS + sub, s_step = G * SUBS;
+    const uint32_t base = (uint32_t)(b * p->heads + h) * (uint32_t)p->seqlen + (uint32_t)row0;
+    auto row_of = [&](int k) __attribute__((always_inline)) { return (wave & (rs - 1)) + k * rs; };
+    auto lse_of = [&](int k) __attribute__((always_inline)) -> float {
+        const int r = row_of(k);
+        return part.get_lse((uint32_t)(lane < ns ? lane : ns - 1) * part.rows + base + (uint32_t)(r < nrows ? r : nrows - 1));
+    };
+    auto request = [&](v4f (&x)[U], int k, int s0) __attribute__((always_inline)) {      // s0: a multiple of U * s_step
+        const int r = row_of(k);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int s = s0 + u * G;                      // past the end: any partial, its weight is zero
-            x[u] = part.get((uint32_t)(s < ns ? s : ns - 1) * part.rows + base + (r < nrows ? r : nrows - 1), D, col);
+            const int s = s0 + u * s_step + s_first;
+            if (s0 + u * s_step < ns)                    // (a scalar test; past the end of a last group: any partial, its weight is zero)
+                x[u] = part.get((uint32_t)(s < ns ? s : ns - 1) * part.rows + base + (uint32_t)(r < nrows ? r : nrows - 1), D, col);
         }
     };
-    request(r_first, g);
-    __builtin_amdgcn_sched_barrier(0);
-    {
-        float mx = -INFINITY, sum = 0.f;
+    char* out0 = p->out + b * p->o_sb + h * p->o_sh + (int64_t)row0 * p->o_sn;
+    v4f x[U], x_next[U];
 #pragma unroll
-        for (int k = 0; k < KL; ++k) {
-            lse[k] = 8 * k + wj < ns ? lse[k] : -INFINITY;
-            mx = fmaxf(mx, lse[k]);
+    for (int u = 0; u < U; ++u) x[u] = x_next[u] = (v4f){0.f, 0.f, 0.f, 0.f};
+    float lse = lse_of(0), lse_next = 0.f;
+    request(x, 0, 0);
+    for (int k = 0; k * rs < nrows; ++k) {
+        const bool more = (k + 1) * rs < nrows;
+        if (more) {
+            lse_next = lse_of(k + 1);
+            if (ns <= U * s_step) request(x_next, k + 1, 0);
         }
-        mx = reduce8(mx, [](float a, float c) { return fmaxf(a, c); });
+        lse = lane < ns ? lse : -INFINITY;
+        float mx = reduce_wave(lse, [](float a, float c) { return fmaxf(a, c); });
         // A row no split saw a key for: zeros with lse = -inf, as in splitkv_combine_kernel.
         const bool empty = mx == -INFINITY;
         if (empty) mx = 0.f;
-#pragma unroll
-        for (int k = 0; k < KL; ++k) sum += fast_exp2(lse[k] - mx);
-        sum = reduce8(sum, [](float a, float c) { return a + c; });
-        const float total = empty ? -INFINITY : __builtin_log2f(sum) + mx;
-#pragma unroll
-        for (int k = 0; k < KL; ++k) w[(8 * k + wj) * 32 + wr] = empty ? 0.f : fast_exp2(lse[k] - total);      // (0 past the last split)
-        if (p.lse != nullptr && wj == 0 && wr < nrows) p.lse[wrow] = total;
-    }
-    __syncthreads();
-    char* out0 = p.out + b * p.o_sb + h * p.o_sh + (int64_t)row0 * p.o_sn;
-    for (int r = r_first; r < nrows || G > 1; r += rs) {   // (G > 1: one trip for every thread, there is a barrier in it)
-        const bool on = r < nrows;
+        const float total = empty ? -INFINITY : __builtin_log2f(reduce_wave(fast_exp2(lse - mx), [](float a, float c) { return a + c; })) + mx;
+        const float w = empty ? 0.f : fast_exp2(lse - total);      // lane s: the weight of split s (0 past the last one)
+        const int r = row_of(k);
+        if (p->lse != nullptr && g == 0 && lane == 0 && r < nrows) p->lse[base + r] = total;
         v4f acc = {0.f, 0.f, 0.f, 0.f};
-        for (int s0 = g; s0 < ns; s0 += U * G) {
-            if (s0 != g || r != r_first) request(r, s0);
+        for (int s0 = 0; s0 < ns; s0 += U * s_step) {
+            if (s0 != 0) request(x, k, s0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int s = s0 + u * G;
-                const float wt = s < ns ? w[s * 32 + (on ? r : 0)] : 0.f;
+                if (s0 + u * s_step >= ns) continue;
+                const int s = s0 + u * s_step + s_first;
+                const float ws = __shfl(w, s & 63);
+                const float wt = s < ns ? ws : 0.f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[i] = fmaf(wt, x[u][i], acc[i]);
             }
         }
-        if (G > 1) {
-            red[tid] = acc;
-            __syncthreads();
-            if (g == 0)
-                for (int k = 1; k < G; ++k) acc += red[tid + k * rs * LPR];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (SUBS == 4) acc[i] = reduce_row_lanes(acc[i], [](float a, float c) { return a + c; });
+            if (SUBS == 2) acc[i] = half_pair_sum(acc[i]);
         }
-        if (on && g == 0) store_out4<OUT_DT>(out0 + (int64_t)r * p.o_sn + col * 2, acc);
-        if (G > 1) break;
+        if (G > 1) {                                     // (one row per wave then: every wave comes here once)
+            v4f* red = (v4f*)smem;
+            if (g > 0) red[wave * 64 + lane] = acc;
+            __syncthreads();
+            if (g > 0) return;
+            for (int j = 1; j < G; ++j) acc += red[(wave + j * rs) * 64 + lane];
+        }
+        if (sub == 0 && r < nrows) store_out4<OUT_DT>(out0 + (int64_t)r * p->o_sn + col * 2, acc);
+        if (more) {
+            lse = lse_next;
+            if (ns <= U * s_step) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) x[u] = x_next[u];
+            } else {
+                request(x, k + 1, 0);
+            }
+        }
     }
 }
 

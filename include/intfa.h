@@ -193,7 +193,7 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
 size_t intfa_fwd_workspace_bytes(const intfa_fwd_params* p);
 
 /* Bytes of workspace with which the split-KV forward merges the partials itself instead of launching a merge kernel
- * behind it: intfa_fwd_workspace_bytes() plus 8 bytes per 32 query rows of every head (0 when num_splits <= 1).  Nothing has to be
+ * behind it: intfa_fwd_workspace_bytes() plus 256 bytes per 16 query rows of every head (0 when num_splits <= 1).  Nothing has to be
  * cleared; with less, down to intfa_fwd_workspace_bytes(), the merge is a second launch.  Two launches that may run at the
  * same time must not share a workspace, with or without the merge. */
 size_t intfa_fwd_merge_workspace_bytes(const intfa_fwd_params* p);

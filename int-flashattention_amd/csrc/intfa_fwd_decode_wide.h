@@ -500,6 +500,12 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                     }
                 }
         }
+        // The products are consumed inside the step: sunk behind the loop's branch, the first register of the last one may be read without the wait
+        // states that an MFMA's result needs (the compiler counts them along the longer of two ways there).
+#pragma unroll
+        for (int j = 0; j < CTW; ++j)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) asm volatile("" : "+v"(o_acc[j][rt]));
     };
 
     if (nb_begin < nb_end) {

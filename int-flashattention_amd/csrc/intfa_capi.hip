@@ -211,11 +211,13 @@ int dispatch(int variant, const intfa_fwd_params* p, KParams kp, bool dump_s, hi
     sel.dump_s = dump_s;
     sel.wide = decode_shaped(kp.seqlen);
     const int64_t wgs = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kDecodeRows - 1) / kDecodeRows) * kp.num_splits;
-    // The decode-shaped kernels' forms, which give the same bits.  Rows past the 16th go to a workgroup of their own while both find a compute
-    // unit to themselves (half-int8 d64, 20 rows, 256 keys 6.0 -> 5.3 us; K and V then come from the L2 twice).  Half steps: two
-    // workgroups per compute unit instead of one (WideGeom).
+    // The decode-shaped kernels' forms.  Rows past the 16th go to a workgroup of their own while both find a compute unit to themselves
+    // (half-int8 d64, 20 rows, 256 keys 6.0 -> 5.3 us; K and V then come from the L2 twice).  Crowded (full-int8 up to head_dim 128): more
+    // workgroups than compute units (head_dim 64, up to 16 rows: than two per unit) get the form of WideGeom with room for more of
+    // them; head_dim 64 with more rows the four-wave kernel, whose 32-row MFMA tiles need half the LDS reads per product (us, eight
+    // waves -> four: B16 H32/8 Nq5 Nk3000, 512 workgroups 19.3 -> 16.1, B9 H8 Nq32 Nk9000 27.0 -> 22.8, 256 workgroups 19.6 both).
     sel.row_tiles = kp.seqlen <= 16 || (2 * wgs <= kComputeUnits && !streams_kv(kp)) ? 1 : 2;
-    sel.half_steps = wgs > kComputeUnits;
+    sel.crowded = wgs > (kp.head_dim == 64 && sel.row_tiles == 1 ? 2 : 1) * kComputeUnits;
     const int d = kp.head_dim;
     if (vblk && kp.vs_sub == 2) {
         if (d == 128) return launch_full_int8_vblk64_d128(kp, sel, stream);
@@ -319,17 +321,19 @@ int intfa_fwd_suggest_splits(const intfa_fwd_params* p, int variant, int num_cus
     const bool decode = decode_shaped(p->seqlen);
     if (decode) {
         wgs = (int64_t)p->batch * p->heads * ((p->seqlen + kDecodeRows - 1) / kDecodeRows);
-        // head_dim 256 with 16-bit V: 96 KiB and more of tiles, one workgroup per compute unit
-        if (p->head_dim == 256 && variant != INTFA_VARIANT_FULL_INT8) slots = cus;
+        // head_dim 256 with 16-bit V: 96 KiB and more of tiles, one workgroup per compute unit.  (Full-int8 there has room for two, and keeps the
+        // count for the sake of its results.)
+        if (p->head_dim == 256) slots = cus;
     }
     else if (p->head_dim == 256) wgs *= 2;     // full-int8: eight-wave workgroups, one per compute unit; the others: column halves
     if (wgs * 5 >= slots * 4) return 1;                                        // at least 80 % of the slots are used anyway
     const int seqlen_k = p->seqlen_k > 0 ? p->seqlen_k : p->seqlen;
     const int bn = block_n_for(variant, p->head_dim);
     const int64_t blocks = (seqlen_k + bn - 1) / bn;
-    // (decode-shaped workgroups are equal in work, so one that starts in a second round doubles the time: full-int8 d128, 36 heads, 16363 keys,
-    // 15 splits on 512 slots 42 us, 14 splits 31)
-    int64_t splits = decode ? slots / wgs : (slots + wgs - 1) / wgs;
+    // Decode-shaped workgroups are equal in work, so one that starts in a second round doubles the time (half-int8 d128, 120 heads, 2805 keys, five
+    // splits on 512 slots 37 us, four 27).  Full-int8 takes them all the same: with fewer, longer ranges P is requantised in coarser frames
+    // (2 splits 3.2e-2 from exact attention, 1 split 3.8e-2, over 320 heads of 4096 keys).
+    int64_t splits = decode && variant != INTFA_VARIANT_FULL_INT8 ? slots / wgs : (slots + wgs - 1) / wgs;
     if (splits < 1) splits = 1;
     if (splits > blocks / 4) splits = blocks / 4;                              // keep four key blocks per split
     // Decode-shaped calls merge inside the launch, so a split costs little (2 us for the first one, then the reading of its partial by

@@ -1,5 +1,6 @@
 // Full-int8 forward whose waves share the keys: for small single-pass problems (decode_kernel_takes, intfa_capi.hip) the kernel of this file,
-// for few query rows per head the one of intfa_fwd_decode_wide.h behind the same name.
+// for few query rows per head the one of intfa_fwd_decode_wide.h behind the same name (but at head_dim 64 with more than 16 rows
+// and more workgroups than compute units: dispatch()).
 //
 // Same arithmetic as fwd_full_int8_kernel (flash_atten_full_int8.py:9-71 per 128-key block: int32 S, dequantise, running
 // max, P = exp2(X c - m), P requantised with the fixed scale 127, int32 P V, fp32 accumulator), other division of labour.
@@ -28,7 +29,7 @@
 namespace intfa {
 
 // Head_dim 128: one 128-key block per step, the block of the general kernel.  Head dims 64 and 256: two 64-key blocks.
-template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool VBLK>
+template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool VBLK, bool FEW /* few query rows: splits, grouped heads as rows, non-temporal K and V */>
 __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_int8_kernel(const KParams p) {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
@@ -58,17 +59,22 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lq = lane & 31, lh = lane >> 5;
 
-    // ---- block -> (head, 32-row query block); whole K/V heads go to one XCD as in the general kernel
+    // ---- block -> (head, 32-row query block, split); whole K/V heads go to one XCD as in the general kernel
     const int n_mblk = (p.seqlen + kDecodeRows - 1) / kDecodeRows;
     const WorkgroupJob wg = deal_workgroup(p, block_after_kernargs());
-    const int mb = p.causal ? n_mblk - 1 - wg.rem : wg.rem;     // heaviest query blocks first
-    const int b = wg.b, h = wg.h, hk = wg.hk;
+    const int n_split = FEW ? p.num_splits : 1;
+    const int mb_idx = FEW ? fast_div(wg.rem, p.d_n_split) : wg.rem, split = wg.rem - mb_idx * n_split;
+    const int mb = p.causal ? n_mblk - 1 - mb_idx : mb_idx;     // heaviest query blocks first
+    const int b = wg.b, h = wg.h, hk = wg.hk, group = (b * p.heads + h) * n_mblk + mb;
 
     const int seqlen_k = keys_of_batch(p, b);
     // causal: row i sees keys 0 .. i + causal_off (mask aligned to the bottom right corner as in the general kernels: a few
     // new tokens against a cache); blocks past the last row's limit are not visited
-    const int causal_off = seqlen_k - p.seqlen;
-    const KeyBlocks kb = key_block_range<BNB>(seqlen_k, p.causal != 0, mb * kDecodeRows + kDecodeRows, causal_off, false, 1, 0, false, 0);
+    // (causal_rows: the rows hold several query heads of one K/V group, causal_rows positions each)
+    const int fold = FEW ? p.causal_rows : 0;
+    const int causal_off = seqlen_k - (fold ? fold : p.seqlen);
+    const KeyBlocks kb = key_block_range<BNB>(seqlen_k, p.causal != 0, fold ? fold : mb * kDecodeRows + kDecodeRows, causal_off, n_split > 1,
+                                              n_split, split, false, FEW ? p.blocks_per_split : 0);
     const int nb_begin = kb.begin, nb_end = kb.end;         // in blocks of BNB keys
     const int key_end = nb_end * BNB < seqlen_k ? nb_end * BNB : seqlen_k;      // one past the last key of the range
     const int q_row = mb * kDecodeRows + lq;
@@ -92,13 +98,20 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const auto k_lane = tile_load_lane<D, SWZ_K, BN>(k_sn, wave, lane);
     const auto v_lane = tile_load_lane<D, SWZ_V8, BN>(v_sn, wave, lane);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    const bool stream = p.stream_kv != 0;
     auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<D, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
-        issue_tile_load<D, SWZ_V8, BN>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        auto issue = [&](auto nt) __attribute__((always_inline)) {
+            issue_tile_load<D, SWZ_K, BN, decltype(nt)::value>(k_rsrc, (uint32_t)(nb * BNB) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
+            issue_tile_load<D, SWZ_V8, BN, decltype(nt)::value>(v_rsrc, (uint32_t)(nb * BNB) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        };
+        if (FEW && stream) issue(BoolTag<true>{});
+        else issue(BoolTag<false>{});
     };
     // The first tiles are requested ahead of everything else: Q, the scales and the lane offsets below arrive or are computed under
     // their way from HBM.
     if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    uint64_t ticket_seen = 0;
+    if (FEW && n_split > 1) ticket_seen = splitkv_look_at_tickets(p, group);
     // ---- Q fragment (B operand of S^T = K Q^T), the same 32 rows in every wave
     v4i qreg[KS];
     load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);
@@ -157,8 +170,8 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     // nothing (the same instruction stream for every wave; a run-time "owns a tile" test around the V fragments and the
     // accumulator update costs the owners a hundred register copies per step)
     // the last visible key of the first row of this query block, and of the lane's row
-    const int first_lim = p.causal ? mb * kDecodeRows + causal_off : 0x3fffffff;
-    const int row_lim = p.causal ? q_row + causal_off : 0x3fffffff;
+    const int first_lim = p.causal ? (fold ? 0 : mb * kDecodeRows) + causal_off : 0x3fffffff;
+    const int row_lim = p.causal ? (fold ? q_row % fold : q_row) + causal_off : 0x3fffffff;
     const bool blk_a = NBS == 1 || wave < 2;                          // this wave's keys belong to the first block of a step
 
     auto step = [&](auto buf_tag, int nb) __attribute__((always_inline)) {
@@ -339,6 +352,31 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     const float out_scale = !seen ? 0.f : (PROUND == 0) ? (vs / l_tot) : (vs / (127.f * l_tot));
     const float l_true = (PROUND == 0) ? l_tot * (1.f / 127.f) : l_tot;
     const float lse = seen ? m_run + __builtin_log2f(l_true) : -INFINITY;
+    if (FEW && n_split > 1) {
+        const KernargPtr pe = kernarg_block();
+        splitkv_open_tickets(pe, group, ticket_seen);
+        const SplitPartials part(pe, D, ((int64_t)(split * pe->batch + b) * pe->heads + h) * pe->seqlen + mb * kDecodeRows);
+        if (q_valid) {
+#pragma unroll
+            for (int j = 0; j < DTW; ++j) {
+                const int dt = wave + 4 * j;
+                if (dt >= DT) continue;
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4) {
+                    v4f o;
+#pragma unroll
+                    for (int b4 = 0; b4 < 4; ++b4) o[b4] = seen ? o_acc[j][4 * a4 + b4] * out_scale : 0.f;
+                    part.put(lq, D, 32 * dt + 8 * a4 + 4 * lh, o);
+                }
+            }
+            if (wave == 0 && lh == 0) part.put_lse(lq, seen ? lse : -INFINITY);
+        }
+        if (pe->ticket == nullptr || !splitkv_last_arrival(pe, smem, group)) return;
+        static_assert(kMergeLds <= LDS_BYTES, "the merge fits the tile memory");
+        const int row0 = mb * kDecodeRows, rows_left = pe->seqlen - row0;
+        splitkv_merge_rows<D, OUT_DT, 4>(pe, smem, b, h, row0, rows_left < kDecodeRows ? rows_left : kDecodeRows);
+        return;
+    }
     if (!q_valid) return;
     char* orow = p.out + b * p.o_sb + h * p.o_sh + (int64_t)q_row * p.o_sn;
 #pragma unroll
@@ -367,7 +405,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 
 // Few query rows per head, split or not: intfa_fwd_decode_wide.h.
 template <int D, class /* WideRows */ R, int OUT_DT, int PROUND, bool VBLK>
-__global__ void __launch_bounds__(kWideThreads, (D == 128 && !R::half_steps) || (D == 256 && VBLK && R::tiles == 2) ? 2 : 4) fwd_decode_full_int8_kernel(const KParams p) {
+__global__ void __launch_bounds__(kWideThreads, (D == 128 && !R::crowded) || (D == 256 && VBLK && R::tiles == 2) ? 2 : D == 64 && R::crowded ? 6 : 4) fwd_decode_full_int8_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     decode_wide<D, true, true, OUT_DT, PROUND, VBLK, R>(p);
 #endif

@@ -14,8 +14,8 @@
 //     16 query rows (RT = 1: up to 16 rows, four values per tile) or of two such row tiles (RT = 2: up to 32);
 //   * wave w computes S^T of its NT tiles; the row maxima of the waves meet in LDS (barrier), every wave then knows the running maximum
 //     of each key block of the step; it exponentiates its keys in their block's frame and publishes P (barrier); every wave multiplies
-//     P of the whole step with its 16 (head_dim 256: 32) columns of V.  Head_dim 64 has four such column tiles: waves 4 - 7 take the second
-//     half of the step's keys, and the two sums meet in the epilogue;
+//     P of the whole step with its 16 (head_dim 256: 32) columns of V.  Head_dim 64 has four such column tiles: waves 4 - 7 take every other
+//     block (16-bit V: the second half) of the step's keys, and the two sums meet in the epilogue;
 //   * the first tiles are requested as soon as their addresses are known, ahead of Q, the scales and the tickets.
 // The frames are those of the general full-int8 kernel: a step holds two blocks of 128 keys (head_dim 128), four of 64 (head_dim 64) or two
 // of 64 (head_dim 256), and m_0 = max(m, max_0), m_1 = max(m_0, max_1), ... with the factors alpha_i = 2^(m_(i-1) - m_i).  The 16-bit P V
@@ -29,30 +29,29 @@
 namespace intfa {
 
 constexpr int kWideWaves = 8, kWideThreads = 64 * kWideWaves;
-// RT: row tiles of 16 query rows.  HALF (full-int8 at head_dim 128): steps of 128 keys instead of 256
-template <int RT, bool HALF> struct WideRows { static constexpr int tiles = RT; static constexpr bool half_steps = HALF; };
+// RT: row tiles of 16 query rows.  CROWDED (full-int8 up to head_dim 128): the form with room for more workgroups per compute unit
+template <int RT, bool CROWDED> struct WideRows { static constexpr int tiles = RT; static constexpr bool crowded = CROWDED; };
 static_assert(kWideWaves == kMergeWaves, "");
 
 // VI8: int8 V (full-int8); KI8: int8 Q, K
-template <int D, bool KI8, bool VI8, bool HALF> struct WideGeom {
+template <int D, bool KI8, bool VI8, typename R> struct WideGeom {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
     static constexpr int KROW = D * (KI8 ? 1 : 2), VROW = D * (VI8 ? 1 : 2);      // bytes per row
     // Two steps of tiles in the LDS, and two workgroups per compute unit: with one, its prologue and its merge (4 - 6 us) overlap with nothing.
-    // Head_dim 256 with 16-bit V has one (fewer than four 16-key tiles are too few).  Full-int8 at head_dim 128 has both
-    // forms, one block per step or two: with no more workgroups than compute units the longer step is better (step of one
-    // request, us: 128 keys 1.0, 256 keys 1.3).
-    static constexpr int KEYS = VI8 && D < 256 && !HALF ? 256 : D == 256 || (D == 128 && !VI8) ? 64 : 128;
+    // Head_dim 256 with 16-bit V has one (fewer than four 16-key tiles are too few).  Full-int8 up to head_dim 128 has a second form with
+    // room for more workgroups: head_dim 128 steps of 128 keys instead of 256 (step of one request, us: 1.0 and 1.3, so the longer one while
+    // there is room), head_dim 64 one step's tiles instead of two, the next ones requested once all waves hold theirs in registers
+    // (three workgroups per unit instead of two, us: 640 workgroups 54 -> 39.7, 960 of 1500 keys 42.1 (128-key steps) -> 37.7).
+    static constexpr int BUFS = VI8 && D == 64 && R::crowded ? 1 : 2;
+    static constexpr int KEYS = VI8 && D < 256 && (!R::crowded || BUFS == 1) ? 256 : D == 256 || (D == 128 && !VI8) ? 64 : 128;
     static constexpr int BNB = VI8 ? (D == 128 ? 128 : 64) : KEYS;                // keys per frame
     static constexpr int BLK = VI8 ? BNB : kBlockN16;                             // key block of the split ranges: intfa_fwd_block_n()
     static constexpr int NB = KEYS / BNB;
     static constexpr int NKT = KEYS / 16;                                         // 16-key tiles per step
     static constexpr int NT = NKT >= kWideWaves ? NKT / kWideWaves : 1;           // ... per wave
     static constexpr int QKW = NKT / NT;                                          // waves with tiles of S^T
-    // The tiles of wave w: NT neighbours of one block, or (two 128-key blocks) tile w of each, so that a lane's row sum is the same
-    // number whichever step length runs.
-    static constexpr bool BOTH = NT == 2 && BNB == 128;
-    __device__ static constexpr int tile(int w, int t) { return BOTH ? w + 8 * t : NT * w + t; }
-    static constexpr int TILE_STEP = BOTH ? 8 : 1;                                // from a wave's tile to its next one
+    // Tile t of wave w: w + 8 t, so that a lane adds the same keys' row sums in the same order whichever step length runs; its frame.
+    __device__ static constexpr int frame_of(int w, int t) { return (w + 8 * t) / (BNB / 16); }
     static constexpr int KS = KROW / 64;                                          // MFMA k-steps of S^T
     static constexpr int TB = VI8 ? 4 : 8;                                        // bytes of P per lane and tile
     static constexpr int TPO = 16 / TB;                                           // tiles per P V MFMA
@@ -62,6 +61,7 @@ template <int D, bool KI8, bool VI8, bool HALF> struct WideGeom {
     static constexpr int CTW = CT / kWideWaves > 0 ? CT / kWideWaves : 1;         // column tiles per wave
     static constexpr int NOPW = NOP / KH;                                         // MFMAs per wave, column tile and row tile
     static constexpr int OPB = NOP / NB;                                          // ... per frame
+    static_assert(!VI8 || KH == 1 || (KH == 2 && OPB == 1), "head_dim 64: waves 0 - 3 take the even blocks of a step, 4 - 7 the odd ones");
     static constexpr int KT = KEYS * KROW, VT = KEYS * VROW;
 };
 
@@ -112,7 +112,7 @@ template <> struct WideAcc<true> { typedef v4i type; };
 // IO_DT: type of the output (and of the 16-bit operands), 0 fp16, 1 bf16.  PROUND, VBLK: full-int8 only (see fwd_full_int8_kernel).
 template <int D, bool KI8, bool VI8, int IO_DT, int PROUND, bool VBLK, class R>
 __device__ __forceinline__ void decode_wide(const KParams& p) {
-    using G = WideGeom<D, KI8, VI8, R::half_steps>;
+    using G = WideGeom<D, KI8, VI8, R>;
     constexpr int RT = R::tiles, ROWS = 16 * RT;
     constexpr int NB = G::NB, NT = G::NT, KS = G::KS, TB = G::TB, TPO = G::TPO, CT = G::CT, KH = G::KH, CTW = G::CTW, NOPW = G::NOPW;
     constexpr int KCH = G::KROW / 16, VCH = G::VROW / 16, BPS = G::KEYS / G::BLK;       // BPS: key blocks per step
@@ -120,13 +120,14 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
     // LDS map (bytes)
     constexpr int OFF_KS = 0;                            // two fp32 k_scale vectors
     constexpr int OFF_XM = 2 * G::KEYS * 4;              // row maxima / row sums of the waves' keys, fp32
-    constexpr int OFF_XP = OFF_XM + 16 * RT * (G::BOTH ? 16 : kWideWaves) * 4;           // P operands: [MFMA][row tile][lane][16 bytes]
+    constexpr int XW = G::NKT > kWideWaves ? G::NKT : kWideWaves;     // words per row there: one per tile; the row sums one per wave
+    constexpr int OFF_XP = OFF_XM + 16 * RT * XW * 4;    // P operands: [MFMA][row tile][lane][16 bytes]
     constexpr int OFF_VS = OFF_XP + G::NOP * RT * 1024;                  // VBLK: two vectors of NV fp32 channel scales
     constexpr int OFF_K = (OFF_VS + (VBLK ? 2 * NV * 4 : 0) + 1023) / 1024 * 1024;
-    constexpr int OFF_V = OFF_K + 2 * G::KT;
+    constexpr int OFF_V = OFF_K + G::BUFS * G::KT;
     // (half-int8 at head_dim 128 would fit three times: a full grid of 1024 workgroups then ends with a third of the card, 247 us for 1.6 GB
     // of K and V against 234 with two)
-    constexpr int LDS_BYTES = OFF_V + 2 * G::VT > 56 * 1024 || D != 128 ? OFF_V + 2 * G::VT : 56 * 1024;
+    constexpr int LDS_BYTES = OFF_V + G::BUFS * G::VT > 56 * 1024 || D != 128 ? OFF_V + G::BUFS * G::VT : 56 * 1024;
     static_assert(LDS_BYTES <= 160 * 1024 && kMergeLds <= LDS_BYTES, "a workgroup fits the LDS of a compute unit, and the merge the workgroup's");
     static_assert(KH == 1 || CT * RT * 1024 <= G::KT, "the sums of the key parts meet in the first K tile");
     __shared__ __attribute__((aligned(1024))) char smem[LDS_BYTES];
@@ -229,26 +230,27 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
     const int k_swz = swz_k<G::KROW>(ln) & (KCH - 1);
     uint32_t k_rd[KS];                                   // row 16 * tile + ln, chunk 4 * ks + lh
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) k_rd[ks] = OFF_K + (16 * G::tile(wave, 0) + ln) * G::KROW + (((4 * ks + lh) ^ k_swz) << 4);
+    for (int ks = 0; ks < KS; ++ks) k_rd[ks] = OFF_K + (16 * wave + ln) * G::KROW + (((4 * ks + lh) ^ k_swz) << 4);
     // V (A operand of O^T = V^T P^T) through the transposing 8-byte loads, 16 lanes (one lh) at a time:
     //   int8:   source lane s at key row 16 * (s >> 3) + 4 * lh + ((s >> 1) & 3), 8-byte half s & 1 of the column tile's 16 bytes: two tiles a load
     //   16-bit: source lane s at key row 4 * lh + (s >> 2), 8-byte quarter s & 3 of the column tile's 32 bytes: one tile a load
     const int s16 = lane & 15;
     const int v_row = VI8 ? 16 * (s16 >> 3) + 4 * lh + ((s16 >> 1) & 3) : 4 * lh + (s16 >> 2);
-    const int kh = KH > 1 ? wave / CT : 0;               // which part of the step's keys
+    // which part of the step's keys: the odd blocks, or (16-bit V) the second half; its MFMA o is number OPS * o + kh * OPH of the step
+    const int kh = KH > 1 ? wave / CT : 0;
+    constexpr int OPS = VI8 ? KH : 1, OPH = VI8 ? 1 : NOPW;
     uint32_t v_rd[CTW];
 #pragma unroll
     for (int j = 0; j < CTW; ++j) {
         const int ct = wave % CT + kWideWaves * j;
         const int chunk = VI8 ? ct : 2 * ct + ((s16 >> 1) & 1);
-        v_rd[j] = OFF_V + (16 * TPO * NOPW * kh + v_row) * G::VROW + ((chunk ^ (swz_v_wide<G::VROW, VI8>(v_row) & (VCH - 1))) << 4) + 8 * (s16 & 1);
+        v_rd[j] = OFF_V + (16 * TPO * OPH * kh + v_row) * G::VROW + ((chunk ^ (swz_v_wide<G::VROW, VI8>(v_row) & (VCH - 1))) << 4) + 8 * (s16 & 1);
     }
-    const uint32_t kk_rd = OFF_KS + 4 * (16 * G::tile(wave, 0) + 4 * lh);
-    // row maxima: [row][wave], twice (BOTH: once per block); row sums: [row][wave]
-    constexpr int XW = G::BOTH ? 16 : kWideWaves;
-    const uint32_t xm_wr = OFF_XM + 4 * (XW * ln + wave), xm_rd = OFF_XM + 4 * XW * ln;     // + 64 * XW per row tile, + 32 per tile (BOTH)
-    const uint32_t xp_wr = OFF_XP + (G::tile(wave, 0) / TPO) * RT * 1024 + 16 * lane + TB * (G::tile(wave, 0) % TPO);    // + 8 / TPO * RT * 1024 per tile (BOTH)
-    const uint32_t xp_rd = OFF_XP + kh * NOPW * RT * 1024 + 16 * lane;
+    const uint32_t kk_rd = OFF_KS + 4 * (16 * wave + 4 * lh);
+    // row maxima: [row][tile]; row sums: [row][wave]
+    const uint32_t xm_wr = OFF_XM + 4 * (XW * ln + wave), xm_rd = OFF_XM + 4 * XW * ln;     // + 64 * XW per row tile, + 32 per tile
+    const uint32_t xp_wr = OFF_XP + (wave / TPO) * RT * 1024 + 16 * lane + TB * (wave % TPO);    // + 8 / TPO * RT * 1024 per tile
+    const uint32_t xp_rd = OFF_XP + kh * OPH * RT * 1024 + 16 * lane;
     const uint32_t vs_wr = OFF_VS + 4 * vs_i;
     const uint32_t vs_rd = OFF_VS + 4 * (16 * (wave % CT) + 4 * lh);                  // + 4 * D per block, + 4 * 16 * kWideWaves per column tile
     const bool qk_wave = wave < G::QKW;
@@ -261,7 +263,6 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
         const int row = row0 + 16 * rt + ln;
         row_lim[rt] = p.causal ? (fold ? row % fold : row) + causal_off : 0x3fffffff;
     }
-    const int my_blk = G::BOTH ? 0 : (NT * wave * 16) / G::BNB;        // the frame of this wave's keys (BOTH: tile t in frame t)
 
     auto mfma_s = [&](v4i a, v4i q, auto c) __attribute__((always_inline)) {
         if constexpr (KI8) return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, q, c, 0, 0, 0);
@@ -272,14 +273,14 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
 
     auto step = [&](auto buf_tag, int nb) __attribute__((always_inline)) {
         constexpr int BUF = decltype(buf_tag)::value ? 1 : 0;
-        constexpr int KB = BUF * G::KT, VB = BUF * G::VT, SB = BUF * G::KEYS * 4, VSB = BUF * NV * 4;
+        constexpr int KB = (G::BUFS - 1) * BUF * G::KT, VB = (G::BUFS - 1) * BUF * G::VT, SB = BUF * G::KEYS * 4, VSB = BUF * NV * 4;
         // (the scales of this step were requested right behind its tiles)
         if (ks_wave) *(float*)(smem + ks_wr + SB) = ks_src.cvt(ks_next);
         if (vs_wave) *(float*)(smem + vs_wr + VSB) = vs_next;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();                                   // the tiles have landed; the other buffer and the exchange areas are free
         if (nb + BPS < nb_end) {
-            issue_loads(nb + BPS, BUF ^ 1);
+            if (G::BUFS == 2) issue_loads(nb + BPS, BUF ^ 1);
             if (ks_wave) ks_next = load_ks(nb + BPS);
             if (vs_wave) vs_next = load_vs(nb + BPS);
         }
@@ -291,8 +292,8 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks) fr[t][ks] = *(const v4i*)(smem + k_rd[ks] + KB + 16 * t * G::TILE_STEP * G::KROW);
-                if (KI8) kk[t] = *(const v4f*)(smem + kk_rd + SB + 64 * t * G::TILE_STEP);
+                for (int ks = 0; ks < KS; ++ks) fr[t][ks] = *(const v4i*)(smem + k_rd[ks] + KB + 128 * t * G::KROW);
+                if (KI8) kk[t] = *(const v4f*)(smem + kk_rd + SB + 512 * t);
             }
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
@@ -309,7 +310,7 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
             for (int o = 0; o < NOPW; ++o)
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const uint32_t a = v_rd[j] + VB + (16 * TPO * o + 8 * TPO * u) * G::VROW;
+                    const uint32_t a = v_rd[j] + VB + (16 * TPO * OPS * o + 8 * TPO * u) * G::VROW;
                     v2i x;
                     if (VI8) x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) v2i*)INTFA_LDS(smem + a));
                     else x = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)INTFA_LDS(smem + a)));
@@ -334,11 +335,11 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                 asm volatile("");
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
-                    const int last = (row_lim[rt] < key_end - 1 ? row_lim[rt] : key_end - 1) - key0 - 16 * G::tile(wave, 0) - 4 * lh;
+                    const int last = (row_lim[rt] < key_end - 1 ? row_lim[rt] : key_end - 1) - key0 - 16 * wave - 4 * lh;
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) x[t][rt][r] = hide_past(x[t][rt][r], last, 16 * t * G::TILE_STEP + r);
+                        for (int r = 0; r < 4; ++r) x[t][rt][r] = hide_past(x[t][rt][r], last, 128 * t + r);
                 }
             }
 #pragma unroll
@@ -346,27 +347,26 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                 float mx[NT];
 #pragma unroll
                 for (int t = 0; t < NT; ++t) mx[t] = fmaxf(fmaxf(x[t][rt][0], x[t][rt][1]), fmaxf(x[t][rt][2], x[t][rt][3]));
-                if (!G::BOTH && NT == 2) mx[0] = fmaxf(mx[0], mx[NT - 1]);
 #pragma unroll
-                for (int t = 0; t < (G::BOTH ? NT : 1); ++t) {
+                for (int t = 0; t < NT; ++t) {
                     mx[t] = reduce_row_lanes(mx[t], [](float a, float c) { return fmaxf(a, c); });
                     if (lh == 0) *(float*)(smem + xm_wr + 64 * XW * rt + 32 * t) = mx[t];
                 }
             }
         }
-        __syncthreads();                                   // the waves' maxima are in LDS
-        float alpha[NB][RT], after[RT], bias[RT][NT];
+        if (G::BUFS == 1) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __syncthreads();                                   // the waves' maxima are in LDS (one buffer: its tiles are in registers)
+        if (G::BUFS == 1 && nb + BPS < nb_end) issue_loads(nb + BPS, 0);
+        float alpha[NB][RT], bias[RT][NT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            float wm[XW];
+            float wm[G::NKT];
 #pragma unroll
-            for (int i = 0; i < XW / 4; ++i)
-                if (G::BOTH || 4 * i < G::QKW) *(v4f*)(wm + 4 * i) = *(const v4f*)(smem + xm_rd + 64 * XW * rt + 16 * i);
+            for (int i = 0; i < G::NKT / 4; ++i) *(v4f*)(wm + 4 * i) = *(const v4f*)(smem + xm_rd + 64 * XW * rt + 16 * i);
             float m = m_run[rt];
-            after[rt] = 1.f;
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
-                constexpr int W = G::BOTH ? kWideWaves : G::QKW / NB;      // waves with keys of one frame
+                constexpr int W = G::NKT / NB;             // tiles per frame
                 float mx = wm[i * W];
 #pragma unroll
                 for (int w = 1; w < W; ++w) mx = fmaxf(mx, wm[i * W + w]);
@@ -374,12 +374,8 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                 alpha[i][rt] = fast_exp2(m - m_new);
                 m = m_new;
                 const float bi = (VI8 && PROUND == 0 ? kLog2_127 : 0.f) - m;
-                if (G::BOTH) bias[rt][i < NT ? i : 0] = bi;
-                else {
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) bias[rt][t] = i == 0 || i == my_blk ? bi : bias[rt][t];
-                    if (i > 0) after[rt] = i > my_blk ? after[rt] * alpha[i][rt] : after[rt];
-                }
+                for (int t = 0; t < NT; ++t) bias[rt][t] = NB == 1 || i == 0 || i == G::frame_of(wave, t) ? bi : bias[rt][t];
             }
             m_run[rt] = m;
         }
@@ -393,14 +389,12 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                     e[i] = fast_exp2(fmaf(x[i / 4][rt][i % 4], qsc[rt], bias[rt][i / 4]));       // RNE mode: 127 * p
                     sum[i / 4] = i % 4 ? sum[i / 4] + e[i] : e[i];
                 }
-                if (G::BOTH || NB == 1) {
 #pragma unroll
-                    for (int i = 0; i < NB; ++i) l_run[rt] = fmaf(l_run[rt], alpha[i][rt], sum[i < NT ? i : 0]);
-                } else {
-                    float total = alpha[0][rt];
+                for (int i = 0; i < NB; ++i) {
+                    float own = 0.f;                       // block after block, so that the sequence does not depend on the step's length
 #pragma unroll
-                    for (int i = 1; i < NB; ++i) total *= alpha[i][rt];
-                    l_run[rt] = fmaf(l_run[rt], total, (NT == 2 ? sum[0] + sum[NT - 1] : sum[0]) * after[rt]);
+                    for (int t = 0; t < NT; ++t) own = NB == 1 || i == G::frame_of(wave, t) ? sum[t] : own;
+                    l_run[rt] = fmaf(l_run[rt], alpha[i][rt], own);
                 }
                 const uint32_t at = xp_wr + 1024 * rt;
                 if constexpr (VI8) {
@@ -415,11 +409,8 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                     } else {
                         requant_p_reference<NT>(e, pk);                                   // the reference's fp16 chain
                     }
-                    if constexpr (G::BOTH) {
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) *(uint32_t*)(smem + at + 8 / TPO * RT * 1024 * t) = pk[t];
-                    } else if constexpr (NT == 2) *(v2i*)(smem + at) = (v2i){(int)pk[0], (int)pk[1]};
-                    else *(uint32_t*)(smem + at) = pk[0];
+                    for (int t = 0; t < NT; ++t) *(uint32_t*)(smem + at + 8 / TPO * RT * 1024 * t) = pk[t];
                 } else {
                     static_assert(VI8 || NT == 1, "16-bit P: one tile per wave");
                     if constexpr (IO_DT == 0) *(v4h*)(smem + at) = __builtin_convertvector((v4f){e[0], e[1], e[2], e[3]}, v4h);
@@ -432,7 +423,7 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
 #pragma unroll
             for (int i = 0; i < NB / KH; ++i)
 #pragma unroll
-                for (int j = 0; j < CTW; ++j) vsc[i][j] = *(const v4f*)(smem + vs_rd + VSB + 4 * D * (kh * (NB / KH) + i) + 64 * kWideWaves * j);
+                for (int j = 0; j < CTW; ++j) vsc[i][j] = *(const v4f*)(smem + vs_rd + VSB + 4 * D * (KH * i + kh) + 64 * kWideWaves * j);
         }
         __syncthreads();                                   // P is in LDS
         // -------- this wave's columns: O^T[d, q] = O^T alpha + V^T[d, key] P^T[key, q], block after block
@@ -440,7 +431,7 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
 #pragma unroll
         for (int o = 0; o < NOPW; ++o)
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) pall[o][rt] = *(const v4i*)(smem + xp_rd + 1024 * (RT * o + rt));
+            for (int rt = 0; rt < RT; ++rt) pall[o][rt] = *(const v4i*)(smem + xp_rd + 1024 * (RT * OPS * o + rt));
         if constexpr (VI8) {
             constexpr int NBW = NB / KH;                   // blocks of this wave's keys
 #pragma unroll
@@ -453,22 +444,16 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
 #pragma unroll
                         for (int o = 0; o < G::OPB; ++o)
                             pv[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf[j][G::OPB * i + o], pall[G::OPB * i + o][rt], o == 0 ? (v4i){0, 0, 0, 0} : pv[i], 0, 0, 0);
-                    float a_in = 1.f, a_out = 1.f;         // factors of the blocks of other waves ahead of and behind this wave's
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        if (KH > 1 && i < NBW) a_in *= alpha[i][rt];
-                        if (KH > 1 && i >= NBW) a_out *= alpha[i][rt];
-                    }
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         float o = o_acc[j][rt][r];
-                        if (KH > 1) o = kh ? o * a_in : o;
 #pragma unroll
                         for (int i = 0; i < NBW; ++i) {
-                            const float al = KH > 1 ? (kh ? alpha[NBW + i][rt] : alpha[i][rt]) : alpha[i][rt];
-                            o = VBLK ? fmaf(o, al, (float)pv[i][r] * vsc[i][j][r]) : fmaf(o, al, (float)pv[i][r]);
+                            float pvf = (float)pv[i][r];
+                            if (VBLK) pvf *= vsc[i][j][r];
+                            if (KH == 1) o = fmaf(o, alpha[i][rt], pvf);
+                            else o = fmaf(fmaf(o, alpha[KH * i][rt], kh ? 0.f : pvf), alpha[KH * i + KH - 1][rt], kh ? pvf : 0.f);
                         }
-                        if (KH > 1) o = kh ? o : o * a_out;
                         o_acc[j][rt][r] = o;
                     }
                 }
@@ -482,7 +467,7 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                 for (int o = 0; o < NOPW; ++o)
 #pragma unroll
                     for (int u = 0; u < 2; ++u)
-                        if (16 * (TPO * (kh * NOPW + o) + u) > seen) {
+                        if (16 * (TPO * (kh * OPH + OPS * o) + u) > seen) {
 #pragma unroll
                             for (int j = 0; j < CTW; ++j) vf[j][o][2 * u] = vf[j][o][2 * u + 1] = 0;
                         }

@@ -218,24 +218,102 @@ template <typename F> __device__ __forceinline__ float reduce_wave(float x, F op
     return reduce_row_lanes(x, op);
 }
 
-// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; kMergeWaves waves, kMergeLds bytes of `smem`.
-// This runs once, at the end of a query block, and its time is a chain of latencies: a wave takes a row, its lanes the row's log-sum-exps
-// (lane s that of split s), which make the weights without a word of LDS, and the partials of the first splits are on their way
-// meanwhile, four columns per lane.  With fewer rows than waves the waves of a row share its splits and meet in LDS.
 constexpr int kMaxSplits = 64;                           // the lanes of a wave
 constexpr int kMergeWaves = 8;
 constexpr int kMergeLds = kMergeWaves * 64 * 16;
-template <int D, int OUT_DT>
+
+// More rows than waves: a wave takes four rows at a time, so that the chains of their weights run side by side, and D / 4 lanes a row of the
+// sums; partials of the next four splits are on their way while four are added.  Row after row, as below, the chains were 0.25 us
+// each: 32 rows, full-int8 d64 B9 H8 Nq32 Nk9000 27.0 -> 24, fp16 d64 B5 H32/8 Nq6 Nk7000 18.9 -> 18.3 us.
+template <int D, int OUT_DT, int WAVES, typename P>
+__device__ __forceinline__ void splitkv_merge_many(P p, const SplitPartials& part, char* smem, uint32_t base, char* out0, int nrows, int ns, int wave, int lane) {
+    constexpr int LPR = D / 4, SUBS = 64 / LPR, U = 4, C = 4;      // C rows side by side
+    const int sub = lane / LPR, col = (lane % LPR) * 4, groups = (ns + U - 1) / U;
+    float* const ws = (float*)smem + wave * (C * 64);      // weights of the wave's rows, of no other wave's concern
+    static_assert(WAVES * C * 64 * 4 <= kMergeLds, "");
+    for (int first = wave; first < nrows; first += C * WAVES) {      // rows first, first + WAVES, ...
+        auto row_of = [&](int i) __attribute__((always_inline)) { const int r = first + WAVES * i; return r < nrows ? r : first; };
+        float lse[C], mx[C], total[C];
+#pragma unroll
+        for (int i = 0; i < C; ++i) lse[i] = part.get_lse((uint32_t)(lane < ns ? lane : ns - 1) * part.rows + base + (uint32_t)row_of(i));
+        v4f x[U], y[U];
+        auto request = [&](v4f (&v)[U], int pass, int g) __attribute__((always_inline)) {
+            const uint32_t row = base + (uint32_t)row_of(pass * SUBS + sub);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int s = g * U + u;
+                v[u] = part.get((uint32_t)(s < ns ? s : ns - 1) * part.rows + row, D, col);
+            }
+        };
+        request(x, 0, 0);
+        bool empty[C];                                     // a row no split saw a key for: zeros with lse = -inf, as in splitkv_combine_kernel
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            lse[i] = lane < ns ? lse[i] : -INFINITY;
+            mx[i] = reduce_wave(lse[i], [](float a, float c) { return fmaxf(a, c); });
+            empty[i] = mx[i] == -INFINITY;
+            if (empty[i]) mx[i] = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            total[i] = reduce_wave(fast_exp2(lse[i] - mx[i]), [](float a, float c) { return a + c; });
+            total[i] = empty[i] ? -INFINITY : __builtin_log2f(total[i]) + mx[i];
+            ws[64 * i + lane] = empty[i] ? 0.f : fast_exp2(lse[i] - total[i]);      // lane s: the weight of split s (0 past the last one)
+            if (p->lse != nullptr && lane == 0 && first + WAVES * i < nrows) p->lse[base + first + WAVES * i] = total[i];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        v4f acc[U] = {zero, zero, zero, zero};             // (four sums, the order of splitkv_merge_rows at head_dim 64)
+        int pass = 0, g = 0;
+        auto add = [&](const v4f (&v)[U]) __attribute__((always_inline)) {
+            const v4f w = *(const v4f*)(ws + 64 * (pass * SUBS + sub) + g * U);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[u][i] = fmaf(w[u], v[u][i], acc[u][i]);
+            if (++g < groups) return;
+            const int r = first + WAVES * (pass * SUBS + sub);
+            if (r < nrows) store_out4<OUT_DT>(out0 + (int64_t)r * p->o_sn + col * 2, (acc[0] + acc[1]) + (acc[2] + acc[3]));
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc[u] = zero;
+            g = 0;
+            ++pass;
+        };
+        constexpr int PASSES = C / SUBS;
+        auto request_next = [&](v4f (&v)[U]) __attribute__((always_inline)) {
+            const bool wrap = g + 1 == groups;
+            if (!wrap || pass + 1 < PASSES) request(v, wrap ? pass + 1 : pass, wrap ? 0 : g + 1);
+        };
+        while (true) {
+            request_next(y);
+            add(x);
+            if (pass == PASSES) break;
+            request_next(x);
+            add(y);
+            if (pass == PASSES) break;
+        }
+    }
+}
+
+// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; WAVES waves, kMergeLds bytes of `smem`.
+// This runs once, at the end of a query block, and its time is a chain of latencies: a wave takes a row, its lanes the row's log-sum-exps
+// (lane s that of split s), which make the weights without a word of LDS, and the partials of the first splits are on their way
+// meanwhile, four columns per lane.  With fewer rows than waves the waves of a row share its splits and meet in LDS.
+template <int D, int OUT_DT, int WAVES = kMergeWaves>
 __device__ __forceinline__ void splitkv_merge_rows(KernargPtr p, char* smem, int b, int h, int row0, int nrows) {
     constexpr int LPR = D / 4, SUBS = 64 / LPR, U = 4;
     const SplitPartials part(p, D, 0);
     const int ns = p->num_splits, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int rs_log = 0;                                      // rows side by side: a power of two; G waves share one
-    while ((1 << rs_log) < nrows && (1 << rs_log) < kMergeWaves) ++rs_log;
-    const int rs = 1 << rs_log, G = kMergeWaves >> rs_log, g = wave >> rs_log;
+    while ((1 << rs_log) < nrows && (1 << rs_log) < WAVES) ++rs_log;
+    const int rs = 1 << rs_log, G = WAVES >> rs_log, g = wave >> rs_log;
     const int sub = lane / LPR, col = (lane % LPR) * 4, s_first = g * SUBS + sub, s_step = G * SUBS;
     const uint32_t base = (uint32_t)(b * p->heads + h) * (uint32_t)p->seqlen + (uint32_t)row0;
+    if (nrows > WAVES) {
+        splitkv_merge_many<D, OUT_DT, WAVES>(p, part, smem, base, p->out + b * p->o_sb + h * p->o_sh + (int64_t)row0 * p->o_sn, nrows, ns, wave, lane);
+        return;
+    }
     auto row_of = [&](int k) __attribute__((always_inline)) { return (wave & (rs - 1)) + k * rs; };
     auto lse_of = [&](int k) __attribute__((always_inline)) -> float {
         const int r = row_of(k);

@@ -247,7 +247,8 @@ __device__ __forceinline__ float q_scale_log2(const KParams& p, uint32_t bits) {
     return c == 0.f ? 0x1p-126f : c;
 }
 __device__ __forceinline__ float load_q_scale_log2(const KParams& p, int b, int h, int q_ld) {
-    return q_scale_log2(p, load_q_scale_bits(p, b, h, q_ld));
+    const float c = load_scale(p.q_scale, b * p.qs_sb + h * p.qs_sh + (int64_t)q_ld * p.qs_sn, p.scale_dtype) * p.qk_scale_log2;
+    return c == 0.f ? 0x1p-126f : c;
 }
 
 // k_scale of the keys of one (batch, K/V head): fetched as raw bits (one key per thread, ahead of the block that uses
@@ -362,7 +363,9 @@ __device__ __forceinline__ void issue_tile_part(v4i rsrc, uint32_t tile_off, uin
                                                 int wave, const TileLoadLane<ROW_BYTES, SWZ, ROWS>& ln, int it) {
     using T = TileLoadLane<ROW_BYTES, SWZ, ROWS>;
     const int i = it * 4 + wave;                     // wave-uniform instruction index
-    issue_copy_1k<NT>(rsrc, ln.off[it % T::NV], tile_off + (uint32_t)(i * T::RPI) * row_stride, lds_tile + (uint32_t)i * 1024u);
+    const uint32_t m0v = lds_tile + (uint32_t)i * 1024u;
+    const uint32_t soff = tile_off + (uint32_t)(i * T::RPI) * row_stride;
+    issue_copy_1k<NT>(rsrc, ln.off[it % T::NV], soff, m0v);
 }
 template <int ROW_BYTES, int SWZ, int ROWS, bool NT = false>
 __device__ __forceinline__ void issue_tile_load(v4i rsrc, uint32_t tile_off, uint32_t row_stride, uint32_t lds_tile,

@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_f16pv_pair_kernel(const K
     // ---- block -> (head, m-block, split): whole K/V heads per XCD
     const int n_mblk = (p.seqlen + kBlockM - 1) / kBlockM;
     const int n_split = SPLIT ? p.num_splits : 1;
-    const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
+    const WorkgroupJob wg = deal_workgroup(p, block_after_kernargs());
     const int rem = wg.rem, head = wg.b * p.heads + wg.h;
     const int mb_idx = fast_div(rem, p.d_n_split);
     const int split = rem - mb_idx * n_split;
@@ -71,12 +71,8 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_f16pv_pair_kernel(const K
     const bool q_valid = q_row < p.seqlen;
     const int q_ld = q_valid ? q_row : p.seqlen - 1;
 
-    // ---- Q fragments (B operand of S^T = K Q^T), resident: 16 bytes per k-step
-    v4i qreg[KS];
-    load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);          // (byte addressing: serves 8- and 16-bit rows alike)
     // exponent scale of this lane's row: q_scale * sm_scale * log2(e) (int8 Q K^T) or sm_scale * log2(e)
-    const float qsc = QK_INT8 ? load_q_scale_log2(p, b, h, q_ld) : p.qk_scale_log2;
-
+    float qsc = p.qk_scale_log2;
     float m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only
     v16f o_acc[DT];
 #pragma unroll
@@ -99,6 +95,15 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_f16pv_pair_kernel(const K
     auto issue_v = [&](int nb, int buf) __attribute__((always_inline)) {
         issue_tile_load<VROW, SWZ_V16, BN>(v_rsrc, (uint32_t)__builtin_amdgcn_readfirstlane((nb * BN) * (int)v_sn), v_sn, lds0 + OFF_V + buf * VT, rw, v_lane);
     };
+    // ---- Q fragments (B operand of S^T = K Q^T), resident: 16 bytes per k-step
+    v4i qreg[KS];
+    load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);          // (byte addressing: serves 8- and 16-bit rows alike)
+    const uint32_t q_scale_bits = QK_INT8 ? load_q_scale_bits(p, b, h, q_ld) : 0u;
+    // (The tiles behind Q: one workgroup per compute unit, and nothing can start without both; the other way round 1 - 3 % slower.)
+    asm volatile("" ::: "memory");
+    if (nb_begin < nb_end) {
+        if (hf == 0) issue_k(nb_begin, 0); else issue_v(nb_begin, 0);
+    }
     // k_scale of a block: thread t < 64 fetches the scale of key t; converted to fp32 when stored to LDS
     const KScaleSource ks_src(p, b, hk, seqlen_k);
     const int ks_key = tid & (BN - 1);
@@ -277,10 +282,10 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_f16pv_pair_kernel(const K
 
     if (nb_begin < nb_end) {
         // prologue: K tile, V tile and k_scale of the first block; its Q K^T chain
-        if (hf == 0) issue_k(nb_begin, 0); else issue_v(nb_begin, 0);
         if (QK_INT8) {
             const uint32_t s0 = load_ks(nb_begin);
             if (wave == 0) *(float*)(smem + ks_wr) = ks_src.cvt(s0);
+            qsc = q_scale_log2(p, q_scale_bits);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();

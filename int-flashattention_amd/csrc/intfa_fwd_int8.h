@@ -187,17 +187,18 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     const uint32_t ks_rd = OFF_KS + 16 * lh;     // + 4 * (32*st + 8*a4) per read
     const uint32_t ks_wr = OFF_KS + 4 * (tid & (BN - 1));
 
-    // One key block out of LDS buffer BUF.  DIAG selects the code for the block on the causal diagonal.
-    // DIAG selects the code instance with masking: keys whose index inside the block exceeds the lane's `lim` are masked
-    // and sub-tiles st > gw (wave-uniform, the sub-tile of the largest lim in the wave) are skipped.  Causal diagonal:
-    // lim = the lane's last visible key; last block of a ragged sequence: lim = the last valid key.
-    auto compute = [&](auto buf_tag, auto diag_tag, int nb, bool more, int gw_in, int lim, int lim_lo) __attribute__((always_inline)) {
-        constexpr int BUF = decltype(buf_tag)::value ? 1 : 0;
+    // One key block out of LDS buffer `buf`.  DIAG selects the code with masking, of which there is one instance per number NACT of
+    // sub-tiles that any row of the wave sees: keys whose index inside the block exceeds the lane's `lim` are masked in the last two of
+    // those (a wave's rows are 32, so the smallest lim lies at most one sub-tile below the largest).  Causal diagonal: lim = the lane's last
+    // visible key; last block of a ragged sequence: lim = the last valid key.  Straight code per instance, and one of it for both
+    // buffers: with run-time tests around sub-tiles and keys a masked block took 1.6 plain ones and more (us, before -> now: d128 B16
+    // H16 N300 25.6 -> 22.2, causal N512 28.8 -> 27.5, B8 H32/8 N1024 74.1 -> 72.2, d64 causal B16 H16 N512 20.0 -> 18.9).
+    auto compute = [&](auto diag_tag, auto nact_tag, int buf, int nb, bool more, int lim) __attribute__((always_inline)) {
         constexpr bool DIAG = decltype(diag_tag)::value;
-        constexpr int KB = BUF * KT, VB = BUF * VT, SB = BUF * BN * 4;
-        const int gw = gw_in;                              // wave-uniform; nact = active sub-tiles
-        const int nact = DIAG ? (gw + 1 < NST ? gw + 1 : NST) : NST;
-        if (DIAG && nact <= 0) return;                     // every key of this block is above the wave's rows
+        constexpr int nact = decltype(nact_tag)::value;
+        const uint32_t KB = buf * KT, VB = buf * VT, SB = buf * BN * 4;
+        int last = lim - 4 * lh;                           // (opaque: 64 thresholds of a ragged end would be computed ahead of the loop)
+        if (DIAG) asm volatile("" : "+v"(last));
         v4i k_next = k_rsrc, v_next = v_rsrc;
         if (!more) { k_next[2] = 0; v_next[2] = 0; }
         // LDS operand fetches are issued one stage ahead of their MFMAs, in program order pinned by scheduling
@@ -210,7 +211,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         auto load_vfrags = [&](v4i (&vf)[NST], int dt) __attribute__((always_inline)) {
 #pragma unroll
             for (int st = 0; st < NST; ++st) {
-                if (DIAG && st > gw && VBLK != 2) continue;     // (VBLK == 2 multiplies every sub-tile: P8 of a hidden one is 0)
+                if (st >= nact) continue;
                 const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
                     (__attribute__((address_space(3))) v2i*)INTFA_LDS(smem + v_rd[dt] + VB + (32 * st) * DV));
                 const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
@@ -249,15 +250,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         // stalls the wave at issue and the matrix core runs entirely under this wave's own vector instructions.
 #pragma unroll
         for (int st = 0; st < NST; ++st) {
-            if (DIAG && st > gw) {                            // sub-tile entirely above the diagonal
-#pragma unroll
-                for (int r = 0; r < 16; ++r) t[st][r] = -INFINITY;
-                continue;
-            }
-            const bool next = st + 1 < NST && st + 1 < nact;
+            if (st >= nact) continue;
+            const bool next = st + 1 < nact;
             __builtin_amdgcn_sched_barrier(0);
-            if (st + 2 < NST && st + 2 < nact) load_kfrags(fr[st & 1], st + 2);
-            if (!DUMP_S && !DIAG) issue_k_slice(k_next, nb + 1, BUF ^ 1, st, NST);
+            if (st + 2 < nact) load_kfrags(fr[st & 1], st + 2);
+            if (!DUMP_S && !DIAG) issue_k_slice(k_next, nb + 1, buf ^ 1, st, NST);
             const v16i& acc = sacc[st & 1];
             v16i& nacc = sacc[(st + 1) & 1];
             if (DUMP_S) {
@@ -284,10 +281,9 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) xq[b4] = (float)acc[4 * a4 + b4] * kk[a4][b4];
                 if (next) load_kk(a4, st + 1);
-                if (DIAG && 32 * st + 31 > lim_lo) {           // wave-uniform: some lane of the wave has a hidden key in this sub-tile
+                if (DIAG && (st + 2 >= nact || VBLK == 2)) {
 #pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4)
-                        if ((32 * st + 8 * a4 + b4 + 4 * lh) > lim) xq[b4] = -INFINITY;
+                    for (int b4 = 0; b4 < 4; ++b4) xq[b4] = hide_past(xq[b4], last, 32 * st + 8 * a4 + b4);
                 }
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) {
@@ -320,10 +316,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             __builtin_amdgcn_sched_barrier(0);
             // V of the next block is requested here, well before the end of this block, so that the copy has landed
             // when the next block waits for it (its buffer was last read before this block's barrier)
-            if (!DIAG) issue_v_slice(v_next, nb + 1, BUF ^ 1, st, NST);
+            if (!DIAG) issue_v_slice(v_next, nb + 1, buf ^ 1, st, NST);
             __builtin_amdgcn_sched_barrier(0);
             float ls = 0.f;
-            if (PROUND == 0) {
+            if (st >= nact) {
+            } else if (PROUND == 0) {
 #pragma unroll
                 for (int w4 = 0; w4 < 4; ++w4) {
                     unsigned pk = 0;
@@ -353,14 +350,14 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             if (VBLK == 2) {                     // keys 0..63 of the block only: the second half is a chain (and a scale row) of its own
                 if (st == 0) oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[0][0], p8[0], (v16i){0}, 0, 0, 0);
                 if (st == 1) oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[0][1], p8[1], oacc[0], 0, 0, 0);
-            } else if (!(DIAG && st > gw)) {
+            } else if (st < nact) {
                 if (st == 0) oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[0][0], p8[0], (v16i){0}, 0, 0, 0);
                 else oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[0][st], p8[st], oacc[0], 0, 0, 0);
             }
         }
         // -------- P V on int8 MFMA: O^T[d, q] += V^T[d, key] P^T[key, q]; the chain of d-tile dt+1 is issued
         // before the accumulator update of d-tile dt, its V fragments were requested two stages earlier.
-        constexpr int VSB = BUF * VSUB * DV * 4;
+        const uint32_t VSB = buf * VSUB * DV * 4;
         v4f vsc[2][4];                          // VBLK: channel scales of the d-tile being folded in / the next one
         if constexpr (VBLK == 2) {
             // Stage s = 2 dt + half: the int32 sum of d-tile dt over the keys 64 half .. 64 half + 63 of the block, times that
@@ -422,7 +419,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
                 if (dt + 1 < DT) {
 #pragma unroll
                     for (int st = a4 * NST / 4; st < (a4 + 1) * NST / 4; ++st) {
-                        if (DIAG && st > gw) continue;
+                        if (st >= nact) continue;
                         if (st == 0) nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[(dt + 1) & 1][0], p8[0], (v16i){0}, 0, 0, 0);
                         else nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[(dt + 1) & 1][st], p8[st], nacc, 0, 0, 0);
                     }
@@ -447,8 +444,8 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 
     // One pipeline step on LDS buffer BUF: wait for this block's tiles (issued one step earlier), make them
     // visible to all four waves, start the copy of the next block into the other buffer, compute.
-    auto step = [&](auto buf_tag, auto diag_tag, int nb, int gw, int lim, int lim_lo) __attribute__((always_inline)) {
-        constexpr int BUF = decltype(buf_tag)::value ? 1 : 0;
+    // (gw: sub-tile of the largest lim of the wave's rows, negative: none)
+    auto step = [&](auto diag_tag, int buf, int nb, int gw, int lim) __attribute__((always_inline)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         const bool more = nb + 1 < nb_end;
@@ -456,18 +453,27 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         float vs_next[VSUB] = {};
         constexpr bool DIAG = decltype(diag_tag)::value;
         if (more) {
-            if (DUMP_S || DIAG) issue_loads(nb + 1, BUF ^ 1);      // (a diagonal block is the last one: more == false)
+            if (DUMP_S || DIAG) issue_loads(nb + 1, buf ^ 1);      // (a diagonal block is the last one: more == false)
             ks_next = load_ks(nb + 1);
             if (vs_thread) {
 #pragma unroll
                 for (int sub = 0; sub < VSUB; ++sub) vs_next[sub] = load_vs(nb + 1, sub);
             }
         }
-        compute(buf_tag, diag_tag, nb, more, gw, lim, lim_lo);
-        if (more && ks_wave) *(float*)(smem + ks_wr + (BUF ^ 1) * BN * 4) = cvt_ks(ks_next);
+        if constexpr (!DIAG) {
+            compute(diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+        } else if constexpr (VBLK == 2) {        // (multiplies every sub-tile, so it masks every one: P8 of a hidden one is 0)
+            if (gw >= 0) compute(diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+        } else {
+            if (gw >= NST - 1) compute(diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+            else if (gw == 0) compute(diag_tag, IntTag<1>{}, buf, nb, more, lim);
+            else if (NST == 4 && gw == 1) compute(diag_tag, IntTag<2>{}, buf, nb, more, lim);
+            else if (NST == 4 && gw == 2) compute(diag_tag, IntTag<3>{}, buf, nb, more, lim);
+        }
+        if (more && ks_wave) *(float*)(smem + ks_wr + (buf ^ 1) * BN * 4) = cvt_ks(ks_next);
         if (more && vs_thread) {
 #pragma unroll
-            for (int sub = 0; sub < VSUB; ++sub) *(float*)(smem + vs_wr + ((BUF ^ 1) * VSUB + sub) * DV * 4) = vs_next[sub];
+            for (int sub = 0; sub < VSUB; ++sub) *(float*)(smem + vs_wr + ((buf ^ 1) * VSUB + sub) * DV * 4) = vs_next[sub];
         }
     };
 
@@ -500,9 +506,9 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         int nb = nb_begin;
         while (true) {
             if (nb >= plain_end) break;
-            step(BoolTag<false>{}, BoolTag<false>{}, nb++, 0, 0, 0);
+            step(BoolTag<false>{}, 0, nb++, 0, 0);
             if (nb >= plain_end) break;
-            step(BoolTag<true>{}, BoolTag<false>{}, nb++, 0, 0, 0);
+            step(BoolTag<false>{}, 1, nb++, 0, 0);
         }
         // masked blocks: the blocks the causal diagonal of this query block crosses (kBlockM / BN of them when the lengths
         // are equal, one more when the offset is not a multiple of the block; keys past the end of a ragged sequence lie above
@@ -512,10 +518,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             // lane: last visible key relative to the block; wave: sub-tile of the largest of them (negative: none)
             const int lim = CAUSAL ? q_row + causal_off - nb * BN : tail_keys - 1;
             const int gw = (CAUSAL ? mb * kBlockM + wave * 32 + 31 + causal_off - nb * BN : tail_keys - 1) >> 5;
-            // smallest lim in the wave: sub-tiles that end at or below it need no per-key test
-            const int lim_lo = CAUSAL ? mb * kBlockM + wave * 32 + causal_off - nb * BN : tail_keys - 1;
-            if (((nb - nb_begin) & 1) == 0) step(BoolTag<false>{}, BoolTag<true>{}, nb, gw, lim, lim_lo);
-            else step(BoolTag<true>{}, BoolTag<true>{}, nb, gw, lim, lim_lo);
+            step(BoolTag<true>{}, (nb - nb_begin) & 1, nb, gw, lim);
         }
     }
     if (DUMP_S) return;

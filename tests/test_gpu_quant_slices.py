@@ -55,3 +55,44 @@ def test_streaming_launch_sizes_bit_exact(steps, dtype):
         q8, s = fn(x)
         ref8, ref_s = ref(x.cpu())
         assert torch.equal(s.cpu(), ref_s) and torch.equal(q8.cpu(), ref8)
+
+
+# 2048 pieces of 32 KiB and more, of slices that fit 256 of them: pieces wait for the maxima of their slice; one piece fewer, and a slice of
+# more than 256 pieces: two passes.  Last pieces of one row, strided rows; old data in the workspace; nobody waits (the debug entry).
+@pytest.mark.parametrize("H,N,d,strided", [(64, 4096, 128, False), (64, 3969, 128, True), (63, 4096, 128, False), (8, 65536, 64, False),
+                                           (8, 65537, 64, False), (683, 257, 256, False), (1024, 2049, 16, True)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_pieces_that_wait_for_their_slice(H, N, d, strided, dtype):
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn((1, H, N, d * (2 if strided else 1)), generator=g, device=DEV).to(dtype)[..., :d]
+    x[:, :, N // 3, d // 2] = 5 + torch.arange(H, device=DEV).to(dtype) / 8      # another maximum in every slice
+    x[0, -1, -1, -1] = 300
+    amax = x.abs().amax((2, 3))
+    want_s = (amax.float() / 127).to(dtype)
+    want = (x.float() / want_s.float()[..., None, None]).to(dtype).float().round().to(torch.int32).to(torch.int8)      # (128 wraps, as in the reference)
+    q8, s = M.quant_pertensor(x)
+    assert torch.equal(s, want_s) and torch.equal(q8, want)
+    lib = _capi.load()
+    need = lib.intfa_quant_pertensor_parts_workspace_bytes(1, H, N, d)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+    for fn in (lib.intfa_quant_pertensor, lib.intfa_debug_quant_pertensor_alone):
+        q8.zero_(); s.zero_()
+        assert fn(x.data_ptr(), *x.stride()[:3], q8.data_ptr(), s.data_ptr(), 1, H, N, d, _capi.INTFA_F16 if dtype == torch.float16 else _capi.INTFA_BF16,
+                  ws.data_ptr(), need, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(s, want_s) and torch.equal(q8, want)
+
+
+def test_pieces_that_wait_under_a_graph():
+    x = torch.randn((1, 64, 4096, 128), device=DEV).half()
+    M.quant_pertensor(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q8, s = M.quant_pertensor(x)
+    for scale in (1.0, 0.25, 3.0):                       # (smaller maxima than those of the replay before, too)
+        x.copy_(torch.randn_like(x) * scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        ref8, ref_s = M.quant_pertensor(x)
+        assert torch.equal(s, ref_s) and torch.equal(q8, ref8)

@@ -165,8 +165,7 @@ def cpu_baseline(budget_s: float, w: dict):
 
 
 def bench_quant(args, variant, x, B, H, N, D, dt):
-    """Times one quantiser; algorithmic bytes = 2 per element read + 1 written (+ scales); the per-(batch, head) variant
-    reads its input twice (maximum, then quantise)."""
+    """Times one quantiser; algorithmic bytes = 2 per element read + 1 written (+ scales)."""
     import torch
     import int_flashattention_amd as M
     if variant == "quant_append":          # K and V of the prompt into an empty cache: reads both inputs once, writes both caches
@@ -182,7 +181,7 @@ def bench_quant(args, variant, x, B, H, N, D, dt):
     # (the per-block variant reads its block twice too, but the second sweep of 32 KiB is served by the cache)
     scale_bytes = {"quant_token": 2 * B * H * N, "quant_tensor": 2 * B * H, "quant_block": 4 * B * H * (N // 128) * D,
                    "quant_append": 2 * B * H * N + 2 * B * H}[variant]
-    alg_bytes = (2 + 1) * n * (2 if variant == "quant_append" else 1) + scale_bytes + (2 * n if variant == "quant_tensor" else 0)
+    alg_bytes = (2 + 1) * n * (2 if variant == "quant_append" else 1) + scale_bytes
     spin = device_spinup(torch, lambda: fn(x), args.spinup_ms)
     for _ in range(args.warmup):
         fn(x)
@@ -203,7 +202,7 @@ def bench_quant(args, variant, x, B, H, N, D, dt):
            "roofline": {"bound": "hbm", "achieved": alg_bytes / (kern_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": alg_bytes / (kern_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
                         "kernel": {"quant_token": "quant_pertoken_kernel", "quant_block": "quant_blockchan_kernel",
-                                   "quant_tensor": "quant_slice_amax_kernel + quant_slice_apply_kernel",
+                                   "quant_tensor": "quant_clear_kernel + quant_slice_wait_kernel",
                                    "quant_append": "kv_append_kernel (keys and values)"}[variant],
                         "avg_launch_ms": kern_ms, "median_launch_ms": statistics.median(per_launch_ms)},
            "peak_check": device_peak_check(torch, x.device), "device_spinup": spin}

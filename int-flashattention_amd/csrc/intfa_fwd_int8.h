@@ -110,13 +110,19 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         issue_tile_load<D, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BN) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
         if (!DUMP_S) issue_tile_load<DV, SWZ_V8, BN>(v_rsrc, (uint32_t)(nb * BN) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
     };
-    // The first tiles ahead of Q and the scales, which arrive under their way from HBM (and the argument lines at once, above:
-    // d128 B4 H16 N2048 causal 66.4 -> 64.9 us, d64 B16 H16 N512 causal 20.6 -> 20.1).
-    if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    // The argument lines at once (above), and the scales converted behind the requests.  Causal: the first tiles ahead of Q, which arrives under
+    // their way from HBM (d128 B4 H16 N2048 66.4 -> 64.9 us, d64 B16 H16 N512 20.6 -> 20.1).  Without a mask grids are longer, most first
+    // tiles come from the L2, and Q, which nobody else reads, is what a workgroup waits for: Q first (the other way round B4 H32
+    // N4096 d128 0.5 % slower, N256 ... N1777 +- 1 %).
+    if (CAUSAL && nb_begin < nb_end) issue_loads(nb_begin, 0);
     // ---- Q fragment (B operand of S^T = K Q^T): 16 bytes per k-step, resident for the whole kernel.
     v4i qreg[KS];
     load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);
     const uint32_t q_scale_bits = DUMP_S ? 0u : load_q_scale_bits(p, b, h, q_ld);
+    if (!CAUSAL) {
+        asm volatile("" ::: "memory");
+        if (nb_begin < nb_end) issue_loads(nb_begin, 0);
+    }
     // The copy of the NEXT block is issued in slices spread over the stages of the current block (one K slice per
     // S^T sub-tile stage, one V slice per output d-tile stage) so that the waves do not queue behind a burst.
     constexpr int DMA_PARTS = TileLoadLane<D, SWZ_K, BN>::NINST / 4;

@@ -212,7 +212,7 @@ int dispatch(int variant, const intfa_fwd_params* p, KParams kp, bool dump_s, hi
     sel.wide = decode_shaped(kp.seqlen);
     const int64_t wgs = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kDecodeRows - 1) / kDecodeRows) * kp.num_splits;
     // The decode-shaped kernels' forms.  Rows past the 16th go to a workgroup of their own while both find a compute unit to themselves
-    // (half-int8 d64, 20 rows, 256 keys 6.0 -> 5.3 us; K and V then come from the L2 twice).  Crowded (full-int8 up to head_dim 128): more
+    // (half-int8 d64, 20 rows, 256 keys 6.0 -> 5.3 us; K and V then come from the L2 twice).  Crowded (full-int8): more
     // workgroups than compute units (head_dim 64, up to 16 rows: than two per unit) get the form of WideGeom with room for more of
     // them; head_dim 64 with more rows the four-wave kernel, whose 32-row MFMA tiles need half the LDS reads per product (us, eight
     // waves -> four: B16 H32/8 Nq5 Nk3000, 512 workgroups 19.3 -> 16.1, B9 H8 Nq32 Nk9000 27.0 -> 22.8, 256 workgroups 19.6 both).

@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 
 // Few query rows per head, split or not: intfa_fwd_decode_wide.h.
 template <int D, class /* WideRows */ R, int OUT_DT, int PROUND, bool VBLK>
-__global__ void __launch_bounds__(kWideThreads, (D == 128 && !R::crowded) || (D == 256 && VBLK && R::tiles == 2) ? 2 : D == 64 && R::crowded ? 6 : 4) fwd_decode_full_int8_kernel(const KParams p) {
+__global__ void __launch_bounds__(kWideThreads, (D >= 128 && !R::crowded) || (D == 256 && VBLK && R::tiles == 2) ? 2 : D == 64 && R::crowded ? 6 : 4) fwd_decode_full_int8_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     decode_wide<D, true, true, OUT_DT, PROUND, VBLK, R>(p);
 #endif

@@ -18,7 +18,7 @@
 //     block (16-bit V: the second half) of the step's keys, and the two sums meet in the epilogue;
 //   * the first tiles are requested as soon as their addresses are known, ahead of Q, the scales and the tickets.
 // The frames are those of the general full-int8 kernel: a step holds two blocks of 128 keys (head_dim 128), four of 64 (head_dim 64) or two
-// of 64 (head_dim 256), and m_0 = max(m, max_0), m_1 = max(m_0, max_1), ... with the factors alpha_i = 2^(m_(i-1) - m_i).  The 16-bit P V
+// of 64 (head_dim 256; one in the crowded form), and m_0 = max(m, max_0), m_1 = max(m_0, max_1), ... with the factors alpha_i = 2^(m_(i-1) - m_i).  The 16-bit P V
 // variants, whose result does not depend on the frame but for the rounding of P, take one frame per step.
 #pragma once
 #include "intfa_device.h"
@@ -29,7 +29,7 @@
 namespace intfa {
 
 constexpr int kWideWaves = 8, kWideThreads = 64 * kWideWaves;
-// RT: row tiles of 16 query rows.  CROWDED (full-int8 up to head_dim 128): the form with room for more workgroups per compute unit
+// RT: row tiles of 16 query rows.  CROWDED (full-int8): the form with room for more workgroups per compute unit
 template <int RT, bool CROWDED> struct WideRows { static constexpr int tiles = RT; static constexpr bool crowded = CROWDED; };
 static_assert(kWideWaves == kMergeWaves, "");
 
@@ -38,15 +38,18 @@ template <int D, bool KI8, bool VI8, typename R> struct WideGeom {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
     static constexpr int KROW = D * (KI8 ? 1 : 2), VROW = D * (VI8 ? 1 : 2);      // bytes per row
     // Two steps of tiles in the LDS, and two workgroups per compute unit: with one, its prologue and its merge (4 - 6 us) overlap with nothing.
-    // Head_dim 256 with 16-bit V has one (fewer than four 16-key tiles are too few).  Full-int8 up to head_dim 128 has a second form with
-    // room for more workgroups: head_dim 128 steps of 128 keys instead of 256 (step of one request, us: 1.0 and 1.3, so the longer one while
+    // Head_dim 256 with 16-bit V has one (fewer than four 16-key tiles are too few).  Full-int8 has a second form with room for more workgroups: head_dim 128 steps of 128 keys instead of 256 (step of one request, us: 1.0 and 1.3, so the longer one while
     // there is room), head_dim 64 one step's tiles instead of two, the next ones requested once all waves hold theirs in registers
-    // (three workgroups per unit instead of two, us: 640 workgroups 54 -> 39.7, 960 of 1500 keys 42.1 (128-key steps) -> 37.7).
+    // (three workgroups per unit instead of two, us: 640 workgroups 54 -> 39.7, 960 of 1500 keys 42.1 (128-key steps) -> 37.7), head_dim 256 steps of 64 keys,
+    // whose S^T keeps half the waves busy, instead of 128 with one workgroup per unit (256 workgroups of 1500 keys 48.7 -> 41.3, 5 requests
+    // of 700 11.6 -> 9.9).
     static constexpr int BUFS = VI8 && D == 64 && R::crowded ? 1 : 2;
-    static constexpr int KEYS = VI8 && D < 256 && (!R::crowded || BUFS == 1) ? 256 : D == 256 || (D == 128 && !VI8) ? 64 : 128;
+    static constexpr int KEYS = VI8 && D < 256 && (!R::crowded || BUFS == 1) ? 256 : (D == 256 && !(VI8 && !R::crowded)) || (D == 128 && !VI8) ? 64 : 128;
     static constexpr int BNB = VI8 ? (D == 128 ? 128 : 64) : KEYS;                // keys per frame
     static constexpr int BLK = VI8 ? BNB : kBlockN16;                             // key block of the split ranges: intfa_fwd_block_n()
     static constexpr int NB = KEYS / BNB;
+    // Full-int8 head_dim 256, one block per step: the row sums of even and odd blocks apart, as the form with two blocks per step has them
+    static constexpr bool EVEN_ODD = VI8 && D == 256 && NB == 1;
     static constexpr int NKT = KEYS / 16;                                         // 16-key tiles per step
     static constexpr int NT = NKT >= kWideWaves ? NKT / kWideWaves : 1;           // ... per wave
     static constexpr int QKW = NKT / NT;                                          // waves with tiles of S^T
@@ -217,11 +220,11 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
     }
     const uint64_t ticket_seen = splitkv_look_at_tickets(p, group);
 
-    float qsc[RT], m_run[RT], l_run[RT];                 // l_run: this lane's keys only
+    float qsc[RT], m_run[RT], l_run[RT], l_odd[RT];      // l_run: this lane's keys only (EVEN_ODD: of even blocks, l_odd: of odd ones)
     v4f o_acc[CTW][RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        qsc[rt] = p.qk_scale_log2; m_run[rt] = -INFINITY; l_run[rt] = 0.f;
+        qsc[rt] = p.qk_scale_log2; m_run[rt] = -INFINITY; l_run[rt] = l_odd[rt] = 0.f;
 #pragma unroll
         for (int j = 0; j < CTW; ++j) o_acc[j][rt] = (v4f){0.f, 0.f, 0.f, 0.f};
     }
@@ -394,7 +397,8 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                     float own = 0.f;                       // block after block, so that the sequence does not depend on the step's length
 #pragma unroll
                     for (int t = 0; t < NT; ++t) own = NB == 1 || i == G::frame_of(wave, t) ? sum[t] : own;
-                    l_run[rt] = fmaf(l_run[rt], alpha[i][rt], own);
+                    l_run[rt] = fmaf(l_run[rt], alpha[i][rt], G::EVEN_ODD && BUF ? 0.f : own);
+                    if (G::EVEN_ODD) l_odd[rt] = fmaf(l_odd[rt], alpha[i][rt], BUF ? own : 0.f);
                 }
                 const uint32_t at = xp_wr + 1024 * rt;
                 if constexpr (VI8) {
@@ -522,7 +526,11 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         l_tot[rt] = reduce_row_lanes(l_run[rt], [](float a, float c) { return a + c; });
-        if (lh == 0) *(float*)(smem + OFF_XM + 4 * kWideWaves * (16 * rt + ln) + 4 * wave) = l_tot[rt];
+        if (lh == 0 && (!G::EVEN_ODD || wave < G::QKW)) *(float*)(smem + OFF_XM + 4 * kWideWaves * (16 * rt + ln) + 4 * wave) = l_tot[rt];
+        if (G::EVEN_ODD && wave < G::QKW) {
+            const float odd = reduce_row_lanes(l_odd[rt], [](float a, float c) { return a + c; });
+            if (lh == 0) *(float*)(smem + OFF_XM + 4 * kWideWaves * (16 * rt + ln) + 4 * (wave + G::QKW)) = odd;
+        }
         if (KH > 1 && kh > 0) *(v4f*)(smem + OFF_K + 1024 * (RT * (wave % CT) + rt) + 16 * lane) = o_acc[0][rt];
     }
     asm volatile("" :: "s"(e_splits), "s"(e_seqlen), "s"(e_heads), "s"(e_batch), "s"(e_scale_dtype), "s"(e_lse), "s"(e_out), "s"(e_sb), "s"(e_sh), "s"(e_sn));

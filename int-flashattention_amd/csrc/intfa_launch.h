@@ -22,7 +22,7 @@ struct LaunchSel {
     bool dump_s;     // full-int8 only: export int32 S and stop
     bool wide;       // decode-shaped kernels: few query rows per head (intfa_fwd_decode_wide.h)
     int row_tiles;   // ... tiles of 16 query rows per workgroup
-    bool crowded;    // ... full-int8 up to head_dim 128: more workgroups than the form with the longer pipeline has room for
+    bool crowded;    // ... full-int8: more workgroups than the form with the longer pipeline has room for
 };
 
 inline FastDiv make_fast_div(int d) {

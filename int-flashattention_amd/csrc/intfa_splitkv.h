@@ -91,7 +91,9 @@ __device__ __forceinline__ void splitkv_open_tickets(KernargPtr p, int group, ui
 }
 
 // Takes this workgroup's ticket of query block `group`; true for the last of the block's num_splits workgroups.
-// Called by every thread of the workgroup after its stores; `smem` is free (16 bytes of it are used).
+// Called by every thread of the workgroup after its stores; `smem` is free.  Its first kArrivalBytes carry the answer, and no barrier follows
+// the reading of it: a wave may read it while another is in the merge already, which therefore leaves these bytes alone.
+constexpr int kArrivalBytes = 16;
 template <typename P> __device__ __forceinline__ bool splitkv_last_arrival(P p, char* smem, int group) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's partials have reached the point of coherence
     __syncthreads();
@@ -220,7 +222,7 @@ template <typename F> __device__ __forceinline__ float reduce_wave(float x, F op
 
 constexpr int kMaxSplits = 64;                           // the lanes of a wave
 constexpr int kMergeWaves = 8;
-constexpr int kMergeLds = kMergeWaves * 64 * 16;
+constexpr int kMergeLds = kArrivalBytes + kMergeWaves * 64 * 16;      // of the workgroup's LDS, from its first byte
 
 // More rows than waves: a wave takes four rows at a time, so that the chains of their weights run side by side, and D / 4 lanes a row of the
 // sums; partials of the next four splits are on their way while four are added.  Row after row, as below, the chains were 0.25 us
@@ -229,8 +231,8 @@ template <int D, int OUT_DT, int WAVES, typename P>
 __device__ __forceinline__ void splitkv_merge_many(P p, const SplitPartials& part, char* smem, uint32_t base, char* out0, int nrows, int ns, int wave, int lane) {
     constexpr int LPR = D / 4, SUBS = 64 / LPR, U = 4, C = 4;      // C rows side by side
     const int sub = lane / LPR, col = (lane % LPR) * 4, groups = (ns + U - 1) / U;
-    float* const ws = (float*)smem + wave * (C * 64);      // weights of the wave's rows, of no other wave's concern
-    static_assert(WAVES * C * 64 * 4 <= kMergeLds, "");
+    float* const ws = (float*)(smem + kArrivalBytes) + wave * (C * 64);      // weights of the wave's rows, of no other wave's concern
+    static_assert(kArrivalBytes + WAVES * C * 64 * 4 <= kMergeLds, "");
     for (int first = wave; first < nrows; first += C * WAVES) {      // rows first, first + WAVES, ...
         auto row_of = [&](int i) __attribute__((always_inline)) { const int r = first + WAVES * i; return r < nrows ? r : first; };
         float lse[C], mx[C], total[C];
@@ -295,7 +297,8 @@ __device__ __forceinline__ void splitkv_merge_many(P p, const SplitPartials& par
     }
 }
 
-// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; WAVES waves, kMergeLds bytes of `smem`.
+// Merges the `nrows` (at most 32) rows from row0 of (b, h) out of the partials; WAVES waves, kMergeLds bytes of `smem` (those behind the
+// first kArrivalBytes).
 // This runs once, at the end of a query block, and its time is a chain of latencies: a wave takes a row, its lanes the row's log-sum-exps
 // (lane s that of split s), which make the weights without a word of LDS, and the partials of the first splits are on their way
 // meanwhile, four columns per lane.  With fewer rows than waves the waves of a row share its splits and meet in LDS.
@@ -368,7 +371,8 @@ __device__ __forceinline__ void splitkv_merge_rows(KernargPtr p, char* smem, int
             if (SUBS == 2) acc[i] = half_pair_sum(acc[i]);
         }
         if (G > 1) {                                     // (one row per wave then: every wave comes here once)
-            v4f* red = (v4f*)smem;
+            v4f* red = (v4f*)(smem + kArrivalBytes);
+            static_assert(kArrivalBytes + WAVES * 64 * 16 <= kMergeLds, "");
             if (g > 0) red[wave * 64 + lane] = acc;
             __syncthreads();
             if (g > 0) return;

@@ -180,8 +180,8 @@ int launch_combine(const intfa_fwd_params* p, const KParams& kp, hipStream_t str
 //     causal B1 H16 N1024 22.7 -> 17.4, B3 H32 N256 (768 workgroups) 10.8 -> 12.8; full-int8 d256 B1 H8 N1024 31.5 -> 20.3,
 //     B1 H16 N1024 32.8 -> 37.6; B1 H8 N256 d64 7.6 -> 5.5.
 // Not half-int8 and fp16 at head_dim 128: there two of the four waves have no share of Q K^T, the gain ends at 10 %, and the
-// kernels differ in the rounding of P.  Everywhere else both kernels give the same bits, so that an output does not depend on how
-// many heads and batch entries it is computed with.
+// kernels differ in the rounding of P.  Everywhere else both kernels give the same bits - and so do the forms of the decode-shaped ones, which
+// dispatch() chooses by the size of the grid - so that an output does not depend on how many heads and batch entries it is computed with.
 bool decode_shaped(int seqlen) { return seqlen <= kDecodeMaxRows; }
 // (scale rows of 64 keys under the 128-key block: the decode kernel has one scale row per block)
 bool decode_kernel_takes(int variant, const KParams& kp) {
@@ -215,7 +215,7 @@ int dispatch(int variant, const intfa_fwd_params* p, KParams kp, bool dump_s, hi
     // (half-int8 d64, 20 rows, 256 keys 6.0 -> 5.3 us; K and V then come from the L2 twice).  Crowded (full-int8): more
     // workgroups than compute units (head_dim 64, up to 16 rows: than two per unit) get the form of WideGeom with room for more of
     // them; head_dim 64 with more rows the four-wave kernel, whose 32-row MFMA tiles need half the LDS reads per product (us, eight
-    // waves -> four: B16 H32/8 Nq5 Nk3000, 512 workgroups 19.3 -> 16.1, B9 H8 Nq32 Nk9000 27.0 -> 22.8, 256 workgroups 19.6 both).
+    // waves -> four: B16 H32/8 Nq5 Nk3000, 512 workgroups 19.3 -> 16.1, B9 H8 Nq32 Nk9000 27.0 -> 22.8, 256 workgroups 19.6 both; the same bits).
     sel.row_tiles = kp.seqlen <= 16 || (2 * wgs <= kComputeUnits && !streams_kv(kp)) ? 1 : 2;
     sel.crowded = wgs > (kp.head_dim == 64 && sel.row_tiles == 1 ? 2 : 1) * kComputeUnits;
     const int d = kp.head_dim;

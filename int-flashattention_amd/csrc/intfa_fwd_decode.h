@@ -1,6 +1,6 @@
 // Full-int8 forward whose waves share the keys: for small single-pass problems (decode_kernel_takes, intfa_capi.hip) the kernel of this file,
 // for few query rows per head the one of intfa_fwd_decode_wide.h behind the same name (but at head_dim 64 with more than 16 rows
-// and more workgroups than compute units: dispatch()).
+// and more workgroups than compute units: dispatch()), whose results are then the same bits.
 //
 // Same arithmetic as fwd_full_int8_kernel (flash_atten_full_int8.py:9-71 per 128-key block: int32 S, dequantise, running
 // max, P = exp2(X c - m), P requantised with the fixed scale 127, int32 P V, fp32 accumulator), other division of labour.
@@ -21,6 +21,11 @@
 // m_A = max(m, max_A), m_B = max(m_A, max_B) and both factors alpha_A = 2^(m - m_A), alpha_B = 2^(m_A - m_B); each wave
 // requantises its keys in its own block's frame, and an output tile is updated as
 // O = (O alpha_A + P8_A V_A) alpha_B + P8_B V_B with one int32 sum per block - the blocks' arithmetic of that kernel.
+// FEW (head_dim 64, few query rows): the sums are those of intfa_fwd_decode_wide.h, which takes the same rows in smaller grids.  Waves 0 and 1
+// multiply the A blocks with the two output tiles, waves 2 and 3 the B blocks, each into a sum of its own, and the row sums stay in the lanes, apart for each
+// quad of keys, until the epilogue: the order in which that kernel's waves and lanes hold them.  Against waves 2 and 3 repeating the products of 0 and 1,
+// and the row sums in the order of the general kernel, us: B16 H32/8 Nq6 Nk16000 causal 56.8 -> 53.2, B32 H16 Nq33 Nk1500 causal 34.9 -> 33.1,
+// B16 H32/8 Nq5 Nk3000 16.3 -> 16.0.
 #pragma once
 #include "intfa_device.h"
 #include "intfa_launch.h"
@@ -31,13 +36,15 @@ namespace intfa {
 // Head_dim 128: one 128-key block per step, the block of the general kernel.  Head dims 64 and 256: two 64-key blocks.
 template <int D, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool VBLK, bool FEW /* few query rows: splits, grouped heads as rows, non-temporal K and V */>
 __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_int8_kernel(const KParams p) {
-    static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
+    static_assert(D == 64 || (!FEW && (D == 128 || D == 256)), "head dims 64, 128, 256; few rows: 64");
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
     constexpr int KS = D / 32;                   // k-steps of Q K^T
     constexpr int DT = D / 32;                   // 32-wide output tiles along head_dim; wave w owns tiles w, w+4, ...
     constexpr int DTW = (DT + 3) / 4;            // output tiles per wave
     constexpr int NST = 4, BN = 32 * NST;        // one 32-key sub-tile per wave
+    constexpr int NSTW = FEW ? NST / 2 : NST;    // sub-tiles that a wave multiplies with V
     constexpr int NBS = D == 128 ? 1 : 2;        // key blocks (of the arithmetic) per step
+    constexpr int NBW = FEW ? 1 : NBS;           // ... that a wave multiplies with V
     constexpr int BNB = BN / NBS;                // key block of the arithmetic: intfa_fwd_block_n()
     constexpr int KT = BN * D, VT = BN * D;      // bytes of one K / V tile
     constexpr int CH = D / 16;                   // 16-byte chunks per row
@@ -83,6 +90,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 
     float qsc = 0.f, m_run = -INFINITY, l_run = 0.f;
     float l_odd = 0.f;                           // head_dim 256: row sums of the odd sub-tiles (a wave of its own in that general kernel)
+    float l_quad[4] = {0.f, 0.f, 0.f, 0.f};      // FEW: row sums of this lane's keys 8 a4 .. 8 a4 + 3 of every sub-tile of the wave
     float o_acc[DTW][16];
 #pragma unroll
     for (int j = 0; j < DTW; ++j)
@@ -141,6 +149,7 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     };
 
     // ---- per-lane LDS offsets
+    const bool blk_a = NBS == 1 || wave < 2;                          // this wave's keys belong to the first block of a step
     const int k_swz = swz_k<D>(lq) & (CH - 1);
     uint32_t k_rd[KS];                            // this wave's 32 keys: row 32*wave + lq, chunk 2*ks + lh
 #pragma unroll
@@ -156,23 +165,23 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
         const int dt = (wave + 4 * j) % DT;          // (head_dim 64: waves 2 and 3 shadow tiles 0 and 1, see below)
         const int c = 2 * dt + (g16 & 1);
         v_rd[j] = OFF_V + v_row0 * D + 8 * (i16 & 1) + (((c & SWM) ^ v_swz) << 4) + ((c & ~SWM) << 4);
+        if (FEW && !blk_a) v_rd[j] += BNB * D;
     }
     const uint32_t ks_rd = OFF_KS + 4 * (32 * wave) + 16 * lh;       // + 4 * 8*a4 per read
     const uint32_t ks_wr = OFF_KS + 4 * (tid & (BN - 1));
     const uint32_t xm_wr = OFF_XM + 4 * (32 * wave + lq);
     const uint32_t xm_rd = OFF_XM + 4 * lq;                          // + 128 per wave
     const uint32_t xp_wr = OFF_XP + 1024 * wave + 16 * lane;
-    const uint32_t xp_rd = OFF_XP + 16 * lane;                       // + 1024 per wave
+    const uint32_t xp_rd = OFF_XP + 16 * lane + (FEW && !blk_a ? 1024 * NSTW : 0);      // + 1024 per wave
     const uint32_t xs_rd = OFF_XS + 16 * lane, xs_wr = xs_rd + 4 * wave;
     const uint32_t vs_wr = OFF_VS + 4 * vs_i;                        // + 4 * kThreads per further value
-    const uint32_t vs_rd = OFF_VS + 16 * lh;                         // + 4 * (D*blk + 32*dt + 8*a4) per read
-    // head_dim 64 has two output tiles for four waves: waves 2 and 3 compute tiles 0 and 1 a second time and store
+    const uint32_t vs_rd = OFF_VS + 16 * lh + (FEW && !blk_a ? 4 * D : 0);      // + 4 * (D*blk + 32*dt + 8*a4) per read
+    // head_dim 64 has two output tiles for four waves: waves 2 and 3 compute tiles 0 and 1 a second time (not FEW) and store
     // nothing (the same instruction stream for every wave; a run-time "owns a tile" test around the V fragments and the
     // accumulator update costs the owners a hundred register copies per step)
     // the last visible key of the first row of this query block, and of the lane's row
     const int first_lim = p.causal ? (fold ? 0 : mb * kDecodeRows) + causal_off : 0x3fffffff;
     const int row_lim = p.causal ? (fold ? q_row % fold : q_row) + causal_off : 0x3fffffff;
-    const bool blk_a = NBS == 1 || wave < 2;                          // this wave's keys belong to the first block of a step
 
     auto step = [&](auto buf_tag, int nb) __attribute__((always_inline)) {
         constexpr int BUF = decltype(buf_tag)::value ? 1 : 0;
@@ -201,11 +210,11 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[ks], qreg[ks], sacc, 0, 0, 0);
         // V fragments of this wave's output tiles travel during the softmax
-        v4i vf[DTW][NST];
+        v4i vf[DTW][NSTW];
 #pragma unroll
         for (int j = 0; j < DTW; ++j)
 #pragma unroll
-            for (int st = 0; st < NST; ++st) {
+            for (int st = 0; st < NSTW; ++st) {
                 const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
                     (__attribute__((address_space(3))) v2i*)INTFA_LDS(smem + v_rd[j] + VB + (32 * st) * D));
                 const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
@@ -252,7 +261,14 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 e[r] = fast_exp2(fmaf(x[r], qsc, bias));                         // RNE mode: 127 * p
-                lsum += e[r];
+                if (!FEW) lsum += e[r];
+            }
+            if (FEW) {
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4) {
+                    const float own = ((e[4 * a4] + e[4 * a4 + 1]) + e[4 * a4 + 2]) + e[4 * a4 + 3];
+                    l_quad[a4] = fmaf(fmaf(l_quad[a4], alpha, blk_a ? own : 0.f), alpha_b, blk_a ? 0.f : own);
+                }
             }
             if (PROUND == 0) {
 #pragma unroll
@@ -267,11 +283,11 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
             }
         }
         *(v4i*)(smem + xp_wr) = p8;
-        *(float*)(smem + xs_wr) = lsum;
-        v4f vsc[NBS][DTW][4];                              // channel scales of the step's blocks for this wave's output tiles
+        if (!FEW) *(float*)(smem + xs_wr) = lsum;
+        v4f vsc[NBW][DTW][4];                              // channel scales of the step's blocks for this wave's output tiles
         if (VBLK) {
 #pragma unroll
-            for (int blk = 0; blk < NBS; ++blk)
+            for (int blk = 0; blk < NBW; ++blk)
 #pragma unroll
                 for (int j = 0; j < DTW; ++j)
 #pragma unroll
@@ -279,14 +295,29 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
                         vsc[blk][j][a4] = *(const v4f*)(smem + vs_rd + VSB + 4 * (D * blk + 32 * ((wave + 4 * j) % DT) + 8 * a4));
         }
         __syncthreads();                                   // the four P8 fragments are in LDS
-        v4i pall[NST];
+        v4i pall[NSTW];
 #pragma unroll
-        for (int st = 0; st < NST; ++st) pall[st] = *(const v4i*)(smem + xp_rd + 1024 * st);
-        const v4f ls = *(const v4f*)(smem + xs_rd);
+        for (int st = 0; st < NSTW; ++st) pall[st] = *(const v4i*)(smem + xp_rd + 1024 * st);
+        v4f ls = {0.f, 0.f, 0.f, 0.f};
+        if (!FEW) ls = *(const v4f*)(smem + xs_rd);
         // -------- this wave's output columns: O^T[d, q] += V^T[d, key] P^T[key, q] over the whole block
 #pragma unroll
         for (int j = 0; j < DTW; ++j) {
-            if (NBS == 1) {
+            if constexpr (FEW) {
+                v16i acc = (v16i){0};
+#pragma unroll
+                for (int st = 0; st < NSTW; ++st) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[j][st], pall[st], acc, 0, 0, 0);
+                auto update = [&](auto first) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        float pv = (float)acc[r];
+                        if (VBLK) pv *= vsc[0][j][r >> 2][r & 3];
+                        o_acc[j][r] = fmaf(fmaf(o_acc[j][r], alpha, decltype(first)::value ? pv : 0.f), alpha_b, decltype(first)::value ? 0.f : pv);
+                    }
+                };
+                if (blk_a) update(BoolTag<true>{});
+                else update(BoolTag<false>{});
+            } else if constexpr (NBS == 1) {
                 v16i acc = (v16i){0};
 #pragma unroll
                 for (int st = 0; st < NST; ++st) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[j][st], pall[st], acc, 0, 0, 0);
@@ -304,14 +335,14 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     if (VBLK) o_acc[j][r] = fmaf(fmaf(o_acc[j][r], alpha, (float)acc_a[r] * vsc[0][j][r >> 2][r & 3]), alpha_b,
-                                                 (float)acc_b[r] * vsc[NBS - 1][j][r >> 2][r & 3]);
+                                                 (float)acc_b[r] * vsc[NBW - 1][j][r >> 2][r & 3]);
                     else o_acc[j][r] = fmaf(fmaf(o_acc[j][r], alpha, (float)acc_a[r]), alpha_b, (float)acc_b[r]);
                 }
             }
         }
         if (D == 128) l_run = fmaf(l_run, alpha, (ls[0] + ls[1]) + (ls[2] + ls[3]));
-        else if (D == 64) l_run = fmaf(fmaf(l_run, alpha, ls[0] + ls[1]), alpha_b, ls[2] + ls[3]);
-        else {
+        else if (D == 64 && !FEW) l_run = fmaf(fmaf(l_run, alpha, ls[0] + ls[1]), alpha_b, ls[2] + ls[3]);
+        else if (D == 256) {
             l_run = fmaf(fmaf(l_run, alpha, ls[0]), alpha_b, ls[2]);
             l_odd = fmaf(fmaf(l_odd, alpha, ls[1]), alpha_b, ls[3]);
         }
@@ -344,7 +375,31 @@ __global__ void __launch_bounds__(kThreads, D <= 128 ? 2 : 1) fwd_decode_full_in
     }
 
     // ---- epilogue: every wave scales and stores its own output columns
-    const float l_tot = half_pair_sum(l_run) + (D == 256 ? half_pair_sum(l_odd) : 0.f);      // units of 1/127 when PROUND == 0
+    float l_tot;                                 // units of 1/127 when PROUND == 0
+    if constexpr (FEW) {
+        // (the words of the row maxima and the K tiles were last read ahead of the step's last barrier)
+        const float t0 = half_pair_sum(l_quad[0]) + half_pair_sum(l_quad[1]), t1 = half_pair_sum(l_quad[2]) + half_pair_sum(l_quad[3]);
+        static_assert(DTW == 1 && 2 * 4096 <= KT, "the sums of the two key blocks meet in the first K tile");
+        if (lh == 0) *(float*)(smem + OFF_XM + 16 * lq + 4 * wave) = t0 + t1;
+        if (!blk_a) {
+#pragma unroll
+            for (int a4 = 0; a4 < 4; ++a4)
+                *(v4f*)(smem + OFF_K + 4096 * (wave - 2) + 1024 * a4 + 16 * lane) = (v4f){o_acc[0][4 * a4], o_acc[0][4 * a4 + 1], o_acc[0][4 * a4 + 2], o_acc[0][4 * a4 + 3]};
+        }
+        __syncthreads();
+        const v4f s = *(const v4f*)(smem + OFF_XM + 16 * lq);
+        l_tot = (s[0] + s[1]) + (s[2] + s[3]);
+        if (blk_a) {
+#pragma unroll
+            for (int a4 = 0; a4 < 4; ++a4) {
+                const v4f odd = *(const v4f*)(smem + OFF_K + 4096 * wave + 1024 * a4 + 16 * lane);
+#pragma unroll
+                for (int b4 = 0; b4 < 4; ++b4) o_acc[0][4 * a4 + b4] += odd[b4];
+            }
+        }
+    } else {
+        l_tot = half_pair_sum(l_run) + (D == 256 ? half_pair_sum(l_odd) : 0.f);
+    }
     const float vs = VBLK ? 1.f : cvt_scale_bits(v_scale_bits, p.scale_dtype);
     // false: an empty split range, an empty cache entry, or a causal row above the first key (zeros, lse = -inf; such a
     // row's accumulators hold NaN from exp2(-inf - -inf), hence the selects below)

@@ -90,14 +90,5 @@ def test_the_forms_give_the_same_bits(variant, D, Nq, Nk, causal, splits):
     few = run(variant, args, causal, D ** -0.5, dt, num_splits=splits)
     many = run(variant, [t.repeat(1, 150, *([1] * (t.dim() - 2))) for t in args], causal, D ** -0.5, dt, num_splits=splits)
     torch.cuda.synchronize()
-    # Full-int8 d64, more than 16 rows in more workgroups than fit at once: another kernel, whose lanes add other keys of a row sum.  Sums of Nk
-    # positive terms in fp32 in any order agree to Nk 2^-24, so the lse to that and the output to one step of its 16-bit type.
-    other = variant == "full" and D == 64 and Nq > 16 and 300 * ((Nq + 31) // 32) * splits > 256
     for a, b in zip(few, many):
-        for c in (b[:, :2], b[:, -2:]):
-            if not other:
-                assert torch.equal(a, c)
-            elif a.dtype == torch.float32:
-                assert (a - c).abs().max().item() <= 1.5 * Nk * 2 ** -24 + 2 ** -20      # (1.5 > log2 e; the last places of the sum m + log2 l)
-            else:
-                assert ((a - c).abs() <= 2 ** -10 * a.abs() + 2 ** -24).all()
+        assert torch.equal(a, b[:, :2]) and torch.equal(a, b[:, -2:])

@@ -9,7 +9,8 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 if HERE not in sys.path:
     sys.path.insert(0, HERE)
-import spill_check  # noqa: E402  (a sibling module; this file also runs as a script)
+import mfma_check  # noqa: E402  (sibling modules; this file also runs as a script)
+import spill_check  # noqa: E402
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libintfa.so")
 # -packed-fp32-ops is switched off on purpose: the compiler must not form v_pk_*_f32 from the float code.
@@ -90,7 +91,7 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
 
     def compile_one(pair):
         # -save-temps=obj leaves the device assembly beside the object: it is scanned for register spills that lose lanes
-        # (spill_check.py) and removed again with the other intermediate files
+        # (spill_check.py) and for early readers of matrix products (mfma_check.py), and removed again with the other intermediate files
         src, obj = pair
         cmd = ["hipcc", *FLAGS, "-save-temps=obj", "-c", src, "-o", obj]
         r = subprocess.run(cmd, capture_output=True, text=True)
@@ -104,17 +105,18 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
             path = os.path.join(objdir, f)
             if f.endswith("gfx950.s"):
                 with open(path) as fh:
-                    findings = [f"{os.path.basename(src)}: {x}" for x in spill_check.scan(fh.read())]
+                    asm = fh.read()
+                findings = [f"{os.path.basename(src)}: {x}" for x in spill_check.scan(asm) + mfma_check.scan(asm)]
                 scanned = True
             os.remove(path)
         if not scanned:      # (a compiler that names its intermediate files otherwise must not pass unchecked)
-            raise RuntimeError(f"no device assembly found for {src}: the spill scan did not run")
+            raise RuntimeError(f"no device assembly found for {src}: its scans did not run")
         return findings
 
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         findings = [x for fs in ex.map(compile_one, todo) for x in fs]
     if findings:
-        raise RuntimeError("the compiler placed register spills where lanes are masked off (wrong results for those lanes):\n  "
+        raise RuntimeError("the compiler placed register spills where lanes are masked off, or readers of a matrix product ahead of its wait states:\n  "
                            + "\n  ".join(findings[:20]))
     r = subprocess.run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", OUT], capture_output=True, text=True)
     if r.returncode != 0:

@@ -38,6 +38,12 @@ template <bool V> struct BoolTag { static constexpr bool value = V; };
 template <int V> struct IntTag { static constexpr int value = V; };
 #define INTFA_GLB(p) ((const __attribute__((address_space(1))) void*)(p))
 
+// The wait states between a 32 x 32 matrix product and the first other instruction on its registers, where that instruction stands behind
+// branches: the compiler counts along the longer of two ways to it, so that scores and accumulators could be read up to three wait states early by waves
+// that skip the products in between (mfma_check.py).
+__device__ __forceinline__ void wait_for_product(v16i& x) { asm volatile("s_nop 11" : "+v"(x)); }
+__device__ __forceinline__ void wait_for_product(v16f& x) { asm volatile("s_nop 11" : "+v"(x)); }
+
 constexpr int kBlockM = 128;
 constexpr int kThreads = 256;
 constexpr float kLog2_127 = 6.98868468677f;   // log2(127)

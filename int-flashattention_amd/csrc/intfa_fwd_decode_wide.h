@@ -489,8 +489,9 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                     }
                 }
         }
-        // The products are consumed inside the step: sunk behind the loop's branch, the first register of the last one may be read without the wait
-        // states that an MFMA's result needs (the compiler counts them along the longer of two ways there).
+        // The products are consumed inside the step (int8 V), or at least not moved out of it: sunk behind the loop's branch, the first register of the
+        // last one was once read without the wait states that an MFMA's result needs (the compiler counts them along the longer of two ways
+        // there).  The statement emits nothing; mfma_check.py proves the distance of every reader at build time.
 #pragma unroll
         for (int j = 0; j < CTW; ++j)
 #pragma unroll

@@ -262,6 +262,10 @@ __global__ void __launch_bounds__(kThreads, 3) fwd_f16pv_kernel(const KParams p)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) qk_mfma(0, ks);
+        if (DIAG) {                                         // (its next reader stands behind the tests for the second sub-tile)
+            if (QK_INT8) wait_for_product(si[0]);
+            else wait_for_product(sf[0]);
+        }
         float t[NST][16];
         float mx = -INFINITY;
 #pragma unroll
@@ -356,6 +360,7 @@ __global__ void __launch_bounds__(kThreads, 3) fwd_f16pv_kernel(const KParams p)
             __builtin_amdgcn_sched_barrier(0);
             if (dt + 2 < DT) load_vfrags(vf[dt & 1], dt + 2);
         }
+        if (DIAG) wait_for_product(o_acc[DT - 1]);          // (the older products of the other tiles with it)
     };
 
     auto step = [&](auto buf_tag, auto diag_tag, int nb, int gw, int lim, int lim_lo) __attribute__((always_inline)) {

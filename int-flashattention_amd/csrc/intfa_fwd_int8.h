@@ -261,6 +261,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             __builtin_amdgcn_sched_barrier(0);
             if (st + 2 < nact) load_kfrags(fr[st & 1], st + 2);
             if (!DUMP_S && !DIAG) issue_k_slice(k_next, nb + 1, buf ^ 1, st, NST);
+            if (DUMP_S) wait_for_product(sacc[st & 1]);
             const v16i& acc = sacc[st & 1];
             v16i& nacc = sacc[(st + 1) & 1];
             if (DUMP_S) {

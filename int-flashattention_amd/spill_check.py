@@ -16,7 +16,7 @@ and fails the build if such a placement appears again.
 from __future__ import annotations
 
 import re
-from typing import List
+from typing import Iterator, List, Tuple
 
 _LABEL = re.compile(r"^\.LBB\d+_\d+:")
 _KERNEL = re.compile(r"^(_Z\w+):")
@@ -30,20 +30,48 @@ _BRANCH = re.compile(r"^\s+s_c?branch\w*\s+(\.LBB\d+_\d+)")
 _NO_FALLTHROUGH = ("s_branch", "s_endpgm", "s_setpc_b64")
 
 
+def kernels(asm: str) -> Iterator[Tuple[str, List[dict]]]:
+    """The kernels of one translation unit's assembly text: name and basic blocks, each its label and its [(line number, text)]."""
+    name, blocks = "?", []
+    for n, line in enumerate(asm.split("\n"), 1):
+        m = _KERNEL.match(line)
+        if m:
+            if blocks:
+                yield name, blocks
+            name, blocks = m.group(1), []
+            continue
+        if _LABEL.match(line) or not blocks or blocks[-1]["done"]:
+            blocks.append({"label": line.split(":")[0] if _LABEL.match(line) else None, "lines": [], "done": False})
+        blocks[-1]["lines"].append((n, line))
+        if _BLOCK_END.match(line):
+            blocks[-1]["done"] = True
+    if blocks:
+        yield name, blocks
+
+
+def successors(blocks: List[dict]) -> List[List[int]]:
+    """Where control goes from the end of each block, by the branches and not by the order of the text."""
+    by_label = {b["label"]: k for k, b in enumerate(blocks) if b["label"]}
+    ways = []
+    for k, b in enumerate(blocks):
+        last = b["lines"][-1][1] if b["lines"] else ""
+        nxt = [by_label[m.group(1)] for m in [_BRANCH.match(last)] if m and m.group(1) in by_label]
+        if not (last.split() and last.split()[0] in _NO_FALLTHROUGH) and k + 1 < len(blocks):
+            nxt.append(k + 1)
+        ways.append(nxt)
+    return ways
+
+
 def scan(asm: str) -> List[str]:
     """Returns one line per suspicious spill / reload in the assembly text of one translation unit.
 
     Which blocks are entered with a narrowed mask follows the branches, not the order of the text: a block that stands behind an
     unconditional branch, inside or after a masked region, is entered from wherever its label is named."""
     findings: List[str] = []
-    kernel = "?"
-    blocks: List[dict] = []            # basic blocks of the current kernel: label, [(line number, text)], last opcode
-
-    def close_kernel():
-        by_label = {b["label"]: k for k, b in enumerate(blocks) if b["label"]}
+    for kernel, blocks in kernels(asm):
+        ways = successors(blocks)
         entry = [0] * len(blocks)      # line of an exec-narrowing instruction that may be in force on entry, 0: none
         work = list(range(len(blocks)))
-        leaves = [0] * len(blocks)
         while work:
             k = work.pop(0)
             state = entry[k]
@@ -52,12 +80,7 @@ def scan(asm: str) -> List[str]:
                     state = n
                 elif _EXEC_RESTORE.match(t):
                     state = 0
-            leaves[k] = state
-            last = blocks[k]["lines"][-1][1] if blocks[k]["lines"] else ""
-            nxt = [by_label[m.group(1)] for m in [_BRANCH.match(last)] if m and m.group(1) in by_label]
-            if not (last.split() and last.split()[0] in _NO_FALLTHROUGH) and k + 1 < len(blocks):
-                nxt.append(k + 1)
-            for j in nxt:
+            for j in ways[k]:
                 if state and not entry[j]:
                     entry[j] = state
                     if j not in work:
@@ -75,18 +98,4 @@ def scan(asm: str) -> List[str]:
                     state = n
                 elif _EXEC_RESTORE.match(t):
                     state = 0
-        blocks.clear()
-
-    for n, line in enumerate(asm.split("\n"), 1):
-        m = _KERNEL.match(line)
-        if m:
-            close_kernel()
-            kernel = m.group(1)
-            continue
-        if _LABEL.match(line) or not blocks or blocks[-1]["done"]:
-            blocks.append({"label": line.split(":")[0] if _LABEL.match(line) else None, "lines": [], "done": False})
-        blocks[-1]["lines"].append((n, line))
-        if _BLOCK_END.match(line):
-            blocks[-1]["done"] = True
-    close_kernel()
     return findings

@@ -1,0 +1,62 @@
+"""The build-time scan for early readers of matrix products (int_flashattention_amd/mfma_check.py) on hand-made assembly: a product of four
+passes (16 x 16) needs eight wait states, one of eight passes (32 x 32) twelve, on every way to an instruction that touches its registers."""
+import os
+import sys
+
+import pytest
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "int-flashattention_amd"))
+import mfma_check  # noqa: E402
+
+HEAD = "_ZN5intfa4kernEv:\n\ts_load_dwordx2 s[0:1], s[4:5], 0x0\n"
+SMALL = "\tv_mfma_f32_16x16x32_f16 v[0:3], v[8:11], v[12:15], v[0:3]\n"
+LARGE = "\tv_mfma_i32_32x32x32_i8 v[16:31], v[8:11], v[12:15], 0\n"
+
+
+@pytest.mark.parametrize("product,states,reader", [
+    (SMALL, 8, "v_mul_f32_e32 v4, v3, v5"), (SMALL, 8, "ds_write_b128 v7, v[0:3]"), (SMALL, 8, "v_mov_b32_e32 v0, 0"),
+    (SMALL, 8, "v_mfma_f32_16x16x32_f16 v[32:35], v[0:3], v[12:15], 0"), (SMALL, 8, "v_mfma_f32_16x16x32_f16 v[32:35], v[8:11], v[12:15], v[2:5]"),
+    (LARGE, 12, "v_cvt_f32_i32_e32 v4, v16"), (LARGE, 12, "global_store_dword v[4:5], v31, off"), (LARGE, 12, "v_accvgpr_write_b32 a0, v20"),
+])
+def test_the_last_wait_state_counts(product, states, reader):
+    for have in (0, states - 1, states):
+        nops = "".join("\ts_mov_b32 s9, s8\n" for _ in range(have % 4)) + (f"\ts_nop {have - have % 4 - 1}\n" if have >= 4 else "")
+        found = mfma_check.scan(HEAD + product + nops + "\t" + reader + " ; a comment naming v0\n\ts_endpgm\n")
+        assert len(found) == (have < states), (have, found)
+        assert all(f"{states - have} wait states too early" in f and "_ZN5intfa4kernEv" in f for f in found)
+
+
+def test_a_chain_and_other_registers_need_no_wait():
+    asm = (HEAD + LARGE + "\tv_mfma_i32_32x32x32_i8 v[16:31], v[8:11], v[12:15], v[16:31]\n"
+           "\tv_mfma_i32_32x32x32_i8 v[40:55], v[8:11], v[12:15], v[16:31]\n\tv_add_f32_e32 v1, v2, v15\n\tv_mov_b32_e32 v32, s16\n\ts_endpgm\n")
+    assert mfma_check.scan(asm) == []
+    # accumulation registers are registers of their own
+    acc = HEAD + LARGE.replace("v[16:31]", "a[16:31]") + "\tv_mov_b32_e32 v16, 0\n\t{}\n\ts_endpgm\n"
+    assert mfma_check.scan(acc.format("s_nop 0")) == []
+    assert len(mfma_check.scan(acc.format("v_accvgpr_read_b32 v0, a16"))) == 1
+
+
+# A product, a way around other products, the reader: the wait must be there on the short way too.
+SKIP = ("\ts_cbranch_scc1 .LBB0_2\n; %bb.1:\n" + 12 * "\tv_mov_b32_e32 v60, 0\n" + ".LBB0_2:\n")
+
+
+def test_the_shorter_of_two_ways_counts():
+    reader = "\tv_cvt_f32_i32_e32 v4, v16\n\ts_endpgm\n"
+    assert len(mfma_check.scan(HEAD + LARGE + SKIP + reader)) == 1
+    assert len(mfma_check.scan(HEAD + LARGE + SKIP + "\ts_nop 9\n" + reader)) == 1
+    assert mfma_check.scan(HEAD + LARGE + SKIP + "\ts_nop 10\n" + reader) == []
+
+
+def test_a_loop_and_its_exit_are_followed():
+    loop = HEAD + ".LBB0_1:\n\tv_mul_f32_e32 v1, v1, v5\n" + 8 * "\ts_mov_b32 s9, s8\n" + SMALL + "{}\ts_cbranch_scc1 .LBB0_1\n; %bb.2:\n{}\tv_add_f32_e32 v6, v0, v0\n\ts_endpgm\n"
+    found = mfma_check.scan(loop.format("", "\ts_nop 6\n"))
+    assert len(found) == 1 and "v_mul_f32_e32 v1" in found[0]      # the next round reads too early, the code behind the loop does not
+    found = mfma_check.scan(loop.format("\ts_nop 6\n", ""))
+    assert found == []
+    found = mfma_check.scan(loop.format("\ts_nop 5\n", ""))
+    assert len(found) == 2
+
+
+def test_an_unknown_product_is_reported():
+    found = mfma_check.scan(HEAD + "\tv_mfma_f64_16x16x4_f64 v[0:7], v[8:9], v[10:11], v[0:7]\n\ts_endpgm\n")
+    assert len(found) == 1 and "table" in found[0]

@@ -106,7 +106,7 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
             if f.endswith("gfx950.s"):
                 with open(path) as fh:
                     asm = fh.read()
-                findings = [f"{os.path.basename(src)}: {x}" for x in spill_check.scan(asm) + mfma_check.scan(asm)]
+                findings = [f"{os.path.basename(src)}: {x}" for x in spill_check.scan(asm) + mfma_check.scan(asm) + mfma_check.scan_waits(asm)]
                 scanned = True
             os.remove(path)
         if not scanned:      # (a compiler that names its intermediate files otherwise must not pass unchecked)
@@ -116,7 +116,8 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         findings = [x for fs in ex.map(compile_one, todo) for x in fs]
     if findings:
-        raise RuntimeError("the compiler placed register spills where lanes are masked off, or readers of a matrix product ahead of its wait states:\n  "
+        raise RuntimeError("the compiler placed register spills where lanes are masked off, or readers of a matrix product ahead of its wait states, "
+                           "or waits for the next tiles ahead of a step's products:\n  "
                            + "\n  ".join(findings[:20]))
     r = subprocess.run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", OUT], capture_output=True, text=True)
     if r.returncode != 0:

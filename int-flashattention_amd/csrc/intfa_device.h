@@ -44,6 +44,16 @@ template <int V> struct IntTag { static constexpr int value = V; };
 __device__ __forceinline__ void wait_for_product(v16i& x) { asm volatile("s_nop 11" : "+v"(x)); }
 __device__ __forceinline__ void wait_for_product(v16f& x) { asm volatile("s_nop 11" : "+v"(x)); }
 
+// Behind the first wait for the tiles: Q was requested with them and has arrived too, and this tells the compiler, which does not know the
+// hand-written waits.  Without it its own wait for Q stands ahead of the products inside the loop over the key blocks, behind the requests for the
+// next tiles, and waits for those: no copy runs under a block's work then (mfma_check.py looks for such waits).  Without -> with it, us: half-int8
+// decode d64 B8 H32 Nq1 Nk4096, one pass, 51.3 -> 37, 320 workgroups of 6000 keys 78 -> 66; 32 rows, fp16, 102 -> 87; bf16 prefill B4 H32 N4096 d128 964 ->
+// 935, causal N2048 d256 425 -> 403.
+template <int N> __device__ __forceinline__ void q_has_arrived(v4i (&q)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(q[i]));
+}
+
 constexpr int kBlockM = 128;
 constexpr int kThreads = 256;
 constexpr float kLog2_127 = 6.98868468677f;   // log2(127)

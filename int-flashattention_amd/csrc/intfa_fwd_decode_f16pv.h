@@ -166,6 +166,7 @@ __global__ void __launch_bounds__(kThreads, D == 256 ? 1 : 2) fwd_decode_f16pv_k
         constexpr int BUF = decltype(buf_tag)::value ? 1 : 0;
         constexpr int KB = BUF * KT, VB = BUF * VT, SB = BUF * BN * 4;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        q_has_arrived(qreg);
         __syncthreads();                                   // the tiles have landed; the other buffer and the exchange areas are free
         const bool more = nb + NBS < nb_end;
         uint32_t ks_next = 0;

@@ -281,6 +281,8 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
         if (ks_wave) *(float*)(smem + ks_wr + SB) = ks_src.cvt(ks_next);
         if (vs_wave) *(float*)(smem + vs_wr + VSB) = vs_next;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) q_has_arrived(qreg[rt]);
         __syncthreads();                                   // the tiles have landed; the other buffer and the exchange areas are free
         if (nb + BPS < nb_end) {
             if (G::BUFS == 2) issue_loads(nb + BPS, BUF ^ 1);

@@ -385,6 +385,7 @@ __global__ void __launch_bounds__(kThreads, 3) fwd_f16pv_kernel(const KParams p)
         const int tail_keys = seqlen_k - (nb_total - 1) * BN;        // valid keys of the last block (BN if it is full)
         const bool ragged = !CAUSAL && tail_keys < BN && nb_end == nb_total;
         const int plain_end = CAUSAL ? (nb_end > diag_begin ? diag_begin : nb_end) : (ragged ? nb_end - 1 : nb_end);
+        q_has_arrived(qreg);
         int nb = nb_begin;
         while (true) {
             if (nb >= plain_end) break;

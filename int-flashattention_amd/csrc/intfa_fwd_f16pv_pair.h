@@ -288,6 +288,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_f16pv_pair_kernel(const K
             qsc = q_scale_log2(p, q_scale_bits);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (CAUSAL) q_has_arrived(qreg);                   // (without the mask a fragment of Q is fetched back from scratch in every block anyway)
         __syncthreads();
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) qk_step(*(const v4i*)(smem + k_rd(ks)), ks);

@@ -333,6 +333,7 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
         store_ks(ks1, !odd0);
         if (QK_INT8) qsc = q_scale_log2(p, q_scale_bits);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        q_has_arrived(qreg);
         __syncthreads();
         int nb = nb_begin;
         if (!odd0) {

@@ -77,3 +77,45 @@ def scan(asm: str) -> List[str]:
                     work.append(j)
         findings += [found[n] for n in sorted(found)]
     return findings
+
+
+_LOAD_WAIT = re.compile(r"^\s+s_waitcnt\b.*\bvmcnt\(")
+
+
+def _in_loops(ways: List[List[int]]) -> List[bool]:
+    """Which blocks can be reached from their own end."""
+    def reach(k):
+        seen, work = set(), list(ways[k])
+        while work:
+            j = work.pop()
+            if j not in seen:
+                seen.add(j)
+                work += ways[j]
+        return seen
+    return [k in reach(k) for k in range(len(ways))]
+
+
+def scan_waits(asm: str) -> List[str]:
+    """Returns one line per wait for loads that the compiler put directly ahead of a product inside a loop.
+
+    Tiles come through LDS, by hand-written copies and waits that the compiler does not know.  A wait of its own ahead of a product in the loop is
+    for Q, which arrived long ago, and holds the products back until the next tiles, requested just before, are there as well: no copy runs under
+    the work of a step (decoding steps lost up to a third).  Kernels that fetch a spilled fragment back from scratch in the loop have to wait there."""
+    findings: List[str] = []
+    for kernel, blocks in spill_check.kernels(asm):
+        found, by_hand, wait, reload = [], False, 0, False
+        if not any("v_mfma" in t for b in blocks for _, t in b["lines"]):
+            continue
+        for b, loop in zip(blocks, _in_loops(spill_check.successors(blocks))):
+            for n, t in b["lines"]:
+                if "#ASMSTART" in t or "#ASMEND" in t:
+                    by_hand = "#ASMSTART" in t
+                m = _INSTRUCTION.match(t)
+                if not m or not loop:
+                    continue
+                reload = reload or "Folded Reload" in t
+                if wait and m.group(1).startswith("v_mfma"):
+                    found.append(f"{kernel}: line {wait}: a wait for loads ahead of the product of line {n}, inside a loop")
+                wait = n if _LOAD_WAIT.match(t) and not by_hand else 0
+        findings += [] if reload else found
+    return findings

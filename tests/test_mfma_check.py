@@ -60,3 +60,16 @@ def test_a_loop_and_its_exit_are_followed():
 def test_an_unknown_product_is_reported():
     found = mfma_check.scan(HEAD + "\tv_mfma_f64_16x16x4_f64 v[0:7], v[8:9], v[10:11], v[0:7]\n\ts_endpgm\n")
     assert len(found) == 1 and "table" in found[0]
+
+
+def test_a_wait_for_loads_ahead_of_a_product_in_a_loop_is_reported():
+    """Q is fetched ahead of the loop; the compiler's wait for it belongs there too."""
+    head = HEAD + "\tglobal_load_dwordx4 v[12:15], v[60:61], off\n{}.LBB0_1: ; =>This Inner Loop Header: Depth=1\n"
+    copy = "\t;;#ASMSTART\n\ts_waitcnt vmcnt(0)\n\t;;#ASMEND\n\ts_barrier\n\t;;#ASMSTART\n\tbuffer_load_dwordx4 v70, s[8:11], s12 offen lds\n\t;;#ASMEND\n"
+    end = LARGE + "\ts_cbranch_scc1 .LBB0_1\n; %bb.2:\n\ts_endpgm\n"
+    found = mfma_check.scan_waits(head.format("") + copy + "\ts_waitcnt vmcnt(0) lgkmcnt(1)\n" + end)
+    assert len(found) == 1 and "_ZN5intfa4kernEv" in found[0]
+    assert mfma_check.scan_waits(head.format("\ts_waitcnt vmcnt(0)\n") + copy + "\ts_waitcnt lgkmcnt(1)\n" + end) == []
+    assert mfma_check.scan_waits(HEAD + "\ts_waitcnt vmcnt(0)\n" + LARGE + "\ts_endpgm\n") == []      # not in a loop
+    spilled = "\tscratch_load_dwordx4 v[12:15], off, off offset:16 ; 16-byte Folded Reload\n\ts_waitcnt vmcnt(0)\n"
+    assert mfma_check.scan_waits(head.format("") + copy + spilled + end) == []

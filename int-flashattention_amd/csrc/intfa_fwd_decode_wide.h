@@ -252,11 +252,16 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
     const uint32_t kk_rd = OFF_KS + 4 * (16 * wave + 4 * lh);
     // row maxima: [row][tile]; row sums: [row][wave]
     const uint32_t xm_wr = OFF_XM + 4 * (XW * ln + wave), xm_rd = OFF_XM + 4 * XW * ln;     // + 64 * XW per row tile, + 32 per tile
+    // 16-bit V and two row tiles (one key tile per wave): a lane's two rows go through the maximum together, in one exchange of lanes and one
+    // store, and both rows' maxima are requested before the first is looked at.  Half-int8 d64, 32 rows of 6000 keys, us: 256 workgroups 60.3 -> 56.3, 320
+    // 79.5 -> 74, 768 167 -> 160 (with all waves known to have keys, see qk_wave).  Not a quarter of the maxima per lane: fewer LDS reads, a longer chain (320: 80).
+    constexpr bool TWO_ROWS = !VI8 && RT == 2;
+    const uint32_t xm_wr2 = xm_wr + 64 * XW * lh;        // of row tile lh
     const uint32_t xp_wr = OFF_XP + (wave / TPO) * RT * 1024 + 16 * lane + TB * (wave % TPO);    // + 8 / TPO * RT * 1024 per tile
     const uint32_t xp_rd = OFF_XP + kh * OPH * RT * 1024 + 16 * lane;
     const uint32_t vs_wr = OFF_VS + 4 * vs_i;
     const uint32_t vs_rd = OFF_VS + 4 * (16 * (wave % CT) + 4 * lh);                  // + 4 * D per block, + 4 * 16 * kWideWaves per column tile
-    const bool qk_wave = wave < G::QKW;
+    const bool qk_wave = G::QKW == kWideWaves || wave < G::QKW;      // (a constant where all have: half-int8 d64 B4 H16 Nq5 Nk3001, one pass, 22.9 -> 21.0 us)
     // the smallest and the largest last visible key of the workgroup's rows, and each lane's own
     const int first_lim = p.causal ? (fold ? 0 : row0) + causal_off : 0x3fffffff;
     const int last_lim = p.causal ? (fold ? fold : row0 + ROWS) - 1 + causal_off : 0x3fffffff;
@@ -347,15 +352,24 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
                         for (int r = 0; r < 4; ++r) x[t][rt][r] = hide_past(x[t][rt][r], last, 128 * t + r);
                 }
             }
+            if constexpr (TWO_ROWS) {
+                static_assert(NT == 1, "one key tile per wave");
+                float mx[RT];
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                float mx[NT];
+                for (int rt = 0; rt < RT; ++rt) mx[rt] = fmaxf(fmaxf(x[0][rt][0], x[0][rt][1]), fmaxf(x[0][rt][2], x[0][rt][3]));
+                const float both = max_of_row_lanes(mx[0], mx[1]);
+                if (lh < RT) *(float*)(smem + xm_wr2) = both;
+            } else {
 #pragma unroll
-                for (int t = 0; t < NT; ++t) mx[t] = fmaxf(fmaxf(x[t][rt][0], x[t][rt][1]), fmaxf(x[t][rt][2], x[t][rt][3]));
+                for (int rt = 0; rt < RT; ++rt) {
+                    float mx[NT];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    mx[t] = reduce_row_lanes(mx[t], [](float a, float c) { return fmaxf(a, c); });
-                    if (lh == 0) *(float*)(smem + xm_wr + 64 * XW * rt + 32 * t) = mx[t];
+                    for (int t = 0; t < NT; ++t) mx[t] = fmaxf(fmaxf(x[t][rt][0], x[t][rt][1]), fmaxf(x[t][rt][2], x[t][rt][3]));
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        mx[t] = reduce_row_lanes(mx[t], [](float a, float c) { return fmaxf(a, c); });
+                        if (lh == 0) *(float*)(smem + xm_wr + 64 * XW * rt + 32 * t) = mx[t];
+                    }
                 }
             }
         }
@@ -363,11 +377,20 @@ __device__ __forceinline__ void decode_wide(const KParams& p) {
         __syncthreads();                                   // the waves' maxima are in LDS (one buffer: its tiles are in registers)
         if (G::BUFS == 1 && nb + BPS < nb_end) issue_loads(nb + BPS, 0);
         float alpha[NB][RT], bias[RT][NT];
+        float wm_all[TWO_ROWS ? RT : 1][G::NKT];
+        auto read_maxima = [&](int rt) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < G::NKT / 4; ++i) *(v4f*)(wm_all[TWO_ROWS ? rt : 0] + 4 * i) = *(const v4f*)(smem + xm_rd + 64 * XW * rt + 16 * i);
+        };
+        if (TWO_ROWS) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) read_maxima(rt);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            float wm[G::NKT];
-#pragma unroll
-            for (int i = 0; i < G::NKT / 4; ++i) *(v4f*)(wm + 4 * i) = *(const v4f*)(smem + xm_rd + 64 * XW * rt + 16 * i);
+            if (!TWO_ROWS) read_maxima(rt);
+            const float* const wm = wm_all[TWO_ROWS ? rt : 0];
             float m = m_run[rt];
 #pragma unroll
             for (int i = 0; i < NB; ++i) {

@@ -212,6 +212,13 @@ template <typename F> __device__ __forceinline__ float reduce_row_lanes(float x,
     const auto c = __builtin_amdgcn_permlane32_swap(w, w, false, false);
     return op(__builtin_bit_cast(float, (unsigned)c[0]), __builtin_bit_cast(float, (unsigned)c[1]));
 }
+// Of two values at once: lanes of even rows of 16 return the maximum of a over their four lanes, those of odd rows that of b.
+__device__ __forceinline__ float max_of_row_lanes(float a, float b) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned w = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)s[0]), __builtin_bit_cast(float, (unsigned)s[1])));
+    const auto c = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return fmaxf(__builtin_bit_cast(float, (unsigned)c[0]), __builtin_bit_cast(float, (unsigned)c[1]));
+}
 template <typename F> __device__ __forceinline__ float reduce_wave(float x, F op) {      // (quad_perm 1,0,3,2 / 2,3,0,1, the mirrored half row, the mirrored row)
     x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true)));
     x = op(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true)));

@@ -250,11 +250,6 @@ size_t intfa_quant_pertensor_parts_workspace_bytes(int32_t batch, int32_t heads,
 int intfa_quant_pertensor(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_n, void* q8, void* scale,
                           int32_t batch, int32_t heads, int32_t seqlen, int32_t head_dim, int32_t dtype,
                           void* workspace, size_t workspace_bytes, void* stream);
-/* The same for tests: where workgroups of a large tensor wait for the maxima of their slice's other pieces, each reads its slice for itself,
- * as it would after a wait that did not end. */
-int intfa_debug_quant_pertensor_alone(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_n, void* q8, void* scale,
-                                      int32_t batch, int32_t heads, int32_t seqlen, int32_t head_dim, int32_t dtype,
-                                      void* workspace, size_t workspace_bytes, void* stream);
 
 /* Quantiser for the blocked V scales of intfa_fwd_params.v_scale_block: one fp32 scale per (batch, head, block of
  * `block` rows, channel), scale = absmax / 127 over the block's rows and q = round-half-even(x / scale), both in fp32

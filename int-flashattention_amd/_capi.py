@@ -59,8 +59,7 @@ EXPORTS = ("intfa_version", "intfa_error_string", "intfa_fwd_block_n", "intfa_fw
            "intfa_fwd_merge_workspace_bytes", "intfa_fwd_suggest_splits",
            "intfa_fwd_full_int8", "intfa_fwd_half_int8", "intfa_fwd_fp16", "intfa_fwd_full_int8_static", "intfa_debug_qk_int32",
            "intfa_quant_pertoken", "intfa_quant_pertensor_workspace_bytes",
-           "intfa_quant_pertensor_parts_workspace_bytes", "intfa_quant_pertensor", "intfa_debug_quant_pertensor_alone",
-           "intfa_quant_perblock_channel", "intfa_kvcache_append_int8")
+           "intfa_quant_pertensor_parts_workspace_bytes", "intfa_quant_pertensor", "intfa_quant_perblock_channel", "intfa_kvcache_append_int8")
 
 _lib = None
 
@@ -103,7 +102,7 @@ def load():
     lib.intfa_quant_pertensor_parts_workspace_bytes.argtypes = [i32, i32, i32, i32]
     lib.intfa_quant_pertensor.restype = ctypes.c_int
     lib.intfa_quant_pertensor.argtypes = [vp, i64, i64, i64, vp, vp, i32, i32, i32, i32, i32, vp, ctypes.c_size_t, vp]
-    lib.intfa_debug_quant_pertensor_alone.restype = ctypes.c_int
+    lib.intfa_debug_quant_pertensor_alone.restype = ctypes.c_int      # (for the tests: not part of intfa.h)
     lib.intfa_debug_quant_pertensor_alone.argtypes = lib.intfa_quant_pertensor.argtypes
     lib.intfa_quant_perblock_channel.restype = ctypes.c_int
     lib.intfa_quant_perblock_channel.argtypes = [vp, i64, i64, i64, vp, vp, i32, i32, i32, i32, i32, i32, vp]

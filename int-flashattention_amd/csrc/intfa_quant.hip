@@ -628,6 +628,8 @@ int intfa_quant_pertensor(const void* x, int64_t stride_b, int64_t stride_h, int
     return quant_pertensor(x, stride_b, stride_h, stride_n, q8, scale, batch, heads, seqlen, head_dim, dtype, workspace, workspace_bytes,
                            kSliceWait, stream);
 }
+// For the tests, and in no header: where workgroups of a large tensor wait for the maxima of their slice's other pieces, each reads its slice for
+// itself, as it would after a wait that did not end.
 int intfa_debug_quant_pertensor_alone(const void* x, int64_t stride_b, int64_t stride_h, int64_t stride_n, void* q8, void* scale,
                                       int32_t batch, int32_t heads, int32_t seqlen, int32_t head_dim, int32_t dtype,
                                       void* workspace, size_t workspace_bytes, void* stream) {

@@ -94,7 +94,7 @@ __device__ __forceinline__ void splitkv_open_tickets(KernargPtr p, int group, ui
 // Called by every thread of the workgroup after its stores; `smem` is free.  Its first kArrivalBytes carry the answer, and no barrier follows
 // the reading of it: a wave may read it while another is in the merge already, which therefore leaves these bytes alone.
 constexpr int kArrivalBytes = 16;
-template <typename P> __device__ __forceinline__ bool splitkv_last_arrival(P p, char* smem, int group) {
+__device__ __forceinline__ bool splitkv_last_arrival(KernargPtr p, char* smem, int group) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's partials have reached the point of coherence
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -109,14 +109,13 @@ template <typename P> __device__ __forceinline__ bool splitkv_last_arrival(P p, 
     if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     return last;
 }
-__device__ __forceinline__ bool splitkv_last_arrival(const KParams& p, char* smem, int group) { return splitkv_last_arrival(&p, smem, group); }
 
 // ---- The same for the general full-int8 kernel, whose waves own 32 query rows each: a ticket per wave and no barrier.  The wave
 // that arrives last reads the partials in the layout of its accumulators, so the row statistics are one value per lane.
 // Instead of a second launch of splitkv_combine_kernel, whose arithmetic and order of splits it keeps (the same bits, whichever
 // wave is last), us: causal chunk B2 H32/8 Nq512 Nk7680 d128 (2 splits) 113 -> 105.5, B4 H12/3 Nq300 Nk3000 (4) 47 -> 43.4, d64 H16/4
 // Nq600 Nk4000 (7) 35.4 -> 31.1.  Not at head_dim 256, whose rows are spread over two waves.
-template <typename P> __device__ __forceinline__ bool splitkv_last_arrival_wave(P p, int group) {
+__device__ __forceinline__ bool splitkv_last_arrival_wave(KernargPtr p, int group) {
     unsigned drew_last = 0;                                // (after the wave's partials have been acknowledged)
     if ((threadIdx.x & 63) == 0) {
         uint64_t* t = p->ticket + group * kTicketStride;

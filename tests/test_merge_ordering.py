@@ -1,6 +1,7 @@
 """The split-KV merge inside the forward launch (csrc/intfa_splitkv.h) reads partials that other workgroups wrote.  What the compiler is given
 must hold the order: stores of partials at agent scope, a wait for them, the ticket's atomic addition, an acquire fence, loads of partials
-at agent scope.  Compiles the two arrival functions, each between a store and a load of a partial, to the compiler's intermediate form."""
+at agent scope.  Compiles the two arrival functions, as the kernels call them and each between a store and a load of a partial, to the compiler's
+intermediate form."""
 import os
 import re
 import subprocess
@@ -12,16 +13,18 @@ SOURCE = """
 using namespace intfa;
 __global__ void arrive_workgroup(const KParams p, float* out) {
     __shared__ __attribute__((aligned(16))) char smem[64];
-    const SplitPartials part(&p, 128, 0);
+    const KernargPtr pe = kernarg_block();
+    const SplitPartials part(pe, 128, 0);
     part.put_lse(threadIdx.x, 1.f);
-    if (!splitkv_last_arrival(p, smem, blockIdx.x)) return;
+    if (!splitkv_last_arrival(pe, smem, blockIdx.x)) return;
     out[threadIdx.x] = part.get_lse(threadIdx.x);
 }
 __global__ void arrive_wave(const KParams p, float* out) {
-    const SplitPartials part(&p, 128, 0);
+    const KernargPtr pe = kernarg_block();
+    const SplitPartials part(pe, 128, 0);
     part.put_lse(threadIdx.x, 1.f);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (!splitkv_last_arrival_wave(&p, blockIdx.x)) return;
+    if (!splitkv_last_arrival_wave(pe, blockIdx.x)) return;
     out[threadIdx.x] = part.get_lse(threadIdx.x);
 }
 """

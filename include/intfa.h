@@ -172,8 +172,10 @@ const char* intfa_error_string(int code);
  * configs.py:13-19).  The running max and, on the full-int8 path, the requantisation of P advance per key block,
  * so a bit-faithful CPU evaluation must use the same value.  Full-int8: 128 at head_dim 128, 64 otherwise; half-int8 and
  * fp16: 64.  At head_dim >= 64 that is a length the reference's kernel admits (flash_atten_full_int8.py:88,
- * static_assert BLOCK_N <= HEAD_DIM); head_dim 16 and 32 are computed zero-padded to 64 and keep the 64-key block.  It holds for every shape: the kernel
- * that takes over decode-shaped calls (at most 64 query rows) walks the same blocks.
+ * static_assert BLOCK_N <= HEAD_DIM); head_dim 16 and 32 are computed zero-padded to 64 and keep the 64-key block.  It holds for every shape: the kernels
+ * that take over decode-shaped calls (at most 64 query rows) walk the same blocks.  Half-int8 and fp16 advance the running maximum by two of
+ * them at head_dim 64 there and add their products in another order: their output of a row may differ by about one rounding of its 16-bit
+ * type from that of the same row in a call of more rows.
  * Negative INTFA_ERR_* for unknown arguments. */
 int intfa_fwd_block_n(int variant, int head_dim);
 

@@ -37,8 +37,9 @@ static_assert(kWideWaves == kMergeWaves, "");
 template <int D, bool KI8, bool VI8, typename R> struct WideGeom {
     static_assert(D == 64 || D == 128 || D == 256, "head dims 64, 128, 256");
     static constexpr int KROW = D * (KI8 ? 1 : 2), VROW = D * (VI8 ? 1 : 2);      // bytes per row
-    // Two steps of tiles in the LDS, and two workgroups per compute unit: with one, its prologue and its merge (4 - 6 us) overlap with nothing.
-    // Head_dim 256 with 16-bit V has one (fewer than four 16-key tiles are too few).  Full-int8 has a second form with room for more workgroups: head_dim 128 steps of 128 keys instead of 256 (step of one request, us: 1.0 and 1.3, so the longer one while
+    // Two steps of tiles in the LDS, and room for two workgroups per compute unit where steps of at least four 16-key tiles allow it: with one, its
+    // prologue and its merge (4 - 6 us) overlap with nothing.  One at head_dim 256 with 16-bit V, and for full-int8 at head_dims 128 (128 KiB of
+    // tiles) and 256 in grids of at most one workgroup per unit.  Full-int8 has a second form with room for more workgroups: head_dim 128 steps of 128 keys instead of 256 (step of one request, us: 1.0 and 1.3, so the longer one while
     // there is room), head_dim 64 one step's tiles instead of two, the next ones requested once all waves hold theirs in registers
     // (three workgroups per unit instead of two, us: 640 workgroups 54 -> 39.7, 960 of 1500 keys 42.1 (128-key steps) -> 37.7), head_dim 256 steps of 64 keys,
     // whose S^T keeps half the waves busy, instead of 128 with one workgroup per unit (256 workgroups of 1500 keys 48.7 -> 41.3, 5 requests

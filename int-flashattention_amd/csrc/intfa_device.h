@@ -90,6 +90,7 @@ struct KParams {
     int32_t causal_rows;                   // decode kernel: query positions per folded query head (0 = the row is the position)
     float qk_scale_log2;                   // sm_scale * log2(e)
     // workgroup -> work mapping of this launch (set by finish_mapping() in intfa_launch.h from the grid size)
+    int32_t items, grid_wgs;               // work items (workgroups, were each to take one), and workgroups of the launch
     int32_t per_head;                      // workgroups per query head
     int32_t heads_kv;                      // heads / kv_group
     int32_t xcd_whole_wgs;                 // workgroups of the K/V heads that are dealt whole to the 8 XCDs (a multiple of 8)
@@ -155,56 +156,58 @@ __device__ __forceinline__ float load_scale(const char* base, int64_t idx, int d
 // ahead of the others: their heavy blocks must not come last either.
 // (All divisors are fixed per launch: fast_div.)
 struct WorkgroupJob { int b, h, hk, rem; };      // batch entry, query head, K/V head, index among the head's workgroups
-__device__ __forceinline__ WorkgroupJob deal_workgroup(const KParams& p, int bid) {
-    const int kv_group = p.kv_group;
-    const int per_head = p.per_head;
+// (Args: const KParams* or KernargPtr)
+template <typename Args> __device__ __forceinline__ WorkgroupJob deal_workgroup(Args p, int bid) {
+    const int kv_group = p->kv_group;
+    const int per_head = p->per_head;
     const int per_kv = per_head * kv_group;              // workgroups per K/V head
     int kv_lin, hq, rem;
-    if (p.causal) {
+    if (p->causal) {
         int idx, first, unit_step, heads;
         FastDiv d_heads;
-        if (bid >= p.rem_wgs) {
-            const int slot = (bid - p.rem_wgs) >> 3;
+        if (bid >= p->rem_wgs) {
+            const int slot = (bid - p->rem_wgs) >> 3;
             unit_step = 8;
-            if (slot < p.run_last_slot) {
-                const int g = fast_div(slot, p.d_run);
-                idx = slot - g * p.run_units * per_kv;
-                first = g * p.run_units; heads = p.run_units * kv_group; d_heads = p.d_run_heads;
+            if (slot < p->run_last_slot) {
+                const int g = fast_div(slot, p->d_run);
+                idx = slot - g * p->run_units * per_kv;
+                first = g * p->run_units; heads = p->run_units * kv_group; d_heads = p->d_run_heads;
             } else {
-                idx = slot - p.run_last_slot;
-                first = fast_div(p.run_last_slot, p.d_per_kv); heads = p.run_units_last * kv_group; d_heads = p.d_run_heads_last;
+                idx = slot - p->run_last_slot;
+                first = fast_div(p->run_last_slot, p->d_per_kv); heads = p->run_units_last * kv_group; d_heads = p->d_run_heads_last;
             }
-            first = first * 8 + ((bid - p.rem_wgs) & 7);
+            first = first * 8 + ((bid - p->rem_wgs) & 7);
         } else {
             idx = bid;
             unit_step = 1;
-            first = fast_div(p.xcd_whole_wgs, p.d_per_kv);
-            heads = (p.batch * p.heads_kv - first) * kv_group; d_heads = p.d_rem_heads;
+            first = fast_div(p->xcd_whole_wgs, p->d_per_kv);
+            heads = (p->batch * p->heads_kv - first) * kv_group; d_heads = p->d_rem_heads;
         }
         rem = fast_div(idx, d_heads);
-        const int u = idx - rem * heads, unit = fast_div(u, p.d_kv_group);
+        const int u = idx - rem * heads, unit = fast_div(u, p->d_kv_group);
         kv_lin = first + unit * unit_step;
         hq = u - unit * kv_group;
     } else {
         int r;
-        if (bid < p.xcd_whole_wgs) {
+        if (bid < p->xcd_whole_wgs) {
             const int xcd = bid & 7, slot = bid >> 3;
-            const int q = fast_div(slot, p.d_per_kv);
+            const int q = fast_div(slot, p->d_per_kv);
             kv_lin = q * 8 + xcd;
             r = slot - q * per_kv;
         } else {
-            const int j = bid - p.xcd_whole_wgs;                        // (xcd_whole_wgs is a multiple of 8: j & 7 is the XCD)
-            const int idx = p.xcd_rem_chunk ? (j & 7) * p.xcd_rem_chunk + (j >> 3) : j;
-            const int q = fast_div(idx, p.d_per_kv);
-            kv_lin = fast_div(p.xcd_whole_wgs, p.d_per_kv) + q;
+            const int j = bid - p->xcd_whole_wgs;                        // (xcd_whole_wgs is a multiple of 8: j & 7 is the XCD)
+            const int idx = p->xcd_rem_chunk ? (j & 7) * p->xcd_rem_chunk + (j >> 3) : j;
+            const int q = fast_div(idx, p->d_per_kv);
+            kv_lin = fast_div(p->xcd_whole_wgs, p->d_per_kv) + q;
             r = idx - q * per_kv;
         }
-        hq = fast_div(r, p.d_per_head);                  // query head inside the group
+        hq = fast_div(r, p->d_per_head);                  // query head inside the group
         rem = r - hq * per_head;
     }
-    const int bb = fast_div(kv_lin, p.d_heads_kv), hk = kv_lin - bb * p.heads_kv;
+    const int bb = fast_div(kv_lin, p->d_heads_kv), hk = kv_lin - bb * p->heads_kv;
     return {bb, hk * kv_group + hq, hk, rem};
 }
+__device__ __forceinline__ WorkgroupJob deal_workgroup(const KParams& p, int bid) { return deal_workgroup(&p, bid); }
 
 // Number of keys of batch entry b: one length for all, or per batch (a cache filled to different lengths), clamped to
 // [0, seqlen_k] so that rows past the allocation are never addressed.
@@ -273,13 +276,14 @@ __device__ __forceinline__ float load_q_scale_log2(const KParams& p, int b, int 
 struct KScaleSource {
     const char* base;
     int stride, dtype, seqlen_k;
-    __device__ __forceinline__ KScaleSource(const KParams& p, int b, int hk, int seqlen_k_) {
-        const int esize = p.scale_dtype == 2 ? 4 : 2;
-        base = p.k_scale + (b * p.ks_sb + hk * p.ks_sh) * esize;
-        stride = (int)(p.ks_sn * esize);
-        dtype = p.scale_dtype;
+    template <typename Args> __device__ __forceinline__ KScaleSource(Args p, int b, int hk, int seqlen_k_) {
+        const int esize = p->scale_dtype == 2 ? 4 : 2;
+        base = p->k_scale + (b * p->ks_sb + hk * p->ks_sh) * esize;
+        stride = (int)(p->ks_sn * esize);
+        dtype = p->scale_dtype;
         seqlen_k = seqlen_k_;
     }
+    __device__ __forceinline__ KScaleSource(const KParams& p, int b, int hk, int seqlen_k_) : KScaleSource(&p, b, hk, seqlen_k_) {}
     __device__ __forceinline__ uint32_t load(int key) const {
         key = key < seqlen_k ? key : seqlen_k - 1;
         const char* src = base + (int64_t)key * stride;

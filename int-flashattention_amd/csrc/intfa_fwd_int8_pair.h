@@ -19,7 +19,7 @@ namespace intfa {
 
 constexpr int kPairThreads = 512;
 
-template <bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK>
+template <bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK, bool RESIDENT>
 __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
     constexpr int D = 256;
@@ -35,7 +35,12 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     constexpr int OFF_XP = OFF_VS + (VBLK ? 2 * D * 4 : 0);   // packed P fragments: [wave][lane] x 16 bytes
     constexpr int OFF_K = (OFF_XP + 8 * 64 * 16 + 1023) & ~1023;
     constexpr int OFF_V = OFF_K + 2 * KT;
-    constexpr int LDS_BYTES = OFF_V + 2 * KT;
+    // several work items per workgroup (below): the next item's Q, and the part of the output staging that the last block's tiles have no room for
+    static_assert(!RESIDENT || (!SPLIT && !VBLK), "");
+    constexpr int OFF_Q = OFF_V + 2 * KT;
+    constexpr int OFF_ST = OFF_Q + (RESIDENT ? kBlockM * D : 0);
+    constexpr int LDS_BYTES = OFF_ST + 4 * OutStage<DVW>::BYTES;
+    static_assert(2 * OutStage<DVW>::BYTES == KT && LDS_BYTES <= 160 * 1024, "output staging");
     __shared__ __attribute__((aligned(1024))) char smem[LDS_BYTES];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -44,44 +49,43 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     const int hf = wave >> 2;                    // key sub-tile of the softmax work and column half of the output
     const int lq = lane & 31, lh = lane >> 5;
 
-    // ---- block -> (head, m-block, split): whole K/V heads per XCD (as in fwd_full_int8_kernel)
-    const int n_mblk = (p.seqlen + kBlockM - 1) / kBlockM;
-    const int n_split = SPLIT ? p.num_splits : 1;
-    const WorkgroupJob wg = deal_workgroup(p, blockIdx.x);
-    const int rem = wg.rem, head = wg.b * p.heads + wg.h;
-    const int mb_idx = fast_div(rem, p.d_n_split);
-    const int split = rem - mb_idx * n_split;
-    const int mb = CAUSAL ? n_mblk - 1 - mb_idx : mb_idx;       // heaviest query blocks first
-    const int b = wg.b, h = wg.h;
-    const int hk = wg.hk;
+    // ---- work item -> (head, m-block, split), key blocks: whole K/V heads per XCD (as in fwd_full_int8_kernel)
+    struct Item { int b, h, hk, mb, split, seqlen_k, nb_begin, nb_end; };
+    // (the arguments of a later item through an opaque copy of the block's address: they are loaded where they are used, and not held in
+    // scalar registers from the first item on)
+    auto locate = [&](auto args, int index, auto later_tag) __attribute__((always_inline)) -> Item {
+        const WorkgroupJob wg = deal_workgroup(args, index);
+        const int n_split = SPLIT ? args->num_splits : 1;
+        const int mb_idx = SPLIT ? fast_div(wg.rem, args->d_n_split) : wg.rem;
+        Item it;
+        it.split = wg.rem - mb_idx * n_split;
+        it.mb = CAUSAL ? (args->seqlen + kBlockM - 1) / kBlockM - 1 - mb_idx : mb_idx;       // heaviest query blocks first
+        it.b = wg.b; it.h = wg.h; it.hk = wg.hk;
+        it.seqlen_k = decltype(later_tag)::value ? args->seqlen_k : keys_of_batch(p, it.b);      // (several items per workgroup: one length for all)
+        // causal mask aligned to the bottom right corner: query row i sees keys 0 .. i + causal_off
+        const KeyBlocks kb = key_block_range<BN>(it.seqlen_k, CAUSAL, it.mb * kBlockM + kBlockM, it.seqlen_k - args->seqlen, SPLIT, n_split,
+                                                 it.split, CAUSAL, args->blocks_per_split);
+        it.nb_begin = kb.begin; it.nb_end = kb.end;
+        return it;
+    };
+    const int bid = block_after_kernargs();
+    Item it = locate(&p, bid, BoolTag<false>{});
+    // query row of this lane, clamped to the last one
+    auto row_of = [&](auto args, const Item& i) __attribute__((always_inline)) -> int {
+        const int r = i.mb * kBlockM + rw * 32 + lq, n = args->seqlen;
+        return r < n ? r : n - 1;
+    };
 
-    const int seqlen_k = keys_of_batch(p, b);
-    // causal mask aligned to the bottom right corner: query row i sees keys 0 .. i + causal_off
-    const int causal_off = seqlen_k - p.seqlen;
-    const KeyBlocks kb = key_block_range<BN>(seqlen_k, CAUSAL, mb * kBlockM + kBlockM, causal_off, SPLIT, n_split, split, CAUSAL,
-                                             p.blocks_per_split);
-    const int nb_total = kb.total, nb_begin = kb.begin, nb_end = kb.end;
-    const int q_row = mb * kBlockM + rw * 32 + lq;
-    const bool q_valid = q_row < p.seqlen;
-    const int q_ld = q_valid ? q_row : p.seqlen - 1;
-
-    // ---- Q fragment (B operand of S^T = K Q^T), resident
-    v4i qreg[KS];
-    load_q8_fragments<KS>(qreg, p, b, h, q_ld, lh);
-    const float qsc = load_q_scale_log2(p, b, h, q_ld);
-
-    float m_run = -INFINITY, l_run = 0.f;        // l_run: this wave's keys only
+    float m_run, l_run;                          // l_run: this wave's keys only
     float o_acc[DT][16];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o_acc[dt][r] = 0.f;
 
     // ---- global -> LDS copies: waves 0-3 the K tile, waves 4-7 the V tile (same geometry, other swizzle and source)
-    const char* Kg = p.k + b * p.k_sb + hk * p.k_sh;
-    const char* Vg = p.v + b * p.v_sb + hk * p.v_sh;
     const uint32_t t_sn = __builtin_amdgcn_readfirstlane((uint32_t)(hf ? p.v_sn : p.k_sn));
-    const v4i t_rsrc = make_rsrc(hf ? Vg : Kg, (uint32_t)((seqlen_k - 1) * (int64_t)t_sn + D));
+    auto tiles_of = [&](auto args, const Item& i) __attribute__((always_inline)) -> v4i {
+        const char* const base = hf ? args->v + i.b * args->v_sb + i.hk * args->v_sh : args->k + i.b * args->k_sb + i.hk * args->k_sh;
+        return make_rsrc(base, (uint32_t)((i.seqlen_k - 1) * (int64_t)t_sn + D));
+    };
+    v4i t_rsrc = tiles_of(&p, it);
     const auto k_lane = tile_load_lane<D, SWZ_K, BN>(t_sn, rw, lane);
     const auto v_lane = tile_load_lane<D, SWZ_V8, BN>(t_sn, rw, lane);
     TileLoadLane<D, SWZ_K, BN> t_lane;
@@ -89,11 +93,26 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     static_assert(TileLoadLane<D, SWZ_K, BN>::NV == 1 && TileLoadLane<D, SWZ_V8, BN>::NV == 1, "one lane offset per tile");
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     const uint32_t t_lds = lds0 + (hf ? OFF_V : OFF_K);
-    auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<D, SWZ_K, BN>(t_rsrc, (uint32_t)(nb * BN) * t_sn, t_sn, t_lds + buf * KT, rw, t_lane);
+    auto issue_loads = [&](const v4i& rsrc, int nb, int buf) __attribute__((always_inline)) {
+        const uint32_t off = __builtin_amdgcn_readfirstlane((nb * BN) * (int)t_sn), lds = __builtin_amdgcn_readfirstlane((int)(t_lds + buf * KT));
+        issue_tile_load<D, SWZ_K, BN>(rsrc, off, t_sn, lds, rw, t_lane);
+    };
+    // The first item's tiles ahead of its Q, which arrives under their way from HBM (as the argument lines, at once).
+    if (it.nb_begin < it.nb_end) issue_loads(t_rsrc, it.nb_begin, 0);
+    // ---- Q fragment (B operand of S^T = K Q^T), resident
+    v4i qreg[KS];
+    load_q8_fragments<KS>(qreg, p, it.b, it.h, row_of(&p, it), lh);
+    uint32_t q_scale_bits = load_q_scale_bits(p, it.b, it.h, row_of(&p, it));
+    // ... of the items after the first: 128 rows through LDS
+    auto issue_q = [&](const Item& i) __attribute__((always_inline)) {
+        const KernargPtr args = kernarg_block();
+        const uint32_t q_sn = (uint32_t)args->q_sn;
+        const int row0 = i.mb * kBlockM, rows = args->seqlen - row0;              // (rows past the last one: zeros)
+        const v4i rsrc = make_rsrc(args->q + i.b * args->q_sb + i.h * args->q_sh + (int64_t)row0 * args->q_sn, (uint32_t)((rows < kBlockM ? rows : kBlockM) - 1) * q_sn + D);
+        issue_tile_load<D, SWZ_K, kBlockM>(rsrc, 0, q_sn, lds0 + OFF_Q, rw, tile_load_lane<D, SWZ_K, kBlockM>(q_sn, rw, lane));
     };
     // k_scale of a block: thread t < 64 fetches the scale of key t; converted to fp32 when stored to LDS
-    const KScaleSource ks_src(p, b, hk, seqlen_k);
+    KScaleSource ks_src(&p, it.b, it.hk, it.seqlen_k);
     const int ks_key = tid & (BN - 1);
     auto load_ks = [&](int nb) __attribute__((always_inline)) -> uint32_t { return ks_src.load(nb * BN + ks_key); };   // raw bits
     auto cvt_ks = [&](uint32_t raw) __attribute__((always_inline)) -> float { return ks_src.cvt(raw); };
@@ -105,7 +124,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     const bool ks_wave = wave == 0;              // threads 0 .. 63: one k_scale each
     const int vs_c = tid - 256;
     const bool vs_thread = VBLK && hf == 1;      // threads 256 .. 511: one channel each
-    const float* Vsg = (const float*)p.v_scale + (b * p.vs_sb + hk * p.vs_sh + (vs_thread ? vs_c : 0));
+    const float* Vsg = (const float*)p.v_scale + (it.b * p.vs_sb + it.hk * p.vs_sh + (vs_thread ? vs_c : 0));
     auto load_vs = [&](int nb) __attribute__((always_inline)) -> float {
         if (!VBLK) return 0.f;
         const int row = p.vs_g == 1 ? nb : nb / p.vs_g;
@@ -142,11 +161,6 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     // S^T accumulators of the block that is processed next (this wave's sub-tile): the MFMA chain of block nb+1 runs
     // under the accumulator update of block nb.
     v16i sacc;
-    auto qk_loadfrags = [&](auto buf_tag, v4i (&fr)[KS]) __attribute__((always_inline)) {
-        constexpr int KB = decltype(buf_tag)::value ? KT : 0;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) fr[ks] = *(const v4i*)(smem + (k_rd(ks) + KB));
-    };
     uint32_t ks_next = 0;                        // raw k_scale of the next block (threads < 64)
     float vs_pend = 0.f;                         // VBLK: channel scale of the current block, not yet in LDS (threads >= 256)
 
@@ -156,13 +170,34 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     //   B2 publishes the row maxima (and this block's V tile and channel scales),
     //   B3 publishes the packed P (and the next block's K tile and k_scale).
     // On entry the K tile and k_scale of this block are visible and `sacc` holds this wave's S^T sub-tile.
-    auto compute = [&](auto buf_tag, int nb) __attribute__((always_inline)) {
-        constexpr int BUF = decltype(buf_tag)::value ? 1 : 0;
-        constexpr int VB = BUF * KT, SB = BUF * BN * 4;
-        // last visible key relative to the block: smallest of the wave (uniform), and the lane's
-        const int lim_lo = CAUSAL ? mb * kBlockM + rw * 32 + causal_off - nb * BN : seqlen_k - 1 - nb * BN;
+    // In the place of a next block's tiles an item's last block requests the first ones of the item `nx`, if has_next.
+    bool has_next = false, v_here = false;       // v_here: this block's V tile was awaited with the K tile
+    Item nx = it;
+    int q_block = -1;                            // the block that requests the next item's Q
+    float qsc = 0.f;
+    uint32_t v_scale_bits = 0;
+    // (LAST: the item's last block, one instance for both buffers.  The others have no run-time test that their place in the item would answer: the
+    // two waves of a SIMD meet at the barriers, so what a scalar branch takes - some twenty of them 12 % of a block - runs under nothing.)
+    auto compute = [&](auto last_tag, const int BUF, int nb) __attribute__((always_inline)) {
+        constexpr bool LAST = RESIDENT && decltype(last_tag)::value, MAYBE_LAST = !RESIDENT;
+        const bool more = MAYBE_LAST ? nb + 1 < it.nb_end : !LAST;
+        const int VB = BUF * KT, SB = BUF * BN * 4;
+        // last visible key relative to the block: smallest of the wave (uniform); the lane's, relative to its first key
+        const int lim_lo = CAUSAL ? it.mb * kBlockM + rw * 32 + it.seqlen_k - p.seqlen - nb * BN : it.seqlen_k - 1 - nb * BN;
         const int lim = CAUSAL ? lim_lo + lq : lim_lo;
-        const bool more = nb + 1 < nb_end;
+        int past = lim - 32 * hf - 4 * lh;
+        if (RESIDENT && (CAUSAL || LAST)) asm volatile("" : "+v"(past));     // (opaque: 16 thresholds would be computed ahead of the loop)
+        const bool request = more || (RESIDENT && has_next);
+        const int nb_next = LAST ? nx.nb_begin : nb + 1;
+        if (LAST) {
+            const KernargPtr args = kernarg_block();
+            if (has_next) {
+                t_rsrc = tiles_of(args, nx);
+                ks_src = KScaleSource(args, nx.b, nx.hk, nx.seqlen_k);
+                q_scale_bits = load_scale_bits(args->q_scale, nx.b * args->qs_sb + nx.h * args->qs_sh + (int64_t)row_of(args, nx) * args->qs_sn, args->scale_dtype);
+            }
+            v_scale_bits = load_scale_bits(args->v_scale, it.b * args->vs_sb + it.hk * args->vs_sh, args->scale_dtype);
+        }
         auto load_vfrag = [&](uint32_t sub, int dt) __attribute__((always_inline)) -> v4i {
             const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
                 (__attribute__((address_space(3))) v2i*)INTFA_LDS(smem + v_rd[dt] + VB + sub));
@@ -171,9 +206,9 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
             return (v4i){lo[0], lo[1], hi[0], hi[1]};
         };
         // the K tile of the next block goes into the other buffer (last read one block ago)
-        if (more && hf == 0) {
-            issue_loads(nb + 1, BUF ^ 1);
-            ks_next = load_ks(nb + 1);
+        if (request && hf == 0) {
+            issue_loads(t_rsrc, nb_next, BUF ^ 1);
+            ks_next = load_ks(nb_next);
         }
         // -------- pass 1: dequantise this wave's S^T sub-tile by k_scale, row maximum
         v4f kk[4];
@@ -186,10 +221,12 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
             float xq[4];
 #pragma unroll
             for (int b4 = 0; b4 < 4; ++b4) xq[b4] = (float)sacc[4 * a4 + b4] * kk[a4][b4];
-            if (32 * hf + 31 > lim_lo) {                       // wave-uniform: some lane of the wave has a hidden key here
+            if ((CAUSAL || LAST || MAYBE_LAST) && 32 * hf + 31 > lim_lo) {   // wave-uniform: some lane of the wave has a hidden key here
 #pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4)
-                    if ((32 * hf + 8 * a4 + b4 + 4 * lh) > lim) xq[b4] = -INFINITY;
+                for (int b4 = 0; b4 < 4; ++b4) {
+                    if (RESIDENT) xq[b4] = hide_past(xq[b4], past, 8 * a4 + b4);
+                    else if (32 * hf + 8 * a4 + b4 + 4 * lh > lim) xq[b4] = -INFINITY;
+                }
             }
 #pragma unroll
             for (int b4 = 0; b4 < 4; ++b4) {
@@ -200,13 +237,14 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         mx = half_pair_max(mx);
         *(float*)(smem + xm_wr) = mx;
         if (hf == 1) {                           // this block's V tile (requested one block ago) and channel scales
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (!RESIDENT || !v_here) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (VBLK) *(float*)(smem + vs_wr + BUF * D * 4) = vs_pend;
         }
         __syncthreads();                         // ---- B2
-        if (more && hf == 1) {                   // the other V buffer was last read before this barrier
-            issue_loads(nb + 1, BUF ^ 1);
+        if (request && hf == 1) {                // the other V buffer was last read before this barrier
+            issue_loads(t_rsrc, nb_next, BUF ^ 1);
             if (VBLK) vs_pend = load_vs(nb + 1);
+            if (RESIDENT && nb == q_block) issue_q(nx);              // a block ahead of the last one (every wave has read this item's Q, and these wait next in a block's time)
         }
         mx = fmaxf(mx, *(const float*)(smem + xm_rd));
         v4i vfo[2], vfp[2];
@@ -249,15 +287,15 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vfo[0], p8o, (v16i){0}, 0, 0, 0);
         vfo[1] = load_vfrag(v_own, 1);
         vfp[1] = load_vfrag(v_oth, 1);
-        if (hf == 0) {                           // the next block's K tile and k_scale
+        if (more && hf == 0) {                   // the next block's K tile and k_scale
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            if (more && ks_wave) *(float*)(smem + ks_wr + (BUF ^ 1) * BN * 4) = cvt_ks(ks_next);
+            if (ks_wave) *(float*)(smem + ks_wr + (BUF ^ 1) * BN * 4) = cvt_ks(ks_next);
         }
         __syncthreads();                         // ---- B3
         const v4i p8p = *(const v4i*)(smem + xp_rd);
         // K fragments of the next block (other buffer), four in flight: k-steps 2dt, 2dt+1 are consumed in stage dt and
         // their registers refilled with k-steps 2dt+4, 2dt+5
-        constexpr int KBN = (BUF ^ 1) * KT;
+        const int KBN = (BUF ^ 1) * KT;
         v4i fr[4];
         if (more) {
 #pragma unroll
@@ -266,7 +304,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         oacc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vfp[0], p8p, oacc[0], 0, 0, 0);
         // -------- P V: O^T[d, q] += V^T[d, key] P^T[key, q]; the chain of d-tile dt+1 and a quarter of the next block's
         // Q K^T chain are issued before the accumulator update of d-tile dt
-        constexpr int VSB = BUF * D * 4;
+        const int VSB = BUF * D * 4;
         v4f vsc[4];
         auto load_vsc = [&](int dt) __attribute__((always_inline)) {
 #pragma unroll
@@ -307,51 +345,99 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         l_run = fmaf(l_run, alpha, lsum);
     };
 
-    if (nb_begin < nb_end) {
-        // prologue: K tile, V tile, k_scale and channel scales of the first block; its Q K^T chain
-        issue_loads(nb_begin, 0);
-        {
-            const uint32_t s0 = load_ks(nb_begin);
-            if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(s0);
-            if (vs_thread) vs_pend = load_vs(nb_begin);
-        }
+    // ---- Work items of this workgroup.  One while all of the launch's workgroups are resident; with more items (RESIDENT) one workgroup per compute
+    // unit takes every grid-th, in the order in which the hardware would deal them (causal: every second round backwards, so that the sums of
+    // the lengths agree).  What it is for: a workgroup fills its compute unit, and nothing ran under its first loads and its last stores (20 % of the time
+    // at 1024 keys).  So an item's last block requests the next one's first tiles, the block before it Q (into the LDS), and nothing waits for the
+    // stores.  us, one item per workgroup -> this: B16 H16 N1024 bf16 268 -> 244, causal 172 -> 161, B4 H32 N4096 1679 -> 1590, B16 H32/4 N200
+    // 49.9 -> 46.4; what bounds it then is the loop over the key blocks.  Launches of one round lose 5 % in the longer code: they run the other form.
+    int buf = 0;                                 // LDS buffer of the item's first block, then of its last
+    int round = 0;
+    if (it.nb_begin < it.nb_end) {
+        const uint32_t s0 = load_ks(it.nb_begin);
+        if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(s0);
+        if (vs_thread) vs_pend = load_vs(it.nb_begin);
+        qsc = q_scale_log2(p, q_scale_bits);
         if (hf == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        {
-            v4i fr[KS];
-            qk_loadfrags(BoolTag<false>{}, fr);
-            sacc = (v16i){0};
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[ks], qreg[ks], sacc, 0, 0, 0);
-        }
-        int nb = nb_begin;
-        while (true) {
-            if (nb >= nb_end) break;
-            compute(BoolTag<false>{}, nb++);
-            if (nb >= nb_end) break;
-            compute(BoolTag<true>{}, nb++);
-        }
     }
+    q_has_arrived(qreg);                         // (outside the branch: see there)
+    while (true) {
+        m_run = -INFINITY; l_run = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o_acc[dt][r] = 0.f;
+        if (RESIDENT) {
+            const KernargPtr args = kernarg_block();
+            const int grid = args->grid_wgs;
+            ++round;
+            const int index = round * grid + (CAUSAL && (round & 1) ? grid - 8 - (bid & ~7) + (bid & 7) : bid);
+            has_next = index < args->items;
+            q_block = -1;
+            if (has_next) {
+                nx = locate(args, index, BoolTag<true>{});
+                q_block = it.nb_end - 2 > it.nb_begin ? it.nb_end - 2 : it.nb_begin;
+            }
+        }
+        if (it.nb_begin < it.nb_end) {
+            {
+                v4i fr[KS];
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) fr[ks] = *(const v4i*)(smem + (k_rd(ks) + buf * KT));
+                sacc = (v16i){0};
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[ks], qreg[ks], sacc, 0, 0, 0);
+            }
+            int nb = it.nb_begin;
+            if (RESIDENT) {
+                const int last = it.nb_end - 1;
+                while (true) {
+                    if (buf == 0) {
+                        if (nb >= last) break;
+                        compute(BoolTag<false>{}, 0, nb++);
+                        v_here = false;
+                    }
+                    buf = 1;
+                    if (nb >= last) break;
+                    compute(BoolTag<false>{}, 1, nb++);
+                    v_here = false;
+                    buf = 0;
+                }
+                compute(BoolTag<true>{}, buf, nb);
+            } else {
+                while (true) {
+                    if (nb >= it.nb_end) break;
+                    compute(BoolTag<false>{}, 0, nb++);
+                    if (nb >= it.nb_end) break;
+                    compute(BoolTag<false>{}, 1, nb++);
+                }
+            }
+        }
 
     // ---- epilogue
     const KernargPtr pe = kernarg_block();
     const int e_heads = pe->heads, e_seqlen = pe->seqlen;
-    const int eb = fast_div(head, pe->d_heads), eh = head - eb * e_heads;
+    const int eb = it.b, eh = it.h;
+    const int q_row = it.mb * kBlockM + rw * 32 + lq;
+    const bool q_valid = q_row < e_seqlen;
     // row sum: this wave's keys plus the partner's (the last block's barriers lie between the last use of the exchange
     // slots and this one)
     float l_tot = half_pair_sum(l_run);          // in units of 1/127 when PROUND == 0
     *(float*)(smem + xm_wr) = l_tot;
     __syncthreads();
     l_tot += *(const float*)(smem + xm_rd);
-    const float vs = VBLK ? 1.f : load_scale(pe->v_scale, eb * pe->vs_sb + fast_div(eh, pe->d_kv_group) * pe->vs_sh, pe->scale_dtype);
+    if (!RESIDENT && !VBLK) v_scale_bits = load_scale_bits(pe->v_scale, eb * pe->vs_sb + it.hk * pe->vs_sh, pe->scale_dtype);
+    asm volatile("" : "+v"(v_scale_bits));       // (arrived here on every way: a load that the compiler takes for pending in the next item makes it wait there)
+    const float vs = VBLK ? 1.f : cvt_scale_bits(v_scale_bits, pe->scale_dtype);
     // (a row without a visible key gives zeros and lse = -inf; its accumulators hold NaN from exp2(-inf - -inf), hence
     // the selects)
-    const bool any_key = nb_begin < nb_end && m_run > -INFINITY;
+    const bool any_key = it.nb_begin < it.nb_end && m_run > -INFINITY;
     const float out_scale = !any_key ? 0.f : (PROUND == 0) ? (vs / l_tot) : (vs / (127.f * l_tot));
     const float l_true = (PROUND == 0) ? l_tot * (1.f / 127.f) : l_tot;
     const float lse = any_key ? m_run + __builtin_log2f(l_true) : -INFINITY;
     if (SPLIT) {
-        const int64_t row = ((int64_t)(split * pe->batch + eb) * e_heads + eh) * e_seqlen + q_row;
+        const int64_t row = ((int64_t)(it.split * pe->batch + eb) * e_heads + eh) * e_seqlen + q_row;
         float* op = pe->o_part + row * D + hf * DVW;
         if (q_valid) {
 #pragma unroll
@@ -368,15 +454,21 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         return;
     }
     {
-    // 16-bit rows go out through LDS (whole lines per store instruction), staged in the tile memory: every wave has
-    // passed the barrier of the row-sum exchange, so no tile is read any more
-    static_assert(OFF_K + 8 * OutStage<DVW>::BYTES <= LDS_BYTES, "output staging fits the tile memory");
+    // the next item's first tiles, k_scale and Q have arrived (ahead of the stores: nothing waits for those)
+    if (RESIDENT && has_next) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("" : "+v"(q_scale_bits));
+        if (ks_wave) *(float*)(smem + ks_wr + (buf ^ 1) * BN * 4) = cvt_ks(ks_next);
+    }
+    // 16-bit rows go out through LDS (whole lines per store instruction): waves 0-3 through the last block's tiles (every wave has
+    // passed the barrier of the row-sum exchange, so none of them is read any more)
     // (an opaque copy of the lane index: the staging addresses depend on the lane only and would otherwise be computed
     // ahead of the main loop and held in registers through it)
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     const int lq_e = lane_e & 31, lh_e = lane_e >> 5;
-    char* stage = smem + OFF_K + wave * OutStage<DVW>::BYTES;
+    constexpr int OSB = OutStage<DVW>::BYTES;
+    char* const stage = smem + (wave < 2 ? OFF_K + buf * KT + wave * OSB : wave < 4 ? OFF_V + buf * KT + (wave - 2) * OSB : OFF_ST + (wave - 4) * OSB);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -394,10 +486,20 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
                 out_stage_put<DVW>(stage, lq_e, d0, __builtin_bit_cast(v2i, o));
             }
         }
-    const int row0 = mb * kBlockM + rw * 32;
+    const int row0 = it.mb * kBlockM + rw * 32;
     out_stage_flush<DVW>(stage, pe->out + eb * pe->o_sb + eh * pe->o_sh + (int64_t)row0 * pe->o_sn + hf * DVW * 2, pe->o_sn,
                          e_seqlen - row0, lane_e);
     if (q_valid && pe->lse != nullptr && lh == 0 && hf == 0) pe->lse[((int64_t)eb * e_heads + eh) * e_seqlen + q_row] = lse;
+    }
+    if (!RESIDENT || !has_next) return;
+    __syncthreads();
+    const uint32_t q_rd0 = OFF_Q + (32 * rw + lq) * D + ((lh ^ k_swz) << 4);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qreg[ks] = *(const v4i*)(smem + (q_rd0 ^ (uint32_t)(32 * ks)));
+    qsc = q_scale_log2(p, q_scale_bits);
+    it = nx;
+    buf ^= 1;
+    v_here = true;
     }
 #endif  // __HIP_DEVICE_COMPILE__
 }

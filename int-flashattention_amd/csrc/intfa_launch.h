@@ -36,6 +36,7 @@ inline FastDiv make_fast_div(int d) {
 inline KParams finish_mapping(const KParams& kp, int grid) {
     KParams k = kp;
     const int n_split = kp.num_splits > 1 ? kp.num_splits : 1;
+    k.items = k.grid_wgs = grid;
     k.per_head = grid / (kp.batch * kp.heads);
     k.heads_kv = kp.heads / kp.kv_group;
     const int per_kv = k.per_head * kp.kv_group, units = kp.batch * k.heads_kv;
@@ -72,6 +73,20 @@ inline KParams finish_mapping(const KParams& kp, int grid) {
 template <typename K> inline int launch_kernel(K kernel, const KParams& kp, hipStream_t stream, int threads = kThreads) {
     const int grid = kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM) * kp.num_splits;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, finish_mapping(kp, grid));
+    return (int)hipGetLastError();
+}
+// The same work items for `slots` workgroups (a multiple of kXcds), which take every slots-th each, where there are more items than that.
+// Not for batches of different lengths (the items of a workgroup would differ in work; the hardware deals single ones as compute units
+// become free), for items that may have no key, or for query rows further apart than a copy's offsets reach.
+inline bool takes_resident(const KParams& kp, int slots) {
+    const int64_t items = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM);
+    return items > slots && kp.num_splits <= 1 && kp.seqlens_k == nullptr && kp.seqlen_k > 0 && !(kp.causal && kp.seqlen_k < kp.seqlen) &&
+           kp.q_sn < (1ll << 31) / kBlockM;
+}
+template <typename K> inline int launch_resident(K kernel, const KParams& kp, hipStream_t stream, int threads, int slots) {
+    KParams k = finish_mapping(kp, kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM));
+    k.grid_wgs = slots;
+    hipLaunchKernelGGL(kernel, dim3(slots), dim3(threads), 0, stream, k);
     return (int)hipGetLastError();
 }
 

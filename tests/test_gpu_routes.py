@@ -20,6 +20,8 @@ CASES = [
     ("full", 128, PAST, N, True, {}, "fwd_full_int8_kernel<128, true"),
     ("full", 128, PAST - 1, N, True, {}, "fwd_decode_full_int8_kernel<128"),
     ("full", 256, PAST, N, False, {}, "fwd_full_int8_pair_kernel<false"),
+    ("full", 256, 129, N, False, {}, "fwd_full_int8_pair_kernel<false, 0, 1, false, false, true"),       # 258 query blocks: several per workgroup
+    ("full", 256, 128, N, False, {}, "fwd_full_int8_pair_kernel<false, 0, 1, false, false, false"),
     ("full", 256, PAST // 2, N, False, {}, "fwd_decode_full_int8_kernel<256"),
     ("full", 128, PAST, N, True, dict(v_block=128), "fwd_full_int8_kernel<128, true"),
     ("full", 128, 1, N, True, dict(v_block=64), "fwd_full_int8_kernel<128, true"),

@@ -211,14 +211,15 @@ __device__ __forceinline__ WorkgroupJob deal_workgroup(const KParams& p, int bid
 
 // Number of keys of batch entry b: one length for all, or per batch (a cache filled to different lengths), clamped to
 // [0, seqlen_k] so that rows past the allocation are never addressed.
-__device__ __forceinline__ int keys_of_batch(const KParams& p, int b) {
-    int seqlen_k = p.seqlen_k;
-    if (p.seqlens_k != nullptr) {
-        const int n = p.seqlens_k[b];
+template <typename Args> __device__ __forceinline__ int keys_of_batch(Args p, int b) {
+    int seqlen_k = p->seqlen_k;
+    if (p->seqlens_k != nullptr) {
+        const int n = p->seqlens_k[b];
         seqlen_k = n < 0 ? 0 : (n < seqlen_k ? n : seqlen_k);
     }
     return seqlen_k;
 }
+__device__ __forceinline__ int keys_of_batch(const KParams& p, int b) { return keys_of_batch(&p, b); }
 
 // Key blocks [begin, end) of BN keys that a workgroup visits.  `visible_end` is the end of the range before a split
 // narrows it (the blocks that hold a key visible to some row of the workgroup).
@@ -247,6 +248,34 @@ __device__ __forceinline__ KeyBlocks key_block_range(int seqlen_k, bool causal, 
         r.end = e < r.end ? e : r.end;
     }
     return r;
+}
+
+// A work item of the general kernels: 128 query rows of one (batch, head), and the key blocks of them (or of one split).
+// LATER: an item after a workgroup's first one (launch_resident in intfa_launch.h: all batch entries have the same length there).  Its
+// arguments come through an opaque copy of the block's address (Args: KernargPtr), so that they are loaded where they are used and not held in scalar
+// registers from the first item on.
+struct WorkItem { int b, h, hk, mb, split, seqlen_k, nb_begin, nb_end; };
+template <int BN, bool CAUSAL, bool SPLIT, bool LATER, typename Args>
+__device__ __forceinline__ WorkItem locate_item(Args args, int index) {
+    const WorkgroupJob wg = deal_workgroup(args, index);
+    const int n_split = SPLIT ? args->num_splits : 1;
+    const int mb_idx = SPLIT ? fast_div(wg.rem, args->d_n_split) : wg.rem;
+    WorkItem it;
+    it.split = wg.rem - mb_idx * n_split;
+    it.mb = CAUSAL ? (args->seqlen + kBlockM - 1) / kBlockM - 1 - mb_idx : mb_idx;       // heaviest query blocks first
+    it.b = wg.b; it.h = wg.h; it.hk = wg.hk;
+    it.seqlen_k = LATER ? args->seqlen_k : keys_of_batch(args, it.b);
+    // causal mask aligned to the bottom right corner: query row i sees keys 0 .. i + (seqlen_k - seqlen)
+    const KeyBlocks kb = key_block_range<BN>(it.seqlen_k, CAUSAL, it.mb * kBlockM + kBlockM, it.seqlen_k - args->seqlen, SPLIT, n_split,
+                                             it.split, CAUSAL, args->blocks_per_split);
+    it.nb_begin = kb.begin; it.nb_end = kb.end;
+    return it;
+}
+// Index of a workgroup's item of the given round (0: its first one), or one past the last item where it has none: every grid-th, and causal
+// every second round backwards (the lengths of two rounds then add up to the same in every workgroup).
+template <bool CAUSAL> __device__ __forceinline__ int item_of_round(KernargPtr args, int bid, int round) {
+    const int grid = args->grid_wgs;
+    return round * grid + (CAUSAL && (round & 1) ? grid - 8 - (bid & ~7) + (bid & 7) : bid);      // (bid & 7: the XCD)
 }
 
 // int8 Q fragments of query row q_ld (B operand of S^T = K Q^T): 16 bytes per k-step of 32, the half lh of the lane.
@@ -462,6 +491,19 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 __device__ __forceinline__ float hide_past(float v, int last, int k_r) {
     const uint32_t t = (uint32_t)(last - k_r);
     return __builtin_fminf(v, __builtin_bit_cast(float, (t & 0x80000000u) | 0x7f800000u));
+}
+// The same for a lane's many keys of a masked block (the general kernels): bit j of hidden_past(last) says that key j of a run of 32 lies past the
+// lane's last visible one (`last` may lie before the run or past it), and hide(v, bits, j) is v or -inf by that bit, the bit spread over a
+// word and a bitwise select: three instructions where the minimum above takes seven with what the compiler puts around it.  us, causal,
+// before -> after: half-int8 d128 B8 H32 N2048 301 -> 296, B4 H12 N1500 38.3 -> 37.4, fp16 B8 H32 N1024 93.8 -> 92.2, full-int8 B8 H32/8 N1024 74.5 -> 73.5.
+__device__ __forceinline__ uint32_t hidden_past(int last) {
+    const int n = last + 1;
+    return (uint32_t)(0xffffffffull << (n < 0 ? 0 : n > 32 ? 32 : n));
+}
+__device__ __forceinline__ float hide(float v, uint32_t bits, int j) {
+    uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)bits, (unsigned)j, 1u);
+    asm("" : "+v"(m));               // (opaque: else a compare and a select of it)
+    return __builtin_bit_cast(float, (m & 0xff800000u) | (~m & __builtin_bit_cast(uint32_t, v)));
 }
 
 // The reference's requantisation of P (flash_atten_full_int8.py:49-51) for the 16 probabilities a lane holds of one 32-key

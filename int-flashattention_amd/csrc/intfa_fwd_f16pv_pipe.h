@@ -287,12 +287,14 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
             const int last = (CAUSAL ? lim_lo + lq : lim_lo) - 4 * lh;
             mx = -INFINITY;
 #pragma unroll
-            for (int st = 0; st < NST; ++st)
+            for (int st = 0; st < NST; ++st) {
+                const uint32_t hidden = hidden_past(last - 32 * st);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    s[PAR][st][r] = hide_past(s[PAR][st][r], last, 32 * st + 8 * (r >> 2) + (r & 3));
+                    s[PAR][st][r] = hide(s[PAR][st][r], hidden, 8 * (r >> 2) + (r & 3));
                     mx = fmaxf(mx, s[PAR][st][r]);
                 }
+            }
         }
         // The exponent's reference point ("frame") follows the running maximum lazily: it moves, and the output and the row
         // sum are rescaled as the reference does in every block (flash_atten_int8.py:48-52), only when some row's block
@@ -323,6 +325,7 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
 #pragma clang fp contract(off)
             l_run += lsum;
         }
+        if (QK_INT8 && decltype(qk_tag)::value) asm volatile("" : "+v"(ks_next));      // (taken for arrived on every way, also where it is not stored)
         if (more) store_ks(ks_next, PAR);
     };
     constexpr BoolTag<false> F{};

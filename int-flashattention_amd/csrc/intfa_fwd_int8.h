@@ -262,6 +262,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             if (st + 2 < nact) load_kfrags(fr[st & 1], st + 2);
             if (!DUMP_S && !DIAG) issue_k_slice(k_next, nb + 1, buf ^ 1, st, NST);
             if (DUMP_S) wait_for_product(sacc[st & 1]);
+            const uint32_t hidden = DIAG ? hidden_past(last - 32 * st) : 0u;
             const v16i& acc = sacc[st & 1];
             v16i& nacc = sacc[(st + 1) & 1];
             if (DUMP_S) {
@@ -290,7 +291,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
                 if (next) load_kk(a4, st + 1);
                 if (DIAG && (st + 2 >= nact || VBLK == 2)) {
 #pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4) xq[b4] = hide_past(xq[b4], last, 32 * st + 8 * a4 + b4);
+                    for (int b4 = 0; b4 < 4; ++b4) xq[b4] = hide(xq[b4], hidden, 8 * a4 + b4);
                 }
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) {

@@ -50,28 +50,10 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     const int lq = lane & 31, lh = lane >> 5;
 
     // ---- work item -> (head, m-block, split), key blocks: whole K/V heads per XCD (as in fwd_full_int8_kernel)
-    struct Item { int b, h, hk, mb, split, seqlen_k, nb_begin, nb_end; };
-    // (the arguments of a later item through an opaque copy of the block's address: they are loaded where they are used, and not held in
-    // scalar registers from the first item on)
-    auto locate = [&](auto args, int index, auto later_tag) __attribute__((always_inline)) -> Item {
-        const WorkgroupJob wg = deal_workgroup(args, index);
-        const int n_split = SPLIT ? args->num_splits : 1;
-        const int mb_idx = SPLIT ? fast_div(wg.rem, args->d_n_split) : wg.rem;
-        Item it;
-        it.split = wg.rem - mb_idx * n_split;
-        it.mb = CAUSAL ? (args->seqlen + kBlockM - 1) / kBlockM - 1 - mb_idx : mb_idx;       // heaviest query blocks first
-        it.b = wg.b; it.h = wg.h; it.hk = wg.hk;
-        it.seqlen_k = decltype(later_tag)::value ? args->seqlen_k : keys_of_batch(p, it.b);      // (several items per workgroup: one length for all)
-        // causal mask aligned to the bottom right corner: query row i sees keys 0 .. i + causal_off
-        const KeyBlocks kb = key_block_range<BN>(it.seqlen_k, CAUSAL, it.mb * kBlockM + kBlockM, it.seqlen_k - args->seqlen, SPLIT, n_split,
-                                                 it.split, CAUSAL, args->blocks_per_split);
-        it.nb_begin = kb.begin; it.nb_end = kb.end;
-        return it;
-    };
     const int bid = block_after_kernargs();
-    Item it = locate(&p, bid, BoolTag<false>{});
+    WorkItem it = locate_item<BN, CAUSAL, SPLIT, false>(&p, bid);
     // query row of this lane, clamped to the last one
-    auto row_of = [&](auto args, const Item& i) __attribute__((always_inline)) -> int {
+    auto row_of = [&](auto args, const WorkItem& i) __attribute__((always_inline)) -> int {
         const int r = i.mb * kBlockM + rw * 32 + lq, n = args->seqlen;
         return r < n ? r : n - 1;
     };
@@ -81,7 +63,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
 
     // ---- global -> LDS copies: waves 0-3 the K tile, waves 4-7 the V tile (same geometry, other swizzle and source)
     const uint32_t t_sn = __builtin_amdgcn_readfirstlane((uint32_t)(hf ? p.v_sn : p.k_sn));
-    auto tiles_of = [&](auto args, const Item& i) __attribute__((always_inline)) -> v4i {
+    auto tiles_of = [&](auto args, const WorkItem& i) __attribute__((always_inline)) -> v4i {
         const char* const base = hf ? args->v + i.b * args->v_sb + i.hk * args->v_sh : args->k + i.b * args->k_sb + i.hk * args->k_sh;
         return make_rsrc(base, (uint32_t)((i.seqlen_k - 1) * (int64_t)t_sn + D));
     };
@@ -104,7 +86,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     load_q8_fragments<KS>(qreg, p, it.b, it.h, row_of(&p, it), lh);
     uint32_t q_scale_bits = load_q_scale_bits(p, it.b, it.h, row_of(&p, it));
     // ... of the items after the first: 128 rows through LDS
-    auto issue_q = [&](const Item& i) __attribute__((always_inline)) {
+    auto issue_q = [&](const WorkItem& i) __attribute__((always_inline)) {
         const KernargPtr args = kernarg_block();
         const uint32_t q_sn = (uint32_t)args->q_sn;
         const int row0 = i.mb * kBlockM, rows = args->seqlen - row0;              // (rows past the last one: zeros)
@@ -172,7 +154,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     // On entry the K tile and k_scale of this block are visible and `sacc` holds this wave's S^T sub-tile.
     // In the place of a next block's tiles an item's last block requests the first ones of the item `nx`, if has_next.
     bool has_next = false, v_here = false;       // v_here: this block's V tile was awaited with the K tile
-    Item nx = it;
+    WorkItem nx = it;
     int q_block = -1;                            // the block that requests the next item's Q
     float qsc = 0.f;
     uint32_t v_scale_bits = 0;
@@ -214,6 +196,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         v4f kk[4];
 #pragma unroll
         for (int a4 = 0; a4 < 4; ++a4) kk[a4] = *(const v4f*)(smem + ks_rd + SB + 32 * a4);
+        const uint32_t hidden = RESIDENT && (CAUSAL || LAST) ? hidden_past(past) : 0u;
         float t[16];
         float mx = -INFINITY;
 #pragma unroll
@@ -224,7 +207,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
             if ((CAUSAL || LAST || MAYBE_LAST) && 32 * hf + 31 > lim_lo) {   // wave-uniform: some lane of the wave has a hidden key here
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) {
-                    if (RESIDENT) xq[b4] = hide_past(xq[b4], past, 8 * a4 + b4);
+                    if (RESIDENT) xq[b4] = hide(xq[b4], hidden, 8 * a4 + b4);
                     else if (32 * hf + 8 * a4 + b4 + 4 * lh > lim) xq[b4] = -INFINITY;
                 }
             }
@@ -370,13 +353,11 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
             for (int r = 0; r < 16; ++r) o_acc[dt][r] = 0.f;
         if (RESIDENT) {
             const KernargPtr args = kernarg_block();
-            const int grid = args->grid_wgs;
-            ++round;
-            const int index = round * grid + (CAUSAL && (round & 1) ? grid - 8 - (bid & ~7) + (bid & 7) : bid);
+            const int index = item_of_round<CAUSAL>(args, bid, ++round);
             has_next = index < args->items;
             q_block = -1;
             if (has_next) {
-                nx = locate(args, index, BoolTag<true>{});
+                nx = locate_item<BN, CAUSAL, SPLIT, true>(args, index);
                 q_block = it.nb_end - 2 > it.nb_begin ? it.nb_end - 2 : it.nb_begin;
             }
         }

@@ -326,6 +326,20 @@ struct KScaleSource {
     }
 };
 
+// The k_scales of a lane's 16 keys of a sub-tile in ONE register: lane i of each row of 16 lanes holds the scale of the lane's i-th key (key
+// 8 (i / 4) + 4 lh + i % 4), and a multiplication takes any of them for the whole row with the DPP modifier row_newbcast, at no instruction of its
+// own.  (Read as quads of a broadcast address they are a quarter of the wave's LDS reads, of which the CU does one per 3 ns whatever it brings.)
+__device__ __forceinline__ uint32_t scale_lane_key(int lane) { return (uint32_t)(8 * ((lane & 15) >> 2) + 4 * (lane >> 5) + (lane & 3)); }
+// c += f * (the scale of the lane's i-th key).  (Reads f like any hand-written instruction: mfma_check.py.)
+__device__ __forceinline__ void fmac_lane_scale(float& c, float scales, int f, int i) {
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(c) : "v"(scales), "v"(f), "i"(i));
+}
+// Int32 scores as fp32 numbers without a conversion: a product chain that starts from the bits of 1.5 * 2^23 instead of zero ends in the bits of
+// 1.5 * 2^23 + S (|S| <= 2^22).  With kScoreBias * k_scale subtracted by the multiplication with k_scale, a score takes one instruction instead of two,
+// to the same bits: the product is exact inside it, and kScoreBias * k_scale is exact for 16-bit scales (at most 11 + 2 significant bits).
+constexpr int kScoreSeed = 0x4B400000;
+constexpr float kScoreBias = 12582912.f;
+
 // ---- LDS swizzles.  A tile row is ROW_BYTES bytes; its 16-byte chunks are XOR-permuted with a function of the
 // row so that the rows touched together by one LDS access cycle (64 banks x 4 bytes = 256 bytes: 16 lanes of a
 // 16-byte read, 32 lanes of an 8-byte read) fall into different bank groups.  Every function depends on the low

@@ -24,7 +24,7 @@ template <int D> struct FullInt8Geom {
     static constexpr int NST = D == 128 ? 4 : 2;
     static constexpr int BN = 32 * NST;
     // occupancy the register budget is held to (a workgroup puts one wave on each SIMD: workgroups per compute unit)
-    static constexpr int waves_per_simd(bool causal, int vblk) { return D == 64 ? (causal || vblk ? 3 : 4) : 2; }
+    static constexpr int waves_per_simd(bool causal, int vblk, bool fold) { return D == 64 ? (causal || vblk || fold ? 3 : 4) : 2; }
 };
 
 // VBLK != 0: V carries one scale per key block and channel (layout of the reference's CUDA kernel,
@@ -34,8 +34,13 @@ template <int D> struct FullInt8Geom {
 // CUDA kernel (kBlockN = 64 at head_dim 128, csrc/flash_fwd_launch_template.h:514-519): the softmax still advances per
 // 128-key block (the running maximum and P8 are those of intfa_fwd_block_n()), but P V is summed in int32 per 64-key
 // half and each half is multiplied by its own scale row.
-template <int D, bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool DUMP_S, bool SPLIT, int VBLK = 0>
-__global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUSAL, VBLK)) fwd_full_int8_kernel(const KParams p) {
+// FOLD: 16-bit k_scales, whose dequantisation is folded into one instruction per score (kScoreSeed): the vector pipe bounds this kernel, with what LDS
+// reads and products add to it, and 64 conversions of 604 vector instructions per wave and 128-key block go.  The biases take as many LDS reads as the
+// scales did.  At head_dim 128 the scales then come as lanes of one register (16 reads become four); at head_dim 64, where no product runs beside
+// most of the vector work, that modifier costs more than the reads, and they stay quads.  us, before -> after: d128 B4 H32 N4096 835 -> 812
+// (causal 449 -> 431), a chunk of 512 rows on 7680 keys B2 H32/8 129 -> 121; d64 B4 H32 N4096 609 -> 599, causal B4 H16 N2048 55.7 -> 49.5.
+template <int D, bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool DUMP_S, bool SPLIT, int VBLK = 0, bool FOLD = false>
+__global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUSAL, VBLK, FOLD)) fwd_full_int8_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
     constexpr int KS = D / 32;                   // k-steps of Q K^T (32 bytes of head_dim each)
     static_assert(D <= 128 || DUMP_S, "head_dim 256 runs fwd_full_int8_pair_kernel");
@@ -50,7 +55,8 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     constexpr int SWM = (CHV < 8 ? CHV : 8) - 1; // swizzle mask of V rows
     // LDS map (bytes)
     constexpr int OFF_KS = 0;                    // two fp32 k_scale vectors
-    constexpr int OFF_K = 2 * BN * 4;            // two K tiles
+    constexpr int OFF_NK = 2 * BN * 4;           // FOLD: two vectors of -kScoreBias * k_scale
+    constexpr int OFF_K = (FOLD ? 4 : 2) * BN * 4;            // two K tiles
     constexpr int OFF_V = OFF_K + 2 * KT;        // two V tiles
     constexpr int VSUB = VBLK == 2 ? 2 : 1;      // V scale rows per key block
     static_assert(VBLK != 2 || NST == 4, "64-key V scale rows belong to the 128-key block");
@@ -191,7 +197,19 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         v_rd[dt] = OFF_V + v_row0 * DV + 8 * (i16 & 1) + (((c & SWM) ^ v_swz) << 4) + ((c & ~SWM) << 4);
     }
     const uint32_t ks_rd = OFF_KS + 16 * lh;     // + 4 * (32*st + 8*a4) per read
+    const uint32_t ks1_rd = OFF_KS + 4 * scale_lane_key(lane);     // + 4 * 32 * st
+    v16i seed = {0};                             // what a score chain starts from
+    if (FOLD) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) seed[r] = kScoreSeed;
+        asm volatile("" : "+v"(seed));           // (opaque: held in its registers, not made anew for each chain)
+    }
     const uint32_t ks_wr = OFF_KS + 4 * (tid & (BN - 1));
+    auto put_ks = [&](uint32_t raw, int buf) __attribute__((always_inline)) {
+        const float s = cvt_ks(raw);
+        *(float*)(smem + ks_wr + buf * BN * 4) = s;
+        if (FOLD) *(float*)(smem + ks_wr + OFF_NK + buf * BN * 4) = -kScoreBias * s;
+    };
 
     // One key block out of LDS buffer `buf`.  DIAG selects the code with masking, of which there is one instance per number NACT of
     // sub-tiles that any row of the wave sees: keys whose index inside the block exceeds the lane's `lim` are masked in the last two of
@@ -236,12 +254,20 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         v16i sacc[2];
         // k_scale of the lane's keys, one quarter (4 keys) per register quad; a quad is refilled for the next sub-tile right
         // after the quarter that consumed it (three quarters of vector work ahead of its next use)
-        v4f kk[4];
+        constexpr bool LANE_SCALES = FOLD && D == 128;
+        v4f kk[4], nk[4];
         auto load_kk = [&](int a4, int st) __attribute__((always_inline)) {
-            kk[a4] = *(const v4f*)(smem + ks_rd + SB + 4 * (32 * st + 8 * a4));
+            const uint32_t at = ks_rd + SB + 4 * (32 * st + 8 * a4);
+            if (FOLD) nk[a4] = *(const v4f*)(smem + at + OFF_NK);
+            if (!LANE_SCALES) kk[a4] = *(const v4f*)(smem + at);
         };
+        float ksv[NST];
+        if (LANE_SCALES) {
+#pragma unroll
+            for (int st = 0; st < NST; ++st) ksv[st] = *(const float*)(smem + ks1_rd + SB + 4 * 32 * st);
+        }
         auto qk_chain = [&](v16i& acc, const v4i (&f)[KS]) __attribute__((always_inline)) {
-            acc = (v16i){0};
+            acc = FOLD ? seed : (v16i){0};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[ks], qreg[ks], acc, 0, 0, 0);
         };
@@ -261,7 +287,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             __builtin_amdgcn_sched_barrier(0);
             if (st + 2 < nact) load_kfrags(fr[st & 1], st + 2);
             if (!DUMP_S && !DIAG) issue_k_slice(k_next, nb + 1, buf ^ 1, st, NST);
-            if (DUMP_S) wait_for_product(sacc[st & 1]);
+            if (DUMP_S || (LANE_SCALES && st == 0)) wait_for_product(sacc[st & 1]);
             const uint32_t hidden = DIAG ? hidden_past(last - 32 * st) : 0u;
             const v16i& acc = sacc[st & 1];
             v16i& nacc = sacc[(st + 1) & 1];
@@ -280,14 +306,24 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
                 if (next) {
 #pragma unroll
                     for (int ks = a4 * KS / 4; ks < (a4 + 1) * KS / 4; ++ks) {
-                        if (ks == 0) nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[(st + 1) & 1][0], qreg[0], (v16i){0}, 0, 0, 0);
+                        if (ks == 0) nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[(st + 1) & 1][0], qreg[0], FOLD ? seed : (v16i){0}, 0, 0, 0);
                         else nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[(st + 1) & 1][ks], qreg[ks], nacc, 0, 0, 0);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 float xq[4];
 #pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) xq[b4] = (float)acc[4 * a4 + b4] * kk[a4][b4];
+                for (int b4 = 0; b4 < 4; ++b4) {
+                    const int sum = acc[4 * a4 + b4];
+                    if constexpr (LANE_SCALES) {
+                        xq[b4] = nk[a4][b4];
+                        fmac_lane_scale(xq[b4], ksv[st], sum, 4 * a4 + b4);
+                    } else if constexpr (FOLD) {
+                        xq[b4] = fmaf(__builtin_bit_cast(float, sum), kk[a4][b4], nk[a4][b4]);
+                    } else {
+                        xq[b4] = (float)sum * kk[a4][b4];
+                    }
+                }
                 if (next) load_kk(a4, st + 1);
                 if (DIAG && (st + 2 >= nact || VBLK == 2)) {
 #pragma unroll
@@ -478,7 +514,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             else if (NST == 4 && gw == 1) compute(diag_tag, IntTag<2>{}, buf, nb, more, lim);
             else if (NST == 4 && gw == 2) compute(diag_tag, IntTag<3>{}, buf, nb, more, lim);
         }
-        if (more && ks_wave) *(float*)(smem + ks_wr + (buf ^ 1) * BN * 4) = cvt_ks(ks_next);
+        if (more && ks_wave) put_ks(ks_next, buf ^ 1);
         if (more && vs_thread) {
 #pragma unroll
             for (int sub = 0; sub < VSUB; ++sub) *(float*)(smem + vs_wr + ((buf ^ 1) * VSUB + sub) * DV * 4) = vs_next[sub];
@@ -497,7 +533,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         open_ticket();
         {
             const uint32_t s0 = load_ks(nb_begin);
-            if (ks_wave) *(float*)(smem + ks_wr) = cvt_ks(s0);
+            if (ks_wave) put_ks(s0, 0);
             qsc = DUMP_S ? p.qk_scale_log2 : q_scale_log2(p, q_scale_bits);
             if (vs_thread) {
 #pragma unroll

@@ -1,0 +1,32 @@
+"""16-bit and 32-bit scales of the same values: the general full-int8 kernels fold the dequantisation of the former into one instruction per
+score (kScoreSeed in csrc/intfa_device.h) and convert with the latter.  Same bits, up to the largest sums there are."""
+import pytest
+import torch
+
+import int_flashattention_amd as M
+from many_heads import repetitions
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("D,causal,Nq,Nk", [(64, False, 300, 333), (64, True, 200, 1100), (64, True, 129, 129), (128, False, 130, 700), (128, True, 257, 257),
+                                            (128, True, 90, 1000), (256, False, 130, 200), (256, True, 200, 200)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_same_bits(D, causal, Nq, Nk, dtype):
+    H = repetitions(1, 1, Nq) + 1
+    g = torch.Generator(device=DEV).manual_seed(D + Nk)
+    q8, k8, v8 = (torch.randint(-128, 128, (1, H, n, D), generator=g, device=DEV, dtype=torch.int32).to(torch.int8) for n in (Nq, Nk, Nk))
+    # the largest sums of either sign: -128 * -128 and -128 * 127 throughout
+    q8[:, :, ::7] = -128
+    k8[:, :, ::5] = -128
+    k8[:, :, 1::5] = 127
+    qs, ks = (torch.rand((1, H, n), generator=g, device=DEV).mul(2e-3).to(dtype) for n in (Nq, Nk))
+    ks[:, :, 3::11] *= 64
+    vs = torch.rand((1, H), generator=g, device=DEV).to(dtype)
+    for p_round in ("reference", "rne"):
+        a, la = M.attention_full_int8(q8, k8, v8, qs, ks, vs, causal, 1.0, out_dtype=dtype, p_round=p_round, return_lse=True)
+        b, lb = M.attention_full_int8(q8, k8, v8, qs.float(), ks.float(), vs.float(), causal, 1.0, out_dtype=dtype, p_round=p_round, return_lse=True)
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+        assert torch.equal(la.view(torch.int32), lb.view(torch.int32))
+        assert bool(torch.isfinite(la).all()) and bool(torch.isfinite(a).all())

@@ -330,6 +330,18 @@ struct KScaleSource {
 // 8 (i / 4) + 4 lh + i % 4), and a multiplication takes any of them for the whole row with the DPP modifier row_newbcast, at no instruction of its
 // own.  (Read as quads of a broadcast address they are a quarter of the wave's LDS reads, of which the CU does one per 3 ns whatever it brings.)
 __device__ __forceinline__ uint32_t scale_lane_key(int lane) { return (uint32_t)(8 * ((lane & 15) >> 2) + 4 * (lane >> 5) + (lane & 3)); }
+// The i-th of them (a constant once inlined), as an operand of the instruction that uses it.
+template <int I> __device__ __forceinline__ float lane_scale_of(float s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0x150 + I, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_scale(float s, int i) {
+    switch (i) {
+        case 0: return lane_scale_of<0>(s); case 1: return lane_scale_of<1>(s); case 2: return lane_scale_of<2>(s); case 3: return lane_scale_of<3>(s);
+        case 4: return lane_scale_of<4>(s); case 5: return lane_scale_of<5>(s); case 6: return lane_scale_of<6>(s); case 7: return lane_scale_of<7>(s);
+        case 8: return lane_scale_of<8>(s); case 9: return lane_scale_of<9>(s); case 10: return lane_scale_of<10>(s); case 11: return lane_scale_of<11>(s);
+        case 12: return lane_scale_of<12>(s); case 13: return lane_scale_of<13>(s); case 14: return lane_scale_of<14>(s); default: return lane_scale_of<15>(s);
+    }
+}
 // c += f * (the scale of the lane's i-th key).  (Reads f like any hand-written instruction: mfma_check.py.)
 __device__ __forceinline__ void fmac_lane_scale(float& c, float scales, int f, int i) {
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(c) : "v"(scales), "v"(f), "i"(i));

@@ -30,3 +30,23 @@ def test_same_bits(D, causal, Nq, Nk, dtype):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
         assert torch.equal(la.view(torch.int32), lb.view(torch.int32))
         assert bool(torch.isfinite(la).all()) and bool(torch.isfinite(a).all())
+
+
+@pytest.mark.parametrize("causal,Nq,Nk", [(False, 130, 64), (False, 200, 333), (True, 129, 129), (True, 257, 700)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_same_bits_16bit_v(causal, Nq, Nk, dtype):
+    """The pipelined half-int8 kernel, in more workgroups than two per compute unit."""
+    H = repetitions(1, 1, Nq, rows=128) + 1
+    g = torch.Generator(device=DEV).manual_seed(Nk)
+    q8, k8 = (torch.randint(-128, 128, (1, H, n, 128), generator=g, device=DEV, dtype=torch.int32).to(torch.int8) for n in (Nq, Nk))
+    q8[:, :, ::7] = -128
+    k8[:, :, ::5] = -128
+    k8[:, :, 1::5] = 127
+    v = torch.randn((1, H, Nk, 128), generator=g, device=DEV).to(dtype)
+    qs, ks = (torch.rand((1, H, n), generator=g, device=DEV).mul(2e-3).to(dtype) for n in (Nq, Nk))
+    ks[:, :, 3::11] *= 64
+    a, la = M.attention_int8(q8, k8, v, qs, ks, causal, 1.0, return_lse=True)
+    b, lb = M.attention_int8(q8, k8, v, qs.float(), ks.float(), causal, 1.0, return_lse=True)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert torch.equal(la.view(torch.int32), lb.view(torch.int32))
+    assert bool(torch.isfinite(la).all()) and bool(torch.isfinite(a).all())

@@ -75,13 +75,44 @@ template <typename K> inline int launch_kernel(K kernel, const KParams& kp, hipS
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, finish_mapping(kp, grid));
     return (int)hipGetLastError();
 }
+// Causal items differ in length, and each of `slots` resident workgroups has a fixed list of them (item_of_round): true if there are two rounds of them
+// and no list is longer than the mean by more than a quarter of an item, and a shortest item where they do not come out even: about what the
+// hardware's dealing of single ones leaves.  (Full-int8
+// head_dim 256, us, dealt by the hardware -> lists: 12 heads of 6000 keys, whose longest list is a third over the mean, 199 -> 248; 8 heads of 6000,
+// 1.5 rounds, 150.7 -> 153.0; 192 heads of 500 47.0 -> 43.4, 24 heads of 3000 119.3 -> 115.7.)  Past 32 rounds it is taken for true.
+inline bool lists_agree(const KParams& kp, int slots) {
+    const int n_mblk = (kp.seqlen + kBlockM - 1) / kBlockM;
+    const KParams k = finish_mapping(kp, kp.batch * kp.heads * n_mblk);
+    const int lists = slots / kXcds, per_xcd = k.xcd_whole_wgs / kXcds;
+    if (k.rem_wgs != 0 || lists > 64 || per_xcd < 2 * lists) return false;
+    if (per_xcd >= 32 * lists) return true;
+    const int xcd_units = per_xcd / (n_mblk * kp.kv_group);
+    int64_t load[64] = {}, total = 0;
+    int list = 0, step = 1;                                       // (to and fro: every second round backwards)
+    for (int unit = 0; unit < xcd_units;) {
+        const int units = unit * n_mblk * kp.kv_group < k.run_last_slot ? k.run_units : k.run_units_last;
+        for (int m = n_mblk; m > 0; --m)
+            for (int head = 0; head < units * kp.kv_group; ++head) {
+                const int64_t keys = (int64_t)m * kBlockM + (kp.seqlen_k - kp.seqlen);
+                load[list] += keys;
+                total += keys;
+                list += step;
+                if (list < 0 || list == lists) { step = -step; list += step; }
+            }
+        unit += units;
+    }
+    int64_t most = 0;
+    for (int i = 0; i < lists; ++i) most = load[i] > most ? load[i] : most;
+    const int64_t shortest = kBlockM + (kp.seqlen_k - kp.seqlen);
+    return most - total / lists <= total / per_xcd / 4 + (per_xcd % lists != 0 ? shortest : 0);
+}
 // The same work items for `slots` workgroups (a multiple of kXcds), which take every slots-th each, where there are more items than that.
 // Not for batches of different lengths (the items of a workgroup would differ in work; the hardware deals single ones as compute units
 // become free), for items that may have no key, or for query rows further apart than a copy's offsets reach.
 inline bool takes_resident(const KParams& kp, int slots) {
     const int64_t items = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM);
     return items > slots && kp.num_splits <= 1 && kp.seqlens_k == nullptr && kp.seqlen_k > 0 && !(kp.causal && kp.seqlen_k < kp.seqlen) &&
-           kp.q_sn < (1ll << 31) / kBlockM;
+           kp.q_sn < (1ll << 31) / kBlockM && (!kp.causal || lists_agree(kp, slots));
 }
 template <typename K> inline int launch_resident(K kernel, const KParams& kp, hipStream_t stream, int threads, int slots) {
     KParams k = finish_mapping(kp, kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM));

@@ -355,7 +355,8 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     // the lengths agree).  What it is for: a workgroup fills its compute unit, and nothing ran under its first loads and its last stores (20 % of the time
     // at 1024 keys).  So an item's last block requests the next one's first tiles, the block before it Q (into the LDS), and nothing waits for the
     // stores.  us, one item per workgroup -> this: B16 H16 N1024 bf16 268 -> 244, causal 172 -> 161, B4 H32 N4096 1679 -> 1590, B16 H32/4 N200
-    // 49.9 -> 46.4; what bounds it then is the loop over the key blocks.  (16-bit scales' dequantisation folded (kScoreSeed): another 1 - 2 %.)  Launches of one round lose 5 % in the longer code: they run the other form.
+    // 49.9 -> 46.4; what bounds it then is the loop over the key blocks.  (16-bit scales' dequantisation folded, kScoreSeed: another 1 - 2 %.)
+    // Launches of one round lose 5 % in the longer code: they run the other form.
     int buf = 0;                                 // LDS buffer of the item's first block, then of its last
     int round = 0;
     if (it.nb_begin < it.nb_end) {

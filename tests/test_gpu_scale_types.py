@@ -50,3 +50,16 @@ def test_same_bits_16bit_v(causal, Nq, Nk, dtype):
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     assert torch.equal(la.view(torch.int32), lb.view(torch.int32))
     assert bool(torch.isfinite(la).all()) and bool(torch.isfinite(a).all())
+
+
+@pytest.mark.parametrize("D,causal,Nq,Nk", [(64, False, 200, 300), (64, True, 130, 1100), (128, False, 200, 300), (128, True, 257, 257)])
+def test_same_bits_blocked_v(D, causal, Nq, Nk):
+    """One V scale per 128 keys and channel."""
+    H = repetitions(1, 1, Nq, rows=128) + 1
+    g = torch.Generator(device=DEV).manual_seed(Nk)
+    q8, k8 = (torch.randint(-128, 128, (1, H, n, D), generator=g, device=DEV, dtype=torch.int32).to(torch.int8) for n in (Nq, Nk))
+    v8, vs = M.quant_perblock_channel(torch.randn((1, H, Nk, D), generator=g, device=DEV).half(), 128)
+    qs, ks = (torch.rand((1, H, n), generator=g, device=DEV).mul(2e-3).half() for n in (Nq, Nk))
+    a = M.attention_full_int8(q8, k8, v8, qs, ks, vs, causal, 1.0, v_scale_block=128)
+    b = M.attention_full_int8(q8, k8, v8, qs.float(), ks.float(), vs, causal, 1.0, v_scale_block=128)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16)) and bool(torch.isfinite(a).all())

@@ -90,7 +90,6 @@ struct KParams {
     int32_t causal_rows;                   // decode kernel: query positions per folded query head (0 = the row is the position)
     float qk_scale_log2;                   // sm_scale * log2(e)
     // workgroup -> work mapping of this launch (set by finish_mapping() in intfa_launch.h from the grid size)
-    int32_t items, grid_wgs;               // work items (workgroups, were each to take one), and workgroups of the launch
     int32_t per_head;                      // workgroups per query head
     int32_t heads_kv;                      // heads / kv_group
     int32_t xcd_whole_wgs;                 // workgroups of the K/V heads that are dealt whole to the 8 XCDs (a multiple of 8)
@@ -102,6 +101,7 @@ struct KParams {
     int32_t kv_key_bytes;                                  // bytes of one key's K and V rows
     int32_t stream_kv;                                     // decode-shaped kernels: K and V tiles are loaded non-temporally
     FastDiv d_run, d_run_heads, d_run_heads_last, d_rem_heads;
+    int32_t items, grid_wgs;               // work items (workgroups, were each to take one), and workgroups of the launch (last: the others keep their places in the lines)
 };
 
 // The kernel's own argument block as the epilogues re-read it: the pointer keeps the constant address space, so its

@@ -349,6 +349,7 @@ __device__ __forceinline__ void fmac_lane_scale(float& c, float scales, int f, i
 // Int32 scores as fp32 numbers without a conversion: a product chain that starts from the bits of 1.5 * 2^23 instead of zero ends in the bits of
 // 1.5 * 2^23 + S (|S| <= 2^22).  With kScoreBias * k_scale subtracted by the multiplication with k_scale, a score takes one instruction instead of two,
 // to the same bits: the product is exact inside it, and kScoreBias * k_scale is exact for 16-bit scales (at most 11 + 2 significant bits).
+// (An infinite scale gives NaN whatever the sum, and so does one past 2.7e31: the quantisers give such scales only to rows of zeros, NaN either way.)
 constexpr int kScoreSeed = 0x4B400000;
 constexpr float kScoreBias = 12582912.f;
 

@@ -348,10 +348,13 @@ __device__ __forceinline__ void fmac_lane_scale(float& c, float scales, int f, i
 }
 // Int32 scores as fp32 numbers without a conversion: a product chain that starts from the bits of 1.5 * 2^23 instead of zero ends in the bits of
 // 1.5 * 2^23 + S (|S| <= 2^22).  With kScoreBias * k_scale subtracted by the multiplication with k_scale, a score takes one instruction instead of two,
-// to the same bits: the product is exact inside it, and kScoreBias * k_scale is exact for 16-bit scales (at most 11 + 2 significant bits).
-// (An infinite scale gives NaN whatever the sum, and so does one past 2.7e31: the quantisers give such scales only to rows of zeros, NaN either way.)
+// to the same bits where the bias is finite (past_fold): the product is exact inside it, and kScoreBias * k_scale is exact for 16-bit scales (at most 11 + 2 significant bits).
 constexpr int kScoreSeed = 0x4B400000;
 constexpr float kScoreBias = 12582912.f;
+// From 2^104 on (keys of bf16 rows of magnitude 2.6e33 have such scales; infinities) the bias is, or may be, past the largest fp32 number and the
+// score would be lost.  A workgroup that meets such a key takes all of its key blocks again with the conversion: the waves that store the
+// scales look for them and leave a word in the LDS, which the others read once, behind the last block.
+__device__ __forceinline__ bool past_fold(float s) { return __builtin_amdgcn_ballot_w64(__builtin_fabsf(s) >= 0x1p104f) != 0; }
 
 // ---- LDS swizzles.  A tile row is ROW_BYTES bytes; its 16-byte chunks are XOR-permuted with a function of the
 // row so that the rows touched together by one LDS access cycle (64 banks x 4 bytes = 256 bytes: 16 lanes of a

@@ -20,11 +20,8 @@ namespace intfa {
 
 // QK_INT8: int8 Q/K with scales (half-int8) or 16-bit Q/K (fp16/bf16 variant).  IO_DT: type of V, P and the output
 // (and of Q/K when !QK_INT8): 0 fp16, 1 bf16.
-// FOLD (QK_INT8): 16-bit k_scales, whose dequantisation is one instruction per score instead of two (kScoreSeed): 32 of 212 vector instructions per
-// wave and block go, for 32 registers of which some are spilled around the loop.  The scales come as lanes of one register in either form.  us, scales as
-// quads -> as lanes -> folded: B8 H32 N2048 484 -> 468 -> 462, causal 299 -> 293 -> 285, B4 H32 N4096 920 -> 904 -> 889; launches of one round,
-// which pay for the spills, 23.9 -> 22.4 -> 23.6 (288 workgroups, N700).
-template <bool QK_INT8, int D, bool CAUSAL, int IO_DT, bool SPLIT, bool FOLD = false>
+// The k_scales come as lanes of one register (scale_lane_key; us, as quads -> as lanes: B8 H32 N2048 484 -> 468, causal 299 -> 293, B4 H32 N4096 920 -> 904).
+template <bool QK_INT8, int D, bool CAUSAL, int IO_DT, bool SPLIT>
 __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     static_assert(D == 64 || D == 128, "head_dim 256 runs fwd_f16pv_pair_kernel (intfa_fwd_f16pv_pair.h)");
@@ -36,9 +33,7 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
     constexpr int KT = BN * KROW, VT = BN * VROW;
     constexpr int KCH = KROW / 16, VCH = VROW / 16;
     constexpr int OFF_KS = 0;
-    static_assert(!FOLD || QK_INT8, "");
-    constexpr int OFF_NK = 2 * BN * 4;                // FOLD: two vectors of -kScoreBias * k_scale
-    constexpr int OFF_K = (FOLD ? 4 : 2) * BN * 4;
+    constexpr int OFF_K = 2 * BN * 4;
     constexpr int OFF_V = OFF_K + 2 * KT;
     constexpr int LDS_BYTES = OFF_V + 2 * VT;
     __shared__ __attribute__((aligned(1024))) char smem[LDS_BYTES];
@@ -118,11 +113,7 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
     };
     const uint32_t ks_wr = OFF_KS + 4 * (tid & (BN - 1));
     auto store_ks = [&](uint32_t raw, int buf) __attribute__((always_inline)) {
-        if (QK_INT8 && ks_wave) {
-            const float sc = ks_src.cvt(raw);
-            *(float*)(smem + ks_wr + buf * BN * 4) = sc;
-            if (FOLD) *(float*)(smem + ks_wr + OFF_NK + buf * BN * 4) = -kScoreBias * sc;
-        }
+        if (QK_INT8 && ks_wave) *(float*)(smem + ks_wr + buf * BN * 4) = ks_src.cvt(raw);
     };
 
     // ---- per-lane LDS read offsets
@@ -158,12 +149,6 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
     constexpr int NQ = NST * KS, NP = DT * 4;         // MFMAs of Q K^T and of P V per block
     constexpr int LA = 4;                             // an MFMA's LDS operands are requested this many MFMAs ahead
     static_assert(NST == 2, "two sub-tiles of 32 keys");
-    v16i seed = {0};                                  // what a score chain starts from
-    if (FOLD) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) seed[r] = kScoreSeed;
-        asm volatile("" : "+v"(seed));                // (opaque: held in its registers)
-    }
     v16f s[2][NST];
     v4i pf[2][NST][2];
     float mx = -INFINITY;
@@ -218,14 +203,7 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
             const int st = j / 8, r = 2 * (j % 8);
             if (QK_INT8) {
 #pragma unroll
-                for (int k = r; k < r + 2; ++k) {
-                    float x = (float)si[st][k] * lane_scale(ksv[st], k);
-                    if constexpr (FOLD) {
-                        x = s[PAR ^ 1][st][k];                       // the bias, from load_nk
-                        fmac_lane_scale(x, ksv[st], si[st][k], k);
-                    }
-                    s[PAR ^ 1][st][k] = x;
-                }
+                for (int k = r; k < r + 2; ++k) s[PAR ^ 1][st][k] = (float)si[st][k] * lane_scale(ksv[st], k);
             }
             mx = fmaxf(fmaxf(mx, s[PAR ^ 1][st][r]), s[PAR ^ 1][st][r + 1]);
             asm volatile("" : "+v"(mx));
@@ -235,11 +213,6 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
 #pragma unroll
                 for (int st = 0; st < NST; ++st) ksv[st] = *(const float*)(smem + ks_rd + SB + 4 * 32 * st);
             }
-        };
-        auto load_nk = [&](int q) __attribute__((always_inline)) {          // quad q of the lane's biases, where the scores are accumulated
-            const v4f n = *(const v4f*)(smem + OFF_NK + 16 * lh + SB + 4 * (32 * (q / 4) + 8 * (q % 4)));
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s[PAR ^ 1][q / 4][4 * (q % 4) + j] = n[j];
         };
         if (QK) mx = -INFINITY;
 #pragma unroll
@@ -257,7 +230,7 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
         for (int i = 0; i < NM; ++i) {
             if (i < NQS) {
                 const int ks = i % KS, st = i / KS;
-                if (QK_INT8) si[st] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[i % LA], qreg[ks], ks ? si[st] : FOLD ? seed : (v16i){0}, 0, 0, 0);
+                if (QK_INT8) si[st] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[i % LA], qreg[ks], ks ? si[st] : (v16i){0}, 0, 0, 0);
                 else s[PAR ^ 1][st] = mfma16(fr[i % LA], qreg[ks], ks ? s[PAR ^ 1][st] : (v16f){0});
             } else {
                 const int k = i - NQS;
@@ -265,11 +238,6 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
             }
             fetch(i + LA);
             if (QK && PV && i == C0 - 4) load_kk();
-            if (FOLD && QK && PV) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    if (C0 - 2 + q * (NM - C0) / 8 == i) load_nk(q);
-            }
             if (E) {
 #pragma unroll
                 for (int j = i * 32 / (NM + !NM); j < (i + 1) * 32 / (NM + !NM); ++j) e_task(j);
@@ -286,11 +254,6 @@ __global__ void __launch_bounds__(kThreads, 2) fwd_f16pv_pipe_kernel(const KPara
         }
         if (QK && !PV) {
             load_kk();
-            if (FOLD) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) load_nk(q);
-                wait_for_product(si[NST - 1]);
-            }
 #pragma unroll
             for (int j = 0; j < 16; ++j) c_task(j);
         }

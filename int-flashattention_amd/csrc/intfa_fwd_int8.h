@@ -37,8 +37,9 @@ template <int D> struct FullInt8Geom {
 // FOLD: 16-bit k_scales, whose dequantisation is folded into one instruction per score (kScoreSeed): the vector pipe bounds this kernel, with what LDS
 // reads and products add to it, and 64 conversions of 604 vector instructions per wave and 128-key block go.  The biases take as many LDS reads as the
 // scales did.  At head_dim 128 the scales then come as lanes of one register (16 reads become four); at head_dim 64, where no product runs beside
-// most of the vector work, that modifier costs more than the reads, and they stay quads.  us, before -> after: d128 B4 H32 N4096 835 -> 812
-// (causal 449 -> 431), a chunk of 512 rows on 7680 keys B2 H32/8 129 -> 121; d64 B4 H32 N4096 609 -> 599, causal B4 H16 N2048 55.7 -> 49.5.
+// most of the vector work, that modifier costs more than the reads, and they stay quads.  Scales too large for it: past_fold.  us, before -> after: d128 B4
+// H32 N4096 834 -> 808 (causal 434 -> 426), a chunk of 512 rows on 7680 keys B2 H32/8 in one pass 124 -> 120, in two splits 106.6 -> 104.1; d64 B4
+// H32 N4096 608 -> 606, N768 29.6 -> 28.7, causal N1024 31.6 -> 29.3.  (Without the way out for such scales: 800, 421, 121, 104.0, 603, 28.6, 28.9.)
 template <int D, bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool DUMP_S, bool SPLIT, int VBLK = 0, bool FOLD = false>
 __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUSAL, VBLK, FOLD)) fwd_full_int8_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
@@ -61,7 +62,8 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     constexpr int VSUB = VBLK == 2 ? 2 : 1;      // V scale rows per key block
     static_assert(VBLK != 2 || NST == 4, "64-key V scale rows belong to the 128-key block");
     constexpr int OFF_VS = OFF_V + 2 * VT;       // VBLK: two vectors of VSUB * DV fp32 channel scales
-    constexpr int LDS_BYTES = OFF_VS + (VBLK ? 2 * VSUB * DV * 4 : 0);
+    constexpr int OFF_PF = OFF_VS + (VBLK ? 2 * VSUB * DV * 4 : 0);      // FOLD: a word per wave that stores k_scales, not zero: past_fold
+    constexpr int LDS_BYTES = OFF_PF + (FOLD ? 16 : 0);
     __shared__ __attribute__((aligned(1024))) char smem[LDS_BYTES];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -113,8 +115,8 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     const auto v_lane = tile_load_lane<DV, SWZ_V8, BN>(v_sn, wave, lane);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_loads = [&](int nb, int buf) __attribute__((always_inline)) {
-        issue_tile_load<D, SWZ_K, BN>(k_rsrc, (uint32_t)(nb * BN) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
-        if (!DUMP_S) issue_tile_load<DV, SWZ_V8, BN>(v_rsrc, (uint32_t)(nb * BN) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
+        issue_tile_load<D, SWZ_K, BN>(k_rsrc, __builtin_amdgcn_readfirstlane((nb * BN) * (int)k_sn), k_sn, lds0 + OFF_K + buf * KT, wave, k_lane);
+        if (!DUMP_S) issue_tile_load<DV, SWZ_V8, BN>(v_rsrc, __builtin_amdgcn_readfirstlane((nb * BN) * (int)v_sn), v_sn, lds0 + OFF_V + buf * VT, wave, v_lane);
     };
     // The argument lines at once (above), and the scales converted behind the requests.  Causal: the first tiles ahead of Q, which arrives under
     // their way from HBM (d128 B4 H16 N2048 66.4 -> 64.9 us, d64 B16 H16 N512 20.6 -> 20.1).  Without a mask grids are longer, most first
@@ -139,13 +141,13 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 #pragma unroll
         for (int it = 0; it < DMA_PARTS; ++it)
             if (it * nstages / DMA_PARTS == stage)
-                issue_tile_part<D, SWZ_K, BN>(rsrc, (uint32_t)(nb * BN) * k_sn, k_sn, lds0 + OFF_K + buf * KT, wave, k_lane, it);
+                issue_tile_part<D, SWZ_K, BN>(rsrc, __builtin_amdgcn_readfirstlane((nb * BN) * (int)k_sn), k_sn, lds0 + OFF_K + buf * KT, wave, k_lane, it);
     };
     auto issue_v_slice = [&](v4i rsrc, int nb, int buf, int stage, int nstages) __attribute__((always_inline)) {
 #pragma unroll
         for (int it = 0; it < V_PARTS; ++it)
             if (it * nstages / V_PARTS == stage)
-                issue_tile_part<DV, SWZ_V8, BN>(rsrc, (uint32_t)(nb * BN) * v_sn, v_sn, lds0 + OFF_V + buf * VT, wave, v_lane, it);
+                issue_tile_part<DV, SWZ_V8, BN>(rsrc, __builtin_amdgcn_readfirstlane((nb * BN) * (int)v_sn), v_sn, lds0 + OFF_V + buf * VT, wave, v_lane, it);
     };
     // k_scale of a block: thread t < 128 fetches the scale of key t; converted to fp32 when stored to LDS
     const KScaleSource ks_src(p, b, hk, seqlen_k);
@@ -205,10 +207,14 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         asm volatile("" : "+v"(seed));           // (opaque: held in its registers, not made anew for each chain)
     }
     const uint32_t ks_wr = OFF_KS + 4 * (tid & (BN - 1));
-    auto put_ks = [&](uint32_t raw, int buf) __attribute__((always_inline)) {
+    auto put_ks = [&](auto fold_tag, uint32_t raw, int buf, bool first) __attribute__((always_inline)) {
         const float s = cvt_ks(raw);
         *(float*)(smem + ks_wr + buf * BN * 4) = s;
-        if (FOLD) *(float*)(smem + ks_wr + OFF_NK + buf * BN * 4) = -kScoreBias * s;
+        if (decltype(fold_tag)::value) {
+            *(float*)(smem + ks_wr + OFF_NK + buf * BN * 4) = -kScoreBias * s;
+            const bool past = past_fold(s);
+            if (first || __builtin_expect(past, 0)) *(int*)(smem + OFF_PF + 4 * wave) = past;
+        }
     };
 
     // One key block out of LDS buffer `buf`.  DIAG selects the code with masking, of which there is one instance per number NACT of
@@ -217,8 +223,8 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     // visible key; last block of a ragged sequence: lim = the last valid key.  Straight code per instance, and one of it for both
     // buffers: with run-time tests around sub-tiles and keys a masked block took 1.6 plain ones and more (us, before -> now: d128 B16
     // H16 N300 25.6 -> 22.2, causal N512 28.8 -> 27.5, B8 H32/8 N1024 74.1 -> 72.2, d64 causal B16 H16 N512 20.0 -> 18.9).
-    auto compute = [&](auto diag_tag, auto nact_tag, int buf, int nb, bool more, int lim) __attribute__((always_inline)) {
-        constexpr bool DIAG = decltype(diag_tag)::value;
+    auto compute = [&](auto fold_tag, auto diag_tag, auto nact_tag, int buf, int nb, bool more, int lim) __attribute__((always_inline)) {
+        constexpr bool F = decltype(fold_tag)::value, DIAG = decltype(diag_tag)::value;
         constexpr int nact = decltype(nact_tag)::value;
         const uint32_t KB = buf * KT, VB = buf * VT, SB = buf * BN * 4;
         int last = lim - 4 * lh;                           // (opaque: 64 thresholds of a ragged end would be computed ahead of the loop)
@@ -254,11 +260,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         v16i sacc[2];
         // k_scale of the lane's keys, one quarter (4 keys) per register quad; a quad is refilled for the next sub-tile right
         // after the quarter that consumed it (three quarters of vector work ahead of its next use)
-        constexpr bool LANE_SCALES = FOLD && D == 128;
+        constexpr bool LANE_SCALES = F && D == 128;
         v4f kk[4], nk[4];
         auto load_kk = [&](int a4, int st) __attribute__((always_inline)) {
             const uint32_t at = ks_rd + SB + 4 * (32 * st + 8 * a4);
-            if (FOLD) nk[a4] = *(const v4f*)(smem + at + OFF_NK);
+            if (F) nk[a4] = *(const v4f*)(smem + at + OFF_NK);
             if (!LANE_SCALES) kk[a4] = *(const v4f*)(smem + at);
         };
         float ksv[NST];
@@ -267,7 +273,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             for (int st = 0; st < NST; ++st) ksv[st] = *(const float*)(smem + ks1_rd + SB + 4 * 32 * st);
         }
         auto qk_chain = [&](v16i& acc, const v4i (&f)[KS]) __attribute__((always_inline)) {
-            acc = FOLD ? seed : (v16i){0};
+            acc = F ? seed : (v16i){0};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[ks], qreg[ks], acc, 0, 0, 0);
         };
@@ -306,7 +312,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
                 if (next) {
 #pragma unroll
                     for (int ks = a4 * KS / 4; ks < (a4 + 1) * KS / 4; ++ks) {
-                        if (ks == 0) nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[(st + 1) & 1][0], qreg[0], FOLD ? seed : (v16i){0}, 0, 0, 0);
+                        if (ks == 0) nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[(st + 1) & 1][0], qreg[0], F ? seed : (v16i){0}, 0, 0, 0);
                         else nacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[(st + 1) & 1][ks], qreg[ks], nacc, 0, 0, 0);
                     }
                 }
@@ -318,14 +324,14 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
                     if constexpr (LANE_SCALES) {
                         xq[b4] = nk[a4][b4];
                         fmac_lane_scale(xq[b4], ksv[st], sum, 4 * a4 + b4);
-                    } else if constexpr (FOLD) {
+                    } else if constexpr (F) {
                         xq[b4] = fmaf(__builtin_bit_cast(float, sum), kk[a4][b4], nk[a4][b4]);
                     } else {
                         xq[b4] = (float)sum * kk[a4][b4];
                     }
                 }
                 if (next) load_kk(a4, st + 1);
-                if (DIAG && (st + 2 >= nact || VBLK == 2)) {
+                if (DIAG && (st + 2 >= nact || VBLK == 2 || FOLD != F)) {
 #pragma unroll
                     for (int b4 = 0; b4 < 4; ++b4) xq[b4] = hide(xq[b4], hidden, 8 * a4 + b4);
                 }
@@ -489,7 +495,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     // One pipeline step on LDS buffer BUF: wait for this block's tiles (issued one step earlier), make them
     // visible to all four waves, start the copy of the next block into the other buffer, compute.
     // (gw: sub-tile of the largest lim of the wave's rows, negative: none)
-    auto step = [&](auto diag_tag, int buf, int nb, int gw, int lim) __attribute__((always_inline)) {
+    auto step = [&](auto fold_tag, auto diag_tag, int buf, int nb, int gw, int lim) __attribute__((always_inline)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         const bool more = nb + 1 < nb_end;
@@ -505,16 +511,16 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             }
         }
         if constexpr (!DIAG) {
-            compute(diag_tag, IntTag<NST>{}, buf, nb, more, lim);
-        } else if constexpr (VBLK == 2) {        // (multiplies every sub-tile, so it masks every one: P8 of a hidden one is 0)
-            if (gw >= 0) compute(diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+            compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+        } else if constexpr (VBLK == 2 || FOLD != decltype(fold_tag)::value) {      // (multiplies every sub-tile, so it masks every one: P8 of a hidden one is 0)
+            if (gw >= 0) compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim);
         } else {
-            if (gw >= NST - 1) compute(diag_tag, IntTag<NST>{}, buf, nb, more, lim);
-            else if (gw == 0) compute(diag_tag, IntTag<1>{}, buf, nb, more, lim);
-            else if (NST == 4 && gw == 1) compute(diag_tag, IntTag<2>{}, buf, nb, more, lim);
-            else if (NST == 4 && gw == 2) compute(diag_tag, IntTag<3>{}, buf, nb, more, lim);
+            if (gw >= NST - 1) compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+            else if (gw == 0) compute(fold_tag, diag_tag, IntTag<1>{}, buf, nb, more, lim);
+            else if (NST == 4 && gw == 1) compute(fold_tag, diag_tag, IntTag<2>{}, buf, nb, more, lim);
+            else if (NST == 4 && gw == 2) compute(fold_tag, diag_tag, IntTag<3>{}, buf, nb, more, lim);
         }
-        if (more && ks_wave) put_ks(ks_next, buf ^ 1);
+        if (more && ks_wave) put_ks(fold_tag, ks_next, buf ^ 1, false);
         if (more && vs_thread) {
 #pragma unroll
             for (int sub = 0; sub < VSUB; ++sub) *(float*)(smem + vs_wr + ((buf ^ 1) * VSUB + sub) * DV * 4) = vs_next[sub];
@@ -529,11 +535,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         if (SPLIT && p.ticket != nullptr && lane == 0 && row_block < row_blocks) splitkv_open_tickets(p, head * row_blocks + row_block);
     };
     if (nb_begin >= nb_end) open_ticket();
-    if (nb_begin < nb_end) {
-        open_ticket();
+    // (the way out for large scales, fold_tag other than FOLD: every block in the code with masking, one instance of it)
+    auto all_blocks = [&](auto fold_tag) __attribute__((always_inline)) {
         {
             const uint32_t s0 = load_ks(nb_begin);
-            if (ks_wave) put_ks(s0, 0);
+            if (ks_wave) put_ks(fold_tag, s0, 0, true);
             qsc = DUMP_S ? p.qk_scale_log2 : q_scale_log2(p, q_scale_bits);
             if (vs_thread) {
 #pragma unroll
@@ -548,11 +554,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         const bool ragged = !CAUSAL && tail_keys < BN && nb_end == nb_total;
         const int plain_end = CAUSAL ? (nb_end > diag_begin ? diag_begin : nb_end) : (ragged ? nb_end - 1 : nb_end);
         int nb = nb_begin;
-        while (true) {
+        while (FOLD == decltype(fold_tag)::value) {
             if (nb >= plain_end) break;
-            step(BoolTag<false>{}, 0, nb++, 0, 0);
+            step(fold_tag, BoolTag<false>{}, 0, nb++, 0, 0);
             if (nb >= plain_end) break;
-            step(BoolTag<false>{}, 1, nb++, 0, 0);
+            step(fold_tag, BoolTag<false>{}, 1, nb++, 0, 0);
         }
         // masked blocks: the blocks the causal diagonal of this query block crosses (kBlockM / BN of them when the lengths
         // are equal, one more when the offset is not a multiple of the block; keys past the end of a ragged sequence lie above
@@ -560,9 +566,28 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 #pragma clang loop unroll(disable)
         for (; nb < nb_end; ++nb) {
             // lane: last visible key relative to the block; wave: sub-tile of the largest of them (negative: none)
-            const int lim = CAUSAL ? q_row + causal_off - nb * BN : tail_keys - 1;
-            const int gw = (CAUSAL ? mb * kBlockM + wave * 32 + 31 + causal_off - nb * BN : tail_keys - 1) >> 5;
-            step(BoolTag<true>{}, (nb - nb_begin) & 1, nb, gw, lim);
+            const int lim = (CAUSAL ? q_row + causal_off : seqlen_k - 1) - nb * BN;
+            const int gw = ((CAUSAL ? mb * kBlockM + wave * 32 + 31 + causal_off : seqlen_k - 1) - nb * BN) >> 5;
+            step(fold_tag, BoolTag<true>{}, (nb - nb_begin) & 1, nb, gw, lim);
+        }
+    };
+    if (nb_begin < nb_end) {
+        open_ticket();
+        all_blocks(BoolTag<FOLD>{});
+        if constexpr (FOLD) {
+            int past = *(const int*)(smem + OFF_PF);
+            if (BN == 128) past |= *(const int*)(smem + OFF_PF + 4);
+            if (__builtin_expect(__builtin_amdgcn_readfirstlane(past), 0)) {
+                m_run = -INFINITY; l_run = 0.f;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o_acc[dt][r] = 0.f;
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // (the slices of a block past the last one write zeros into the tiles)
+                __syncthreads();
+                issue_loads(nb_begin, 0);
+                all_blocks(BoolTag<false>{});
+            }
         }
     }
     if (DUMP_S) return;

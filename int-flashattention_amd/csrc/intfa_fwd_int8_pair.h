@@ -19,7 +19,7 @@ namespace intfa {
 
 constexpr int kPairThreads = 512;
 
-template <bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK, bool RESIDENT, bool FOLD = false>
+template <bool CAUSAL, int OUT_DT /*0 f16, 1 bf16*/, int PROUND, bool SPLIT, bool VBLK, bool RESIDENT>
 __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(const KParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass only needs the kernel's symbol
     constexpr int D = 256;
@@ -30,8 +30,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     constexpr int KT = BN * D;                   // bytes of one K tile, and of one V tile
     // LDS map (bytes)
     constexpr int OFF_KS = 0;                    // two fp32 k_scale vectors
-    constexpr int OFF_NK = OFF_KS + 2 * BN * 4;  // FOLD: two vectors of -kScoreBias * k_scale
-    constexpr int OFF_XM = OFF_NK + (FOLD ? 2 * BN * 4 : 0);  // row maxima (and, in the epilogue, row sums): [wave][32]
+    constexpr int OFF_XM = OFF_KS + 2 * BN * 4;  // row maxima (and, in the epilogue, row sums): [wave][32]
     constexpr int OFF_VS = OFF_XM + 8 * 32 * 4;  // VBLK: two vectors of D fp32 channel scales
     constexpr int OFF_XP = OFF_VS + (VBLK ? 2 * D * 4 : 0);   // packed P fragments: [wave][lane] x 16 bytes
     constexpr int OFF_K = (OFF_XP + 8 * 64 * 16 + 1023) & ~1023;
@@ -136,19 +135,8 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     }
     const uint32_t v_own = 32 * hf * D, v_oth = 32 * (hf ^ 1) * D;      // sub-tile of this wave's P, of the partner's
     const uint32_t ks_rd = OFF_KS + 4 * 32 * hf + 16 * lh;              // + 32 * a4 per read
-    const uint32_t ks1_rd = OFF_KS + 4 * 32 * hf + 4 * scale_lane_key(lane);
     const uint32_t ks_wr = OFF_KS + 4 * (tid & (BN - 1));
-    auto put_ks = [&](uint32_t raw, int buf) __attribute__((always_inline)) {
-        const float s = cvt_ks(raw);
-        *(float*)(smem + ks_wr + buf * BN * 4) = s;
-        if (FOLD) *(float*)(smem + ks_wr + (OFF_NK - OFF_KS) + buf * BN * 4) = -kScoreBias * s;
-    };
-    v16i seed = {0};                             // what a score chain starts from
-    if (FOLD) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) seed[r] = kScoreSeed;
-        asm volatile("" : "+v"(seed));           // (opaque: held in its registers)
-    }
+    auto put_ks = [&](uint32_t raw, int buf) __attribute__((always_inline)) { *(float*)(smem + ks_wr + buf * BN * 4) = cvt_ks(raw); };
     const uint32_t xm_wr = OFF_XM + 4 * (wave * 32 + lq), xm_rd = OFF_XM + 4 * ((wave ^ 4) * 32 + lq);
     const uint32_t xp_wr = OFF_XP + 16 * (wave * 64 + lane), xp_rd = OFF_XP + 16 * ((wave ^ 4) * 64 + lane);
 
@@ -208,9 +196,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         // -------- pass 1: dequantise this wave's S^T sub-tile by k_scale, row maximum
         v4f kk[4];
 #pragma unroll
-        for (int a4 = 0; a4 < 4; ++a4) kk[a4] = *(const v4f*)(smem + ks_rd + (FOLD ? OFF_NK - OFF_KS : 0) + SB + 32 * a4);
-        const float ksv = FOLD ? *(const float*)(smem + ks1_rd + SB) : 0.f;
-        if (FOLD) wait_for_product(sacc);
+        for (int a4 = 0; a4 < 4; ++a4) kk[a4] = *(const v4f*)(smem + ks_rd + SB + 32 * a4);
         const uint32_t hidden = RESIDENT && (CAUSAL || LAST) ? hidden_past(past) : 0u;
         float t[16];
         float mx = -INFINITY;
@@ -218,14 +204,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         for (int a4 = 0; a4 < 4; ++a4) {
             float xq[4];
 #pragma unroll
-            for (int b4 = 0; b4 < 4; ++b4) {
-                if constexpr (FOLD) {
-                    xq[b4] = kk[a4][b4];
-                    fmac_lane_scale(xq[b4], ksv, sacc[4 * a4 + b4], 4 * a4 + b4);
-                } else {
-                    xq[b4] = (float)sacc[4 * a4 + b4] * kk[a4][b4];
-                }
-            }
+            for (int b4 = 0; b4 < 4; ++b4) xq[b4] = (float)sacc[4 * a4 + b4] * kk[a4][b4];
             if ((CAUSAL || LAST || MAYBE_LAST) && 32 * hf + 31 > lim_lo) {   // wave-uniform: some lane of the wave has a hidden key here
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) {
@@ -327,7 +306,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
             if (more) {
 #pragma unroll
                 for (int ks = 2 * dt; ks < 2 * dt + 2; ++ks) {
-                    if (ks == 0) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[0], qreg[0], FOLD ? seed : (v16i){0}, 0, 0, 0);
+                    if (ks == 0) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[0], qreg[0], (v16i){0}, 0, 0, 0);
                     else sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[ks & 3], qreg[ks], sacc, 0, 0, 0);
                 }
             }
@@ -355,7 +334,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     // the lengths agree).  What it is for: a workgroup fills its compute unit, and nothing ran under its first loads and its last stores (20 % of the time
     // at 1024 keys).  So an item's last block requests the next one's first tiles, the block before it Q (into the LDS), and nothing waits for the
     // stores.  us, one item per workgroup -> this: B16 H16 N1024 bf16 268 -> 244, causal 172 -> 161, B4 H32 N4096 1679 -> 1590, B16 H32/4 N200
-    // 49.9 -> 46.4; what bounds it then is the loop over the key blocks.  (16-bit scales' dequantisation folded, kScoreSeed: another 1 - 2 %.)
+    // 49.9 -> 46.4; what bounds it then is the loop over the key blocks.
     // Launches of one round lose 5 % in the longer code: they run the other form.
     int buf = 0;                                 // LDS buffer of the item's first block, then of its last
     int round = 0;
@@ -389,7 +368,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
                 v4i fr[KS];
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) fr[ks] = *(const v4i*)(smem + (k_rd(ks) + buf * KT));
-                sacc = FOLD ? seed : (v16i){0};
+                sacc = (v16i){0};
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[ks], qreg[ks], sacc, 0, 0, 0);
             }

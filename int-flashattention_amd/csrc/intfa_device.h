@@ -523,9 +523,10 @@ __device__ __forceinline__ float hide_past(float v, int last, int k_r) {
     return __builtin_fminf(v, __builtin_bit_cast(float, (t & 0x80000000u) | 0x7f800000u));
 }
 // The same for a lane's many keys of a masked block (the general kernels): bit j of hidden_past(last) says that key j of a run of 32 lies past the
-// lane's last visible one (`last` may lie before the run or past it), and hide(v, bits, j) is v or -inf by that bit, the bit spread over a
-// word and a bitwise select: three instructions where the minimum above takes seven with what the compiler puts around it.  us, causal,
-// before -> after: half-int8 d128 B8 H32 N2048 301 -> 296, B4 H12 N1500 38.3 -> 37.4, fp16 B8 H32 N1024 93.8 -> 92.2, full-int8 B8 H32/8 N1024 74.5 -> 73.5.
+// lane's last visible one (`last` may lie before the run or past it), and hide(v, bits, j) is the smaller of v and an infinity with that bit for
+// its sign: three instructions where the minimum above takes seven with what the compiler puts around it.  A visible score that is not a number
+// becomes +infinity, as there: its row's maximum shows it, also where the row has no other key.  us, causal, minimum -> this: half-int8 d128 B8 H32 N2048
+// 286 -> 278, N512 32.2 -> 31.1, full-int8 d128 B4 H32 N4096 432 -> 424, N1024 blocked V scales 39.9 -> 39.6 (with the fold, where it runs).
 __device__ __forceinline__ uint32_t hidden_past(int last) {
     const int n = last + 1;
     return (uint32_t)(0xffffffffull << (n < 0 ? 0 : n > 32 ? 32 : n));
@@ -533,6 +534,15 @@ __device__ __forceinline__ uint32_t hidden_past(int last) {
 __device__ __forceinline__ float hide(float v, uint32_t bits, int j) {
     uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)bits, (unsigned)j, 1u);
     asm("" : "+v"(m));               // (opaque: else a compare and a select of it)
+    const uint32_t most = m << 31 | 0x7f800000u;
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(v), "v"(most));
+    return r;
+}
+// ... and the one that leaves a visible NaN what it is (head_dim 256).
+__device__ __forceinline__ float hide_number(float v, uint32_t bits, int j) {
+    uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)bits, (unsigned)j, 1u);
+    asm("" : "+v"(m));
     return __builtin_bit_cast(float, (m & 0xff800000u) | (~m & __builtin_bit_cast(uint32_t, v)));
 }
 

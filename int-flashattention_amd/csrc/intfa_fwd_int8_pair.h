@@ -208,7 +208,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
             if ((CAUSAL || LAST || MAYBE_LAST) && 32 * hf + 31 > lim_lo) {   // wave-uniform: some lane of the wave has a hidden key here
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) {
-                    if (RESIDENT) xq[b4] = hide(xq[b4], hidden, 8 * a4 + b4);
+                    if (RESIDENT) xq[b4] = hide_number(xq[b4], hidden, 8 * a4 + b4);
                     else if (32 * hf + 8 * a4 + b4 + 4 * lh > lim) xq[b4] = -INFINITY;
                 }
             }

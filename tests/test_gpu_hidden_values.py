@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import int_flashattention_amd as M
+from many_heads import repetitions
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -142,3 +143,30 @@ def test_hidden_keys_of_a_row_without_scores(variant, D, reps, Nq, Nk, splits, c
         for r in rows:
             n = r + 1 + Nk - Nq if causal else Nk
             assert (out[0, :, r].float() - v[0, :, :n].float().mean(1)).abs().max().item() <= tol, (r, n)
+
+
+# A score that is not a number, of a key that rows do see: they are NaN, also the row that sees no other key (the first one) and rows of a cache
+# with one ragged block in which every key is like that.  The first key of every head; grids past the decode-shaped kernels
+@pytest.mark.parametrize("variant,D,v_block", [("full", 64, None), ("full", 64, 64), ("full", 128, None), ("full", 128, 128), ("full", 128, 64), ("half", 128, None),
+                                               ("fp", 128, None)])
+@pytest.mark.parametrize("scale_dtype", [torch.float16, torch.float32])
+def test_visible_scores_that_are_not_numbers(variant, D, v_block, scale_dtype):
+    for Nq, Nk, causal in ((200, 200, True), (600, 600, True), (200, 45, False)):
+        H = repetitions(1, 1, Nq)
+        q, k, v = (torch.randn((1, H, n, D), generator=torch.Generator(device=DEV).manual_seed(n + i), device=DEV).half() for i, n in enumerate((Nq, Nk, Nk)))
+        bad = slice(0, 1) if causal else slice(None)
+        if variant == "fp":
+            k[:, :, bad, 3] = NAN
+            out, lse = M.attention(q, k, v, causal, 0.1, return_lse=True)
+        else:
+            (q8, qs), (k8, ks) = M.quant_pertoken(q), M.quant_pertoken(k)
+            ks[:, :, bad] = NAN
+            qs, ks = qs.to(scale_dtype), ks.to(scale_dtype)
+            if variant == "half":
+                out, lse = M.attention_int8(q8, k8, v, qs, ks, causal, 0.1, return_lse=True)
+            else:
+                v8, vs = M.quant_perblock_channel(v, v_block) if v_block else M.quant_pertensor(v)
+                vs = vs if v_block else vs.to(scale_dtype)
+                out, lse = M.attention_full_int8(q8, k8, v8, qs, ks, vs, causal, 0.1, return_lse=True, v_scale_block=v_block)
+        torch.cuda.synchronize()
+        assert bool(lse.isnan().all()) and bool(out.isnan().all()), (Nq, Nk, causal, int((~lse.isnan()).sum()))

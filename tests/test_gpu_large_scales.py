@@ -18,8 +18,8 @@ def same(a, b):
 
 
 # (16-bit scales of the general kernels; D 256: past 256 query blocks of 128 rows, several per workgroup)
-KERNELS = [("full", 64, 300, 333, False, None, 1), ("full", 64, 300, 300, True, None, 1), ("full", 64, 130, 700, True, None, 2), ("full", 64, 130, 128, False, 64, 1),
-           ("full", 64, 300, 300, True, 128, 1), ("full", 128, 300, 333, False, None, 1), ("full", 128, 300, 300, True, None, 1), ("full", 128, 90, 256, False, None, 1),
+KERNELS = [("full", 64, 300, 333, False, None, 1), ("full", 64, 300, 300, True, None, 1), ("full", 64, 130, 700, True, None, 2), ("full", 64, 130, 129, False, 64, 1),
+           ("full", 64, 300, 300, True, 128, 1), ("full", 128, 300, 333, False, None, 1), ("full", 128, 300, 300, True, None, 1), ("full", 128, 90, 257, False, None, 1),
            ("full", 128, 300, 700, True, None, 2), ("full", 128, 300, 300, True, 128, 1), ("full", 256, 130, 200, False, None, 1),
            ("full", 256, 200, 200, True, None, 1), ("half", 128, 200, 333, False, None, 1), ("half", 128, 257, 257, True, None, 1), ("half", 64, 300, 300, False, None, 1)]
 

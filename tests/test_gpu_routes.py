@@ -27,6 +27,28 @@ CASES = [
     ("full", 128, 1, N, True, dict(v_block=64), "fwd_full_int8_kernel<128, true"),
     ("full", 128, 1, N, False, dict(num_splits=2), "fwd_full_int8_kernel<128, false"),
     ("full", 128, 1, 64, False, {}, "fwd_decode_full_int8_kernel<128"),
+    # the folded dequantisation (last argument), on both sides of each line: more than two key blocks, blocks per split, 16-bit scales; head_dim 64:
+    # 768 workgroups, 2048 keys, causal 640 keys and 1536 workgroups; V scales per 128 keys
+    ("full", 128, PAST, 257, False, {}, "fwd_full_int8_kernel<128, false, 0, 1, false, false, 0, true>"),
+    ("full", 128, PAST, 256, False, {}, "fwd_full_int8_kernel<128, false, 0, 1, false, false, 0, false>"),
+    ("full", 128, PAST, 257, False, dict(scales=torch.float32), "fwd_full_int8_kernel<128, false, 0, 1, false, false, 0, false>"),
+    ("full", 128, 20, 513, True, dict(num_splits=2), "fwd_full_int8_kernel<128, true, 0, 1, false, true, 0, true>"),
+    ("full", 128, 20, 512, True, dict(num_splits=2), "fwd_full_int8_kernel<128, true, 0, 1, false, true, 0, false>"),
+    ("full", 128, PAST, 600, False, dict(v_block=128), "fwd_full_int8_kernel<128, false, 0, 1, false, false, 1, false>"),
+    ("full", 128, PAST, 600, False, dict(v_block=64), "fwd_full_int8_kernel<128, false, 0, 1, false, false, 2, false>"),
+    ("full", 64, 256, 129, False, {}, "fwd_full_int8_kernel<64, false, 0, 1, false, false, 0, true>"),
+    ("full", 64, 256, 128, False, {}, "fwd_full_int8_kernel<64, false, 0, 1, false, false, 0, false>"),
+    ("full", 64, 256, 384, True, {}, "fwd_full_int8_kernel<64, true, 0, 1, false, false, 0, true>"),
+    ("full", 64, 257, 384, True, {}, "fwd_full_int8_kernel<64, true, 0, 1, false, false, 0, false>"),
+    ("full", 64, 49, 2047, False, {}, "fwd_full_int8_kernel<64, false, 0, 1, false, false, 0, false>"),
+    ("full", 64, 49, 2048, False, {}, "fwd_full_int8_kernel<64, false, 0, 1, false, false, 0, true>"),
+    ("full", 64, 155, 639, True, {}, "fwd_full_int8_kernel<64, true, 0, 1, false, false, 0, false>"),
+    ("full", 64, 155, 640, True, {}, "fwd_full_int8_kernel<64, true, 0, 1, false, false, 0, true>"),
+    ("full", 64, 255, 700, True, {}, "fwd_full_int8_kernel<64, true, 0, 1, false, false, 0, true>"),
+    ("full", 64, 256, 700, True, {}, "fwd_full_int8_kernel<64, true, 0, 1, false, false, 0, false>"),
+    ("full", 64, 300, 384, True, dict(v_block=128), "fwd_full_int8_kernel<64, true, 0, 1, false, false, 1, true>"),
+    ("full", 64, 300, 128, True, dict(v_block=128), "fwd_full_int8_kernel<64, true, 0, 1, false, false, 1, false>"),
+    ("full", 64, 300, 384, True, dict(v_block=128, scales=torch.float32), "fwd_full_int8_kernel<64, true, 0, 1, false, false, 1, false>"),
     ("half", 64, PAST - 1, N, False, {}, "fwd_decode_f16pv_kernel<true, 64"),
     ("half", 64, PAST, N, False, {}, "fwd_f16pv_pipe_kernel<true, 64"),
     ("half", 64, PAST, N, True, {}, "fwd_f16pv_kernel<true, 64"),                       # fewer than eight key blocks
@@ -42,16 +64,18 @@ def test_kernels_of_calls():
     calls = []
     for variant, D, H, Nq, causal, kw, _ in CASES:
         kw = dict(kw)
-        v_block = kw.pop("v_block", None)
+        v_block, scales = kw.pop("v_block", None), kw.pop("scales", torch.float16)
         q, k, v = (torch.randn((1, H, Nq, D), device=DEV).half() for _ in range(3))
         if variant == "fp":
             calls.append(lambda a=(q, k, v, causal, 0.1), kw=kw: M.attention(*a, **kw))
             continue
         (q8, qs), (k8, ks) = M.quant_pertoken(q), M.quant_pertoken(k)
+        qs, ks = qs.to(scales), ks.to(scales)
         if variant == "half":
             calls.append(lambda a=(q8, k8, v, qs, ks, causal, 0.1), kw=kw: M.attention_int8(*a, **kw))
             continue
         v8, vs = M.quant_perblock_channel(v, v_block) if v_block else M.quant_pertensor(v)
+        vs = vs if v_block else vs.to(scales)
         kw["v_scale_block"] = v_block
         calls.append(lambda a=(q8, k8, v8, qs, ks, vs, causal, 0.1), kw=kw: M.attention_full_int8(*a, **kw))
     torch.cuda.synchronize()

@@ -91,7 +91,7 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
 
     def compile_one(pair):
         # -save-temps=obj leaves the device assembly beside the object: it is scanned for register spills that lose lanes
-        # (spill_check.py) and for early readers of matrix products (mfma_check.py), and removed again with the other intermediate files
+        # (spill_check.py) and for early readers of matrix products and of other lanes' registers (mfma_check.py), and removed again with the other intermediate files
         src, obj = pair
         cmd = ["hipcc", *FLAGS, "-save-temps=obj", "-c", src, "-o", obj]
         r = subprocess.run(cmd, capture_output=True, text=True)
@@ -106,7 +106,7 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
             if f.endswith("gfx950.s"):
                 with open(path) as fh:
                     asm = fh.read()
-                findings = [f"{os.path.basename(src)}: {x}" for x in spill_check.scan(asm) + mfma_check.scan(asm) + mfma_check.scan_waits(asm)]
+                findings = [f"{os.path.basename(src)}: {x}" for x in spill_check.scan(asm) + mfma_check.scan(asm) + mfma_check.scan_lanes(asm) + mfma_check.scan_waits(asm)]
                 scanned = True
             os.remove(path)
         if not scanned:      # (a compiler that names its intermediate files otherwise must not pass unchecked)
@@ -117,7 +117,7 @@ def build(verbose: bool = True, jobs: int = 8, only=None) -> str:
         findings = [x for fs in ex.map(compile_one, todo) for x in fs]
     if findings:
         raise RuntimeError("the compiler placed register spills where lanes are masked off, or readers of a matrix product ahead of its wait states, "
-                           "or waits for the next tiles ahead of a step's products:\n  "
+                           "or of another lane's register, or waits for the next tiles ahead of a step's products:\n  "
                            + "\n  ".join(findings[:20]))
     r = subprocess.run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", OUT], capture_output=True, text=True)
     if r.returncode != 0:

@@ -342,7 +342,8 @@ __device__ __forceinline__ float lane_scale(float s, int i) {
         case 12: return lane_scale_of<12>(s); case 13: return lane_scale_of<13>(s); case 14: return lane_scale_of<14>(s); default: return lane_scale_of<15>(s);
     }
 }
-// c += f * (the scale of the lane's i-th key).  (Reads f like any hand-written instruction: mfma_check.py.)
+// c += f * (the scale of the lane's i-th key).  (Hand-written: the wait states ahead of it, of the product in f and of a vector instruction that writes `scales`,
+// are not the compiler's; mfma_check.py looks for them.)
 __device__ __forceinline__ void fmac_lane_scale(float& c, float scales, int f, int i) {
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(c) : "v"(scales), "v"(f), "i"(i));
 }

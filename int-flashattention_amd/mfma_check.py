@@ -79,6 +79,52 @@ def scan(asm: str) -> List[str]:
     return findings
 
 
+_DPP = re.compile(r"_dpp\b|\b(quad_perm|row_newbcast|row_shl|row_shr|row_ror|row_mirror|row_half_mirror|row_bcast|wave_)")
+
+
+def scan_lanes(asm: str) -> List[str]:
+    """Returns one line per instruction that takes another lane's register (DPP, its first source) less than two wait states after a vector instruction wrote
+    it, or less than five after one wrote the exec mask, along all ways through the kernel.  The hardware does not hold it back; the compiler
+    keeps the distance for its own instructions only, and the kernels' hand-written ones read registers that it may copy or fetch back from an
+    accumulation register just ahead."""
+    findings: List[str] = []
+    for kernel, blocks in spill_check.kernels(asm):
+        code = [[(n, t, *m.groups()) for n, t in b["lines"] for m in [_INSTRUCTION.match(t)] if m] for b in blocks]
+        if not any(_DPP.search(t) for c in code for _, t, _, _ in c):
+            continue
+        ways = spill_check.successors(blocks)
+        entry: List[Dict[object, Tuple[int, int]]] = [{} for _ in blocks]      # register, or "exec" -> (wait states still needed, line of the write)
+        found: Dict[int, str] = {}
+        work = list(range(len(blocks)))
+        while work:
+            k = work.pop(0)
+            pending = dict(entry[k])
+            for n, text, op, operands in code[k]:
+                args = re.split(r",\s*(?![^\[]*\])", operands.strip())
+                if pending and op.startswith("v_") and _DPP.search(text):
+                    early = [pending[r] for r in ["exec", *_registers(args[1].split()[0] if len(args) > 1 else "")] if r in pending]
+                    if early:
+                        need, line = max(early)
+                        found[n] = f"{kernel}: line {n}: `{op} {operands.strip()}` comes {need} wait states too early for the write of line {line}"
+                states = int(operands, 0) + 1 if op == "s_nop" else 1
+                pending = {r: (need - states, line) for r, (need, line) in pending.items() if need > states}
+                if op.startswith("v_"):
+                    for r in _registers(args[0]):
+                        pending[r] = (2, n)
+                    if op.startswith("v_cmpx"):
+                        pending["exec"] = (5, n)
+            for j in ways[k]:
+                grown = False
+                for r, p in pending.items():
+                    if p[0] > entry[j].get(r, (0, 0))[0]:
+                        entry[j][r] = p
+                        grown = True
+                if grown and j not in work:
+                    work.append(j)
+        findings += [found[n] for n in sorted(found)]
+    return findings
+
+
 _LOAD_WAIT = re.compile(r"^\s+s_waitcnt\b.*\bvmcnt\(")
 
 

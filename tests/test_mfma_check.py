@@ -1,4 +1,4 @@
-"""The build-time scan for early readers of matrix products (int_flashattention_amd/mfma_check.py) on hand-made assembly: a product of four
+"""The build-time scans for early readers of matrix products and of other lanes' registers (int_flashattention_amd/mfma_check.py) on hand-made assembly: a product of four
 passes (16 x 16) needs eight wait states, one of eight passes (32 x 32) twelve, on every way to an instruction that touches its registers."""
 import os
 import sys
@@ -73,3 +73,37 @@ def test_a_wait_for_loads_ahead_of_a_product_in_a_loop_is_reported():
     assert mfma_check.scan_waits(HEAD + "\ts_waitcnt vmcnt(0)\n" + LARGE + "\ts_endpgm\n") == []      # not in a loop
     spilled = "\tscratch_load_dwordx4 v[12:15], off, off offset:16 ; 16-byte Folded Reload\n\ts_waitcnt vmcnt(0)\n"
     assert mfma_check.scan_waits(head.format("") + copy + spilled + end) == []
+
+
+LANES = "\tv_fmac_f32_dpp v7, v1, v9 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+
+
+@pytest.mark.parametrize("writer,states", [("v_mov_b32_e32 v1, v50", 2), ("v_accvgpr_read_b32 v1, a3", 2), ("v_cmpx_gt_f32_e32 v2, v3", 5)])
+def test_another_lanes_register_is_not_read_too_early(writer, states):
+    for have in range(states + 1):
+        nops = f"\ts_nop {have - 1}\n" if have else ""
+        found = mfma_check.scan_lanes(HEAD + f"\t{writer}\n" + nops + LANES + "\ts_endpgm\n")
+        assert len(found) == (have < states), (have, found)
+        assert all(f"{states - have} wait states too early" in f and "_ZN5intfa4kernEv" in f for f in found)
+
+
+def test_only_the_lanes_source_waits():
+    # loads from the LDS are waited for; the other source and the addend are the lane's own; instructions without DPP read what they like
+    for writer in ("ds_read_b32 v1, v2", "v_mov_b32_e32 v9, 0", "v_mov_b32_e32 v7, 0", "v_cmp_gt_f32_e32 vcc, v1, v3", "s_mov_b32 s1, s2"):
+        assert mfma_check.scan_lanes(HEAD + f"\t{writer}\n" + LANES + "\ts_endpgm\n") == []
+    assert mfma_check.scan_lanes(HEAD + "\tv_mov_b32_e32 v1, v50\n\tv_add_f32_e32 v3, v1, v1\n" + "\ts_nop 0\n" + LANES + "\ts_endpgm\n") == []
+    # (operands of several registers, and the modifier in the place of the suffix)
+    wide = HEAD + "\tv_lshlrev_b64 v[0:1], 1, v[4:5]\n\tv_mov_b32 v7, v1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\ts_endpgm\n"
+    assert len(mfma_check.scan_lanes(wide)) == 1
+
+
+def test_another_lanes_register_on_every_way():
+    asm = HEAD + "\tv_mov_b32_e32 v1, v50\n{}" + SKIP + "{}" + LANES + "\ts_endpgm\n"
+    # (the branch is a wait state)
+    assert len(mfma_check.scan_lanes(asm.format("", ""))) == 1
+    assert mfma_check.scan_lanes(asm.format("\ts_nop 0\n", "")) == []
+    assert mfma_check.scan_lanes(asm.format("", "\ts_nop 0\n")) == []
+    # over the back edge of a loop
+    loop = HEAD + ".LBB0_1:\n" + LANES + 4 * "\ts_mov_b32 s9, s8\n" + "\tv_mov_b32_e32 v1, v50\n{}\ts_cbranch_scc1 .LBB0_1\n; %bb.2:\n\ts_endpgm\n"
+    assert len(mfma_check.scan_lanes(loop.format(""))) == 1
+    assert mfma_check.scan_lanes(loop.format("\ts_nop 0\n")) == []

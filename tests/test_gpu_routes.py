@@ -20,8 +20,16 @@ CASES = [
     ("full", 128, PAST, N, True, {}, "fwd_full_int8_kernel<128, true"),
     ("full", 128, PAST - 1, N, True, {}, "fwd_decode_full_int8_kernel<128"),
     ("full", 256, PAST, N, False, {}, "fwd_full_int8_pair_kernel<false"),
-    ("full", 256, 129, N, False, {}, "fwd_full_int8_pair_kernel<false, 0, 1, false, false, true"),       # 258 query blocks: several per workgroup
-    ("full", 256, 128, N, False, {}, "fwd_full_int8_pair_kernel<false, 0, 1, false, false, false"),
+    ("full", 256, 129, N, False, {}, "fwd_full_int8_pair_kernel<false, 0, 1, false, false, true>"),       # 258 query blocks: several per workgroup
+    ("full", 256, 128, N, False, {}, "fwd_full_int8_pair_kernel<false, 0, 1, false, false, false>"),
+    ("full", 256, 129, N, False, dict(scales=torch.float32), "fwd_full_int8_pair_kernel<false, 0, 1, false, false, true>"),
+    # ... causal: two rounds of 256, whole rounds of K/V heads per XCD, lists that agree; one length for all entries, no more rows than keys
+    ("full", 256, 256, N, True, {}, "fwd_full_int8_pair_kernel<true, 0, 1, false, false, true>"),
+    ("full", 256, 248, N, True, {}, "fwd_full_int8_pair_kernel<true, 0, 1, false, false, false>"),
+    ("full", 256, 257, N, True, {}, "fwd_full_int8_pair_kernel<true, 0, 1, false, false, false>"),
+    ("full", 256, 12, 6000, True, {}, "fwd_full_int8_pair_kernel<true, 0, 1, false, false, false>"),
+    ("full", 256, 129, N, False, dict(seqlens=True), "fwd_full_int8_pair_kernel<false, 0, 1, false, false, false>"),
+    ("full", 256, 256, N, True, dict(keys=N - 1), "fwd_full_int8_pair_kernel<true, 0, 1, false, false, false>"),
     ("full", 256, PAST // 2, N, False, {}, "fwd_decode_full_int8_kernel<256"),
     ("full", 128, PAST, N, True, dict(v_block=128), "fwd_full_int8_kernel<128, true"),
     ("full", 128, 1, N, True, dict(v_block=64), "fwd_full_int8_kernel<128, true"),
@@ -64,8 +72,10 @@ def test_kernels_of_calls():
     calls = []
     for variant, D, H, Nq, causal, kw, _ in CASES:
         kw = dict(kw)
-        v_block, scales = kw.pop("v_block", None), kw.pop("scales", torch.float16)
-        q, k, v = (torch.randn((1, H, Nq, D), device=DEV).half() for _ in range(3))
+        v_block, scales, Nk = kw.pop("v_block", None), kw.pop("scales", torch.float16), kw.pop("keys", Nq)
+        if kw.pop("seqlens", False):
+            kw["seqlens_k"] = torch.tensor([Nk], dtype=torch.int32, device=DEV)
+        q, k, v = (torch.randn((1, H, n, D), device=DEV).half() for n in (Nq, Nk, Nk))
         if variant == "fp":
             calls.append(lambda a=(q, k, v, causal, 0.1), kw=kw: M.attention(*a, **kw))
             continue

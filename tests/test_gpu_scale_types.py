@@ -1,5 +1,6 @@
-"""16-bit and 32-bit scales of the same values: the general full-int8 kernels fold the dequantisation of the former into one instruction per
-score (kScoreSeed in csrc/intfa_device.h) and convert with the latter.  Same bits, up to the largest sums there are."""
+"""16-bit and 32-bit scales of the same values: the general full-int8 kernels up to head_dim 128 fold the dequantisation of the former into one instruction
+per score (kScoreSeed in csrc/intfa_device.h; which calls: test_gpu_routes.py) and convert with the latter; the other kernels convert both.  Same bits,
+up to the largest sums there are."""
 import pytest
 import torch
 
@@ -14,7 +15,8 @@ DEV = "cuda"
                                             (128, True, 90, 1000), (256, False, 130, 200), (256, True, 200, 200)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_same_bits(D, causal, Nq, Nk, dtype):
-    H = repetitions(1, 1, Nq) + 1
+    # (head_dim 256: more than 256 query blocks of 128 rows, several per workgroup, for which causal lists take whole rounds of K/V heads)
+    H = repetitions(1, 1, Nq) + 1 if D < 256 else -(-(repetitions(1, 1, Nq, rows=128) + 1) // 8) * 8
     g = torch.Generator(device=DEV).manual_seed(D + Nk)
     q8, k8, v8 = (torch.randint(-128, 128, (1, H, n, D), generator=g, device=DEV, dtype=torch.int32).to(torch.int8) for n in (Nq, Nk, Nk))
     # the largest sums of either sign: -128 * -128 and -128 * 127 throughout
@@ -35,7 +37,7 @@ def test_same_bits(D, causal, Nq, Nk, dtype):
 @pytest.mark.parametrize("causal,Nq,Nk", [(False, 130, 64), (False, 200, 333), (True, 129, 129), (True, 257, 700)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_same_bits_16bit_v(causal, Nq, Nk, dtype):
-    """The pipelined half-int8 kernel, in more workgroups than two per compute unit."""
+    """The pipelined half-int8 kernel."""
     H = repetitions(1, 1, Nq, rows=128) + 1
     g = torch.Generator(device=DEV).manual_seed(Nk)
     q8, k8 = (torch.randint(-128, 128, (1, H, n, 128), generator=g, device=DEV, dtype=torch.int32).to(torch.int8) for n in (Nq, Nk))

@@ -332,10 +332,10 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
     // ---- Work items of this workgroup.  One while all of the launch's workgroups are resident; with more items (RESIDENT) one workgroup per compute
     // unit takes every grid-th, in the order in which the hardware would deal them (causal: every second round backwards, so that the sums of
     // the lengths agree).  What it is for: a workgroup fills its compute unit, and nothing ran under its first loads and its last stores (20 % of the time
-    // at 1024 keys).  So an item's last block requests the next one's first tiles, the block before it Q (into the LDS), and nothing waits for the
-    // stores.  us, one item per workgroup -> this: B16 H16 N1024 bf16 268 -> 244, causal 172 -> 161, B4 H32 N4096 1679 -> 1590, B16 H32/4 N200
-    // 49.9 -> 46.4; what bounds it then is the loop over the key blocks.
-    // Launches of one round lose 5 % in the longer code: they run the other form.
+    // at 1024 keys).  So an item's last block requests the next one's first tiles and the block before it Q (into the LDS), and the stores have until
+    // the next item's first wait for tiles, a part of a key block (waves 4-7: one more block; an item of one block: its end).  us, one item
+    // per workgroup -> this: B16 H16 N1024 bf16 255 -> 238, causal 169 -> 155, B4 H32 N2048 448 -> 422, B32 H32 N128 causal 43.7 -> 37.6; what
+    // bounds it then is the loop over the key blocks.  Launches of one round lose 5 % in the longer code: they run the other form.
     int buf = 0;                                 // LDS buffer of the item's first block, then of its last
     int round = 0;
     if (it.nb_begin < it.nb_end) {
@@ -437,7 +437,7 @@ __global__ void __launch_bounds__(kPairThreads, 1) fwd_full_int8_pair_kernel(con
         return;
     }
     {
-    // the next item's first tiles, k_scale and Q have arrived (ahead of the stores: nothing waits for those)
+    // the next item's first tiles, k_scale and Q have arrived (ahead of the stores)
     if (RESIDENT && has_next) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         asm volatile("" : "+v"(q_scale_bits));

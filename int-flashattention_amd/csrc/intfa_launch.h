@@ -109,6 +109,10 @@ inline bool lists_agree(const KParams& kp, int slots) {
 // The same work items for `slots` workgroups (a multiple of kXcds), which take every slots-th each, where there are more items than that.
 // Not for batches of different lengths (the items of a workgroup would differ in work; the hardware deals single ones as compute units
 // become free), for items that may have no key, or for query rows further apart than a copy's offsets reach.
+// (The lists are fixed: a compute unit is held until its list ends, and beside another stream's kernels a workgroup that starts late runs all of its items late.
+// Full-int8 head_dim 256 B16 H16 N1024, twenty launches beside as much other work on a second stream, ms, until both have ended, dealt singly -> lists:
+// 256 MiB copies 10.0 -> 6.9, fp16 decodes 10.9 -> 9.6, d128 prefills 10.3 -> 10.1, the same again 10.5 -> 10.1; small prefills that leave most units idle,
+// which now wait for a launch's end instead of an item's, 8.2 -> 9.8, the twenty launches themselves 6.6 -> 5.6.)
 inline bool takes_resident(const KParams& kp, int slots) {
     const int64_t items = (int64_t)kp.batch * kp.heads * ((kp.seqlen + kBlockM - 1) / kBlockM);
     return items > slots && kp.num_splits <= 1 && kp.seqlens_k == nullptr && kp.seqlen_k > 0 && !(kp.causal && kp.seqlen_k < kp.seqlen) &&

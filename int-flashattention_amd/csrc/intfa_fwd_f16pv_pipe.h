@@ -8,7 +8,7 @@
 // that load (1.86 -> 1.63 GHz, 1.90 -> 1.81), so the time falls by less than the clocks.  Causal half-int8 B8 H32 N2048 keeps 2.03 GHz and has neither
 // pipe full (matrix 35 %, 30 % of the waves' time in waits): its workgroups are 17 key blocks long on average and fill and drain the
 // pipeline each for itself, 2120 clocks per wave and block where the non-causal launch takes 1670.
-// (Half-int8 with scales as lanes of a register and folded, below: 1.59 M clocks, 50 % busy; causal 1990 clocks per wave and block, non-causal 1550.)
+// (Half-int8 with scales as lanes of a register, below: 1.65 M clocks, 48 % busy; causal 2044 clocks per wave and block, non-causal 1616.)
 // B4 H32 d128, us, before -> with the pipeline: N4096 fp16 1106 -> 1038, causal 608 -> 563, half-int8 969 -> 929; N512 fp16 causal
 // 27.6 -> 21.0, half-int8 30.3 -> 21.0, causal 30.1 -> 18.5.
 // (Two row blocks per wave at one wave per SIMD halve the LDS reads per MFMA: fp16 N4096 another 6 %, but half-int8, whose dequantisation

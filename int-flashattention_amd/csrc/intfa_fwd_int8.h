@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
     // visible key; last block of a ragged sequence: lim = the last valid key.  Straight code per instance, and one of it for both
     // buffers: with run-time tests around sub-tiles and keys a masked block took 1.6 plain ones and more (us, before -> now: d128 B16
     // H16 N300 25.6 -> 22.2, causal N512 28.8 -> 27.5, B8 H32/8 N1024 74.1 -> 72.2, d64 causal B16 H16 N512 20.0 -> 18.9).
-    auto compute = [&](auto fold_tag, auto diag_tag, auto nact_tag, int buf, int nb, bool more, int lim) __attribute__((always_inline)) {
+    auto compute = [&](auto fold_tag, auto diag_tag, auto nact_tag, int buf, int nb, bool more, int lim, int number_tiles) __attribute__((always_inline)) {
         constexpr bool F = decltype(fold_tag)::value, DIAG = decltype(diag_tag)::value;
         constexpr int nact = decltype(nact_tag)::value;
         const uint32_t KB = buf * KT, VB = buf * VT, SB = buf * BN * 4;
@@ -333,7 +333,11 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
                 if (next) load_kk(a4, st + 1);
                 if (DIAG && (st + 2 >= nact || VBLK == 2 || FOLD != F)) {
 #pragma unroll
-                    for (int b4 = 0; b4 < 4; ++b4) xq[b4] = hide(xq[b4], hidden, 8 * a4 + b4);
+                    for (int b4 = 0; b4 < 4; ++b4) {
+                        const float x = xq[b4];
+                        xq[b4] = hide(x, hidden, 8 * a4 + b4);
+                        if (FOLD != F && st < number_tiles) xq[b4] = hide_number(x, hidden, 8 * a4 + b4);
+                    }
                 }
 #pragma unroll
                 for (int b4 = 0; b4 < 4; ++b4) {
@@ -494,8 +498,9 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
 
     // One pipeline step on LDS buffer BUF: wait for this block's tiles (issued one step earlier), make them
     // visible to all four waves, start the copy of the next block into the other buffer, compute.
-    // (gw: sub-tile of the largest lim of the wave's rows, negative: none)
-    auto step = [&](auto fold_tag, auto diag_tag, int buf, int nb, int gw, int lim) __attribute__((always_inline)) {
+    // (gw: sub-tile of the largest lim of the wave's rows, negative: none.  number_tiles, on the way out of the fold: the sub-tiles that the other
+    // instances do not mask, in which a score that is not a number stays what it is)
+    auto step = [&](auto fold_tag, auto diag_tag, int buf, int nb, int gw, int lim, int number_tiles) __attribute__((always_inline)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         const bool more = nb + 1 < nb_end;
@@ -511,14 +516,14 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             }
         }
         if constexpr (!DIAG) {
-            compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+            compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim, 0);
         } else if constexpr (VBLK == 2 || FOLD != decltype(fold_tag)::value) {      // (multiplies every sub-tile, so it masks every one: P8 of a hidden one is 0)
-            if (gw >= 0) compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim);
+            if (gw >= 0) compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim, number_tiles);
         } else {
-            if (gw >= NST - 1) compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim);
-            else if (gw == 0) compute(fold_tag, diag_tag, IntTag<1>{}, buf, nb, more, lim);
-            else if (NST == 4 && gw == 1) compute(fold_tag, diag_tag, IntTag<2>{}, buf, nb, more, lim);
-            else if (NST == 4 && gw == 2) compute(fold_tag, diag_tag, IntTag<3>{}, buf, nb, more, lim);
+            if (gw >= NST - 1) compute(fold_tag, diag_tag, IntTag<NST>{}, buf, nb, more, lim, 0);
+            else if (gw == 0) compute(fold_tag, diag_tag, IntTag<1>{}, buf, nb, more, lim, 0);
+            else if (NST == 4 && gw == 1) compute(fold_tag, diag_tag, IntTag<2>{}, buf, nb, more, lim, 0);
+            else if (NST == 4 && gw == 2) compute(fold_tag, diag_tag, IntTag<3>{}, buf, nb, more, lim, 0);
         }
         if (more && ks_wave) put_ks(fold_tag, ks_next, buf ^ 1, false);
         if (more && vs_thread) {
@@ -556,9 +561,9 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
         int nb = nb_begin;
         while (FOLD == decltype(fold_tag)::value) {
             if (nb >= plain_end) break;
-            step(fold_tag, BoolTag<false>{}, 0, nb++, 0, 0);
+            step(fold_tag, BoolTag<false>{}, 0, nb++, 0, 0, 0);
             if (nb >= plain_end) break;
-            step(fold_tag, BoolTag<false>{}, 1, nb++, 0, 0);
+            step(fold_tag, BoolTag<false>{}, 1, nb++, 0, 0, 0);
         }
         // masked blocks: the blocks the causal diagonal of this query block crosses (kBlockM / BN of them when the lengths
         // are equal, one more when the offset is not a multiple of the block; keys past the end of a ragged sequence lie above
@@ -568,7 +573,7 @@ __global__ void __launch_bounds__(kThreads, FullInt8Geom<D>::waves_per_simd(CAUS
             // lane: last visible key relative to the block; wave: sub-tile of the largest of them (negative: none)
             const int lim = (CAUSAL ? q_row + causal_off : seqlen_k - 1) - nb * BN;
             const int gw = ((CAUSAL ? mb * kBlockM + wave * 32 + 31 + causal_off : seqlen_k - 1) - nb * BN) >> 5;
-            step(fold_tag, BoolTag<true>{}, (nb - nb_begin) & 1, nb, gw, lim);
+            step(fold_tag, BoolTag<true>{}, (nb - nb_begin) & 1, nb, gw, lim, nb < plain_end ? NST : (gw < NST ? gw : NST - 1) - 1);
         }
     };
     if (nb_begin < nb_end) {

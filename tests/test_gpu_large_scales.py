@@ -19,14 +19,15 @@ def same(a, b):
 
 # (16-bit scales of the general kernels; D 256: past 256 query blocks of 128 rows, several per workgroup)
 KERNELS = [("full", 64, 300, 333, False, None, 1), ("full", 64, 300, 300, True, None, 1), ("full", 64, 130, 700, True, None, 2), ("full", 64, 130, 129, False, 64, 1),
-           ("full", 64, 300, 300, True, 128, 1), ("full", 128, 300, 333, False, None, 1), ("full", 128, 300, 300, True, None, 1), ("full", 128, 90, 257, False, None, 1),
+           ("full", 64, 300, 300, True, 128, 1), ("full", 64, 130, 192, False, None, 1), ("full", 128, 130, 384, False, None, 1), ("full", 128, 300, 333, False, None, 1), ("full", 128, 300, 300, True, None, 1), ("full", 128, 90, 257, False, None, 1),
            ("full", 128, 300, 700, True, None, 2), ("full", 128, 300, 300, True, 128, 1), ("full", 256, 130, 200, False, None, 1),
            ("full", 256, 200, 200, True, None, 1), ("half", 128, 200, 333, False, None, 1), ("half", 128, 257, 257, True, None, 1), ("half", 64, 300, 300, False, None, 1)]
 
 
 @pytest.mark.parametrize("variant,D,Nq,Nk,causal,v_block,splits", KERNELS)
 @pytest.mark.parametrize("kind,dtype", [("one", torch.bfloat16), ("some", torch.bfloat16), ("all", torch.bfloat16), ("infinite", torch.bfloat16),
-                                        ("infinite", torch.float16), ("infinite_hidden_sign", torch.bfloat16), ("infinite_hidden_sign", torch.float16)])
+                                        ("infinite", torch.float16), ("infinite_hidden_sign", torch.bfloat16), ("infinite_hidden_sign", torch.float16),
+                                        ("infinite_zeros", torch.bfloat16), ("infinite_zeros", torch.float16)])
 def test_large_scales(variant, D, Nq, Nk, causal, v_block, splits, kind, dtype):
     H = -(-(repetitions(1, 1, Nq, rows=128) + 1) // 8) * 8
     g = torch.Generator(device=DEV).manual_seed(D + Nk)
@@ -44,6 +45,10 @@ def test_large_scales(variant, D, Nq, Nk, causal, v_block, splits, kind, dtype):
         qs.mul_(1e-40 if D == 64 else 1e-39)
     elif kind == "infinite":
         ks[:, :, 3::50] = INF
+    elif kind == "infinite_zeros":           # no score is a number: of any key, of the first ones
+        k8[:, ::2] = 0
+        k8[:, 1::2, :2 * Nk // 3] = 0
+        ks[:] = INF
     else:                                    # sums of one sign: the scores are -infinity, the keys weigh nothing
         q8.abs_().clamp_(min=1)
         k8[:, :, 3::50] = -1
